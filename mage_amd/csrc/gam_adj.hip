@@ -56,8 +56,9 @@ static inline dim3 agrid(const Box &b)
 
 // Point kernels whose stencils run along j and k: the box's rows (the
 // points of one (j, k) along i) in slabs of RBA j-rows, j fastest within a
-// slab, then k, then the next slab, cut into 256-point chunks numbered as
-// in POINT_IN (one contiguous run per XCD).  The rows at j +- 4 and at
+// slab, then k, then the next slab, cut into 256-point chunks of which
+// each XCD takes runs of 16 (as the step's launches do, see XCD_RUN in
+// gam_step.hip).  The rows at j +- 4 and at
 // k +- 4 of a point are then at most 4 RBA rows away in the order the
 // workgroups run, so the 8-point stencils of neighbouring workgroups meet
 // in L2; with the plane-by-plane order of POINT_IN the k neighbours lie a
@@ -67,7 +68,7 @@ static inline dim3 agrid_slab(const Box &b)
 {
     const long pts = (long)(b.i1 - b.i0 + 1) * (b.j1 - b.j0 + 1) * (b.k1 - b.k0 + 1);
     const long nc = (pts + ABT - 1) / ABT;
-    return dim3((unsigned)(((nc + 7) / 8) * 8));
+    return dim3((unsigned)(((nc + 127) / 128) * 128));
 }
 
 __device__ __forceinline__ void slab_row(const Box &b, unsigned nj, unsigned R, int &j, int &k)
@@ -87,7 +88,7 @@ __device__ __forceinline__ void slab_row(const Box &b, unsigned nj, unsigned R, 
 
 #define POINT_SLAB(b)                                                                            \
     const unsigned ni_ = (unsigned)((b).i1 - (b).i0 + 1), nj_ = (unsigned)((b).j1 - (b).j0 + 1); \
-    const unsigned L_ = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);                \
+    const unsigned L_ = (blockIdx.x & ~127u) + ((blockIdx.x & 7u) << 4) + ((blockIdx.x >> 3) & 15u); \
     const unsigned p_ = L_ * ABT + threadIdx.x;                                                  \
     if (p_ >= ni_ * nj_ * (unsigned)((b).k1 - (b).k0 + 1)) return;                               \
     const unsigned R_ = p_ / ni_;                                                                \
