@@ -226,9 +226,10 @@ int gam_get_solver(gam_ctx *ctx, int which, double *out);
  * launch shapes that give the same results: the chunk tiling of the box's
  * points, value = row order (1 = j fastest, 2 = k fastest, 3 = slabs of 8
  * j-rows) + 8 x chunk extent (0: 256 points per workgroup, 1: 512,
- * 2: 128), and, for the j and k fluxes, the LDS-staged face tile of
- * 64 x 4 (4) or 64 x 8 (5) faces, or those tiles with their rows brought
- * to LDS by direct global-to-LDS loads (6: 64 x 4, 7: 64 x 8).
+ * 2: 128), and, for the fluxes, the LDS-staged forms: 4 (tiles numbered
+ * along i first; i fluxes: rows j fastest) and 5 (along the flux direction
+ * first; rows k fastest).  For the j and k fluxes 6 and 7 are other names
+ * of 4 and 5.
  * gam_autotune times every candidate of every slot on the context's own
  * grid (reps steps per candidate, hipEvents around that slot's launch),
  * keeps the fastest (the current shape unless another is more than 1 %

@@ -102,6 +102,19 @@ __device__ __forceinline__ void stp(double *__restrict__ plane, unsigned off, do
 {
     *(double *)((char *)plane + off) = v;
 }
+// Plane n of a buffer, as a base the compiler keeps in scalar registers:
+// without the barrier it folds the plane offset into a 64-bit vector address
+// per load, one vector instruction each.
+__device__ __forceinline__ const double *pln(const double *base, long off)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    __attribute__((address_space(1))) const double *q = (__attribute__((address_space(1))) const double *)(base + off);
+    asm("" : "+s"(q));
+    return (const double *)q;
+#else
+    return base + off;
+#endif
+}
 // Point c + d*s of a plane whose stencil runs along axis AX (stride s):
 // along i (AX = 0) plain indexing, which the compiler turns into wide loads
 // of contiguous points; along j and k a 32-bit byte offset from the plane

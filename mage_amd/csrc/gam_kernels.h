@@ -54,16 +54,15 @@ void order_wait(hipStream_t s, hipEvent_t e, int ev);
 
 // Launch plan: the shape of every tunable launch of the step.  Values
 // 1, 2, 3 are the Tile row orders (ax1: j fastest, k fastest, j-slabs);
-// PLAN_LDS and PLAN_LDS8 select the LDS-staged form of the j/k interface
-// fluxes (a 64 x 4 or 64 x 8 face tile with its stencil halo rows in LDS);
-// PLAN_LDSDMA and PLAN_LDS8DMA the 64 x 4 and 64 x 8 tiles whose rows reach
-// LDS by global_load_lds.
+// PLAN_LDS and PLAN_LDS_D select the LDS-staged interface fluxes, tiles
+// numbered along i first or along the flux direction first (i fluxes: rows j
+// or k fastest).  PLAN_ALIAS added to either names the same launch: plans
+// saved when these were separate shapes stay valid.
 enum { TS_PREDICT = 0, TS_EMF_I, TS_EMF_J, TS_EMF_K, TS_FLUX_I, TS_FLUX_J, TS_FLUX_K, TS_UPDATE,
        TS_COUNT };
 #define PLAN_LDS 4
-#define PLAN_LDS8 5
-#define PLAN_LDSDMA 6
-#define PLAN_LDS8DMA 7
+#define PLAN_LDS_D 5
+#define PLAN_ALIAS 2
 struct Plan {
     int v[TS_COUNT];
 };
@@ -95,6 +94,13 @@ void launch_emf(hipStream_t s, int eD, int ax, const Geo &g, const MParm &m, con
 // vf's three planes of direction d
 void launch_flux(hipStream_t s, int d, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
                  const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
+// one face direction each, one source file each
+void launch_flux_i(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
+                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
+void launch_flux_j(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
+                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
+void launch_flux_k(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
+                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
 void launch_update(hipStream_t s, int ax, const Geo &g, const MParm &m, const Box &fb, const Box &ctb,
                    const Box *eboxes, const Box &ab, const Box &dtb, Clock *clk, const double *So,
                    double *Sn, const double *gf, const double *mf, const double *met, const double *bg);

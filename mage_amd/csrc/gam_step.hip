@@ -3,10 +3,10 @@
 // Kernel sequence of one stepGamera (gamapp.F90:73-113):
 //   k_predict    Predictor: AB2 face fluxes, half-step B and gas, plus the
 //                primitives used by the flux sweeps
-//   k_flux       Lyon gas/magnetic fluxes, one per direction, and the face
-//                velocities (Mom2Face) of the same faces
+//   k_flux_t     Lyon gas/magnetic fluxes, one per direction, and the face
+//                velocities (Mom2Face) of the same faces (gam_flux.h)
 //   k_vface_rim  face velocities the EMF stencils read past the flux faces
-//   k_emf        edge EMFs
+//   k_emf        edge EMFs (gam_emf.hip)
 //   k_update     CT face-flux update, cell B of the new state, flux
 //                divergence, Reynolds, Maxwell/Boris and the CFL
 //                min-reduction of the new state
@@ -17,230 +17,11 @@
 // State and oState are two buffers that swap roles every step, which
 // replaces CopyState (mhdgroup.F90:204-255): the update reads the current
 // buffer and writes every point of the other.
-#include "gam_phys.h"
-#include "gam_kernels.h"
-#include <type_traits>
+#include "gam_launch.h"
 
-#define BX 64
-#define BY 4
-
-__device__ __forceinline__ bool in_box(const Box &b, int i, int j, int k)
-{
-    return i >= b.i0 && i <= b.i1 && j >= b.j0 && j <= b.j1 && k >= b.k0 && k <= b.k1;
-}
-
-#define THREAD_IJK(b)                                   \
-    const int i = (b).i0 + blockIdx.x * BX + threadIdx.x; \
-    const int j = (b).j0 + blockIdx.y * BY + threadIdx.y; \
-    const int k = (b).k0 + blockIdx.z;                  \
-    if (i > (b).i1 || j > (b).j1) return;
-
-// XCD-aware tiling.  A launch covers box b row by row (a row = the points
-// of one (j, k) along i) and cuts the rows, i fastest, into chunks of 256
-// consecutive points, one per workgroup, so no lane idles however the row
-// length falls against 64.  Row order, by ax1:
-//   1: j fastest, then k;   2: k fastest, then j;
-//   3: slabs of RB j-rows: j fastest within the slab, then k, then the
-//      next slab -- the rows at j+1 and at k+1 are both at most RB rows
-//      away, for kernels that read neighbours along j and along k.
-// The hardware hands workgroup w to XCD w % 8; xcd_tile numbers the chunks
-// so that each XCD takes runs of 2^xs consecutive ones: neighbouring chunks,
-// which share stencil rows, meet in one L2, while the eight runs in flight
-// stay side by side in memory.  Runs of 16 (XCD_RUN): on the 256x256x384
-// shell the step takes 17.30 ms with runs of 4, 17.12 with 16 or 32, 17.19
-// with 128, 17.40 with 1024 and 17.55 with one run of nb / 8 per XCD (eight
-// far-apart streams, each a slower mix of DRAM pages); 96x96x128: 1.037,
-// 1.027, 1.068, 1.32 and 1.09.
-#define RB 8
-struct Tile {
-    Box b;
-    int ax1;
-    int ni, nj, nk;   // extents
-    int nb;           // chunks in all
-    int ch;           // points per chunk (= threads per workgroup)
-    int xs;           // log2 of an XCD's run of consecutive chunks
-};
-
-#define XCD_RUN 4     // log2 of the run length of a large launch
-__device__ __forceinline__ int xcd_tile(int w, int xs)
-{
-    return ((w >> (3 + xs)) << (3 + xs)) + ((w & 7) << xs) + ((w >> 3) & ((1 << xs) - 1));
-}
-// Run length (log2) of a launch of nb chunks, and its workgroup count: a
-// whole number of rounds of eight runs.
-static inline int xcd_shift(long nb)
-{
-    int xs = 0;
-    while (xs < XCD_RUN && (16L << xs) <= nb) xs++;
-    return xs;
-}
-static inline unsigned xcd_grid(long nb, int xs)
-{
-    const long r = 8L << xs;
-    return (unsigned)((nb + r - 1) / r * r);
-}
-
-__device__ __forceinline__ bool tile_point(const Tile &t, int w, int &i, int &j, int &k)
-{
-    const int L = xcd_tile(w, t.xs);
-    i = j = k = 0x40000000;
-    if (L >= t.nb) return false;
-    const unsigned p = (unsigned)L * (unsigned)t.ch + threadIdx.x + BX * threadIdx.y;
-    if (p >= (unsigned)t.ni * (unsigned)(t.nj * t.nk)) return false;
-    const unsigned R = p / (unsigned)t.ni;
-    i = t.b.i0 + (int)(p - R * (unsigned)t.ni);
-    int jj, kk;
-    if (t.ax1 == 1) {
-        kk = (int)(R / (unsigned)t.nj); jj = (int)(R - (unsigned)kk * t.nj);
-    } else if (t.ax1 == 2) {
-        jj = (int)(R / (unsigned)t.nk); kk = (int)(R - (unsigned)jj * t.nk);
-    } else {
-        const unsigned slab = (unsigned)RB * t.nk;
-        const unsigned nfull = (unsigned)(t.nj / RB);
-        const unsigned sb = R / slab;
-        if (sb < nfull) {
-            const unsigned r = R - sb * slab;
-            kk = (int)(r / RB);
-            jj = (int)(sb * RB + (r % RB));
-        } else {
-            const unsigned r = R - nfull * slab;
-            const unsigned rj = (unsigned)t.nj - nfull * RB;
-            kk = (int)(r / rj);
-            jj = (int)(nfull * RB + (r - (unsigned)kk * rj));
-        }
-    }
-    j = t.b.j0 + jj;
-    k = t.b.k0 + kk;
-    return true;
-}
-
-#define TILE_IJK(t)                  \
-    int i, j, k;                     \
-    if (!tile_point((t), (int)bi.x, i, j, k)) return;
-
-static inline Tile tile_of(const Box &b, int ax1, int ch = BX * BY)
-{
-    Tile t;
-    t.b = b;
-    t.ax1 = ax1;
-    t.ni = b.i1 - b.i0 + 1;
-    t.nj = b.j1 - b.j0 + 1;
-    t.nk = b.k1 - b.k0 + 1;
-    t.ch = ch;
-    const long pts = (long)t.ni * t.nj * t.nk;
-    t.nb = (int)((pts + ch - 1) / ch);
-    t.xs = xcd_shift(t.nb);
-    return t;
-}
-
-// A launch plan value of a chunk-tiled slot: the row order in its low 3
-// bits, the chunk size (threads per workgroup) above them.
-static inline int plan_ax(int v) { return v & 7; }
-static inline int plan_chunk(int v) { return (v >> 3) == 1 ? 512 : (v >> 3) == 2 ? 128 : BX * BY; }
-static inline dim3 tgrid(const Tile &t) { return dim3(xcd_grid(t.nb, t.xs)); }
-
-static inline dim3 grid_of(const Box &b)
-{
-    return dim3((unsigned)((b.i1 - b.i0 + BX) / BX), (unsigned)((b.j1 - b.j0 + BY) / BY),
-                (unsigned)(b.k1 - b.k0 + 1));
-}
-
-// ====================================================================
-// Launch forms.  Every kernel of the step is a functor whose body takes its
-// workgroup's block index bi.  k_one<F> runs F over its own grid (one
-// context); k_ens<F> runs F for many contexts in one launch: the
-// concatenated grid of the members, each member's workgroups starting at a
-// multiple of 8 (so a member's chunk-to-XCD mapping is the same as in its
-// own launch) and each with its own argument record.  A table after the
-// header names the member of every run of 8 workgroups.
-// ====================================================================
-// Threads per workgroup of functor F: F::NT where it declares one, else 256.
-template <class F, class = void> struct nthreads { static constexpr int v = BX * BY; };
-template <class F> struct nthreads<F, std::void_t<decltype(F::NT)>> { static constexpr int v = F::NT; };
-
-template <class F, class... A>
-__global__ __launch_bounds__(nthreads<F>::v) void k_one(A... a)
-{
-    F{}(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), a...);
-}
-
-// Pointers read from an argument record are generic pointers to the
-// compiler; every one of them addresses device (global) memory, and saying
-// so lets it use global instead of flat loads and stores.
-template <class T>
-__device__ __forceinline__ const T &in_global(const T &v)
-{
-    return v;
-}
-template <class T>
-__device__ __forceinline__ T *in_global(T *const &p)
-{
-    __attribute__((address_space(1))) T *q = (__attribute__((address_space(1))) T *)p;
-    asm("" : "+s"(q));   // keeps the cast from folding back to a generic pointer
-    return (T *)q;
-}
-
-// Call F with the record's fields, in order (passed by reference into the
-// record, so that arrays in them are read where they lie).
-template <class F, class... B>
-__device__ __forceinline__ void pcall(const Pack<> &, uint3 bi, const B &...b)
-{
-    F{}(bi, in_global(b)...);
-}
-template <class F, class A0, class... A, class... B>
-__device__ __forceinline__ void pcall(const Pack<A0, A...> &p, uint3 bi, const B &...b)
-{
-    pcall<F>(p.r, bi, b..., p.a0);
-}
-
-template <class F, class... A>
-__global__ __launch_bounds__(nthreads<F>::v) void k_ens(const EnsHdr *__restrict__ h,
-                                             const Pack<A...> *__restrict__ rec)
-{
-    const unsigned w = blockIdx.x;
-    // owner of each run of 8 workgroups, stored right after the header
-    const unsigned lo = reinterpret_cast<const unsigned short *>(h + 1)[w >> 3];
-    const unsigned gx = h->gx[lo], gy = h->gy[lo], gz = h->gz[lo];
-    unsigned l = w - h->wg0[lo];
-    if (l >= gx * gy * gz) return;   // padding of the member's range
-    uint3 bi;
-    bi.x = l % gx;
-    l /= gx;
-    bi.y = l % gy;
-    bi.z = l / gy;
-    pcall<F>(rec[lo], bi);
-}
-
-template <class F, class... A>
-static void launch_ens(hipStream_t s, const void *hdr, const void *rec, unsigned nwg, dim3 block)
-{
-    hipLaunchKernelGGL((k_ens<F, A...>), dim3(nwg), block, 0, s, (const EnsHdr *)hdr,
-                       (const Pack<A...> *)rec);
-}
-
-// Batchable launch: issued at once, or appended to this thread's recorder.
 static thread_local std::vector<EnsLaunch> *g_rec = nullptr;
 void set_launch_recorder(std::vector<EnsLaunch> *r) { g_rec = r; }
-
-template <class F, class... A>
-static void launch_f(dim3 grid, dim3 block, hipStream_t s, A... a)
-{
-    if (g_rec) {
-        const Pack<A...> p = make_pack(a...);
-        EnsLaunch e;
-        e.launch = &launch_ens<F, A...>;
-        e.grid = grid;
-        e.block = block;
-        e.rec.resize(sizeof(p));
-        memcpy(e.rec.data(), &p, sizeof(p));
-        e.stream = s;
-        e.mark = 0;
-        e.ev = -1;
-        g_rec->push_back(std::move(e));
-        return;
-    }
-    hipLaunchKernelGGL((k_one<F, A...>), grid, block, 0, s, a...);
-}
+std::vector<EnsLaunch> *launch_recorder() { return g_rec; }
 
 static void order_mark(hipStream_t s, int mark, int ev)
 {
@@ -392,440 +173,6 @@ struct k_vface_rim {
 #pragma unroll
             for (int n = 0; n < 8; n++) q8[n] = wv[x * N3 + c + (n - 4) * s];
             Vf[(3 * d + x) * N3 + c] = mom2face(q8, Vi, rVi);
-        }
-    }
-};
-
-// ====================================================================
-// Edge EMF: GetCornerV/GetCornerD/GetCornerB/EdgeLRs + VxB
-// (fields.F90:187-224, 288-517).  One thread per active edge of ED.
-// ====================================================================
-template <int FD, int SD, int RM>
-__device__ __forceinline__ void edge_lr(const Geo &g, const MParm &m, long c,
-                                        const double *__restrict__ met,
-                                        const double *__restrict__ mfH,
-                                        const double *__restrict__ mfL,
-                                        double &bL, double &bR, double &fA)
-{
-    // EdgeLRs (fields.F90:288-362) for FD faces stacked along SD, area weighted
-    const long N3 = g.N3;
-    const long s = STRIDE<SD>(g);
-    double A[8], q[8], nq[4];
-#pragma unroll
-    for (int n = 0; n < 8; n++) {
-        A[n] = ldx<SD>(met + (M_FACE + FD) * N3, c, s, n - 4);
-        q[n] = ldx<SD>(mfH + FD * N3, c, s, n - 4) / dmax(A[n], GAM_TINY);
-    }
-    // the limiter faces are the middle four of the stencil
-#pragma unroll
-    for (int n = 0; n < 4; n++) nq[n] = ldx<SD>(mfL + FD * N3, c, s, n - 2) / dmax(A[n + 2], GAM_TINY);
-    double Vi = wsum8([&](int n) { return A[n]; });
-    double l, r;
-    recon_lr<RM>(m.pdmb, A, 1.0 / Vi, nq, q, l, r);
-    fA = Vi;
-    bL = l * fA;
-    bR = r * fA;
-}
-
-template <int ED, int RM, bool BG, bool BORIS, int NTH = BX * BY>
-struct k_emf {
-    static constexpr int NT = NTH;
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m,
-                                               Tile b, const Clock *clk,
-                                               const double *__restrict__ H,
-                                               const double *__restrict__ S,
-                                               const double *__restrict__ Vf,
-                                               const double *__restrict__ met,
-                                               const double *__restrict__ bg,
-                                               double *__restrict__ E) const
-    {
-        TILE_IJK(b);
-        constexpr int T1 = (ED == 0) ? 1 : (ED == 1) ? 2 : 0;
-        constexpr int T2 = (ED == 0) ? 2 : (ED == 1) ? 0 : 1;
-        // getNormalPlane (metric.F90:151-167)
-        constexpr int E1 = (ED == 0) ? 1 : 0;
-        constexpr int E2 = (ED == 2) ? 1 : 2;
-        const long N3 = g.N3;
-        const long c = IX(g, i, j, k);
-        const long s2 = STRIDE<T2>(g);
-
-        // GetCornerV (fields.F90:457-517), doVdA
-        double A[8];
-#pragma unroll
-        for (int n = 0; n < 8; n++) A[n] = ldx<T2>(met + (M_FACE + T1) * N3, c, s2, n - 4);
-        const double rdA = 1.0 / dmax(wsum8([&](int n) { return A[n]; }), GAM_TINY);
-        double vc[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++)
-            vc[d] = wsum8([&](int n) { return A[n] * ldx<T2>(Vf + d * N3, c, s2, n - 4); }) * rdA;
-        const double *Te = met + (long)(M_TE + 9 * ED) * N3 + c;
-        const double v1 = vc[0] * Te[3 * N3] + vc[1] * Te[4 * N3] + vc[2] * Te[5 * N3];
-        const double v2 = vc[0] * Te[6 * N3] + vc[1] * Te[7 * N3] + vc[2] * Te[8 * N3];
-        double vDiff = sqrt(v1 * v1 + v2 * v2);
-
-        // GetCornerD (fields.F90:427-454)
-        const long se1 = STRIDE<E1>(g), se2 = STRIDE<E2>(g);
-        const double *Dh = H + (H_GAS + DEN) * N3;
-        const double Dc = 0.25 * (Dh[c] + Dh[c - se1] + Dh[c - se2] + Dh[c - se1 - se2]);
-
-        // GetCornerB (fields.F90:365-424)
-        const double *mfH = H + H_MF * N3;
-        const double *mfL = m.doLFM ? S + S_MF * N3 : mfH;
-        double bT1L, bT1R, fA1, bT2L, bT2R, fA2;
-        edge_lr<T1, T2, RM>(g, m, c, met, mfH, mfL, bT1L, bT1R, fA1);
-        edge_lr<T2, T1, RM>(g, m, c, met, mfH, mfL, bT2L, bT2R, fA2);
-        const double *Tb = met + (long)(M_TEB + 4 * ED) * N3 + c;
-        const double xni = Tb[0], yni = Tb[N3], xnj = Tb[2 * N3], ynj = Tb[3 * N3];
-        const double detT = 1.0 / (xni * ynj - xnj * yni);
-        const double rA1 = 1.0 / fA1, rA2 = 1.0 / fA2;
-        const double bT1 = 0.5 * (bT1L + bT1R) * rA1;
-        const double bT2 = 0.5 * (bT2L + bT2R) * rA2;
-        const double db1 = (bT1R - bT1L) * rA1;
-        const double db2 = (bT2R - bT2L) * rA2;
-        const double Jd = db2 - db1;
-        double b1 = detT * (ynj * bT1 - yni * bT2);
-        double b2 = detT * (-(xnj * bT1) + xni * bT2);
-        if (BG) {
-            b1 = b1 + bg[(B_EDGB0 + 0 + 2 * ED) * N3 + c];
-            b2 = b2 + bg[(B_EDGB0 + 1 + 2 * ED) * N3 + c];
-        }
-        const double edge = met[(M_EDGE + ED) * N3 + c];
-        double vA = sqrt(b1 * b1 + b2 * b2) / sqrt(Dc);
-        if (BORIS) vA = m.Ca * vA / sqrt(m.Ca * m.Ca + vA * vA);
-        vDiff = vDiff + vA;
-        vDiff = dmin(vDiff, m.CFL * edge / clk->dt);
-        const double e = -(v1 * b2 - v2 * b1) + m.Vd0 * vDiff * Jd;
-        E[ED * N3 + c] = e * edge;
-    }
-};
-
-// ====================================================================
-// The fluxes of one face from its reconstructed L/R states (the part of
-// Fluxes, stress.F90:204-429, after BlockStateLRs): magnetic kinetic flux
-// with the B0 terms, Boris mag-HOGS, gas kinetic flux, HOGS and the nuke
-// term, times the face area, stored to gFlx/mFlx of direction D.  AT(p)
-// reads plane p at the face point, AT_M(p) one cell below it along D;
-// RECON_B(BL, BR) fills the magnetic L/R states (called only with MHD on,
-// after the metric loads, which keeps the register peak of the fused
-// kernel at that of the gas part); oc is the face's byte offset for the
-// stores.
-// ====================================================================
-template <int D, bool BG, bool BORIS, class AtF, class AtMF, class ReconB>
-__device__ __forceinline__ void face_flux_lr(const Geo &g, const MParm &m,
-                                             const double *__restrict__ H,
-                                             const double *__restrict__ met,
-                                             const double *__restrict__ bg, AtF AT, AtMF AT_M,
-                                             ReconB RECON_B, const double *WL,
-                                             const double *WR, double *BL, double *BR,
-                                             unsigned oc,
-                                             double *__restrict__ gflx,
-                                             double *__restrict__ mflx)
-{
-    const long N3 = g.N3;
-    double T[9];
-#pragma unroll
-    for (int q = 0; q < 9; q++) T[q] = AT(met + (M_TF + q + 9 * D) * N3);
-    const double faB = AT(met + (M_FACE + D) * N3);
-
-    double VaD = 0.0;
-    if (m.doMHD) {
-        RECON_B(BL, BR);
-        const double iFaB = 1.0 / faB;
-        const double Bn = AT(H + (H_MF + D) * N3) * iFaB;
-        double B0[3] = {0.0, 0.0, 0.0}, B0n = 0.0;
-        if (BG) {
-#pragma unroll
-            for (int x = 0; x < 3; x++) B0[x] = AT(bg + (B_FCB0 + x + 3 * D) * N3);
-            B0n = AT(bg + (B_BFLUX0 + D) * N3) * iFaB;
-        }
-        double mF[3] = {0.0, 0.0, 0.0}, bbD = 0.0;
-        mag_kin<BG, BORIS>(m, -1.0, WL, BL, Bn, T, B0, B0n, mF, bbD, VaD);
-        mag_kin<BG, BORIS>(m, +1.0, WR, BR, Bn, T, B0, B0n, mF, bbD, VaD);
-        if (BORIS) {
-#pragma unroll
-            for (int x = 0; x < 3; x++) {
-                double deeP = bbD * (WR[1 + x] - WL[1 + x]) * m.iCa2;
-                mF[x] = mF[x] - m.cHogM * VaD * deeP;
-            }
-        }
-#pragma unroll
-        for (int x = 0; x < 3; x++) stp(mflx + (x + 3 * D) * N3, oc, faB * mF[x]);
-    }
-
-    double gF[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, dW[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    gas_kin(m.igm1, -1.0, WL, T, gF, dW);
-    gas_kin(m.igm1, +1.0, WR, T, gF, dW);
-#pragma unroll
-    for (int v = 0; v < 5; v++) gF[v] = gF[v] - m.cHogH * VaD * dW[v];
-    if (BORIS) {   // "nuclear option" (stress.F90:399-417)
-        double vL = sqrt(WL[1] * WL[1] + WL[2] * WL[2] + WL[3] * WL[3]);
-        double vR = sqrt(WR[1] * WR[1] + WR[2] * WR[2] + WR[3] * WR[3]);
-        double vn = sqrt(vL * vL + vR * vR) / GAM_SQRT2_SP;
-        if (vn >= 1.5 * m.Ca) {
-#pragma unroll
-            for (int v = 0; v < 5; v++) {
-                double dU = AT(H + (H_GAS + v) * N3) - AT_M(H + (H_GAS + v) * N3);
-                gF[v] = gF[v] - m.Ca * dU;
-            }
-        }
-    }
-#pragma unroll
-    for (int v = 0; v < 5; v++) stp(gflx + (v + 5 * D) * N3, oc, faB * gF[v]);
-}
-
-// ====================================================================
-// Interface fluxes of one direction (Fluxes, stress.F90:204-429), every
-// stencil point read from global memory (used along i, where the 8 points
-// are contiguous and merge into wide loads)
-// ====================================================================
-template <int D, int RM, bool BG, bool BORIS, int NTH = BX * BY>
-struct k_flux {
-    static constexpr int NT = NTH;
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m,
-                                               Tile b, const double *__restrict__ H,
-                                               const double *__restrict__ S,
-                                               const double *__restrict__ met,
-                                               const double *__restrict__ bg,
-                                               double *__restrict__ gflx,
-                                               double *__restrict__ mflx,
-                                               double *__restrict__ Vf) const
-    {
-        TILE_IJK(b);
-        const long N3 = g.N3;
-        const long c = IX(g, i, j, k);
-        const long s = STRIDE<D>(g);
-        // byte offsets of the 8 stencil points (cells c-4s .. c+3s), shared by
-        // every plane; o[4] is the face point c itself.  Along i the points are
-        // contiguous and the compiler merges them into wide loads from one
-        // address, so that direction keeps plain indexing.
-        unsigned o[8];
-#pragma unroll
-        for (int n = 0; n < 8; n++) o[n] = (unsigned)((c + (n - 4) * s) * 8);
-        auto LD = [&](const double *__restrict__ plane, int n) -> double {
-            if (D == 0) return plane[c + (n - 4)];
-            return ldp(plane, o[n]);
-        };
-
-        double vol[8];
-#pragma unroll
-        for (int n = 0; n < 8; n++) vol[n] = LD(met + M_VOL * N3, n);
-        const double Vi = wsum8([&](int n) { return vol[n]; });
-        const double rVi = 1.0 / Vi;
-
-        // L/R primitives (BlockStateLRs, recon.F90:39-93); Wv holds V*W
-        const double *Wv = H + H_WH * N3;
-        const double *Wl = H + H_WN * N3;
-        double WL[5], WR[5];
-#pragma unroll
-        for (int v = 0; v < 5; v++) {
-            double qv[8], nq[4];
-#pragma unroll
-            for (int n = 0; n < 8; n++) qv[n] = LD(Wv + v * N3, n);
-#pragma unroll
-            for (int n = 0; n < 4; n++) nq[n] = LD(Wl + v * N3, n + 2);
-            recon_lr_w<RM>(m.pdmb, rVi, nq, qv, WL[v], WR[v]);
-            // Mom2Face of this face from the same velocity stencil
-            // (written without a condition on Vf: a branch here keeps the
-            // stencils alive and costs ~30 VGPRs)
-            if (v >= 1 && v <= 3) stp(Vf + (v - 1) * N3, o[4], mom2face(qv, Vi, rVi));
-        }
-        auto recon_b = [&](double *BL, double *BR) {
-            const double *Bh = H + H_B * N3;
-            const double *Bl = m.doLFM ? S + S_B * N3 : Bh;
-#pragma unroll
-            for (int x = 0; x < 3; x++) {
-                double q[8], nq[4];
-#pragma unroll
-                for (int n = 0; n < 8; n++) q[n] = LD(Bh + x * N3, n);
-#pragma unroll
-                for (int n = 0; n < 4; n++) nq[n] = LD(Bl + x * N3, n + 2);
-                recon_lr<RM>(m.pdmb, vol, rVi, nq, q, BL[x], BR[x]);
-            }
-        };
-        double BL[3], BR[3];
-        face_flux_lr<D, BG, BORIS>(
-            g, m, H, met, bg, [&](const double *p) { return LD(p, 4); },
-            [&](const double *p) { return LD(p, 3); }, recon_b, WL, WR, BL, BR, o[4], gflx, mflx);
-    }
-};
-
-// ====================================================================
-// Interface fluxes along j or k (D = 1, 2) with the stencil planes staged
-// in LDS.  A workgroup owns 64 (i) x FH (along D) faces, FH = 4 or 8 (a
-// launch-plan choice: the taller tile loads FH + 7 rows for FH face rows,
-// fewer halo rows per face, with twice the waves per barrier); the rows
-// of the 8-point stencil (faces' cells a-4 .. a+FH+2) and of the 4-point
-// limiter stencil (a-2 .. a+FH) of one variable at a time go to LDS with
-// coalesced loads, double-buffered so the next variable's rows are in
-// flight while the current one is reconstructed.  Each row is loaded once
-// per workgroup instead of once per stencil point.
-// ====================================================================
-struct FluxTile {
-    int i0, i1, a0, a1, b0, b1;   // faces along i, along D, along the third axis
-    int nti, nta, nb, xs;
-};
-
-template <int D, int RM, bool BG, bool BORIS, int FH = BY, bool DMA = false>
-struct k_flux_s {
-    static constexpr int NT = BX * FH;                         // threads
-    static constexpr int SR8 = FH + 7;                         // rows of an 8-point stage
-    static constexpr int SR4 = FH + 3;                         // rows of a 4-point stage
-    static constexpr int SRW = SR8 + SR4;                      // rows of one variable's stage
-    static constexpr int SLD = (SRW * BX + NT - 1) / NT;       // loads per thread per stage
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m,
-                                               FluxTile t, const double *__restrict__ H,
-                                               const double *__restrict__ S,
-                                               const double *__restrict__ met,
-                                               const double *__restrict__ bg,
-                                               double *__restrict__ gflx,
-                                               double *__restrict__ mflx,
-                                               double *__restrict__ Vf) const
-    {
-        __shared__ double vs[SR8][BX];
-        __shared__ double buf[2][SRW][BX];
-        const int L = xcd_tile((int)bi.x, t.xs);
-        if (L >= t.nb) return;                   // whole workgroup
-        const int ti = L % t.nti;
-        const int r = L / t.nti;
-        const int ta = r % t.nta;
-        const int bb = t.b0 + r / t.nta;
-        const int tx = threadIdx.x, ty = threadIdx.y, tid = tx + BX * ty;
-        const int i0 = t.i0 + ti * BX, a0 = t.a0 + ta * FH;
-        const int i = i0 + tx, a = a0 + ty;
-        const bool act = i <= t.i1 && a <= t.a1;
-        const long N3 = g.N3;
-        const long s = STRIDE<D>(g);
-        // point (i', a', bb) of the box's index space
-        auto at = [&](int ii, int aa) -> long {
-            return D == 1 ? IX(g, ii, aa, bb) : IX(g, ii, bb, aa);
-        };
-        // rows that exist: the stencils of the active faces reach a1 + 3
-        const int aTop = t.a1 + 3;
-        // stage loaders: element e of a stage -> (row, column)
-        auto fetch = [&](const double *p8, const double *p4, double *reg) {
-#pragma unroll
-            for (int q = 0; q < SLD; q++) {
-                const int e = tid + q * NT;
-                const int row = e / BX, col = e % BX;
-                const int ii = i0 + col;
-                double v = 0.0;
-                if (row < SRW && ii <= t.i1) {
-                    const int aa = row < SR8 ? a0 - 4 + row : a0 - 2 + (row - SR8);
-                    const double *p = row < SR8 ? p8 : p4;
-                    if (aa <= aTop) v = p[at(ii, aa)];
-                }
-                reg[q] = v;
-            }
-        };
-        auto store = [&](int bsel, const double *reg) {
-#pragma unroll
-            for (int q = 0; q < SLD; q++) {
-                const int e = tid + q * NT;
-                if (e < SRW * BX) buf[bsel][e / BX][e % BX] = reg[q];
-            }
-        };
-        // DMA form: the stage's rows go straight from global memory to LDS
-        // (global_load_lds, 16 B per lane): one instruction moves two rows,
-        // lanes 0-31 the even row and 32-63 the odd one, into consecutive
-        // LDS rows.  Columns past t.i1 read the tile's first pair and rows
-        // past aTop the row aTop instead (valid cells; only the lanes of
-        // faces outside the box read those LDS entries).
-        auto dma = [&](const double *p8, const double *p4, int bsel) {
-            const int wv = tid >> 6, ln = tid & 63;
-            for (int q = wv; q < SRW / 2; q += NT / 64) {
-                const int row = 2 * q + (ln >> 5);
-                int ii = i0 + 2 * (ln & 31);
-                if (ii > t.i1) ii = i0;
-                int aa = row < SR8 ? a0 - 4 + row : a0 - 2 + (row - SR8);
-                if (aa > aTop) aa = aTop;
-                const double *src = (row < SR8 ? p8 : p4) + at(ii, aa);
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
-                                                 (__attribute__((address_space(3))) void *)&buf[bsel][2 * q][0],
-                                                 16, 0, 0);
-            }
-        };
-        // volumes (8-point rows) and the first stage
-        {
-            const double *pv = met + M_VOL * N3;
-            for (int e = tid; e < SR8 * BX; e += NT) {
-                const int row = e / BX, col = e % BX;
-                const int ii = i0 + col, aa = a0 - 4 + row;
-                vs[row][col] = (ii <= t.i1 && aa <= aTop) ? pv[at(ii, aa)] : 0.0;
-            }
-        }
-        const int nst = m.doMHD ? 8 : 5;
-        const double *Wv = H + H_WH * N3, *Wl = H + H_WN * N3;
-        const double *Bh = H + H_B * N3, *Bl = m.doLFM ? S + S_B * N3 : Bh;
-        auto planes = [&](int st, const double *&p8, const double *&p4) {
-            if (st < 5) { p8 = Wv + st * N3; p4 = Wl + st * N3; }
-            else { p8 = Bh + (st - 5) * N3; p4 = Bl + (st - 5) * N3; }
-        };
-        double reg[DMA ? 1 : SLD];
-        {
-            const double *p8, *p4;
-            planes(0, p8, p4);
-            if (DMA) {
-                dma(p8, p4, 0);
-                __builtin_amdgcn_s_waitcnt(0);
-            } else {
-                fetch(p8, p4, reg);
-                store(0, reg);
-            }
-        }
-        __syncthreads();
-        const double Vi = wsum8([&](int n) { return vs[ty + n][tx]; });
-        const double rVi = 1.0 / Vi;
-        double WL[5], WR[5], BL[3] = {0.0, 0.0, 0.0}, BR[3] = {0.0, 0.0, 0.0};
-        // kept a loop: unrolled, the compiler hoists later stages' loads and
-        // the register count doubles
-#pragma unroll 1
-        for (int st = 0; st < 8; st++) {
-            if (st >= nst) break;
-            const int cur = st & 1;
-            if (!DMA && st + 1 < nst) {
-                const double *p8, *p4;
-                planes(st + 1, p8, p4);
-                fetch(p8, p4, reg);
-            }
-            double q[8], nq[4], vq[8];
-#pragma unroll
-            for (int n = 0; n < 8; n++) q[n] = buf[cur][ty + n][tx];
-#pragma unroll
-            for (int n = 0; n < 4; n++) nq[n] = buf[cur][SR8 + ty + n][tx];
-            if (DMA) {
-                // this stage's LDS reads come first, then the next stage's
-                // DMA, so that no LDS read waits behind the DMA in flight
-                if (st >= 5) {
-#pragma unroll
-                    for (int n = 0; n < 8; n++) vq[n] = vs[ty + n][tx];
-                }
-                if (st + 1 < nst) {
-                    const double *p8, *p4;
-                    planes(st + 1, p8, p4);
-                    dma(p8, p4, cur ^ 1);
-                }
-            }
-            if (st < 5) {
-                recon_lr_w<RM>(m.pdmb, rVi, nq, q, WL[st], WR[st]);
-                // Mom2Face of this face from the same velocity stencil
-                if (st >= 1 && st <= 3 && act) Vf[(st - 1) * N3 + at(i, a)] = mom2face(q, Vi, rVi);
-            } else {
-                // cell B is not volume-weighted in H: weight it here (LDS volumes)
-#pragma unroll
-                for (int n = 0; n < 8; n++) q[n] = (DMA ? vq[n] : vs[ty + n][tx]) * q[n];
-                recon_lr_w<RM>(m.pdmb, rVi, nq, q, BL[st - 5], BR[st - 5]);
-            }
-            if (DMA) __builtin_amdgcn_s_waitcnt(0);
-            else if (st + 1 < nst) store(cur ^ 1, reg);
-            __syncthreads();
-        }
-        if (act) {
-            const long c = at(i, a);
-            const unsigned oc = (unsigned)(c * 8);
-            face_flux_lr<D, BG, BORIS>(
-                g, m, H, met, bg, [&](const double *p) { return ldp(p, oc); },
-                [&](const double *p) { return p[c - s]; },
-                [](double *, double *) {}, WL, WR, BL, BR, oc, gflx, mflx);
         }
     }
 };
@@ -1498,9 +845,9 @@ Plan default_plan()
     p.v[TS_EMF_I] = 3;    // stencils along j and k
     p.v[TS_EMF_J] = 2;    // along i and k
     p.v[TS_EMF_K] = 1;    // along i and j
-    p.v[TS_FLUX_I] = 1;
-    p.v[TS_FLUX_J] = PLAN_LDSDMA;
-    p.v[TS_FLUX_K] = PLAN_LDSDMA;
+    p.v[TS_FLUX_I] = PLAN_LDS;
+    p.v[TS_FLUX_J] = PLAN_LDS;
+    p.v[TS_FLUX_K] = PLAN_LDS;
     p.v[TS_UPDATE] = 3;
     return p;
 }
@@ -1513,11 +860,13 @@ int plan_candidates(int slot, int *vals)
     // row order x chunk size (256, 512, 128 points per workgroup)
     for (int c = 0; c < 3; c++)
         for (int a = 1; a <= maxax; a++) vals[n++] = a + 8 * c;
-    if (slot == TS_FLUX_J || slot == TS_FLUX_K) {
+    if (slot >= TS_FLUX_I && slot <= TS_FLUX_K) {
         vals[n++] = PLAN_LDS;
-        vals[n++] = PLAN_LDS8;
-        vals[n++] = PLAN_LDSDMA;
-        vals[n++] = PLAN_LDS8DMA;
+        vals[n++] = PLAN_LDS_D;
+        if (slot != TS_FLUX_I) {
+            vals[n++] = PLAN_LDS + PLAN_ALIAS;
+            vals[n++] = PLAN_LDS_D + PLAN_ALIAS;
+        }
     }
     return n;
 }
@@ -1552,110 +901,10 @@ void launch_vface_rim(hipStream_t s, const Geo &g, const double *H, const double
     launch_f<k_vface_rim>(dim3((unsigned)tot), dim3(BX, BY), s, g, r, H, met, Vf);
 }
 
-template <int ED, int RM, bool BG, bool BO>
-static void emf_t(hipStream_t s, int plan, const Geo &g, const MParm &m, const Box &b, const Clock *clk,
-                  const double *H, const double *S, const double *Vf, const double *met,
-                  const double *bg, double *E)
-{
-    const int ch = plan_chunk(plan);
-    const Tile t = tile_of(b, plan_ax(plan), ch);
-    if (ch == 512)
-        launch_f<k_emf<ED, RM, BG, BO, 512>>(tgrid(t), dim3(BX, 8), s, g, m, t, clk, H, S, Vf, met, bg, E);
-    else if (ch == 128)
-        launch_f<k_emf<ED, RM, BG, BO, 128>>(tgrid(t), dim3(BX, 2), s, g, m, t, clk, H, S, Vf, met, bg, E);
-    else
-        launch_f<k_emf<ED, RM, BG, BO>>(tgrid(t), dim3(BX, BY), s, g, m, t, clk, H, S, Vf, met, bg, E);
-}
-
-template <int ED>
-static void emf_d(hipStream_t s, int ax, const Geo &g, const MParm &m, const Box &b, const Clock *clk,
-                  const double *H, const double *S, const double *Vf, const double *met,
-                  const double *bg, double *E)
-{
-    const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
-    switch (sel) {
-    case 0: emf_t<ED, 0, false, false>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 1: emf_t<ED, 0, false, true>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 2: emf_t<ED, 0, true, false>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 3: emf_t<ED, 0, true, true>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 4: emf_t<ED, 1, false, false>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 5: emf_t<ED, 1, false, true>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 6: emf_t<ED, 1, true, false>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    default: emf_t<ED, 1, true, true>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    }
-}
-
-void launch_emf(hipStream_t s, int eD, int ax, const Geo &g, const MParm &m, const Box &b, const Clock *clk,
-                const double *H, const double *S, const double *Vf, const double *met,
-                const double *bg, double *E)
-{
-    if (eD == 0) emf_d<0>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E);
-    else if (eD == 1) emf_d<1>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E);
-    else emf_d<2>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E);
-}
-
-template <int D, int RM, bool BG, bool BO>
-static void flux_t(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
-                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
-{
-    if constexpr (D != 0) {
-        if (form >= PLAN_LDS && form <= PLAN_LDS8DMA) {
-            const int fh = (form == PLAN_LDS8 || form == PLAN_LDS8DMA) ? 8 : BY;
-            FluxTile t;
-            t.i0 = b.i0;
-            t.i1 = b.i1;
-            if (D == 1) { t.a0 = b.j0; t.a1 = b.j1; t.b0 = b.k0; t.b1 = b.k1; }
-            else { t.a0 = b.k0; t.a1 = b.k1; t.b0 = b.j0; t.b1 = b.j1; }
-            t.nti = (t.i1 - t.i0 + BX) / BX;
-            t.nta = (t.a1 - t.a0 + fh) / fh;
-            t.nb = t.nti * t.nta * (t.b1 - t.b0 + 1);
-            t.xs = xcd_shift(t.nb);
-            const dim3 grid(xcd_grid(t.nb, t.xs));
-            if (form == PLAN_LDS8DMA)
-                launch_f<k_flux_s<D, RM, BG, BO, 8, true>>(grid, dim3(BX, 8), s, g, m, t, H, S, met, bg, gf, mf, vf);
-            else if (fh == 8)
-                launch_f<k_flux_s<D, RM, BG, BO, 8>>(grid, dim3(BX, 8), s, g, m, t, H, S, met, bg, gf, mf, vf);
-            else if (form == PLAN_LDSDMA)
-                launch_f<k_flux_s<D, RM, BG, BO, BY, true>>(grid, dim3(BX, BY), s, g, m, t, H, S, met, bg, gf, mf,
-                                                            vf);
-            else
-                launch_f<k_flux_s<D, RM, BG, BO>>(grid, dim3(BX, BY), s, g, m, t, H, S, met, bg, gf, mf, vf);
-            return;
-        }
-    }
-    const int ch = plan_chunk(form);
-    const Tile t = tile_of(b, plan_ax(form), ch);
-    if (ch == 512)
-        launch_f<k_flux<D, RM, BG, BO, 512>>(tgrid(t), dim3(BX, 8), s, g, m, t, H, S, met, bg, gf, mf, vf);
-    else if (ch == 128)
-        launch_f<k_flux<D, RM, BG, BO, 128>>(tgrid(t), dim3(BX, 2), s, g, m, t, H, S, met, bg, gf, mf, vf);
-    else
-        launch_f<k_flux<D, RM, BG, BO>>(tgrid(t), dim3(BX, BY), s, g, m, t, H, S, met, bg, gf, mf, vf);
-}
-
-template <int D>
-static void flux_d(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
-                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
-{
-    const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
-    switch (sel) {
-    case 0: flux_t<D, 0, false, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 1: flux_t<D, 0, false, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 2: flux_t<D, 0, true, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 3: flux_t<D, 0, true, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 4: flux_t<D, 1, false, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 5: flux_t<D, 1, false, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 6: flux_t<D, 1, true, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    default: flux_t<D, 1, true, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    }
-}
-
 void launch_flux(hipStream_t s, int d, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
                  const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
 {
-    if (d == 0) flux_d<0>(s, form, g, m, b, H, S, met, bg, gf, mf, vf);
-    else if (d == 1) flux_d<1>(s, form, g, m, b, H, S, met, bg, gf, mf, vf);
-    else flux_d<2>(s, form, g, m, b, H, S, met, bg, gf, mf, vf);
+    (d == 0 ? launch_flux_i : d == 1 ? launch_flux_j : launch_flux_k)(s, form, g, m, b, H, S, met, bg, gf, mf, vf);
 }
 
 template <bool BG, bool BO>
