@@ -200,11 +200,13 @@ extern "C" int gam_create(gam_ctx **out, const gam_dims *d, const gam_model *m)
     g.Ni = d->Nip + 8; g.Nj = d->Njp + 8; g.Nk = d->Nkp + 8;
     g.is = 1; g.ie = d->Nip; g.js = 1; g.je = d->Njp; g.ks = 1; g.ke = d->Nkp;
     g.isg = -3; g.ieg = g.ie + 4; g.jsg = -3; g.jeg = g.je + 4; g.ksg = -3; g.keg = g.ke + 4;
-    g.P = ((g.Ni + 1 + 4) + 7) / 8 * 8;
+    // rows of whole 128-byte lines with the first active cell i = is at the
+    // start of one (index 16), the i ghosts below it at the end of the row
+    // before: tiles of 16 or 32 points from i = is read whole lines
+    g.P = (g.Ni + 1 + 15) / 16 * 16;
     g.PP = (long)g.P * (g.Nj + 1);
-    // i=isg lands at offset 4 of its row, so i=is (=isg+4) is 64-byte aligned
-    g.c0 = 4 - g.isg - (long)g.P * g.jsg - g.PP * g.ksg;
-    long n3 = g.PP * (g.Nk + 1);
+    g.c0 = 16 - g.is - (long)g.P * g.jsg - g.PP * g.ksg;
+    long n3 = g.PP * (g.Nk + 1) + 16;
     g.N3 = (n3 + 63) / 64 * 64;
     const size_t pl = (size_t)g.N3 * sizeof(double);
 

@@ -3,8 +3,8 @@
 // Device layout: every field is a structure-of-arrays "plane" of N3 doubles
 // over ONE padded index space shared by cell-, face- and edge-centred data:
 //     IX(i,j,k) = c0 + i + P*j + PP*k
-// with P = roundup(Ni+1+4, 8) (i fastest, rows 64-byte aligned so that the
-// first active cell i=1 sits on a 64-byte boundary), PP = P*(Nj+1).
+// with P = roundup(Ni+1, 16) (i fastest, rows of whole 128-byte lines, the
+// first active cell i=1 at the start of one), PP = P*(Nj+1).
 // Cell (i,j,k), its low I/J/K faces and its low edges share the index, as
 // in the reference's (isg:ieg[+1], ...) Fortran arrays.
 #pragma once

@@ -171,11 +171,13 @@ struct k_flux {
 // Two phases share the LDS planes: the five gas variables, then the three
 // field components, whose loads wait in registers meanwhile; 37 KB (33 for
 // D = 0) and 128 registers leave room for four workgroups per CU.
+// The tile's 32 points are two whole 128-byte lines of every row.
 // Bound by memory traffic, close behind by FP64 issue (1075 vector
 // instructions per face; at 1580 the clock fell to 1.8 GHz).  256x256x384
 // shell, per launch: a 64 x 4 tile staged one variable at a time took 2.35
 // ms for D = 1, 2 (9.15 GB), direct loads 2.02 ms for D = 0 (9.1 GB); this
-// form 2.0-2.15 ms and 1.94 ms.
+// form 1.75-1.84 ms and 1.92 ms (9.0 GB at 5.0 TB/s; the streaming rate of
+// 32 read and 11 written planes is 5.2-5.5).
 // ====================================================================
 struct FluxTile {
     Tile t;                       // D = 0: the face rows; D = 1, 2: t.nb and t.xs
