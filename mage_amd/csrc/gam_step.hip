@@ -841,14 +841,16 @@ __global__ void k_mask_e(Geo g, Box all, EdgeBoxes eb, double *__restrict__ E)
 Plan default_plan()
 {
     Plan p;
-    p.v[TS_PREDICT] = 3;
+    // pointwise but for the next row and plane: row order 1 takes the
+    // 256x256x384 step from 16.28 to 16.09 ms for either (slabs: 3)
+    p.v[TS_PREDICT] = 1;
     p.v[TS_EMF_I] = 3;    // stencils along j and k
     p.v[TS_EMF_J] = 2;    // along i and k
     p.v[TS_EMF_K] = 1;    // along i and j
     p.v[TS_FLUX_I] = PLAN_LDS;
     p.v[TS_FLUX_J] = PLAN_LDS;
     p.v[TS_FLUX_K] = PLAN_LDS;
-    p.v[TS_UPDATE] = 3;
+    p.v[TS_UPDATE] = 1;
     return p;
 }
 
