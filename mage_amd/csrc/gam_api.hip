@@ -573,32 +573,18 @@ static int check_ready(gam_ctx *c, const char *who)
 
 static Box empty_box() { return mkbox(1, 0, 1, 0, 1, 0); }
 
-// bFlux2Fld over all cells, or over the ghost cells only when the active
-// cells' faces are known to be unchanged since their B was computed.
-static void enq_bflux2fld(gam_ctx *c, double *S, bool ghosts_only = false)
+// bFlux2Fld over all cells
+static void enq_bflux2fld(gam_ctx *c, double *S)
 {
     const long N3 = c->g.N3;
-    if (ghosts_only)
-        launch_bflux2fld_ghosts(c->stream, c->g, S + S_MF * N3, S + S_B * N3, c->met);
-    else
-        launch_bflux2fld(c->stream, c->g, cell_box(c->g), empty_box(), S + S_MF * N3, S + S_B * N3, c->met);
+    launch_bflux2fld(c->stream, c->g, cell_box(c->g), empty_box(), S + S_MF * N3, S + S_B * N3, c->met);
 }
 
-// ghostB: whether BCs also set ghost-cell B (EnforceBCs on its own does;
-// inside stepGamera the bFlux2Fld that follows rewrites every ghost cell).
-// clk: the clock whose time the inflow BC reads (the context's by default).
-static void enq_bcs(gam_ctx *c, double *S, bool ghostB = true, const Clock *clk = nullptr)
+// EnforceBCs on its own.  clk: the clock whose time the inflow BC reads (the
+// context's by default).
+static void enq_bcs(gam_ctx *c, double *S, Clock *clk = nullptr)
 {
-    for (int ax = 0; ax < 3; ax++) {
-        const int lo = 2 * ax, hi = lo + 1;
-        if (c->model.bc[lo] == GAM_BC_PERIODIC && c->model.bc[hi] == GAM_BC_PERIODIC) {
-            launch_bc_periodic_pair(c->stream, ax, c->g, S);
-            continue;
-        }
-        for (int side = lo; side <= hi; side++)
-            launch_bc(c->stream, side, c->model.bc[side], c->g, c->mp, clk ? clk : c->clk, &c->wd, S, c->met,
-                      ghostB);
-    }
+    launch_bcs(c->stream, c->model.bc, false, 0, c->g, c->mp, clk ? clk : c->clk, c->wd, S, c->met);
 }
 
 // While a slot is being tuned, its launches are bracketed by events.
@@ -686,7 +672,7 @@ static void enq_advance(gam_ctx *c, int finmode)
     tune_mark(c, TS_UPDATE);
     prof_end(c, KG_UPDATE);
 
-    launch_finalize(s, c->mp, c->clk, finmode);
+    if (finmode) launch_finalize(s, c->mp, c->clk, finmode);
     if (c->snx) {
         c->st[1 - c->cur] = c->snx;
         c->snx = nullptr;
@@ -716,16 +702,17 @@ static void enq_intermediates(gam_ctx *c)
 
 static void enq_step(gam_ctx *c)
 {
-    enq_advance(c, FIN_ADVANCE | FIN_MODEL | FIN_CALCDT | FIN_SETDT);
+    const int fin = FIN_ADVANCE | FIN_MODEL | FIN_CALCDT | FIN_SETDT;
+    // the boundary launch does the time bookkeeping, unless CalcDT's argmin
+    // is recorded, which needs the new dt before it
+    const bool rec = c->dtrec != nullptr;
+    enq_advance(c, rec ? fin : 0);
     double *S = S_cur(c);
-    if (c->dtrec)
+    if (rec)
         launch_dt_record(c->stream, c->g, c->mp, dt_box(c->g), S, c->met, c->bg, c->clk, c->dtrec_part, c->dtrec);
     prof_begin(c, KG_BC);
-    enq_bcs(c, S, false);
+    launch_bcs(c->stream, c->model.bc, true, rec ? 0 : fin, c->g, c->mp, c->clk, c->wd, S, c->met);
     prof_end(c, KG_BC);
-    prof_begin(c, KG_BFLD);
-    enq_bflux2fld(c, S, true);
-    prof_end(c, KG_BFLD);
 }
 
 // n steps: pairs as one launch of a graph of two steps (captured on first
@@ -2040,7 +2027,7 @@ static int adj_replay(gam_adj *a, const double *Gas, const double *oGas, const d
         enq_bflux2fld(c, S_old(c));
     }
     enq_bcs(c, S_cur(c));    // ghosts from the given interiors, oState's at its time
-    enq_bcs(c, S_old(c), true, a->oclk);
+    enq_bcs(c, S_old(c), a->oclk);
     if (c->mp.doMHD) {       // cell B from the face fluxes
         enq_bflux2fld(c, S_cur(c));
         enq_bflux2fld(c, S_old(c));

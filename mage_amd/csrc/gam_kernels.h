@@ -109,12 +109,10 @@ void launch_calc_dt(hipStream_t s, const Geo &g, const MParm &m, const Box &dtb,
 void launch_finalize(hipStream_t s, const MParm &m, Clock *clk, int mode);
 void launch_bflux2fld(hipStream_t s, const Geo &g, const Box &cb, const Box &skip, const double *mf,
                       double *B, const double *met);
-void launch_bflux2fld_ghosts(hipStream_t s, const Geo &g, const double *mf, double *B, const double *met);
-// ghostB = false skips ghost-cell B that a following ghost bFlux2Fld rewrites
-// both sides of axis ax (0 = I, 1 = J, 2 = K) when both are periodic
-void launch_bc_periodic_pair(hipStream_t s, int ax, const Geo &g, double *S);
-void launch_bc(hipStream_t s, int side, int kind, const Geo &g, const MParm &m, const Clock *clk,
-               const WindDev *w, double *S, const double *met, bool ghostB);
+// EnforceBCs of S: alone (field = false) or inside a step, with cell B of
+// the ghost cells from their faces and, with finmode, launch_finalize's work
+void launch_bcs(hipStream_t s, const int *kind, bool field, int finmode, const Geo &g, const MParm &m, Clock *clk,
+                const WindDev &w, double *S, const double *met);
 void launch_divb(hipStream_t s, const Geo &g, const Box &ab, const double *mf, const double *bg,
                  int useBG, double *part, int *nparts);
 void launch_repack(hipStream_t s, int dir_in, const Geo &g, int ni, int nj, int nk,

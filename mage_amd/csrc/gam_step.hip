@@ -10,10 +10,9 @@
 //   k_update     CT face-flux update, cell B of the new state, flux
 //                divergence, Reynolds, Maxwell/Boris and the CFL
 //                min-reduction of the new state
-//   k_finalize   time bookkeeping and CalcDT checks (1 thread)
-//   k_bc_*       boundary conditions
-//   k_bflux2fld  cell B after the BCs; active cells keep theirs,
-//                since no BC writes a face of an active cell
+//   k_bc_i, k_bc_copy  boundary conditions, cell B of the ghost cells (the
+//                active cells keep theirs: no BC writes a face of one),
+//                time bookkeeping and CalcDT checks (gam_bc.hip)
 // State and oState are two buffers that swap roles every step, which
 // replaces CopyState (mhdgroup.F90:204-255): the update reads the current
 // buffer and writes every point of the other.
@@ -416,356 +415,6 @@ struct k_calc_dt {
     }
 };
 
-// ====================================================================
-// Time bookkeeping and CalcDT checks (step.F90:103-166); one thread.
-// ====================================================================
-struct k_finalize {
-    __device__ __forceinline__ void operator()(const uint3 bi, MParm m, Clock *clk, int mode) const
-    {
-        if (threadIdx.x != 0 || bi.x != 0) return;
-        Clock c = *clk;
-        if (mode & FIN_ADVANCE) {          // applyUpdate: oState%time=State%time; State%time+=dt
-            c.ost = c.st;
-            c.st = c.st + c.dtA;
-        }
-        if (mode & FIN_MODEL) {            // UpdateStateData (gamapp.F90:108-110)
-            c.ts = c.ts + 1;
-            c.t = c.t + c.dt;
-        }
-        if (mode & FIN_CALCDT) {
-            const double dtMin = __longlong_as_double((long long)c.dtBits);
-            int st = 0;
-            if (dtMin == GAM_HUGE) st = 2;
-            double dt = dtMin;
-            if (c.ts > 0) {
-                if (c.dt / dtMin >= 10) st = st > 1 ? st : 1;
-                if ((m.dt0 > GAM_TINY) && (dtMin / m.dt0 <= m.limDT0)) st = st > 1 ? st : 1;
-                if (dtMin <= GAM_TINY) st = 2;
-            }
-            if ((c.t + dt) > m.tFin) dt = dmax(m.tFin - c.t, GAM_TINY);
-            if (m.dt0 > GAM_TINY && dt > (10.0 * m.dt0)) dt = 10.0 * m.dt0;
-            c.dtRet = dt;
-            c.lastStatus = st;
-            c.status = c.status > st ? c.status : st;
-            if (mode & FIN_SETDT) { c.dt = dt; c.dtA = dt; }
-            if (mode & FIN_INIT) c.ost = c.st - c.dt;
-        }
-        c.dtBits = (unsigned long long)__double_as_longlong(GAM_HUGE);
-        *clk = c;
-    }
-};
-
-// ====================================================================
-// bFlux2Fld (gridutils.F90:281-301) over all cells
-// ====================================================================
-struct k_bflux2fld {
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g,
-                                               Tile cb, Box skip, const double *__restrict__ mf,
-                                               double *__restrict__ B,
-                                               const double *__restrict__ met) const
-    {
-        TILE_IJK(cb);
-        if (in_box(skip, i, j, k)) return;
-        const long N3 = g.N3, c = IX(g, i, j, k);
-        double b[3];
-        cell_b(g, met, c, mf[c], mf[N3 + c], mf[2 * N3 + c], mf[c + 1], mf[N3 + c + g.P],
-               mf[2 * N3 + c + g.PP], b);
-        for (int x = 0; x < 3; x++) B[x * N3 + c] = b[x];
-    }
-};
-
-// bFlux2Fld over the ghost shell only: up to six boxes (the i, j and k
-// ghost slabs, disjoint), each cut into 64 x 4 (i, j) tiles; workgroup w
-// finds its box from the running tile counts.
-// A tile of BX*BY threads covers iw[q] points along i by BX*BY/iw[q] along
-// j: 64 x 4 in the wide boxes, 4 x 64 in the 4-wide i-ghost slabs (every
-// lane busy, 32 contiguous bytes per row).
-struct GhostBoxes {
-    Box b[6];
-    int start[7];     // first tile of each box; start[n] = total
-    int n0[6], n1[6], iw[6];
-    int n;
-};
-
-struct k_bflux2fld_ghosts {
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g,
-                                               const GhostBoxes &gb, const double *__restrict__ mf,
-                                               double *__restrict__ B,
-                                               const double *__restrict__ met) const
-    {
-        const int w = (int)bi.x;
-        int q = 0;
-        while (q + 1 < gb.n && w >= gb.start[q + 1]) q++;
-        const int L = w - gb.start[q];
-        const Box &b = gb.b[q];
-        const int t0 = L % gb.n0[q];
-        const int r = L / gb.n0[q];
-        const int tid = (int)(threadIdx.x + BX * threadIdx.y), iw = gb.iw[q];
-        const int i = b.i0 + t0 * iw + tid % iw;
-        const int j = b.j0 + (r % gb.n1[q]) * (BX * BY / iw) + tid / iw;
-        const int k = b.k0 + r / gb.n1[q];
-        if (i > b.i1 || j > b.j1 || k > b.k1) return;
-        const long N3 = g.N3, c = IX(g, i, j, k);
-        double bb[3];
-        cell_b(g, met, c, mf[c], mf[N3 + c], mf[2 * N3 + c], mf[c + 1], mf[N3 + c + g.P],
-               mf[2 * N3 + c + g.PP], bb);
-        for (int x = 0; x < 3; x++) B[x * N3 + c] = bb[x];
-    }
-};
-
-// ====================================================================
-// Boundary conditions.  One thread per transverse ghost column with the n
-// loop inside as in the reference (j and k sides), or per column and
-// ghost layer (i sides, below).  Kernels of the six faces run in the
-// reference order INI, OUTI, INJ, OUTJ, INK, OUTK.
-// ====================================================================
-__device__ __forceinline__ void copy_cell(double *S, long N3, long dst, long src)
-{
-    for (int v = 0; v < 5; v++) S[(S_GAS + v) * N3 + dst] = S[(S_GAS + v) * N3 + src];
-}
-__device__ __forceinline__ void copy_b(double *S, long N3, long dst, long src)
-{
-    for (int x = 0; x < 3; x++) S[(S_B + x) * N3 + dst] = S[(S_B + x) * N3 + src];
-}
-__device__ __forceinline__ bool is_cell(const Geo &g, int i, int j, int k)
-{
-    return i >= g.isg && i <= g.ieg && j >= g.jsg && j <= g.jeg && k >= g.ksg && k <= g.keg;
-}
-
-// Ghost layers n = 1..4: the i-side kernels (points (j, k) with 4-wide
-// ghost slabs along i) run one layer per thread, the four layers of a point
-// in adjacent lanes (a 64-lane block covers 16 points along j), so that one
-// load reads 32 contiguous bytes along i rather than 8; the j- and k-side
-// kernels (threads along i, coalesced) loop over n.  TA = the thread's
-// transverse offset along the first transverse axis.
-#define NL0(side) (((side) <= 1) ? 1 + (int)(threadIdx.x & 3) : 1)
-#define NL1(side) (((side) <= 1) ? 1 + (int)(threadIdx.x & 3) : 4)
-#define TA(side) (((side) <= 1) ? (int)(bi.x * 16 + (threadIdx.x >> 2)) : (int)(bi.x * blockDim.x + threadIdx.x))
-
-// periodic (bcs.F90:279-450).  side: 0..5.  (a,b) = transverse indices
-template <int SIDE>
-struct k_bc_periodic {
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, Box t,
-                                               double *__restrict__ S) const
-    {
-        const int a = t.i0 + TA(SIDE);
-        const int b = t.j0 + bi.y;
-        if (a > t.i1 || b > t.j1) return;
-        const long N3 = g.N3;
-        double *mf = S + S_MF * N3;
-        for (int n = NL0(SIDE); n <= NL1(SIDE); n++) {
-            if (SIDE == 0) {        // inner I: a=j, b=k
-                const int ig = g.is - n, sr = g.ie - n + 1;
-                const long d = IX(g, ig, a, b), s = IX(g, sr, a, b);
-                if (is_cell(g, ig, a, b)) { copy_cell(S, N3, d, s); copy_b(S, N3, d, s); }
-                for (int x = 0; x < 3; x++) mf[x * N3 + d] = mf[x * N3 + s];
-            } else if (SIDE == 1) { // outer I
-                const int ig = g.ie + n, sr = g.is + n - 1;
-                const long d = IX(g, ig, a, b), s = IX(g, sr, a, b);
-                if (is_cell(g, ig, a, b)) { copy_cell(S, N3, d, s); copy_b(S, N3, d, s); }
-                mf[1 * N3 + d] = mf[1 * N3 + s];
-                mf[2 * N3 + d] = mf[2 * N3 + s];
-                mf[IX(g, ig + 1, a, b)] = mf[IX(g, g.is + n, a, b)];
-            } else if (SIDE == 2) { // inner J: a=i, b=k
-                const int jg = g.js - n, sr = g.je - n + 1;
-                const long d = IX(g, a, jg, b), s = IX(g, a, sr, b);
-                if (is_cell(g, a, jg, b)) { copy_cell(S, N3, d, s); copy_b(S, N3, d, s); }
-                for (int x = 0; x < 3; x++) mf[x * N3 + d] = mf[x * N3 + s];
-            } else if (SIDE == 3) { // outer J
-                const int jg = g.je + n, sr = g.js + n - 1;
-                const long d = IX(g, a, jg, b), s = IX(g, a, sr, b);
-                if (is_cell(g, a, jg, b)) { copy_cell(S, N3, d, s); copy_b(S, N3, d, s); }
-                mf[0 * N3 + d] = mf[0 * N3 + s];
-                mf[2 * N3 + d] = mf[2 * N3 + s];
-                mf[1 * N3 + IX(g, a, jg + 1, b)] = mf[1 * N3 + IX(g, a, g.js + n, b)];
-            } else if (SIDE == 4) { // inner K: a=i, b=j
-                const int kg = g.ks - n, sr = g.ke - n + 1;
-                const long d = IX(g, a, b, kg), s = IX(g, a, b, sr);
-                if (is_cell(g, a, b, kg)) { copy_cell(S, N3, d, s); copy_b(S, N3, d, s); }
-                for (int x = 0; x < 3; x++) mf[x * N3 + d] = mf[x * N3 + s];
-            } else {                // outer K
-                const int kg = g.ke + n, sr = g.ks + n - 1;
-                const long d = IX(g, a, b, kg), s = IX(g, a, b, sr);
-                if (is_cell(g, a, b, kg)) { copy_cell(S, N3, d, s); copy_b(S, N3, d, s); }
-                mf[0 * N3 + d] = mf[0 * N3 + s];
-                mf[1 * N3 + d] = mf[1 * N3 + s];
-                mf[2 * N3 + IX(g, a, b, kg + 1)] = mf[2 * N3 + IX(g, a, b, g.ks + n)];
-            }
-        }
-    }
-};
-
-// zero-gradient (bcs.F90:799-930), sphere in/out (934-982)
-template <int SIDE, int KIND>
-struct k_bc_copy {
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, Box t,
-                                               double *__restrict__ S,
-                                               const double *__restrict__ met) const
-    {
-        const int a = t.i0 + TA(SIDE);
-        const int b = t.j0 + bi.y;
-        if (a > t.i1 || b > t.j1) return;
-        const long N3 = g.N3;
-        double *mf = S + S_MF * N3;
-        if (SIDE == 0) {            // inner I: a=j, b=k
-            const long s = IX(g, g.is, a, b);
-            for (int n = NL0(SIDE); n <= NL1(SIDE); n++) {
-                const long d = IX(g, g.is - n, a, b);
-                copy_cell(S, N3, d, s);
-                for (int x = 0; x < 3; x++) mf[x * N3 + d] = mf[x * N3 + s];
-                if (KIND == 2) copy_b(S, N3, d, s);      // SphIn also copies Bxyz
-            }
-        } else if (SIDE == 1) {     // outer I
-            const long s = IX(g, g.ie, a, b);
-            if (KIND == 3) {        // SphOut
-                for (int n = NL0(SIDE); n <= NL1(SIDE); n++) {
-                    const int ig = g.ie + n;
-                    const long d = IX(g, ig, a, b);
-                    copy_cell(S, N3, d, s);
-                    mf[IX(g, ig + 1, a, b)] = mf[s];
-                    mf[N3 + d] = mf[N3 + s];
-                    mf[2 * N3 + d] = mf[2 * N3 + s];
-                    copy_b(S, N3, d, s);
-                }
-            } else {                // zeroGrad_obcI: fluxes of the last physical cell's B
-                double B[3];
-                cell_b(g, met, s, mf[s], mf[N3 + s], mf[2 * N3 + s], mf[s + 1], mf[N3 + s + g.P],
-                       mf[2 * N3 + s + g.PP], B);
-                for (int n = NL0(SIDE); n <= NL1(SIDE); n++) {
-                    const int ig = g.ie + n;
-                    const long d = IX(g, ig, a, b);
-                    copy_cell(S, N3, d, s);
-                    const long fi[3] = {IX(g, ig + 1, a, b), d, d};
-                    for (int x = 0; x < 3; x++) {
-                        const long f = fi[x];
-                        const double *nrm = met + (long)(M_TF + 9 * x) * N3 + f;
-                        mf[x * N3 + f] = met[(M_FACE + x) * N3 + f] * (B[0] * nrm[0] + B[1] * nrm[N3] + B[2] * nrm[2 * N3]);
-                    }
-                }
-            }
-        } else if (SIDE == 2) {     // inner J: a=i, b=k
-            const long s = IX(g, a, g.js, b);
-            for (int n = NL0(SIDE); n <= NL1(SIDE); n++) {
-                const long d = IX(g, a, g.js - n, b);
-                copy_cell(S, N3, d, s);
-                for (int x = 0; x < 3; x++) mf[x * N3 + d] = mf[x * N3 + s];
-            }
-        } else if (SIDE == 3) {     // outer J
-            const long s = IX(g, a, g.je, b);
-            for (int n = NL0(SIDE); n <= NL1(SIDE); n++) {
-                const long d = IX(g, a, g.je + n, b);
-                copy_cell(S, N3, d, s);
-                mf[d] = mf[s];
-                mf[2 * N3 + d] = mf[2 * N3 + s];
-                mf[N3 + IX(g, a, g.je + n + 1, b)] = mf[N3 + IX(g, a, g.je + 1, b)];
-            }
-        } else if (SIDE == 4) {     // inner K: a=i, b=j
-            const long s = IX(g, a, b, g.ks);
-            for (int n = NL0(SIDE); n <= NL1(SIDE); n++) {
-                const long d = IX(g, a, b, g.ks - n);
-                copy_cell(S, N3, d, s);
-                for (int x = 0; x < 3; x++) mf[x * N3 + d] = mf[x * N3 + s];
-            }
-        } else {                    // outer K; the k+1 face takes the J flux (bcs.F90:925)
-            const long s = IX(g, a, b, g.ke);
-            for (int n = NL0(SIDE); n <= NL1(SIDE); n++) {
-                const long d = IX(g, a, b, g.ke + n);
-                copy_cell(S, N3, d, s);
-                mf[d] = mf[s];
-                mf[N3 + d] = mf[N3 + s];
-                mf[2 * N3 + IX(g, a, b, g.ke + n + 1)] = mf[N3 + IX(g, a, b, g.ke + 1)];
-            }
-        }
-    }
-};
-
-// ---------------------------------------------------------------- wind
-#include "gam_wind.h"
-
-// WindBC part 1 (wind.F90:226-335): ghost gas and blended face fluxes.
-// Transverse: a = j in jsg..jeg+1, b = k in ksg..keg+1.
-struct k_bc_wind {
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, Box t,
-                                               const Clock *clk, WindDev w, double *__restrict__ S,
-                                               const double *__restrict__ met) const
-    {
-        const int j = t.i0 + TA(1);
-        const int k = t.j0 + bi.y;
-        if (j > t.i1 || k > t.j1) return;
-        const long N3 = g.N3;
-        double *mf = S + S_MF * N3;
-        const double tm = clk->t;
-        double vF[3];
-        wind_front(w, tm, vF);
-        const int ip = g.ie;
-        for (int n = NL0(1); n <= NL1(1); n++) {
-            const int ig = g.ie + n;
-            if (k <= g.keg && j <= g.jeg) {
-                const long cg = IX(g, ig, j, k), cp = IX(g, ip, j, k);
-                const double xc[3] = {met[(M_XYZCC + 0) * N3 + cg], met[(M_XYZCC + 1) * N3 + cg], met[(M_XYZCC + 2) * N3 + cg]};
-                double r, p, V[3], B[3];
-                wind_at(w, vF, xc, tm, &r, &p, V, B);
-                const double wSW = wind_wgt_v(xc, V), wMHD = 1.0 - wSW;
-                double gs[5] = {0, 0, 0, 0, 0}, gi[5] = {0, 0, 0, 0, 0};
-                if (wSW > GAM_TINY) {
-                    gs[0] = r; gs[1] = V[0]; gs[2] = V[1]; gs[3] = V[2]; gs[4] = p;
-                }
-                if (wMHD > GAM_TINY) {
-                    double U[5], Bi[3];
-                    for (int v = 0; v < 5; v++) U[v] = S[(S_GAS + v) * N3 + cp];
-                    for (int x = 0; x < 3; x++) Bi[x] = S[(S_B + x) * N3 + cp];
-                    const long fp = IX(g, ip + 1, j, k);
-                    const double nH[3] = {met[(M_TF + 0) * N3 + fp], met[(M_TF + 1) * N3 + fp], met[(M_TF + 2) * N3 + fp]};
-                    wind_inner(m, U, Bi, nH, gi);
-                }
-                double gw[5], U[5];
-                for (int v = 0; v < 5; v++) gw[v] = wSW * gs[v] + wMHD * gi[v];
-                p2c_cell(m, gw, U);
-                for (int v = 0; v < 5; v++) S[(S_GAS + v) * N3 + cg] = U[v];
-            }
-            const int fi[3] = {ig + 1, ig, ig};
-            const int ii[3] = {ip + 1, ip, ip};
-            for (int d = 0; d < 3; d++) {
-                const long f = IX(g, fi[d], j, k);
-                const double xf[3] = {met[(M_XFC + 0 + 3 * d) * N3 + f], met[(M_XFC + 1 + 3 * d) * N3 + f], met[(M_XFC + 2 + 3 * d) * N3 + f]};
-                double r, p, V[3], B[3];
-                wind_at(w, vF, xf, tm, &r, &p, V, B);
-                const double wSW = wind_wgt_v(xf, V);
-                const double *nrm = met + (long)(M_TF + 9 * d) * N3 + f;
-                const double sw = met[(M_FACE + d) * N3 + f] * (nrm[0] * B[0] + nrm[N3] * B[1] + nrm[2 * N3] * B[2]);
-                const double in = mf[d * N3 + IX(g, ii[d], j, k)];
-                mf[d * N3 + f] = wSW * sw + (1 - wSW) * in;
-            }
-        }
-    }
-};
-
-// WindBC part 2 (wind.F90:338-348): ghost Bxyz from the blended fluxes with
-// the periodic k mapping of lfmIJKcc (ringutils.F90:482-518).
-struct k_bc_wind_b {
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, Box t,
-                                               double *__restrict__ S,
-                                               const double *__restrict__ met) const
-    {
-        const int j = t.i0 + TA(1);
-        const int k = t.j0 + bi.y;
-        if (j > t.i1 || k > t.j1) return;
-        const long N3 = g.N3;
-        const double *mf = S + S_MF * N3;
-        int kp = k;
-        if (k < g.ks) kp = k + g.Nkp;
-        else if (k > g.ke) kp = k - g.Nkp;
-        for (int n = NL0(1); n <= NL1(1); n++) {
-            const int ig = g.ie + n;
-            const long s = IX(g, ig, j, kp);
-            double B[3];
-            cell_b(g, met, s, mf[s], mf[N3 + s], mf[2 * N3 + s], mf[s + 1], mf[N3 + s + g.P], mf[2 * N3 + s + g.PP], B);
-            const long d = IX(g, ig, j, k);
-            for (int x = 0; x < 3; x++) S[(S_B + x) * N3 + d] = B[x];
-        }
-    }
-};
-
 // DivB partial sums (gridutils.F90:717-770)
 __global__ void k_divb(Geo g, Box ab, const double *__restrict__ mf, const double *__restrict__ bg,
                        int useBG, double *__restrict__ part)
@@ -952,118 +601,6 @@ void launch_calc_dt(hipStream_t s, const Geo &g, const MParm &m, const Box &dtb,
     case 1: launch_f<k_calc_dt<false, true>>(tgrid(t), dim3(BX, BY), s, g, m, t, clk, S, met, bg); break;
     case 2: launch_f<k_calc_dt<true, false>>(tgrid(t), dim3(BX, BY), s, g, m, t, clk, S, met, bg); break;
     default: launch_f<k_calc_dt<true, true>>(tgrid(t), dim3(BX, BY), s, g, m, t, clk, S, met, bg); break;
-    }
-}
-
-void launch_finalize(hipStream_t s, const MParm &m, Clock *clk, int mode)
-{
-    launch_f<k_finalize>(dim3(1), dim3(64), s, m, clk, mode);
-}
-
-void launch_bflux2fld(hipStream_t s, const Geo &g, const Box &cb, const Box &skip, const double *mf,
-                      double *B, const double *met)
-{
-    const Tile t = tile_of(cb, 1);
-    launch_f<k_bflux2fld>(tgrid(t), dim3(BX, BY), s, g, t, skip, mf, B, met);
-}
-
-void launch_bflux2fld_ghosts(hipStream_t s, const Geo &g, const double *mf, double *B, const double *met)
-{
-    GhostBoxes gb;
-    const Box bx[6] = {
-        {g.isg, g.ieg, g.jsg, g.jeg, g.ksg, g.ks - 1},      // k ghosts, all i, j
-        {g.isg, g.ieg, g.jsg, g.jeg, g.ke + 1, g.keg},
-        {g.isg, g.ieg, g.jsg, g.js - 1, g.ks, g.ke},        // j ghosts, active k
-        {g.isg, g.ieg, g.je + 1, g.jeg, g.ks, g.ke},
-        {g.isg, g.is - 1, g.js, g.je, g.ks, g.ke},          // i ghosts, active j, k
-        {g.ie + 1, g.ieg, g.js, g.je, g.ks, g.ke}};
-    int tot = 0;
-    for (int q = 0; q < 6; q++) {
-        gb.b[q] = bx[q];
-        gb.start[q] = tot;
-        gb.iw[q] = (q >= 4) ? 4 : BX;
-        const int jw = BX * BY / gb.iw[q];
-        gb.n0[q] = (bx[q].i1 - bx[q].i0 + gb.iw[q]) / gb.iw[q];
-        gb.n1[q] = (bx[q].j1 - bx[q].j0 + jw) / jw;
-        tot += gb.n0[q] * gb.n1[q] * (bx[q].k1 - bx[q].k0 + 1);
-    }
-    gb.start[6] = tot;
-    gb.n = 6;
-    launch_f<k_bflux2fld_ghosts>(dim3((unsigned)tot), dim3(BX, BY), s, g, gb, mf, B, met);
-}
-
-static inline dim3 grid2(const Box &t) { return dim3((unsigned)((t.i1 - t.i0 + 64) / 64), (unsigned)(t.j1 - t.j0 + 1)); }
-
-// Both periodic sides of one axis in one launch: each reads only interior
-// cells and faces and writes its own ghosts, so the two commute.  Blocks
-// with z = 0 run the low side, z = 1 the high side.
-template <int AX>
-struct k_bc_periodic_pair {
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, Box t, double *__restrict__ S) const
-    {
-        if (bi.z == 0) k_bc_periodic<2 * AX>{}(bi, g, t, S);
-        else k_bc_periodic<2 * AX + 1>{}(make_uint3(bi.x, bi.y, 0), g, t, S);
-    }
-};
-
-void launch_bc_periodic_pair(hipStream_t s, int ax, const Geo &g, double *S)
-{
-    Box t;   // the transverse boxes of launch_bc's periodic sides
-    if (ax == 0) { t.i0 = g.jsg; t.i1 = g.jeg + 1; t.j0 = g.ksg; t.j1 = g.keg + 1; }
-    else if (ax == 1) { t.i0 = g.isg; t.i1 = g.ieg + 1; t.j0 = g.ksg; t.j1 = g.keg + 1; }
-    else { t.i0 = g.isg; t.i1 = g.ieg + 1; t.j0 = g.jsg; t.j1 = g.jeg + 1; }
-    t.k0 = t.k1 = 0;
-    dim3 gr = grid2(t), bl(64);
-    if (ax == 0) gr.x = (unsigned)((t.i1 - t.i0 + 16) / 16);   // 16 points x 4 layers per block
-    gr.z = 2;
-    if (ax == 0) launch_f<k_bc_periodic_pair<0>>(gr, bl, s, g, t, S);
-    else if (ax == 1) launch_f<k_bc_periodic_pair<1>>(gr, bl, s, g, t, S);
-    else launch_f<k_bc_periodic_pair<2>>(gr, bl, s, g, t, S);
-}
-
-void launch_bc(hipStream_t s, int side, int kind, const Geo &g, const MParm &m, const Clock *clk,
-               const WindDev *w, double *S, const double *met, bool ghostB)
-{
-    // Transverse boxes (a,b) per side as in the reference loops
-    Box t;
-    const bool pi = (kind == 0);
-    if (side <= 1) { t.i0 = g.jsg; t.i1 = g.jeg + (pi ? 1 : 0); t.j0 = g.ksg; t.j1 = g.keg + (pi ? 1 : 0); }
-    else if (side <= 3) { t.i0 = g.isg; t.i1 = g.ieg + (pi ? 1 : 0); t.j0 = g.ksg; t.j1 = g.keg + (pi ? 1 : 0); }
-    else { t.i0 = g.isg; t.i1 = g.ieg + (pi ? 1 : 0); t.j0 = g.jsg; t.j1 = g.jeg + (pi ? 1 : 0); }
-    t.k0 = t.k1 = 0;
-    dim3 gr = grid2(t), bl(64);
-    if (side <= 1) gr.x = (unsigned)((t.i1 - t.i0 + 16) / 16);   // 16 points x 4 layers per block
-    if (kind == 0) {
-        switch (side) {
-        case 0: launch_f<k_bc_periodic<0>>(gr, bl, s, g, t, S); break;
-        case 1: launch_f<k_bc_periodic<1>>(gr, bl, s, g, t, S); break;
-        case 2: launch_f<k_bc_periodic<2>>(gr, bl, s, g, t, S); break;
-        case 3: launch_f<k_bc_periodic<3>>(gr, bl, s, g, t, S); break;
-        case 4: launch_f<k_bc_periodic<4>>(gr, bl, s, g, t, S); break;
-        default: launch_f<k_bc_periodic<5>>(gr, bl, s, g, t, S); break;
-        }
-    } else if (kind == 1) {
-        switch (side) {
-        case 0: launch_f<k_bc_copy<0, 1>>(gr, bl, s, g, t, S, met); break;
-        case 1: launch_f<k_bc_copy<1, 1>>(gr, bl, s, g, t, S, met); break;
-        case 2: launch_f<k_bc_copy<2, 1>>(gr, bl, s, g, t, S, met); break;
-        case 3: launch_f<k_bc_copy<3, 1>>(gr, bl, s, g, t, S, met); break;
-        case 4: launch_f<k_bc_copy<4, 1>>(gr, bl, s, g, t, S, met); break;
-        default: launch_f<k_bc_copy<5, 1>>(gr, bl, s, g, t, S, met); break;
-        }
-    } else if (kind == 2) {
-        launch_f<k_bc_copy<0, 2>>(gr, bl, s, g, t, S, met);
-    } else if (kind == 3) {
-        launch_f<k_bc_copy<1, 3>>(gr, bl, s, g, t, S, met);
-    } else if (kind == 4) {
-        Box tw = t;
-        tw.i1 = g.jeg + 1; tw.j1 = g.keg + 1;
-        dim3 gw = grid2(tw);
-        gw.x = (unsigned)((tw.i1 - tw.i0 + 16) / 16);
-        launch_f<k_bc_wind>(gw, bl, s, g, m, tw, clk, *w, S, met);
-        // ghost-cell B of the wind BC (wind.F90:338-348); skipped when a
-        // bFlux2Fld over every ghost cell follows, which overwrites it
-        if (ghostB) launch_f<k_bc_wind_b>(gr, bl, s, g, t, S, met);
     }
 }
 
