@@ -461,7 +461,8 @@ def main():
     kernels = {k: {"ms_total": v[0], "launches": v[1],
                    "ms_per_launch": (v[0] / v[1]) if v[1] else None} for k, v in kt.items()}
     flux = kt["flux"]
-    flux_ms = flux[0] / flux[1]
+    # per direction: a step's three directions may share one launch
+    flux_ms = flux[0] / (3 * args.profile_steps)
     faces = ((N[0] + 1) * N[1] * N[2] + N[0] * (N[1] + 1) * N[2] + N[0] * N[1] * (N[2] + 1)) / 3.0
     flux_gbs = FLUX_BYTES_PER_FACE * faces / (flux_ms * 1e-3) / 1e9
     step_gbs = STEP_BYTES_PER_CELL * value / 1e9

@@ -13,7 +13,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 LIB = os.path.join(HERE, "libgamhip.so")
-SOURCES = ["gam_api.hip", "gam_step.hip", "gam_flux_i.hip", "gam_flux_j.hip", "gam_flux_k.hip", "gam_emf.hip", "gam_bc.hip", "gam_grid.hip", "gam_adj.hip", "gam_noalloc.hip"]
+SOURCES = ["gam_api.hip", "gam_step.hip", "gam_flux_i.hip", "gam_flux_j.hip", "gam_flux_k.hip", "gam_flux3.hip", "gam_emf.hip", "gam_bc.hip", "gam_grid.hip", "gam_adj.hip", "gam_noalloc.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

@@ -594,6 +594,86 @@ static void tune_mark(gam_ctx *c, int slot)
     hipEventRecord(c->tev[c->ntev++], c->stream);
 }
 
+static void flux_boxes(const Geo &g, Box *fb)
+{   // active faces of each direction
+    for (int d = 0; d < 3; d++) fb[d] = act_box(g);
+    fb[0].i1++;
+    fb[1].j1++;
+    fb[2].k1++;
+}
+
+// The fluxes of every direction and the Mom2Face rim as one launch, if the
+// plan's shapes allow it for them and for the EMFs; false: nothing enqueued.
+// While a slot is tuned its launch stays apart, and so does every launch of
+// an ensemble's members, whose batched grids are long enough without it (and
+// whose branches the batched graph runs side by side).
+static bool enq_fluxes_merged(gam_ctx *c)
+{
+    const int *form = &c->plan.v[TS_FLUX_I];
+    if (c->tune_slot >= 0 || launch_recorder() || !flux3_ok(form) || !emf3_ok(&c->plan.v[TS_EMF_I])) return false;
+    Box fb[3];
+    flux_boxes(c->g, fb);
+    prof_begin(c, KG_FLUX);
+    launch_flux3(c->stream, form, c->g, c->mp, fb, c->H, S_cur(c), c->met, c->bg, c->gflx, c->mflx, c->vf);
+    prof_end(c, KG_FLUX);
+    return true;
+}
+
+// One launch per direction of the fluxes and EMFs.  Inside a captured graph
+// (fork) the j and k fluxes and the EMFs that take their face velocities run
+// on two more streams: the graph then has three branches between the
+// predictor and the update, which the device may overlap.  The launches and
+// their arguments are the same either way.
+static void enq_fluxes_emfs_apart(gam_ctx *c, const Box *eb, double *E)
+{
+    const Geo &g = c->g;
+    const long N3 = g.N3;
+    hipStream_t s = c->stream;
+    double *S = S_cur(c);
+    const bool fork = c->fork && c->mp.doMHD;
+    hipStream_t fs[3] = {s, s, s};   // stream of the flux of direction d and of its EMF
+    if (fork) {
+        order_record(s, c->fev[0], 0);
+        for (int q = 0; q < 2; q++) {
+            order_wait(c->aux[q], c->fev[0], 0);
+            fs[1 + q] = c->aux[q];
+        }
+    }
+    Box fb[3];
+    flux_boxes(g, fb);
+    for (int d = 0; d < 3; d++) {
+        prof_begin(c, KG_FLUX);
+        tune_mark(c, TS_FLUX_I + d);
+        launch_flux(fs[d], d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb[d], c->H, S, c->met, c->bg, c->gflx, c->mflx,
+                    c->vf + (long)3 * d * N3);
+        tune_mark(c, TS_FLUX_I + d);
+        prof_end(c, KG_FLUX);
+    }
+    if (!c->mp.doMHD) return;
+    prof_begin(c, KG_MOM2FACE);
+    launch_vface_rim(s, g, c->H, c->met, c->vf);
+    prof_end(c, KG_MOM2FACE);
+    if (fork) {
+        order_record(s, c->fev[1], 1);
+        for (int q = 0; q < 2; q++) order_wait(c->aux[q], c->fev[1], 1);
+    }
+    for (int eD = 0; eD < 3; eD++) {
+        // edge direction eD takes the face velocities along dT1
+        const int dT1 = (eD == 0) ? 1 : (eD == 1) ? 2 : 0;
+        prof_begin(c, KG_EMF);
+        tune_mark(c, TS_EMF_I + eD);
+        launch_emf(fs[dT1], eD, c->plan.v[TS_EMF_I + eD], g, c->mp, eb[eD], c->clk, c->H, S,
+                   c->vf + (long)3 * dT1 * N3, c->met, c->bg, E);
+        tune_mark(c, TS_EMF_I + eD);
+        prof_end(c, KG_EMF);
+    }
+    if (fork)
+        for (int q = 0; q < 2; q++) {
+            order_record(c->aux[q], c->fev[2 + q], 2 + q);
+            order_wait(s, c->fev[2 + q], 2 + q);
+        }
+}
+
 // AdvanceMHD on the device (mhdgroup.F90:16-76); swaps State/oState.
 static void enq_advance(gam_ctx *c, int finmode)
 {
@@ -610,58 +690,16 @@ static void enq_advance(gam_ctx *c, int finmode)
     tune_mark(c, TS_PREDICT);
     prof_end(c, KG_PREDICT);
 
-    // interface fluxes (CalcStress), with Mom2Face of the same faces; the
-    // EMFs do not depend on the fluxes, so they run after them.  Inside a
-    // captured graph (fork) the j and k fluxes and the EMFs that take their
-    // face velocities run on two more streams: the graph then has three
-    // branches between the predictor and the update, which the device may
-    // overlap.  The launches and their arguments are the same either way.
-    const bool fork = c->fork && c->mp.doMHD;
-    hipStream_t fs[3] = {s, s, s};   // stream of the flux of direction d and of its EMF
-    if (fork) {
-        order_record(s, c->fev[0], 0);
-        for (int q = 0; q < 2; q++) {
-            order_wait(c->aux[q], c->fev[0], 0);
-            fs[1 + q] = c->aux[q];
-        }
-    }
-    for (int d = 0; d < 3; d++) {
-        Box fb = act_box(g);
-        if (d == 0) fb.i1 += 1; else if (d == 1) fb.j1 += 1; else fb.k1 += 1;
-        prof_begin(c, KG_FLUX);
-        tune_mark(c, TS_FLUX_I + d);
-        launch_flux(fs[d], d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb, c->H, S, c->met, c->bg, c->gflx, c->mflx,
-                    c->vf + (long)3 * d * N3);
-        tune_mark(c, TS_FLUX_I + d);
-        prof_end(c, KG_FLUX);
-    }
+    // interface fluxes (CalcStress), with Mom2Face of the same faces and of
+    // the rim the EMF stencils read (fields.F90:119-175); the EMFs do not
+    // depend on the fluxes, so they run after them
     Box eb[3];
     edge_boxes(g, eb);
-    if (c->mp.doMHD) {
-        // Mom2Face on the rest of the ranges the EMF stencils read
-        // (fields.F90:119-175)
-        prof_begin(c, KG_MOM2FACE);
-        launch_vface_rim(s, g, c->H, c->met, c->vf);
-        prof_end(c, KG_MOM2FACE);
-        if (fork) {
-            order_record(s, c->fev[1], 1);
-            for (int q = 0; q < 2; q++) order_wait(c->aux[q], c->fev[1], 1);
-        }
-        for (int eD = 0; eD < 3; eD++) {
-            // edge direction eD takes the face velocities along dT1
-            const int dT1 = (eD == 0) ? 1 : (eD == 1) ? 2 : 0;
-            prof_begin(c, KG_EMF);
-            tune_mark(c, TS_EMF_I + eD);
-            launch_emf(fs[dT1], eD, c->plan.v[TS_EMF_I + eD], g, c->mp, eb[eD], c->clk, c->H, S,
-                       c->vf + (long)3 * dT1 * N3, c->met, c->bg, Sn + S_E * N3);
-            tune_mark(c, TS_EMF_I + eD);
-            prof_end(c, KG_EMF);
-        }
-        if (fork)
-            for (int q = 0; q < 2; q++) {
-                order_record(c->aux[q], c->fev[2 + q], 2 + q);
-                order_wait(s, c->fev[2 + q], 2 + q);
-            }
+    if (!enq_fluxes_merged(c)) enq_fluxes_emfs_apart(c, eb, Sn + S_E * N3);
+    else if (c->mp.doMHD) {
+        prof_begin(c, KG_EMF);
+        launch_emf3(s, &c->plan.v[TS_EMF_I], g, c->mp, eb, c->clk, c->H, S, c->vf, c->met, c->bg, Sn + S_E * N3);
+        prof_end(c, KG_EMF);
     }
 
     prof_begin(c, KG_UPDATE);
@@ -691,12 +729,12 @@ static void enq_intermediates(gam_ctx *c)
     hipStream_t s = c->stream;
     double *S = S_cur(c), *O = S_old(c);
     launch_predict(s, c->plan.v[TS_PREDICT], g, c->mp, face_box(g), c->clk, S, O, c->met, c->H);
-    for (int d = 0; d < 3; d++) {
-        Box fb = act_box(g);
-        if (d == 0) fb.i1 += 1; else if (d == 1) fb.j1 += 1; else fb.k1 += 1;
-        launch_flux(s, d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb, c->H, S, c->met, c->bg, c->gflx, c->mflx,
+    if (enq_fluxes_merged(c)) return;
+    Box fb[3];
+    flux_boxes(g, fb);
+    for (int d = 0; d < 3; d++)
+        launch_flux(s, d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb[d], c->H, S, c->met, c->bg, c->gflx, c->mflx,
                     c->vf + (long)3 * d * N3);
-    }
     if (c->mp.doMHD) launch_vface_rim(s, g, c->H, c->met, c->vf);
 }
 

@@ -30,11 +30,10 @@ __device__ __forceinline__ void edge_lr(const Geo &g, const MParm &m, long c,
     recon_lr_w<RM>(m.pdmb, gam_rcp(wsum8([&](int n) { return A[n]; })), nq, q, bL, bR);
 }
 
-template <int ED, int RM, bool BG, bool BORIS, int NTH = BX * BY>
-struct k_emf {
-    static constexpr int NT = NTH;
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m,
-                                               Tile b, const Clock *clk,
+template <int ED, int RM, bool BG, bool BORIS>
+struct edge_emf {
+    __device__ __forceinline__ void operator()(int w, const Geo &g, const MParm &m,
+                                               const Tile &b, const Clock *clk,
                                                const double *__restrict__ H,
                                                const double *__restrict__ S,
                                                const double *__restrict__ Vf,
@@ -42,7 +41,8 @@ struct k_emf {
                                                const double *__restrict__ bg,
                                                double *__restrict__ E) const
     {
-        TILE_IJK(b);
+        int i, j, k;
+        if (!tile_point(b, w, i, j, k)) return;
         constexpr int T1 = (ED == 0) ? 1 : (ED == 1) ? 2 : 0;
         constexpr int T2 = (ED == 0) ? 2 : (ED == 1) ? 0 : 1;
         // getNormalPlane (metric.F90:151-167)
@@ -99,6 +99,89 @@ struct k_emf {
         E[ED * N3 + c] = e * edge;
     }
 };
+
+template <int ED, int RM, bool BG, bool BORIS, int NTH = BX * BY>
+struct k_emf {
+    static constexpr int NT = NTH;
+    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m,
+                                               Tile b, const Clock *clk,
+                                               const double *__restrict__ H,
+                                               const double *__restrict__ S,
+                                               const double *__restrict__ Vf,
+                                               const double *__restrict__ met,
+                                               const double *__restrict__ bg,
+                                               double *__restrict__ E) const
+    {
+        edge_emf<ED, RM, BG, BORIS>{}((int)bi.x, g, m, b, clk, H, S, Vf, met, bg, E);
+    }
+};
+
+// The three edge directions in one launch, one range of workgroups after
+// another.  Vf: the face velocities of all three directions; direction eD
+// takes those of the faces along dT1.
+struct Emf3 {
+    Tile t[3];
+    int start[2];     // first workgroup of edge direction 1, of direction 2
+};
+
+template <int RM, bool BG, bool BORIS>
+struct k_emf3 {
+    static constexpr int NT = BX * BY;
+    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, const Emf3 &f, const Clock *clk,
+                                               const double *__restrict__ H,
+                                               const double *__restrict__ S,
+                                               const double *__restrict__ Vf,
+                                               const double *__restrict__ met,
+                                               const double *__restrict__ bg,
+                                               double *__restrict__ E) const
+    {
+        const int w = (int)bi.x;
+        if (w < f.start[0])
+            edge_emf<0, RM, BG, BORIS>{}(w, g, m, f.t[0], clk, H, S, Vf + 3 * g.N3, met, bg, E);
+        else if (w < f.start[1])
+            edge_emf<1, RM, BG, BORIS>{}(w - f.start[0], g, m, f.t[1], clk, H, S, Vf + 6 * g.N3, met, bg, E);
+        else
+            edge_emf<2, RM, BG, BORIS>{}(w - f.start[1], g, m, f.t[2], clk, H, S, Vf, met, bg, E);
+    }
+};
+
+template <int RM, bool BG, bool BO>
+static void emf3_t(hipStream_t s, const int *plan, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
+                   const double *H, const double *S, const double *Vf, const double *met, const double *bg,
+                   double *E)
+{
+    Emf3 f;
+    int tot = 0;
+    for (int d = 0; d < 3; d++) {
+        f.t[d] = tile_of(b[d], plan_ax(plan[d]));
+        tot += (int)tgrid(f.t[d]).x;
+        if (d < 2) f.start[d] = tot;
+    }
+    launch_f<k_emf3<RM, BG, BO>>(dim3((unsigned)tot), dim3(BX, BY), s, g, m, f, clk, H, S, Vf, met, bg, E);
+}
+
+bool emf3_ok(const int *plan)
+{
+    for (int d = 0; d < 3; d++)
+        if (plan_chunk(plan[d]) != BX * BY) return false;
+    return true;
+}
+
+void launch_emf3(hipStream_t s, const int *plan, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
+                 const double *H, const double *S, const double *Vf, const double *met, const double *bg, double *E)
+{
+    const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
+    switch (sel) {
+    case 0: emf3_t<0, false, false>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 1: emf3_t<0, false, true>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 2: emf3_t<0, true, false>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 3: emf3_t<0, true, true>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 4: emf3_t<1, false, false>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 5: emf3_t<1, false, true>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 6: emf3_t<1, true, false>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    default: emf3_t<1, true, true>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    }
+}
 
 template <int ED, int RM, bool BG, bool BO>
 static void emf_t(hipStream_t s, int plan, const Geo &g, const MParm &m, const Box &b, const Clock *clk,

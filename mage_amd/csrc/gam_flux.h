@@ -187,16 +187,19 @@ struct FluxTile {
     FastDiv q7;                   // D = 0: by ni + 7
 };
 
+#define FLUX_LDS ((8 + 3) * 376 > (8 + 7) * 32 * 6 + (8 + 3) * 32 * 5 ? (8 + 3) * 376 : (8 + 7) * 32 * 6 + (8 + 3) * 32 * 5)
+
 template <int D, int RM, bool BG, bool BORIS>
-struct k_flux_t {
-    static constexpr int NT = 256;
+struct flux_tile {
     static constexpr int TI = 32, TA = 8;
     static constexpr int NE = D == 0 ? 376 : (TA + 7) * TI;   // cells staged (D = 0: at most)
     static constexpr int NL = D == 0 ? 376 : (TA + 3) * TI;   // limiter cells staged
     static constexpr int SN = D == 0 ? 1 : TI;                // LDS step of the stencil
     static constexpr int LO = D == 0 ? 0 : 2 * TI;            // first staged cell with a limiter entry
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, FluxTile t,
-                                               const double *__restrict__ H,
+    static_assert(6 * NE + 5 * NL <= FLUX_LDS, "LDS planes");
+    // workgroup w of the launch's range for this direction; lds: FLUX_LDS doubles
+    __device__ __forceinline__ void operator()(double *lds, int w, const Geo &g, const MParm &m,
+                                               const FluxTile &t, const double *__restrict__ H,
                                                const double *__restrict__ S,
                                                const double *__restrict__ met,
                                                const double *__restrict__ bg,
@@ -204,8 +207,10 @@ struct k_flux_t {
                                                double *__restrict__ mflx,
                                                double *__restrict__ Vf) const
     {
-        __shared__ double sv[NE], sq[5][NE], sl[5][NL];
-        const int L = xcd_tile((int)bi.x, t.t.xs);
+        double *sv = lds;                                     // volumes
+        auto sq = [&](int n) { return lds + (1 + n) * NE; };  // weighted values
+        auto sl = [&](int n) { return lds + 6 * NE + n * NL; };   // limiter values
+        const int L = xcd_tile(w, t.t.xs);
         if (L >= t.t.nb) return;                   // whole workgroup
         const int tid = (int)(threadIdx.x + BX * threadIdx.y);
         const long N3 = g.N3;
@@ -287,10 +292,10 @@ struct k_flux_t {
             if (put[q]) {
                 sv[e] = v[q];
 #pragma unroll
-                for (int n = 0; n < 5; n++) sq[n][e] = wq[q][n];
+                for (int n = 0; n < 5; n++) sq(n)[e] = wq[q][n];
                 if (lim(e))
 #pragma unroll
-                    for (int n = 0; n < 5; n++) sl[n][e - LO] = wl[q][n];
+                    for (int n = 0; n < 5; n++) sl(n)[e - LO] = wl[q][n];
             }
         }
         __syncthreads();
@@ -299,9 +304,9 @@ struct k_flux_t {
         auto recon = [&](int n, double &l, double &r, double *vel) {
             double qv[8], nq[4];
 #pragma unroll
-            for (int x = 0; x < 8; x++) qv[x] = sq[n][f0 + x * SN];
+            for (int x = 0; x < 8; x++) qv[x] = sq(n)[f0 + x * SN];
 #pragma unroll
-            for (int x = 0; x < 4; x++) nq[x] = sl[n][f0 + (D == 0 ? x + 2 : x * SN)];
+            for (int x = 0; x < 4; x++) nq[x] = sl(n)[f0 + (D == 0 ? x + 2 : x * SN)];
             recon_lr_w<RM>(m.pdmb, rVi, nq, qv, l, r);
             if (vel) *vel = mom2face(qv, Vi, rVi);
             // hold the two results here: their use lies inside the branch on
@@ -324,10 +329,10 @@ struct k_flux_t {
                 const int e = tid + 256 * q;
                 if (put[q]) {
 #pragma unroll
-                    for (int x = 0; x < 3; x++) sq[x][e] = v[q] * bq[q][x];
+                    for (int x = 0; x < 3; x++) sq(x)[e] = v[q] * bq[q][x];
                     if (lim(e))
 #pragma unroll
-                        for (int x = 0; x < 3; x++) sl[x][e - LO] = bl[q][x];
+                        for (int x = 0; x < 3; x++) sl(x)[e - LO] = bl[q][x];
                 }
             }
             __syncthreads();
@@ -342,27 +347,53 @@ struct k_flux_t {
     }
 };
 
+template <int D, int RM, bool BG, bool BORIS>
+struct k_flux_t {
+    static constexpr int NT = 256;
+    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, FluxTile t,
+                                               const double *__restrict__ H,
+                                               const double *__restrict__ S,
+                                               const double *__restrict__ met,
+                                               const double *__restrict__ bg,
+                                               double *__restrict__ gflx,
+                                               double *__restrict__ mflx,
+                                               double *__restrict__ Vf) const
+    {
+        __shared__ double lds[FLUX_LDS];
+        flux_tile<D, RM, BG, BORIS>{}(lds, (int)bi.x, g, m, t, H, S, met, bg, gflx, mflx, Vf);
+    }
+};
+
+// The tiles of one direction's faces (box b); alt: the other numbering
+// (PLAN_LDS_D)
+static inline FluxTile flux_tiles(int D, const Box &b, bool alt)
+{
+    FluxTile t;
+    t.t = tile_of(b, D == 0 && alt ? 2 : 1);
+    t.q7 = fast_div((unsigned)t.t.ni + 7);
+    t.byD = alt;
+    t.q1 = t.q2 = t.q7;
+    t.i0 = b.i0;
+    t.i1 = b.i1;
+    t.a0 = t.a1 = t.b0 = 0;
+    if (D != 0) {
+        if (D == 1) { t.a0 = b.j0; t.a1 = b.j1; t.b0 = b.k0; }
+        else { t.a0 = b.k0; t.a1 = b.k1; t.b0 = b.j0; }
+        const int nti = (t.i1 - t.i0 + 32) / 32, nta = (t.a1 - t.a0 + 8) / 8;
+        t.t.nb = nti * nta * (D == 1 ? b.k1 - b.k0 + 1 : b.j1 - b.j0 + 1);
+        t.t.xs = xcd_shift(t.t.nb);
+        t.q1 = fast_div((unsigned)(alt ? nta : nti));
+        t.q2 = fast_div((unsigned)(alt ? nti : nta));
+    }
+    return t;
+}
+
 template <int D, int RM, bool BG, bool BO>
 static void flux_t(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
                    const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
 {
     if (plan_ax(form) >= PLAN_LDS) {
-        const bool alt = form & 1;       // PLAN_LDS_D and its alias
-        FluxTile t;
-        t.t = tile_of(b, D == 0 && alt ? 2 : 1);
-        t.q7 = fast_div((unsigned)t.t.ni + 7);
-        t.byD = alt;
-        if (D != 0) {
-            t.i0 = b.i0;
-            t.i1 = b.i1;
-            if (D == 1) { t.a0 = b.j0; t.a1 = b.j1; t.b0 = b.k0; }
-            else { t.a0 = b.k0; t.a1 = b.k1; t.b0 = b.j0; }
-            const int nti = (t.i1 - t.i0 + 32) / 32, nta = (t.a1 - t.a0 + 8) / 8;
-            t.t.nb = nti * nta * (D == 1 ? b.k1 - b.k0 + 1 : b.j1 - b.j0 + 1);
-            t.t.xs = xcd_shift(t.t.nb);
-            t.q1 = fast_div((unsigned)(alt ? nta : nti));
-            t.q2 = fast_div((unsigned)(alt ? nti : nta));
-        }
+        const FluxTile t = flux_tiles(D, b, form & 1);
         launch_f<k_flux_t<D, RM, BG, BO>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, met, bg, gf, mf, vf);
         return;
     }

@@ -1,0 +1,88 @@
+// gam_flux3.hip -- the interface fluxes of all three directions and the
+// Mom2Face rim in one launch.
+#include "gam_flux.h"
+#include "gam_rim.h"
+
+// The workgroups of the three directions and of the rim one after another
+// (starts are multiples of 8, so each keeps its chunk-to-XCD mapping).  One
+// launch instead of four (or of three graph branches joined by events, whose
+// waits cost more than the overlap gave).  Step with this and k_emf3: 16^3
+// box 0.079 -> 0.037 ms, 64^3 box 0.225 -> 0.195, 48x48x64 shell 0.171 ->
+// 0.142, 96x96x128 0.869 -> 0.850, 256x256x384 15.87 -> 15.88.
+struct Flux3 {
+    FluxTile t[3];
+    RimSet rim;
+    int start[4];     // first workgroup of direction 1, of direction 2, of the rim; the end
+};
+
+template <int RM, bool BG, bool BORIS>
+struct k_flux3 {
+    static constexpr int NT = 256;
+    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, const Flux3 &f,
+                                               const double *__restrict__ H,
+                                               const double *__restrict__ S,
+                                               const double *__restrict__ met,
+                                               const double *__restrict__ bg,
+                                               double *__restrict__ gflx,
+                                               double *__restrict__ mflx,
+                                               double *__restrict__ Vf) const
+    {
+        __shared__ double lds[FLUX_LDS];
+        const int w = (int)bi.x;
+        const long N3 = g.N3;
+        if (w < f.start[0])
+            flux_tile<0, RM, BG, BORIS>{}(lds, w, g, m, f.t[0], H, S, met, bg, gflx, mflx, Vf);
+        else if (w < f.start[1])
+            flux_tile<1, RM, BG, BORIS>{}(lds, w - f.start[0], g, m, f.t[1], H, S, met, bg, gflx, mflx, Vf + 3 * N3);
+        else if (w < f.start[2])
+            flux_tile<2, RM, BG, BORIS>{}(lds, w - f.start[1], g, m, f.t[2], H, S, met, bg, gflx, mflx, Vf + 6 * N3);
+        else
+            vface_rim{}(w - f.start[2], g, f.rim, H, met, Vf);
+    }
+};
+
+template <int RM, bool BG, bool BO>
+static void flux3_t(hipStream_t s, const int *form, const Geo &g, const MParm &m, const Box *b, const double *H,
+                    const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
+{
+    Flux3 f;
+    int tot = 0;
+    for (int d = 0; d < 3; d++) {
+        f.t[d] = flux_tiles(d, b[d], form[d] & 1);
+        tot += (int)tgrid(f.t[d].t).x;
+        f.start[d] = tot;
+    }
+    f.rim = rim_set(g);
+    if (m.doMHD) tot += f.rim.start[6];
+    f.start[3] = tot;
+    launch_f<k_flux3<RM, BG, BO>>(dim3((unsigned)tot), dim3(BX, BY), s, g, m, f, H, S, met, bg, gf, mf, vf);
+}
+
+bool flux3_ok(const int *form)
+{
+    for (int d = 0; d < 3; d++)
+        if (plan_ax(form[d]) < PLAN_LDS) return false;
+    return true;
+}
+
+void launch_flux3(hipStream_t s, const int *form, const Geo &g, const MParm &m, const Box *b, const double *H,
+                  const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
+{
+    const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
+    switch (sel) {
+    case 0: flux3_t<0, false, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
+    case 1: flux3_t<0, false, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
+    case 2: flux3_t<0, true, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
+    case 3: flux3_t<0, true, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
+    case 4: flux3_t<1, false, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
+    case 5: flux3_t<1, false, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
+    case 6: flux3_t<1, true, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
+    default: flux3_t<1, true, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
+    }
+}
+
+void launch_vface_rim(hipStream_t s, const Geo &g, const double *H, const double *met, double *Vf)
+{
+    const RimSet r = rim_set(g);
+    launch_f<k_vface_rim>(dim3((unsigned)r.start[6]), dim3(BX, BY), s, g, r, H, met, Vf);
+}

@@ -46,6 +46,7 @@ struct EnsLaunch {
 // While r is set, the step kernels that this thread would launch are
 // appended to *r instead (nothing is issued); nullptr restores launching.
 void set_launch_recorder(std::vector<EnsLaunch> *r);
+std::vector<EnsLaunch> *launch_recorder();   // r, or nullptr
 // Stream order of a branching step: hipEventRecord(e, s) and
 // hipStreamWaitEvent(s, e) at once, or, while a recorder is set, appended
 // to it as markers naming the event by its index ev.
@@ -94,6 +95,15 @@ void launch_emf(hipStream_t s, int eD, int ax, const Geo &g, const MParm &m, con
 // vf's three planes of direction d
 void launch_flux(hipStream_t s, int d, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
                  const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
+// All three directions (forms of the three slots, face boxes b[3]) and, with
+// MHD, the Mom2Face rim in one launch; flux3_ok: the forms allow it
+bool flux3_ok(const int *form);
+void launch_flux3(hipStream_t s, const int *form, const Geo &g, const MParm &m, const Box *b, const double *H,
+                  const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
+// the three edge directions (plans of the three slots, edge boxes b[3]) in one launch
+bool emf3_ok(const int *plan);
+void launch_emf3(hipStream_t s, const int *plan, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
+                 const double *H, const double *S, const double *Vf, const double *met, const double *bg, double *E);
 // one face direction each, one source file each
 void launch_flux_i(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
                    const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);

@@ -239,7 +239,6 @@ static void launch_ens(hipStream_t s, const void *hdr, const void *rec, unsigned
 }
 
 // Batchable launch: issued at once, or appended to this thread's recorder.
-std::vector<EnsLaunch> *launch_recorder();
 
 template <class F, class... A>
 static void launch_f(dim3 grid, dim3 block, hipStream_t s, A... a)
