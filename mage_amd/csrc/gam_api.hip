@@ -59,6 +59,7 @@ struct gam_ctx {
     double *stage;        // one-plane staging buffer for layout conversion
     double *part;         // reduction partials
     Clock *clk;
+    Clock *hclk;          // pinned host copy of *clk (read_clock)
     double *wind;         // device wind series
     WindDev wd;
     int haveGrid, haveBG, haveWind;
@@ -236,6 +237,7 @@ extern "C" int gam_create(gam_ctx **out, const gam_dims *d, const gam_model *m)
     ALLOC(c->part, 1);
 #undef ALLOC
     if (e == hipSuccess) e = hipMalloc((void **)&c->clk, sizeof(Clock));
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->hclk, sizeof(Clock), hipHostMallocDefault);
     if (e == hipSuccess) {
         Clock ck;
         memset(&ck, 0, sizeof(ck));
@@ -271,6 +273,7 @@ extern "C" int gam_destroy(gam_ctx *c)
     double *bufs[] = {c->st[0], c->st[1], c->H, c->met, c->bg, c->gflx, c->mflx, c->vf, c->stage, c->part, c->wind};
     for (double *b : bufs) if (b) hipFree(b);
     if (c->clk) hipFree(c->clk);
+    if (c->hclk) hipHostFree(c->hclk);
     for (int q = 0; q < (int)(sizeof(c->ev) / sizeof(c->ev[0])); q++) if (c->ev[q]) hipEventDestroy(c->ev[q]);
     for (int q = 0; q < 2 * GAM_TUNE_MAXREPS; q++) if (c->tev[q]) hipEventDestroy(c->tev[q]);
     for (int q = 0; q < 2; q++) if (c->aux[q]) hipStreamDestroy(c->aux[q]);
@@ -282,36 +285,73 @@ extern "C" int gam_destroy(gam_ctx *c)
 }
 
 // ------------------------------------------------------------ transfers
+// The Fortran arrays of a call may sit in host memory or in device memory of
+// the context's GPU.  Device memory of the current GPU is read and written
+// by the layout kernels themselves, every component in one launch; anything
+// else goes through the one-plane staging buffer (hipMemcpyDefault lets the
+// runtime pick the direction).
+static bool on_this_gpu(const void *p)
+{
+    hipPointerAttribute_t at;
+    int dev = -1;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
+        hipGetLastError();   // plain host memory is no error of this call
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == dev;
+}
+
 // Upload ncomp consecutive Fortran planes of (ni,nj,nk) into device planes.
-// The Fortran arrays may sit in host memory or in device memory of the
-// context's GPU (hipMemcpyDefault lets the runtime pick the direction), so
-// a caller holding its state on the GPU (torch tensors) moves nothing over
-// PCIe.
-static int upload(gam_ctx *c, const double *src, int face, int ncomp, double *dst)
+// With sync the caller's array is free for reuse on return; without, once the
+// context's stream has been waited for.
+static int upload(gam_ctx *c, const double *src, int face, int ncomp, double *dst, bool sync = true)
 {
     const Geo &g = c->g;
     const int ni = g.Ni + face, nj = g.Nj + face, nk = g.Nk + face;
     const size_t n = (size_t)ni * nj * nk;
-    for (int q = 0; q < ncomp; q++) {
-        HIPCHK(hipMemcpyAsync(c->stage, src + q * n, n * sizeof(double), hipMemcpyDefault, c->stream));
-        launch_repack(c->stream, 1, g, ni, nj, nk, c->stage, dst + (size_t)q * g.N3);
+    if (on_this_gpu(src)) {
+        launch_repack(c->stream, 1, g, ni, nj, nk, ncomp, src, dst);
         HIPCHK(hipGetLastError());
+    } else {
+        for (int q = 0; q < ncomp; q++) {
+            HIPCHK(hipMemcpyAsync(c->stage, src + q * n, n * sizeof(double), hipMemcpyDefault, c->stream));
+            launch_repack(c->stream, 1, g, ni, nj, nk, 1, c->stage, dst + (size_t)q * g.N3);
+            HIPCHK(hipGetLastError());
+        }
     }
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if (sync) HIPCHK(hipStreamSynchronize(c->stream));
     return GAM_OK;
 }
 
-static int download(gam_ctx *c, const double *src, int face, int ncomp, double *dst)
+// The reverse; host arrays are complete on return, device arrays with sync
+// (else once the stream has been waited for).
+static int download(gam_ctx *c, const double *src, int face, int ncomp, double *dst, bool sync = true)
 {
     const Geo &g = c->g;
     const int ni = g.Ni + face, nj = g.Nj + face, nk = g.Nk + face;
     const size_t n = (size_t)ni * nj * nk;
+    if (on_this_gpu(dst)) {
+        launch_repack(c->stream, 0, g, ni, nj, nk, ncomp, src, dst);
+        HIPCHK(hipGetLastError());
+        if (sync) HIPCHK(hipStreamSynchronize(c->stream));
+        return GAM_OK;
+    }
     for (int q = 0; q < ncomp; q++) {
-        launch_repack(c->stream, 0, g, ni, nj, nk, src + (size_t)q * g.N3, c->stage);
+        launch_repack(c->stream, 0, g, ni, nj, nk, 1, src + (size_t)q * g.N3, c->stage);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(dst + q * n, c->stage, n * sizeof(double), hipMemcpyDefault, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
     }
+    return GAM_OK;
+}
+
+// The device clock as it is once everything enqueued so far has run: one
+// copy to pinned memory behind it and one wait.
+static int read_clock(gam_ctx *c, Clock *ck)
+{
+    HIPCHK(hipMemcpyAsync(c->hclk, c->clk, sizeof(Clock), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    *ck = *c->hclk;
     return GAM_OK;
 }
 
@@ -460,19 +500,18 @@ extern "C" int gam_put_state(gam_ctx *c, int which, const double *Gas, const dou
     if (!S) return fail(GAM_E_ARG, "gam_put_state: which must be GAM_STATE or GAM_OSTATE");
     const long N3 = c->g.N3;
     int rc;
-    if (Gas && (rc = upload(c, Gas, 0, 5, S + S_GAS * N3))) return rc;
-    if (magFlux && (rc = upload(c, magFlux, 1, 3, S + S_MF * N3))) return rc;
-    if (Bxyz && (rc = upload(c, Bxyz, 0, 3, S + S_B * N3))) return rc;
+    if (Gas && (rc = upload(c, Gas, 0, 5, S + S_GAS * N3, false))) return rc;
+    if (magFlux && (rc = upload(c, magFlux, 1, 3, S + S_MF * N3, false))) return rc;
+    if (Bxyz && (rc = upload(c, Bxyz, 0, 3, S + S_B * N3, false))) return rc;
     if (Efld) {
-        if ((rc = upload(c, Efld, 0, 3, S + S_E * N3))) return rc;
+        if ((rc = upload(c, Efld, 0, 3, S + S_E * N3, false))) return rc;
         Box eb[3];
         edge_boxes(c->g, eb);
         launch_mask_e(c->stream, c->g, cell_box(c->g), eb, S + S_E * N3);
-        HIPCHK(hipGetLastError());
     }
     // State%time / oState%time
-    const size_t off = (which == GAM_STATE) ? offsetof(Clock, st) : offsetof(Clock, ost);
-    HIPCHK(hipMemcpyAsync((char *)c->clk + off, &time, sizeof(double), hipMemcpyHostToDevice, c->stream));
+    launch_clock_state(c->stream, c->clk, which == GAM_STATE, time);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
     return GAM_OK;
 }
@@ -493,15 +532,13 @@ extern "C" int gam_get_state(gam_ctx *c, int which, double *Gas, double *magFlux
         return GAM_OK;
     }
     if (!S) return fail(GAM_E_ARG, "gam_get_state: bad selector %d", which);
-    if (Gas && (rc = download(c, S + S_GAS * N3, 0, 5, Gas))) return rc;
-    if (magFlux && (rc = download(c, S + S_MF * N3, 1, 3, magFlux))) return rc;
-    if (Bxyz && (rc = download(c, S + S_B * N3, 0, 3, Bxyz))) return rc;
-    if (Efld && (rc = download(c, S + S_E * N3, 0, 3, Efld))) return rc;
-    if (time) {
-        Clock ck;
-        HIPCHK(hipMemcpy(&ck, c->clk, sizeof(Clock), hipMemcpyDeviceToHost));
-        *time = (which == GAM_STATE) ? ck.st : ck.ost;
-    }
+    if (Gas && (rc = download(c, S + S_GAS * N3, 0, 5, Gas, false))) return rc;
+    if (magFlux && (rc = download(c, S + S_MF * N3, 1, 3, magFlux, false))) return rc;
+    if (Bxyz && (rc = download(c, S + S_B * N3, 0, 3, Bxyz, false))) return rc;
+    if (Efld && (rc = download(c, S + S_E * N3, 0, 3, Efld, false))) return rc;
+    Clock ck;
+    if ((rc = read_clock(c, &ck))) return rc;
+    if (time) *time = (which == GAM_STATE) ? ck.st : ck.ost;
     return GAM_OK;
 }
 
@@ -516,11 +553,8 @@ extern "C" int gam_get_solver(gam_ctx *c, int which, double *out)
 extern "C" int gam_set_time(gam_ctx *c, double t, double dt, int ts)
 {
     if (!c) return fail(GAM_E_ARG, "gam_set_time: NULL context");
-    HIPCHK(hipStreamSynchronize(c->stream));
-    Clock ck;
-    HIPCHK(hipMemcpy(&ck, c->clk, sizeof(Clock), hipMemcpyDeviceToHost));
-    ck.t = t; ck.dt = dt; ck.dtA = dt; ck.ts = ts;
-    HIPCHK(hipMemcpy(c->clk, &ck, sizeof(Clock), hipMemcpyHostToDevice));
+    launch_clock_time(c->stream, c->clk, t, dt, ts);
+    HIPCHK(hipGetLastError());
     return GAM_OK;
 }
 
@@ -552,8 +586,8 @@ extern "C" int gam_get_time(gam_ctx *c, double *t, double *dt, int *ts)
 {
     if (!c) return fail(GAM_E_ARG, "gam_get_time: NULL context");
     Clock ck;
-    HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(&ck, c->clk, sizeof(Clock), hipMemcpyDeviceToHost));
+    int rc = read_clock(c, &ck);
+    if (rc) return rc;
     if (t) *t = ck.t;
     if (dt) *dt = ck.dt;
     if (ts) *ts = ck.ts;
@@ -786,13 +820,6 @@ static int enq_steps(gam_ctx *c, int nsteps)
     return GAM_OK;
 }
 
-static int read_clock(gam_ctx *c, Clock *ck)
-{
-    HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(ck, c->clk, sizeof(Clock), hipMemcpyDeviceToHost));
-    return GAM_OK;
-}
-
 static int status_code(int st)
 {
     if (st >= 2) return fail(GAM_E_DT_DISASTER, "<Timestep too small or no timestep below HUGE>");
@@ -823,7 +850,7 @@ extern "C" int gam_advance_mhd(gam_ctx *c, double dt)
 {
     int rc = check_ready(c, "gam_advance_mhd");
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync((char *)c->clk + offsetof(Clock, dtA), &dt, sizeof(double), hipMemcpyHostToDevice, c->stream));
+    launch_clock_dta(c->stream, c->clk, dt);
     enq_advance(c, FIN_ADVANCE);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));

@@ -116,6 +116,11 @@ void launch_update(hipStream_t s, int ax, const Geo &g, const MParm &m, const Bo
                    double *Sn, const double *gf, const double *mf, const double *met, const double *bg);
 void launch_calc_dt(hipStream_t s, const Geo &g, const MParm &m, const Box &dtb, Clock *clk,
                     const double *S, const double *met, const double *bg);
+// Clock fields set from the host: State%time (st) or oState%time; Model%t,
+// dt, ts; AdvanceMHD's dt
+void launch_clock_state(hipStream_t s, Clock *clk, bool st, double time);
+void launch_clock_time(hipStream_t s, Clock *clk, double t, double dt, int ts);
+void launch_clock_dta(hipStream_t s, Clock *clk, double dt);
 void launch_finalize(hipStream_t s, const MParm &m, Clock *clk, int mode);
 void launch_bflux2fld(hipStream_t s, const Geo &g, const Box &cb, const Box &skip, const double *mf,
                       double *B, const double *met);
@@ -125,7 +130,8 @@ void launch_bcs(hipStream_t s, const int *kind, bool field, int finmode, const G
                 const WindDev &w, double *S, const double *met);
 void launch_divb(hipStream_t s, const Geo &g, const Box &ab, const double *mf, const double *bg,
                  int useBG, double *part, int *nparts);
-void launch_repack(hipStream_t s, int dir_in, const Geo &g, int ni, int nj, int nk,
+// ncomp consecutive Fortran planes of (ni,nj,nk) to (dir_in) or from device planes
+void launch_repack(hipStream_t s, int dir_in, const Geo &g, int ni, int nj, int nk, int ncomp,
                    const double *src, double *dst);
 void launch_mask_e(hipStream_t s, const Geo &g, const Box &all, const Box *eboxes, double *E);
 

@@ -397,33 +397,37 @@ __global__ void k_divb(Geo g, Box ab, const double *__restrict__ mf, const doubl
     if (tid == 0) part[blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)] = red[0];
 }
 
-// Layout conversion between Fortran host arrays and the padded device index
-// space.  src/dst plane of an (ni,nj,nk) Fortran array starting at isg.
-__global__ void k_repack_in(Geo g, int ni, int nj, int nk, const double *__restrict__ src,
-                            double *__restrict__ dst)
+// Layout conversion between Fortran arrays and the padded device index
+// space: planes of an (ni,nj,nk) Fortran array starting at isg, one plane per
+// block y.  (Per plane and with a staging copy each, a 16^3 state took 38
+// launches, 30 copies and 25 waits to put and get.)
+template <bool IN>
+__global__ __launch_bounds__(256) void k_repack(Geo g, int ni, int nj, int nk, FastDiv qi, FastDiv qj,
+                                                const double *__restrict__ src, double *__restrict__ dst)
 {
-    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long tot = (long)ni * nj * nk;
+    const long q = (long)blockIdx.x * 256 + threadIdx.x;
     if (q >= tot) return;
-    const int ii = (int)(q % ni);
-    const long r = q / ni;
-    const int jj = (int)(r % nj);
-    const int kk = (int)(r / nj);
-    dst[IX(g, g.isg + ii, g.jsg + jj, g.ksg + kk)] = src[q];
+    const unsigned r = (unsigned)q / qi, kk = r / qj;
+    const int ii = (int)((unsigned)q - r * (unsigned)ni), jj = (int)(r - kk * (unsigned)nj);
+    const long c = IX(g, g.isg + ii, g.jsg + jj, g.ksg + (int)kk);
+    if (IN) dst[blockIdx.y * g.N3 + c] = src[blockIdx.y * tot + q];
+    else dst[blockIdx.y * tot + q] = src[blockIdx.y * g.N3 + c];
 }
 
-__global__ void k_repack_out(Geo g, int ni, int nj, int nk, const double *__restrict__ src,
-                             double *__restrict__ dst)
+__global__ void k_clock_state(Clock *clk, int st, double time)
 {
-    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long tot = (long)ni * nj * nk;
-    if (q >= tot) return;
-    const int ii = (int)(q % ni);
-    const long r = q / ni;
-    const int jj = (int)(r % nj);
-    const int kk = (int)(r / nj);
-    dst[q] = src[IX(g, g.isg + ii, g.jsg + jj, g.ksg + kk)];
+    if (st) clk->st = time;
+    else clk->ost = time;
 }
+__global__ void k_clock_time(Clock *clk, double t, double dt, int ts)
+{
+    clk->t = t;
+    clk->dt = dt;
+    clk->dtA = dt;
+    clk->ts = ts;
+}
+__global__ void k_clock_dta(Clock *clk, double dt) { clk->dtA = dt; }
 
 // Zero the E entries outside the active EMF boxes (CalcElecField zeroes E
 // before filling the active edges, fields.F90:89).
@@ -545,13 +549,27 @@ void launch_divb(hipStream_t s, const Geo &g, const Box &ab, const double *mf, c
     LAUNCH(k_divb, gr, dim3(BX, BY), s, g, ab, mf, bg, useBG, part);
 }
 
-void launch_repack(hipStream_t s, int dir_in, const Geo &g, int ni, int nj, int nk,
+void launch_repack(hipStream_t s, int dir_in, const Geo &g, int ni, int nj, int nk, int ncomp,
                    const double *src, double *dst)
 {
-    const long tot = (long)ni * nj * nk;
-    dim3 gr((unsigned)((tot + 255) / 256));
-    if (dir_in) LAUNCH(k_repack_in, gr, dim3(256), s, g, ni, nj, nk, src, dst);
-    else LAUNCH(k_repack_out, gr, dim3(256), s, g, ni, nj, nk, src, dst);
+    const long tot = (long)ni * nj * nk;   // a plane: below 2^31 points, as everywhere
+    const dim3 gr((unsigned)((tot + 255) / 256), (unsigned)ncomp);
+    const FastDiv qi = fast_div((unsigned)ni), qj = fast_div((unsigned)nj);
+    if (dir_in) LAUNCH(k_repack<true>, gr, dim3(256), s, g, ni, nj, nk, qi, qj, src, dst);
+    else LAUNCH(k_repack<false>, gr, dim3(256), s, g, ni, nj, nk, qi, qj, src, dst);
+}
+
+void launch_clock_state(hipStream_t s, Clock *clk, bool st, double time)
+{
+    LAUNCH(k_clock_state, dim3(1), dim3(1), s, clk, st ? 1 : 0, time);
+}
+void launch_clock_time(hipStream_t s, Clock *clk, double t, double dt, int ts)
+{
+    LAUNCH(k_clock_time, dim3(1), dim3(1), s, clk, t, dt, ts);
+}
+void launch_clock_dta(hipStream_t s, Clock *clk, double dt)
+{
+    LAUNCH(k_clock_dta, dim3(1), dim3(1), s, clk, dt);
 }
 
 void launch_mask_e(hipStream_t s, const Geo &g, const Box &all, const Box *eboxes, double *E)
