@@ -424,7 +424,7 @@ __device__ __forceinline__ void dt_cell_in(const Geo &g, const MParm &m, long c,
     const long N3 = g.N3;
     for (int v = 0; v < 5; v++) U[v] = S[(S_GAS + v) * N3 + c];
     for (int x = 0; x < 3; x++) B[x] = m.doMHD ? S[(S_B + x) * N3 + c] + (m.doBG ? bg[(B_B0 + x) * N3 + c] : 0.0) : 0.0;
-    dl = dmin(dmin(met[M_DI * N3 + c], met[M_DJ * N3 + c]), met[M_DK * N3 + c]);
+    dl = met[M_DL * N3 + c];
 }
 
 __device__ __forceinline__ void min_pair(double *rv, double *ri, int a, int b)

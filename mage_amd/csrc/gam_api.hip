@@ -355,6 +355,24 @@ static int read_clock(gam_ctx *c, Clock *ck)
     return GAM_OK;
 }
 
+// After new metrics: the plane derived from them, and whether the active
+// faces' triads are orthonormal to rounding (those of Corners2Grid are, to a
+// few 1e-16; the two forms of the fluxes then differ by that much).
+static int derive_metrics(gam_ctx *c)
+{
+    launch_min_length(c->stream, c->g, c->met);
+    unsigned long long *err = (unsigned long long *)c->part, h = 0;
+    HIPCHK(hipMemsetAsync(err, 0, sizeof(h), c->stream));
+    launch_triad_error(c->stream, c->g, c->met, err);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(&h, err, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    double e;
+    memcpy(&e, &h, sizeof(e));
+    c->mp.ortho = e <= 1.0e-14;
+    return GAM_OK;
+}
+
 extern "C" int gam_set_grid(gam_ctx *c, const gam_grid_arrays *a)
 {
     if (!c || !a) return fail(GAM_E_ARG, "gam_set_grid: NULL argument");
@@ -375,6 +393,7 @@ extern "C" int gam_set_grid(gam_ctx *c, const gam_grid_arrays *a)
     if ((rc = upload(c, a->Teb, 1, 12, c->met + M_TEB * N3))) return rc;
     if ((rc = upload(c, a->face, 1, 3, c->met + M_FACE * N3))) return rc;
     if ((rc = upload(c, a->edge, 1, 3, c->met + M_EDGE * N3))) return rc;
+    if ((rc = derive_metrics(c))) return rc;
     c->haveGrid = 1;
     return GAM_OK;
 }
@@ -387,7 +406,7 @@ extern "C" int gam_grid_from_corners(gam_ctx *c, const double *xyz)
     if (rc) return rc;
     launch_grid_from_corners(c->stream, c->g, c->met);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if ((rc = derive_metrics(c))) return rc;
     c->haveGrid = 1;
     return GAM_OK;
 }

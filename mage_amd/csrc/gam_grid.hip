@@ -277,6 +277,53 @@ __global__ void k_teb(Geo g, Box b, double *__restrict__ met)
     met[(M_TEB + C0 + 1 + 4 * DN) * N3 + c] = dyT / dS;
 }
 
+__global__ __launch_bounds__(256) void k_min_length(long n, double *__restrict__ met)
+{
+    const long q = (long)blockIdx.x * 256 + threadIdx.x;
+    if (q < n) met[M_DL * n + q] = dmin(dmin(met[M_DI * n + q], met[M_DJ * n + q]), met[M_DK * n + q]);
+}
+
+void launch_min_length(hipStream_t s, const Geo &g, double *met)
+{
+    hipLaunchKernelGGL(k_min_length, dim3((unsigned)((g.N3 + 255) / 256)), dim3(256), 0, s, g.N3, met);
+}
+
+// How far the face triads are from orthonormal: the largest |T T^t - 1| over
+// the faces of box b (all directions), as the bits of a positive double in
+// *err (0 before; NaN counts as 1).  The flux kernels read only the normals
+// of triads that are orthonormal to rounding.
+__global__ __launch_bounds__(256) void k_triad_error(Geo g, Box b, const double *__restrict__ met,
+                                                     unsigned long long *__restrict__ err)
+{
+    const int i = b.i0 + blockIdx.x * 64 + threadIdx.x;
+    const int j = b.j0 + blockIdx.y * 4 + threadIdx.y;
+    const int k = b.k0 + blockIdx.z;
+    double e = 0.0;
+    if (i <= b.i1 && j <= b.j1) {
+        const long N3 = g.N3, c = IX(g, i, j, k);
+        for (int d = 0; d < 3; d++) {
+            if ((d != 0 && i == b.i1) || (d != 1 && j == b.j1) || (d != 2 && k == b.k1)) continue;
+            double T[9];
+            for (int q = 0; q < 9; q++) T[q] = met[(M_TF + q + 9 * d) * N3 + c];
+            for (int p = 0; p < 3; p++)
+                for (int q = p; q < 3; q++) {
+                    const double x = fabs(T[3 * p] * T[3 * q] + T[3 * p + 1] * T[3 * q + 1] +
+                                          T[3 * p + 2] * T[3 * q + 2] - (p == q ? 1.0 : 0.0));
+                    e = x <= e ? e : (x < 1.0 ? x : 1.0);
+                }
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) e = fmax(e, __shfl_xor(e, off, 64));
+    if ((threadIdx.x & 63) == 0 && e > 0.0) atomicMax(err, (unsigned long long)__double_as_longlong(e));
+}
+
+void launch_triad_error(hipStream_t s, const Geo &g, const double *met, unsigned long long *err)
+{
+    const Box b = {g.is, g.ie + 1, g.js, g.je + 1, g.ks, g.ke + 1};
+    const dim3 gr((unsigned)((b.i1 - b.i0 + 64) / 64), (unsigned)((b.j1 - b.j0 + 4) / 4), (unsigned)(b.k1 - b.k0 + 1));
+    hipLaunchKernelGGL(k_triad_error, gr, dim3(64, 4), 0, s, g, b, met, err);
+}
+
 __global__ void k_fill(long n, double v, double *__restrict__ p)
 {
     const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;

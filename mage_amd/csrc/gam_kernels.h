@@ -137,6 +137,10 @@ void launch_mask_e(hipStream_t s, const Geo &g, const Box &all, const Box *eboxe
 
 // Grid pre-compute (gam_grid.hip)
 void launch_grid_from_corners(hipStream_t s, const Geo &g, double *met);
+// the M_DL plane from di, dj, dk
+void launch_min_length(hipStream_t s, const Geo &g, double *met);
+// largest |T T^t - 1| of the active faces' triads into *err (set to 0 before)
+void launch_triad_error(hipStream_t s, const Geo &g, const double *met, unsigned long long *err);
 void launch_dipole_b0(hipStream_t s, const Geo &g, double M0, const double *met, double *bg,
                       double *scratch9);
 

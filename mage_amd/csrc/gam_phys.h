@@ -148,35 +148,58 @@ __device__ __forceinline__ double mom2face(const double *qv, double Vi, double r
 }
 
 // ---------------------------------------------------------- fluxes
+// Velocity across a face with triad T (N, T1, T2): what T1 and T2 take of it.
+__device__ __forceinline__ void face_tangent(const double *T, const double *W, double *vt)
+{
+    const double t1 = T[3] * W[1] + T[4] * W[2] + T[5] * W[3];
+    const double t2 = T[6] * W[1] + T[7] * W[2] + T[8] * W[3];
+#pragma unroll
+    for (int x = 0; x < 3; x++) vt[x] = T[3 + x] * t1 + T[6 + x] * t2;
+}
+// The same where T is orthonormal: what the normal leaves of it.
+__device__ __forceinline__ void face_tangent_n(const double *N, const double *W, double *vt)
+{
+    const double vn = N[0] * W[1] + N[1] * W[2] + N[2] * W[3];
+#pragma unroll
+    for (int x = 0; x < 3; x++) vt[x] = W[1 + x] - N[x] * vn;
+}
+
 // One side (s = -1 left, +1 right) of the Lyon gas-kinetic flux,
-// GasKinFlux (stress.F90:432-511).  T = face triad (N, T1, T2).
-// 1/sqrt(lam) and sqrt(lam) come from one reciprocal square root of 1/lam.
-__device__ __forceinline__ void gas_kin(double igm1, double s, const double *W, const double *T,
-                                        double *gF, double *dW)
+// GasKinFlux (stress.F90:432-511).  N = face normal, vt = the velocity along
+// the face (face_tangent).  1/sqrt(lam) and sqrt(lam) come from one
+// reciprocal square root of 1/lam.
+__device__ __forceinline__ void gas_kin_vt(double igm1, double s, const double *W, const double *N,
+                                           const double *vt, double *gF, double *dW)
 {
     double d = W[DEN], p = W[PRS], vx = W[1], vy = W[2], vz = W[3];
     double e = 0.5 * d * (vx * vx + vy * vy + vz * vz) + p * igm1;
     double rl, sl;                          // 1/sqrt(lam), sqrt(lam); lam = d / (2 p)
     gam_sqrt_rsqrt(2 * p * gam_rcp(d), rl, sl);
-    double vn = T[0] * vx + T[1] * vy + T[2] * vz;
-    double vt1 = T[3] * vx + T[4] * vy + T[5] * vz;
-    double vt2 = T[6] * vx + T[7] * vy + T[8] * vz;
+    double vn = N[0] * vx + N[1] * vy + N[2] * vz;
     // erfc(s sqrt(lam) vn) and exp(-lam vn^2) from one evaluation
     double ez;
     double vn0 = 0.5 * gam_erfc_exp(s * sl * vn, ez);
     double vn1 = vn * vn0 - 0.5 * s * ez * (rl * GAM_RSQRT_PI);
-    gF[DEN] = gF[DEN] + d * vn1;
+    double dv = d * vn1;
+    gF[DEN] = gF[DEN] + dv;
     gF[ENER] = gF[ENER] + (e + 0.5 * p) * vn1 + 0.5 * p * vn0 * vn;
-    double fn = d * vn * vn1 + p * vn0;
-    double ft1 = d * vt1 * vn1, ft2 = d * vt2 * vn1;
-    gF[MOMX] = gF[MOMX] + (T[0] * fn + T[3] * ft1 + T[6] * ft2);
-    gF[MOMY] = gF[MOMY] + (T[1] * fn + T[4] * ft1 + T[7] * ft2);
-    gF[MOMZ] = gF[MOMZ] + (T[2] * fn + T[5] * ft1 + T[8] * ft2);
+    double fn = dv * vn + p * vn0;
+    gF[MOMX] = gF[MOMX] + (N[0] * fn + dv * vt[0]);
+    gF[MOMY] = gF[MOMY] + (N[1] * fn + dv * vt[1]);
+    gF[MOMZ] = gF[MOMZ] + (N[2] * fn + dv * vt[2]);
     dW[DEN] = dW[DEN] + s * d;
     dW[MOMX] = dW[MOMX] + s * d * vx;
     dW[MOMY] = dW[MOMY] + s * d * vy;
     dW[MOMZ] = dW[MOMZ] + s * d * vz;
     dW[ENER] = dW[ENER] + s * e;
+}
+// with the face triad T (N, T1, T2)
+__device__ __forceinline__ void gas_kin(double igm1, double s, const double *W, const double *T,
+                                        double *gF, double *dW)
+{
+    double vt[3];
+    face_tangent(T, W, vt);
+    gas_kin_vt(igm1, s, W, T, vt, gF, dW);
 }
 
 // One side of the magnetic kinetic flux, MagKinFlux (stress.F90:513-599),

@@ -334,7 +334,7 @@ struct k_update {
                     by = by + ldp(bg + (B_B0 + 1) * N3, oc);
                     bz = bz + ldp(bg + (B_B0 + 2) * N3, oc);
                 }
-                const double dl = dmin(dmin(ldp(met + M_DI * N3, oc), ldp(met + M_DJ * N3, oc)), ldp(met + M_DK * N3, oc));
+                const double dl = ldp(met + M_DL * N3, oc);
                 dtc = cell_dt<BORIS>(m, U, bx, by, bz, dl);
                 if (!(dtc == dtc)) dtc = GAM_HUGE;
             }
@@ -360,7 +360,7 @@ struct k_calc_dt {
             for (int v = 0; v < 5; v++) U[v] = S[(S_GAS + v) * N3 + c];
             double bx = S[(S_B + 0) * N3 + c], by = S[(S_B + 1) * N3 + c], bz = S[(S_B + 2) * N3 + c];
             if (BG) { bx = bx + bg[(B_B0 + 0) * N3 + c]; by = by + bg[(B_B0 + 1) * N3 + c]; bz = bz + bg[(B_B0 + 2) * N3 + c]; }
-            const double dl = dmin(dmin(met[M_DI * N3 + c], met[M_DJ * N3 + c]), met[M_DK * N3 + c]);
+            const double dl = met[M_DL * N3 + c];
             dtc = cell_dt<BORIS>(m, U, bx, by, bz, dl);
             if (!(dtc == dtc)) dtc = GAM_HUGE;
         }
