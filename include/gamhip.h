@@ -228,7 +228,7 @@ int gam_get_solver(gam_ctx *ctx, int which, double *out);
  * launch shapes that give the same results: the chunk tiling of the box's
  * points, value = row order (1 = j fastest, 2 = k fastest, 3 = slabs of 8
  * j-rows) + 8 x chunk extent (0: 256 points per workgroup, 1: 512,
- * 2: 128), and, for the fluxes, the LDS-staged forms: 4 (tiles numbered
+ * 2: 128), and the LDS-staged forms: 4 for the EMFs; for the fluxes 4 (tiles numbered
  * along i first; i fluxes: rows j fastest) and 5 (along the flux direction
  * first; rows k fastest).  For the j and k fluxes 6 and 7 are other names
  * of 4 and 5.

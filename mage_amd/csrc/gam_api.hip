@@ -751,7 +751,7 @@ static void enq_advance(gam_ctx *c, int finmode)
     if (!enq_fluxes_merged(c)) enq_fluxes_emfs_apart(c, eb, Sn + S_E * N3);
     else if (c->mp.doMHD) {
         prof_begin(c, KG_EMF);
-        launch_emf3(s, &c->plan.v[TS_EMF_I], g, c->mp, eb, c->clk, c->H, S, c->vf, c->met, c->bg, Sn + S_E * N3);
+        launch_emf3(s, g, c->mp, eb, c->clk, c->H, S, c->vf, c->met, c->bg, Sn + S_E * N3);
         prof_end(c, KG_EMF);
     }
 

@@ -30,76 +30,6 @@ __device__ __forceinline__ void edge_lr(const Geo &g, const MParm &m, long c,
     recon_lr_w<RM>(m.pdmb, gam_rcp(wsum8([&](int n) { return A[n]; })), nq, q, bL, bR);
 }
 
-template <int ED, int RM, bool BG, bool BORIS>
-struct edge_emf {
-    __device__ __forceinline__ void operator()(int w, const Geo &g, const MParm &m,
-                                               const Tile &b, const Clock *clk,
-                                               const double *__restrict__ H,
-                                               const double *__restrict__ S,
-                                               const double *__restrict__ Vf,
-                                               const double *__restrict__ met,
-                                               const double *__restrict__ bg,
-                                               double *__restrict__ E) const
-    {
-        int i, j, k;
-        if (!tile_point(b, w, i, j, k)) return;
-        constexpr int T1 = (ED == 0) ? 1 : (ED == 1) ? 2 : 0;
-        constexpr int T2 = (ED == 0) ? 2 : (ED == 1) ? 0 : 1;
-        // getNormalPlane (metric.F90:151-167)
-        constexpr int E1 = (ED == 0) ? 1 : 0;
-        constexpr int E2 = (ED == 2) ? 1 : 2;
-        const long N3 = g.N3;
-        const long c = IX(g, i, j, k);
-        const long s2 = STRIDE<T2>(g);
-
-        // GetCornerV (fields.F90:457-517), doVdA
-        double A[8];
-#pragma unroll
-        for (int n = 0; n < 8; n++) A[n] = ldx<T2>(met + (M_FACE + T1) * N3, c, s2, n - 4);
-        const double rdA = gam_rcp(dmax(wsum8([&](int n) { return A[n]; }), GAM_TINY));
-        double vc[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++)
-            vc[d] = wsum8([&](int n) { return A[n] * ldx<T2>(Vf + d * N3, c, s2, n - 4); }) * rdA;
-        const double *Te = met + (long)(M_TE + 9 * ED) * N3 + c;
-        const double v1 = vc[0] * Te[3 * N3] + vc[1] * Te[4 * N3] + vc[2] * Te[5 * N3];
-        const double v2 = vc[0] * Te[6 * N3] + vc[1] * Te[7 * N3] + vc[2] * Te[8 * N3];
-        double vDiff = gam_sqrt(v1 * v1 + v2 * v2);
-
-        // GetCornerD (fields.F90:427-454)
-        const long se1 = STRIDE<E1>(g), se2 = STRIDE<E2>(g);
-        const double *Dh = H + (H_GAS + DEN) * N3;
-        const double Dc = 0.25 * (Dh[c] + Dh[c - se1] + Dh[c - se2] + Dh[c - se1 - se2]);
-
-        // GetCornerB (fields.F90:365-424)
-        const double *mfH = H + H_MF * N3;
-        const double *mfL = m.doLFM ? S + S_MF * N3 : mfH;
-        double bT1L, bT1R, bT2L, bT2R;
-        edge_lr<T1, T2, RM>(g, m, c, met, mfH, mfL, bT1L, bT1R);
-        edge_lr<T2, T1, RM>(g, m, c, met, mfH, mfL, bT2L, bT2R);
-        const double *Tb = met + (long)(M_TEB + 4 * ED) * N3 + c;
-        const double xni = Tb[0], yni = Tb[N3], xnj = Tb[2 * N3], ynj = Tb[3 * N3];
-        const double detT = gam_rcp(xni * ynj - xnj * yni);
-        const double bT1 = 0.5 * (bT1L + bT1R);
-        const double bT2 = 0.5 * (bT2L + bT2R);
-        const double Jd = (bT2R - bT2L) - (bT1R - bT1L);
-        double b1 = detT * (ynj * bT1 - yni * bT2);
-        double b2 = detT * (-(xnj * bT1) + xni * bT2);
-        if (BG) {
-            b1 = b1 + bg[(B_EDGB0 + 0 + 2 * ED) * N3 + c];
-            b2 = b2 + bg[(B_EDGB0 + 1 + 2 * ED) * N3 + c];
-        }
-        const double edge = met[(M_EDGE + ED) * N3 + c];
-        // vA = |b| / sqrt(D), with Boris Ca vA / sqrt(Ca^2 + vA^2)
-        const double bb = b1 * b1 + b2 * b2, Ca2 = m.Ca * m.Ca;
-        const double vA = gam_sqrt(BORIS ? Ca2 * bb * gam_rcp(Ca2 * Dc + bb) : bb * gam_rcp(Dc));
-        vDiff = vDiff + vA;
-        vDiff = dmin(vDiff, m.CFL * edge * gam_rcp(clk->dt));
-        const double e = -(v1 * b2 - v2 * b1) + m.Vd0 * vDiff * Jd;
-        E[ED * N3 + c] = e * edge;
-    }
-};
-
 // The EMF of one edge from its corner velocity vc, corner density Dc and the
 // L/R normal fields of its two face pairs.
 template <int ED, bool BG, bool BORIS>
@@ -130,6 +60,63 @@ __device__ __forceinline__ double edge_value(const MParm &m, const double *vc, d
     return e * edge;
 }
 
+template <int ED, int RM, bool BG, bool BORIS, int NTH = BX * BY>
+struct k_emf {
+    static constexpr int NT = NTH;
+    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m,
+                                               Tile b, const Clock *clk,
+                                               const double *__restrict__ H,
+                                               const double *__restrict__ S,
+                                               const double *__restrict__ Vf,
+                                               const double *__restrict__ met,
+                                               const double *__restrict__ bg,
+                                               double *__restrict__ E) const
+    {
+        int i, j, k;
+        if (!tile_point(b, (int)bi.x, i, j, k)) return;
+        constexpr int T1 = (ED == 0) ? 1 : (ED == 1) ? 2 : 0;
+        constexpr int T2 = (ED == 0) ? 2 : (ED == 1) ? 0 : 1;
+        // getNormalPlane (metric.F90:151-167)
+        constexpr int E1 = (ED == 0) ? 1 : 0;
+        constexpr int E2 = (ED == 2) ? 1 : 2;
+        const long N3 = g.N3;
+        const long c = IX(g, i, j, k);
+        const long s2 = STRIDE<T2>(g);
+
+        // GetCornerV (fields.F90:457-517), doVdA
+        double A[8];
+#pragma unroll
+        for (int n = 0; n < 8; n++) A[n] = ldx<T2>(met + (M_FACE + T1) * N3, c, s2, n - 4);
+        const double rdA = gam_rcp(dmax(wsum8([&](int n) { return A[n]; }), GAM_TINY));
+        double vc[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+            vc[d] = wsum8([&](int n) { return A[n] * ldx<T2>(Vf + d * N3, c, s2, n - 4); }) * rdA;
+        // GetCornerD (fields.F90:427-454)
+        const long se1 = STRIDE<E1>(g), se2 = STRIDE<E2>(g);
+        const double *Dh = H + (H_GAS + DEN) * N3;
+        const double Dc = 0.25 * (Dh[c] + Dh[c - se1] + Dh[c - se2] + Dh[c - se1 - se2]);
+
+        // GetCornerB (fields.F90:365-424)
+        const double *mfH = H + H_MF * N3;
+        const double *mfL = m.doLFM ? S + S_MF * N3 : mfH;
+        double bT1L, bT1R, bT2L, bT2R;
+        edge_lr<T1, T2, RM>(g, m, c, met, mfH, mfL, bT1L, bT1R);
+        edge_lr<T2, T1, RM>(g, m, c, met, mfH, mfL, bT2L, bT2R);
+        double Te[6], Tb[4], b0[2] = {0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 6; q++) Te[q] = met[(M_TE + 9 * ED + 3 + q) * N3 + c];
+#pragma unroll
+        for (int q = 0; q < 4; q++) Tb[q] = met[(M_TEB + 4 * ED + q) * N3 + c];
+        if (BG) {
+            b0[0] = bg[(B_EDGB0 + 0 + 2 * ED) * N3 + c];
+            b0[1] = bg[(B_EDGB0 + 1 + 2 * ED) * N3 + c];
+        }
+        E[ED * N3 + c] = edge_value<ED, BG, BORIS>(m, vc, Dc, bT1L, bT1R, bT2L, bT2R, Te, Tb, b0,
+                                                   met[(M_EDGE + ED) * N3 + c], clk->dt);
+    }
+};
+
 // ====================================================================
 // EMFs with the face stencils in LDS.  A workgroup of 256 threads owns a
 // tile of edges, brings the areas, face velocities and fluxes of every face
@@ -142,6 +129,11 @@ __device__ __forceinline__ double edge_value(const MParm &m, const double *vc, d
 //              stencil plane is across i: the 16 are one 128-byte line).
 // The velocities are weighted and the limiter fluxes divided by their areas
 // once per face staged instead of once per edge and stencil point.
+// Bound by memory traffic: 256x256x384 shell 4.05 ms for the three directions
+// with direct loads (76 to 80 registers, six waves per SIMD waiting on L1),
+// 3.34 ms here (19.7 GB at 5.9 TB/s).  Numbering the tiles so that an XCD's
+// run of 16 is a block of the stencil plane (4 x 4, or 2 x 8) fetches less
+// but took 3.38 to 3.49 ms.
 // ====================================================================
 struct EdgeTile {
     int i0, i1, j0, j1, k0, k1;   // edges
@@ -344,6 +336,22 @@ struct edge_tile {
     }
 };
 
+template <int ED, int RM, bool BG, bool BORIS>
+struct k_emf_t {
+    static constexpr int NT = BX * BY;
+    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, EdgeTile b, const Clock *clk,
+                                               const double *__restrict__ H,
+                                               const double *__restrict__ S,
+                                               const double *__restrict__ Vf,
+                                               const double *__restrict__ met,
+                                               const double *__restrict__ bg,
+                                               double *__restrict__ E) const
+    {
+        __shared__ double lds[edge_geom<ED>::LDS];
+        edge_tile<ED, RM, BG, BORIS>{}(lds, (int)bi.x, g, m, b, clk, H, S, Vf, met, bg, E);
+    }
+};
+
 static inline EdgeTile edge_tiles(int ED, const Box &b)
 {
     EdgeTile t;
@@ -357,22 +365,6 @@ static inline EdgeTile edge_tiles(int ED, const Box &b)
     t.xs = xcd_shift(t.nb);
     return t;
 }
-
-template <int ED, int RM, bool BG, bool BORIS, int NTH = BX * BY>
-struct k_emf {
-    static constexpr int NT = NTH;
-    __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m,
-                                               Tile b, const Clock *clk,
-                                               const double *__restrict__ H,
-                                               const double *__restrict__ S,
-                                               const double *__restrict__ Vf,
-                                               const double *__restrict__ met,
-                                               const double *__restrict__ bg,
-                                               double *__restrict__ E) const
-    {
-        edge_emf<ED, RM, BG, BORIS>{}((int)bi.x, g, m, b, clk, H, S, Vf, met, bg, E);
-    }
-};
 
 // The three edge directions in one launch, one range of workgroups after
 // another.  Vf: the face velocities of all three directions; direction eD
@@ -405,7 +397,7 @@ struct k_emf3 {
 };
 
 template <int RM, bool BG, bool BO>
-static void emf3_t(hipStream_t s, const int *plan, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
+static void emf3_t(hipStream_t s, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
                    const double *H, const double *S, const double *Vf, const double *met, const double *bg,
                    double *E)
 {
@@ -422,23 +414,23 @@ static void emf3_t(hipStream_t s, const int *plan, const Geo &g, const MParm &m,
 bool emf3_ok(const int *plan)
 {
     for (int d = 0; d < 3; d++)
-        if (plan_chunk(plan[d]) != BX * BY) return false;
+        if (plan[d] != PLAN_LDS) return false;
     return true;
 }
 
-void launch_emf3(hipStream_t s, const int *plan, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
+void launch_emf3(hipStream_t s, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
                  const double *H, const double *S, const double *Vf, const double *met, const double *bg, double *E)
 {
     const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
     switch (sel) {
-    case 0: emf3_t<0, false, false>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 1: emf3_t<0, false, true>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 2: emf3_t<0, true, false>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 3: emf3_t<0, true, true>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 4: emf3_t<1, false, false>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 5: emf3_t<1, false, true>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 6: emf3_t<1, true, false>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    default: emf3_t<1, true, true>(s, plan, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 0: emf3_t<0, false, false>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 1: emf3_t<0, false, true>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 2: emf3_t<0, true, false>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 3: emf3_t<0, true, true>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 4: emf3_t<1, false, false>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 5: emf3_t<1, false, true>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 6: emf3_t<1, true, false>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    default: emf3_t<1, true, true>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
     }
 }
 
@@ -447,6 +439,12 @@ static void emf_t(hipStream_t s, int plan, const Geo &g, const MParm &m, const B
                   const double *H, const double *S, const double *Vf, const double *met,
                   const double *bg, double *E)
 {
+    if (plan == PLAN_LDS) {
+        const EdgeTile t = edge_tiles(ED, b);
+        launch_f<k_emf_t<ED, RM, BG, BO>>(dim3(xcd_grid(t.nb, t.xs)), dim3(BX, BY), s, g, m, t, clk, H, S, Vf, met,
+                                          bg, E);
+        return;
+    }
     const int ch = plan_chunk(plan);
     const Tile t = tile_of(b, plan_ax(plan), ch);
     if (ch == 512)

@@ -55,8 +55,8 @@ void order_wait(hipStream_t s, hipEvent_t e, int ev);
 
 // Launch plan: the shape of every tunable launch of the step.  Values
 // 1, 2, 3 are the Tile row orders (ax1: j fastest, k fastest, j-slabs);
-// PLAN_LDS and PLAN_LDS_D select the LDS-staged interface fluxes, tiles
-// numbered along i first or along the flux direction first (i fluxes: rows j
+// PLAN_LDS selects the LDS-staged EMFs; it and PLAN_LDS_D the LDS-staged
+// interface fluxes, tiles numbered along i first or along the flux direction first (i fluxes: rows j
 // or k fastest).  PLAN_ALIAS added to either names the same launch: plans
 // saved when these were separate shapes stay valid.
 enum { TS_PREDICT = 0, TS_EMF_I, TS_EMF_J, TS_EMF_K, TS_FLUX_I, TS_FLUX_J, TS_FLUX_K, TS_UPDATE,
@@ -100,9 +100,10 @@ void launch_flux(hipStream_t s, int d, int form, const Geo &g, const MParm &m, c
 bool flux3_ok(const int *form);
 void launch_flux3(hipStream_t s, const int *form, const Geo &g, const MParm &m, const Box *b, const double *H,
                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
-// the three edge directions (plans of the three slots, edge boxes b[3]) in one launch
+// the three edge directions (edge boxes b[3]) in one launch, if the plans of
+// the three slots allow it
 bool emf3_ok(const int *plan);
-void launch_emf3(hipStream_t s, const int *plan, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
+void launch_emf3(hipStream_t s, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
                  const double *H, const double *S, const double *Vf, const double *met, const double *bg, double *E);
 // one face direction each, one source file each
 void launch_flux_i(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,

@@ -450,9 +450,9 @@ Plan default_plan()
     // pointwise but for the next row and plane: row order 1 takes the
     // 256x256x384 step from 16.28 to 16.09 ms for either (slabs: 3)
     p.v[TS_PREDICT] = 1;
-    p.v[TS_EMF_I] = 3;    // stencils along j and k
-    p.v[TS_EMF_J] = 2;    // along i and k
-    p.v[TS_EMF_K] = 1;    // along i and j
+    p.v[TS_EMF_I] = PLAN_LDS;
+    p.v[TS_EMF_J] = PLAN_LDS;
+    p.v[TS_EMF_K] = PLAN_LDS;
     p.v[TS_FLUX_I] = PLAN_LDS;
     p.v[TS_FLUX_J] = PLAN_LDS;
     p.v[TS_FLUX_K] = PLAN_LDS;
@@ -468,6 +468,7 @@ int plan_candidates(int slot, int *vals)
     // row order x chunk size (256, 512, 128 points per workgroup)
     for (int c = 0; c < 3; c++)
         for (int a = 1; a <= maxax; a++) vals[n++] = a + 8 * c;
+    if (slot >= TS_EMF_I && slot <= TS_EMF_K) vals[n++] = PLAN_LDS;
     if (slot >= TS_FLUX_I && slot <= TS_FLUX_K) {
         vals[n++] = PLAN_LDS;
         vals[n++] = PLAN_LDS_D;
