@@ -108,15 +108,6 @@ __device__ __forceinline__ bool inside(const Box &b, int i, int j, int k)
     return i >= b.i0 && i <= b.i1 && j >= b.j0 && j <= b.j1 && k >= b.k0 && k <= b.k1;
 }
 
-// AB2 weight of the predictor from a step's clock (k_predict)
-__device__ __forceinline__ double ab2_weight(const Clock *clk)
-{
-    const double st = clk->st, dtM = clk->dt;
-    double ost = clk->ost;
-    if (fabs(ost - st) < GAM_TINY) ost = st - dtM;
-    return (0.5 * clk->dtA) / (st - ost);
-}
-
 // ------------------------------------------------------------ objective
 // J = sum_c w_c P_c over cells (P from CellC2P); seeds the adjoint of the
 // final State's gas and writes one partial sum per block.

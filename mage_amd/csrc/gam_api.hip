@@ -92,6 +92,16 @@ struct gam_ctx {
     // gflx, mflx): steps, step and ensemble graph launches, the adjoint's
     // recomputes
     unsigned long itgen;
+    // State buffer as a step leaves it (HalfSrc): gas floored, S_W its
+    // primitives, cell B that of its face fluxes, everywhere.  Two such
+    // states let a step take its half state from them without the predictor.
+    int std[2];
+    int general;         // > 0: steps run the predictor whatever std says
+    int direct;          // recording an ensemble's steps without the predictor
+    // where the last step's half state is (gam_get_state of GAM_HFSTATE): 0 in
+    // H; 1 to be formed from oState and the oState before it, kept in
+    // planes HF_O of H; 2 the same with State at the step's start kept in vf
+    int hf;
     // when set, the next step writes its new State there instead of over
     // oState's buffer, and that buffer becomes State (the adjoint's interval
     // recompute steps through its tape this way)
@@ -126,6 +136,8 @@ static void edge_boxes(const Geo &g, Box *e)
     e[1] = mkbox(g.is, g.ie + 1, g.js, g.je, g.ks, g.ke + 1);
     e[2] = mkbox(g.is, g.ie + 1, g.js, g.je + 1, g.ks, g.ke);
 }
+
+enum { HF_O = H_NPL - 8 };   // gas and face fluxes: 8 planes
 
 static double *S_cur(gam_ctx *c) { return c->st[c->cur]; }
 static double *S_old(gam_ctx *c) { return c->st[1 - c->cur]; }
@@ -355,6 +367,33 @@ static int read_clock(gam_ctx *c, Clock *ck)
     return GAM_OK;
 }
 
+// The buffers of State and oState have been written by something other than
+// a step: their primitives and ghost B need not fit any more.
+static void not_std(gam_ctx *c, bool cur, bool old)
+{
+    if (cur) c->std[c->cur] = 0;
+    if (old) c->std[1 - c->cur] = 0;
+}
+
+// The two states a half state is formed from are kept (hf_keep: what the
+// step about to run takes as oState, or run over by its new State) or still
+// there; hf_flush forms it in H before either goes.
+static int hf_keep(gam_ctx *c, hipStream_t s, const double *O)
+{
+    HIPCHK(hipMemcpyAsync(c->H + (size_t)HF_O * c->g.N3, O, (size_t)8 * c->g.N3 * sizeof(double),
+                          hipMemcpyDeviceToDevice, s));
+    return GAM_OK;
+}
+static int hf_flush(gam_ctx *c)
+{
+    if (!c->hf) return GAM_OK;
+    launch_predict(c->stream, c->plan.v[TS_PREDICT], c->g, c->mp, face_box(c->g), c->clk,
+                   c->hf == 2 ? c->vf : S_old(c), c->H + (size_t)HF_O * c->g.N3, c->met, c->H, 1);
+    HIPCHK(hipGetLastError());
+    c->hf = 0;
+    return GAM_OK;
+}
+
 // After new metrics: the plane derived from them, and whether the active
 // faces' triads are orthonormal to rounding (those of Corners2Grid are, to a
 // few 1e-16; the two forms of the fluxes then differ by that much).
@@ -382,6 +421,8 @@ extern "C" int gam_set_grid(gam_ctx *c, const gam_grid_arrays *a)
         return fail(GAM_E_ARG, "gam_set_grid: every metric array is required");
     const long N3 = c->g.N3;
     int rc;
+    if ((rc = hf_flush(c))) return rc;
+    not_std(c, true, true);
     if ((rc = upload(c, a->xyzcc, 0, 3, c->met + M_XYZCC * N3))) return rc;
     if ((rc = upload(c, a->xfc, 1, 9, c->met + M_XFC * N3))) return rc;
     if ((rc = upload(c, a->di, 0, 1, c->met + M_DI * N3))) return rc;
@@ -402,8 +443,10 @@ extern "C" int gam_grid_from_corners(gam_ctx *c, const double *xyz)
 {
     if (!c || !xyz) return fail(GAM_E_ARG, "gam_grid_from_corners: NULL argument");
     graphs_drop(c);   // launch arguments change
-    int rc = upload(c, xyz, 1, 3, c->met + (long)M_XYZ * c->g.N3);
+    int rc = hf_flush(c);
     if (rc) return rc;
+    not_std(c, true, true);
+    if ((rc = upload(c, xyz, 1, 3, c->met + (long)M_XYZ * c->g.N3))) return rc;
     launch_grid_from_corners(c->stream, c->g, c->met);
     HIPCHK(hipGetLastError());
     if ((rc = derive_metrics(c))) return rc;
@@ -519,6 +562,8 @@ extern "C" int gam_put_state(gam_ctx *c, int which, const double *Gas, const dou
     if (!S) return fail(GAM_E_ARG, "gam_put_state: which must be GAM_STATE or GAM_OSTATE");
     const long N3 = c->g.N3;
     int rc;
+    if (which == GAM_OSTATE && c->hf == 1 && (rc = hf_flush(c))) return rc;
+    not_std(c, which == GAM_STATE, which == GAM_OSTATE);
     if (Gas && (rc = upload(c, Gas, 0, 5, S + S_GAS * N3, false))) return rc;
     if (magFlux && (rc = upload(c, magFlux, 1, 3, S + S_MF * N3, false))) return rc;
     if (Bxyz && (rc = upload(c, Bxyz, 0, 3, S + S_B * N3, false))) return rc;
@@ -543,6 +588,7 @@ extern "C" int gam_get_state(gam_ctx *c, int which, double *Gas, double *magFlux
     double *S = state_ptr(c, which);
     int rc;
     if (which == GAM_HFSTATE) {
+        if ((rc = hf_flush(c))) return rc;
         if (Gas && (rc = download(c, c->H + H_GAS * N3, 0, 5, Gas))) return rc;
         if (magFlux && (rc = download(c, c->H + H_MF * N3, 1, 3, magFlux))) return rc;
         if (Bxyz && (rc = download(c, c->H + H_B * N3, 0, 3, Bxyz))) return rc;
@@ -637,7 +683,7 @@ static void enq_bflux2fld(gam_ctx *c, double *S)
 // context's by default).
 static void enq_bcs(gam_ctx *c, double *S, Clock *clk = nullptr)
 {
-    launch_bcs(c->stream, c->model.bc, false, 0, c->g, c->mp, clk ? clk : c->clk, c->wd, S, c->met);
+    launch_bcs(c->stream, c->model.bc, false, false, 0, c->g, c->mp, clk ? clk : c->clk, c->wd, S, c->met);
 }
 
 // While a slot is being tuned, its launches are bracketed by events.
@@ -660,14 +706,14 @@ static void flux_boxes(const Geo &g, Box *fb)
 // While a slot is tuned its launch stays apart, and so does every launch of
 // an ensemble's members, whose batched grids are long enough without it (and
 // whose branches the batched graph runs side by side).
-static bool enq_fluxes_merged(gam_ctx *c)
+static bool enq_fluxes_merged(gam_ctx *c, const HalfSrc &h)
 {
     const int *form = &c->plan.v[TS_FLUX_I];
     if (c->tune_slot >= 0 || launch_recorder() || !flux3_ok(form) || !emf3_ok(&c->plan.v[TS_EMF_I])) return false;
     Box fb[3];
     flux_boxes(c->g, fb);
     prof_begin(c, KG_FLUX);
-    launch_flux3(c->stream, form, c->g, c->mp, fb, c->H, S_cur(c), c->met, c->bg, c->gflx, c->mflx, c->vf);
+    launch_flux3(c->stream, form, c->g, c->mp, fb, h, c->met, c->bg, c->gflx, c->mflx, c->vf);
     prof_end(c, KG_FLUX);
     return true;
 }
@@ -677,12 +723,11 @@ static bool enq_fluxes_merged(gam_ctx *c)
 // on two more streams: the graph then has three branches between the
 // predictor and the update, which the device may overlap.  The launches and
 // their arguments are the same either way.
-static void enq_fluxes_emfs_apart(gam_ctx *c, const Box *eb, double *E)
+static void enq_fluxes_emfs_apart(gam_ctx *c, const HalfSrc &h, const Box *eb, double *E)
 {
     const Geo &g = c->g;
     const long N3 = g.N3;
     hipStream_t s = c->stream;
-    double *S = S_cur(c);
     const bool fork = c->fork && c->mp.doMHD;
     hipStream_t fs[3] = {s, s, s};   // stream of the flux of direction d and of its EMF
     if (fork) {
@@ -697,14 +742,14 @@ static void enq_fluxes_emfs_apart(gam_ctx *c, const Box *eb, double *E)
     for (int d = 0; d < 3; d++) {
         prof_begin(c, KG_FLUX);
         tune_mark(c, TS_FLUX_I + d);
-        launch_flux(fs[d], d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb[d], c->H, S, c->met, c->bg, c->gflx, c->mflx,
+        launch_flux(fs[d], d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb[d], h, c->met, c->bg, c->gflx, c->mflx,
                     c->vf + (long)3 * d * N3);
         tune_mark(c, TS_FLUX_I + d);
         prof_end(c, KG_FLUX);
     }
     if (!c->mp.doMHD) return;
     prof_begin(c, KG_MOM2FACE);
-    launch_vface_rim(s, g, c->H, c->met, c->vf);
+    launch_vface_rim(s, g, h, c->met, c->vf);
     prof_end(c, KG_MOM2FACE);
     if (fork) {
         order_record(s, c->fev[1], 1);
@@ -715,8 +760,8 @@ static void enq_fluxes_emfs_apart(gam_ctx *c, const Box *eb, double *E)
         const int dT1 = (eD == 0) ? 1 : (eD == 1) ? 2 : 0;
         prof_begin(c, KG_EMF);
         tune_mark(c, TS_EMF_I + eD);
-        launch_emf(fs[dT1], eD, c->plan.v[TS_EMF_I + eD], g, c->mp, eb[eD], c->clk, c->H, S,
-                   c->vf + (long)3 * dT1 * N3, c->met, c->bg, E);
+        launch_emf(fs[dT1], eD, c->plan.v[TS_EMF_I + eD], g, c->mp, eb[eD], h, c->vf + (long)3 * dT1 * N3, c->met,
+                   c->bg, E);
         tune_mark(c, TS_EMF_I + eD);
         prof_end(c, KG_EMF);
     }
@@ -727,31 +772,47 @@ static void enq_fluxes_emfs_apart(gam_ctx *c, const Box *eb, double *E)
         }
 }
 
+// Whether the launch plan's fluxes and EMFs can form the half state themselves.
+static bool plan_direct(const gam_ctx *c)
+{
+    return c->mp.doMHD && flux3_ok(&c->plan.v[TS_FLUX_I]) && emf3_ok(&c->plan.v[TS_EMF_I]);
+}
+// Whether the next step will.
+static bool step_direct(const gam_ctx *c)
+{
+    return plan_direct(c) && (c->direct || (!c->general && !c->snx && c->std[0] && c->std[1]));
+}
+
 // AdvanceMHD on the device (mhdgroup.F90:16-76); swaps State/oState.
-static void enq_advance(gam_ctx *c, int finmode)
+// writeW: leave the new State's primitives (active cells).
+static void enq_advance(gam_ctx *c, int finmode, bool writeW)
 {
     c->itgen++;
     const Geo &g = c->g;
-    const long N3 = g.N3;
     hipStream_t s = c->stream;
     double *S = S_cur(c), *O = S_old(c);
     double *Sn = c->snx ? c->snx : O;   // becomes State
 
-    prof_begin(c, KG_PREDICT);
-    tune_mark(c, TS_PREDICT);
-    launch_predict(s, c->plan.v[TS_PREDICT], g, c->mp, face_box(g), c->clk, S, O, c->met, c->H);
-    tune_mark(c, TS_PREDICT);
-    prof_end(c, KG_PREDICT);
+    const bool direct = step_direct(c);
+    const HalfSrc h = {c->H, S, direct ? O : nullptr, c->clk};
+    if (!direct) {
+        prof_begin(c, KG_PREDICT);
+        tune_mark(c, TS_PREDICT);
+        launch_predict(s, c->plan.v[TS_PREDICT], g, c->mp, face_box(g), c->clk, S, O, c->met, c->H);
+        tune_mark(c, TS_PREDICT);
+        prof_end(c, KG_PREDICT);
+        c->hf = 0;
+    }
 
     // interface fluxes (CalcStress), with Mom2Face of the same faces and of
     // the rim the EMF stencils read (fields.F90:119-175); the EMFs do not
     // depend on the fluxes, so they run after them
     Box eb[3];
     edge_boxes(g, eb);
-    if (!enq_fluxes_merged(c)) enq_fluxes_emfs_apart(c, eb, Sn + S_E * N3);
+    if (!enq_fluxes_merged(c, h)) enq_fluxes_emfs_apart(c, h, eb, Sn + S_E * g.N3);
     else if (c->mp.doMHD) {
         prof_begin(c, KG_EMF);
-        launch_emf3(s, g, c->mp, eb, c->clk, c->H, S, c->vf, c->met, c->bg, Sn + S_E * N3);
+        launch_emf3(s, g, c->mp, eb, h, c->vf, c->met, c->bg, Sn + S_E * g.N3);
         prof_end(c, KG_EMF);
     }
 
@@ -759,7 +820,7 @@ static void enq_advance(gam_ctx *c, int finmode)
     Box ctb = mkbox(g.is, g.ie + 1, g.js, g.je + 1, g.ks, g.ke + 1);
     tune_mark(c, TS_UPDATE);
     launch_update(s, c->plan.v[TS_UPDATE], g, c->mp, face_box(g), ctb, eb, act_box(g), dt_box(g), c->clk,
-                  S, Sn, c->gflx, c->mflx, c->met, c->bg);
+                  S, Sn, writeW, c->gflx, c->mflx, c->met, c->bg);
     tune_mark(c, TS_UPDATE);
     prof_end(c, KG_UPDATE);
 
@@ -769,6 +830,7 @@ static void enq_advance(gam_ctx *c, int finmode)
         c->snx = nullptr;
     }
     c->cur = 1 - c->cur;
+    c->std[c->cur] = 0;      // until the boundary pass
 }
 
 // The forward intermediates of one step as enq_advance computes them
@@ -781,47 +843,64 @@ static void enq_intermediates(gam_ctx *c)
     const long N3 = g.N3;
     hipStream_t s = c->stream;
     double *S = S_cur(c), *O = S_old(c);
+    const HalfSrc h = {c->H, S, nullptr, c->clk};
     launch_predict(s, c->plan.v[TS_PREDICT], g, c->mp, face_box(g), c->clk, S, O, c->met, c->H);
-    if (enq_fluxes_merged(c)) return;
+    if (enq_fluxes_merged(c, h)) return;
     Box fb[3];
     flux_boxes(g, fb);
     for (int d = 0; d < 3; d++)
-        launch_flux(s, d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb[d], c->H, S, c->met, c->bg, c->gflx, c->mflx,
+        launch_flux(s, d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb[d], h, c->met, c->bg, c->gflx, c->mflx,
                     c->vf + (long)3 * d * N3);
-    if (c->mp.doMHD) launch_vface_rim(s, g, c->H, c->met, c->vf);
+    if (c->mp.doMHD) launch_vface_rim(s, g, h, c->met, c->vf);
 }
 
-static void enq_step(gam_ctx *c)
+// keep: hold on to what the step's half state is formed from, if the step
+// does not leave it in H (the last step of a call).
+static int enq_step(gam_ctx *c, bool keep = true)
 {
     const int fin = FIN_ADVANCE | FIN_MODEL | FIN_CALCDT | FIN_SETDT;
     // the boundary launch does the time bookkeeping, unless CalcDT's argmin
-    // is recorded, which needs the new dt before it
-    const bool rec = c->dtrec != nullptr;
-    enq_advance(c, rec ? fin : 0);
+    // is recorded, which needs the new dt before it, or an ensemble's launches
+    const bool apart = c->dtrec || launch_recorder();
+    const bool writeW = c->mp.doMHD && !c->general && !c->snx;
+    const bool direct = step_direct(c);
+    if (direct && keep) {
+        const int rc = hf_keep(c, c->stream, S_old(c));
+        if (rc) return rc;
+    }
+    enq_advance(c, apart ? fin : 0, writeW);
     double *S = S_cur(c);
-    if (rec)
+    if (c->dtrec)
         launch_dt_record(c->stream, c->g, c->mp, dt_box(c->g), S, c->met, c->bg, c->clk, c->dtrec_part, c->dtrec);
     prof_begin(c, KG_BC);
-    launch_bcs(c->stream, c->model.bc, true, rec ? 0 : fin, c->g, c->mp, c->clk, c->wd, S, c->met);
+    launch_bcs(c->stream, c->model.bc, true, writeW, apart ? 0 : fin, c->g, c->mp, c->clk, c->wd, S, c->met);
     prof_end(c, KG_BC);
+    c->std[c->cur] = writeW;
+    c->hf = direct ? 1 : 0;
+    return GAM_OK;
 }
 
 // n steps: pairs as one launch of a graph of two steps (captured on first
 // use for the current State buffer; a step is only kernels, so the graph
 // replays exactly what enq_step launches), the odd one plainly.  While
-// profiling or tuning every step is enqueued plainly (those add events).
+// profiling or tuning every step is enqueued plainly (those add events), and
+// so are the first steps of a state that was put (they run the predictor,
+// the recorded ones do not).
 static int enq_steps(gam_ctx *c, int nsteps)
 {
-    int n = 0;
+    int n = 0, rc;
     const bool graph = !c->prof && c->tune_slot < 0;
+    for (; n < nsteps && plan_direct(c) && !step_direct(c); n++)
+        if ((rc = enq_step(c, false))) return rc;
+    const bool direct = step_direct(c);
     for (; graph && n + 2 <= nsteps; n += 2) {
         const int p = c->cur;
         if (!c->gx[p]) {
             hipGraph_t gr = nullptr;
             HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             c->fork = c->concurrent;
-            enq_step(c);
-            enq_step(c);
+            enq_step(c, false);
+            enq_step(c, false);
             c->fork = 0;
             hipError_t e = hipStreamEndCapture(c->stream, &gr);
             c->cur = p;
@@ -832,10 +911,14 @@ static int enq_steps(gam_ctx *c, int nsteps)
                 return fail(GAM_E_HIP, "step graph capture: %s", hipGetErrorString(e));
             }
         }
+        // the second step of a pair runs over the State the first starts from
+        if (direct && n + 2 == nsteps && (rc = hf_keep(c, c->stream, S_cur(c)))) return rc;
         HIPCHK(hipGraphLaunch(c->gx[p], c->stream));   // two steps: the parity comes back to p
         c->itgen++;
+        c->hf = direct ? 1 : 0;
     }
-    for (; n < nsteps; n++) enq_step(c);
+    for (; n < nsteps; n++)
+        if ((rc = enq_step(c, n + 1 == nsteps))) return rc;
     return GAM_OK;
 }
 
@@ -851,7 +934,12 @@ extern "C" int gam_init_run(gam_ctx *c, double *dt)
     int rc = check_ready(c, "gam_init_run");
     if (rc) return rc;
     double *S = S_cur(c), *O = S_old(c);
-    const size_t bytes = (size_t)S_NPL * c->g.N3 * sizeof(double);
+    const size_t bytes = (size_t)ST_NPL * c->g.N3 * sizeof(double);
+    if (c->hf == 1) {   // the last step's half state outlives its State(n)
+        HIPCHK(hipMemcpyAsync(c->vf, O, (size_t)8 * c->g.N3 * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+        c->hf = 2;
+    }
+    not_std(c, true, true);
     if (c->mp.doMHD) enq_bflux2fld(c, S);
     enq_bcs(c, S);
     HIPCHK(hipMemcpyAsync(O, S, bytes, hipMemcpyDeviceToDevice, c->stream));
@@ -870,7 +958,9 @@ extern "C" int gam_advance_mhd(gam_ctx *c, double dt)
     int rc = check_ready(c, "gam_advance_mhd");
     if (rc) return rc;
     launch_clock_dta(c->stream, c->clk, dt);
-    enq_advance(c, FIN_ADVANCE);
+    c->general++;
+    enq_advance(c, FIN_ADVANCE, false);
+    c->general--;
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
     return prof_flush(c);
@@ -893,6 +983,7 @@ extern "C" int gam_enforce_bcs(gam_ctx *c)
 {
     int rc = check_ready(c, "gam_enforce_bcs");
     if (rc) return rc;
+    not_std(c, true, false);
     enq_bcs(c, S_cur(c));
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -915,7 +1006,7 @@ extern "C" int gam_step(gam_ctx *c, double *dt_next)
 {
     int rc = check_ready(c, "gam_step");
     if (rc) return rc;
-    enq_step(c);
+    if ((rc = enq_step(c))) return rc;
     HIPCHK(hipGetLastError());
     if (!dt_next) return GAM_OK;
     Clock ck;
@@ -952,7 +1043,7 @@ extern "C" int gam_advance_model(gam_ctx *c, double dt, int *nsteps)
     const double target = ck.t + dt;
     int n = 0;
     do {
-        enq_step(c);
+        if ((rc = enq_step(c))) break;
         HIPCHK(hipGetLastError());
         n++;
         if ((rc = read_clock(c, &ck))) break;
@@ -1068,16 +1159,19 @@ struct gam_ens {
     hipStream_t aux[2];              // branch streams of the capture
     hipEvent_t ev[4];                // fork/join events of the capture
     unsigned char *dev;              // headers and argument records
-    std::vector<EnsPhase> ph[2];
-    hipGraph_t graph[2];
-    hipGraphExec_t exec[2];
+    // the recorded step from each State buffer role, r: with the predictor
+    // (ph[r]) and, where every member's plan allows, without (ph[2 + r])
+    int direct;
+    std::vector<EnsPhase> ph[4];
+    hipGraph_t graph[4];
+    hipGraphExec_t exec[4];
 };
 
 extern "C" int gam_ens_destroy(gam_ens *e)
 {
     if (!e) return GAM_OK;
     if (e->stream) hipStreamSynchronize(e->stream);
-    for (int q = 0; q < 2; q++) {
+    for (int q = 0; q < 4; q++) {
         if (e->exec[q]) hipGraphExecDestroy(e->exec[q]);
         if (e->graph[q]) hipGraphDestroy(e->graph[q]);
     }
@@ -1088,8 +1182,7 @@ extern "C" int gam_ens_destroy(gam_ens *e)
     free(e->m);
     free(e->cur0);
     free(e->gen0);
-    e->ph[0].~vector<EnsPhase>();
-    e->ph[1].~vector<EnsPhase>();
+    for (int q = 0; q < 4; q++) e->ph[q].~vector<EnsPhase>();
     free(e);
     return GAM_OK;
 }
@@ -1120,8 +1213,10 @@ extern "C" int gam_ens_create(gam_ens **out, int n, gam_ctx *const *members)
     }
     gam_ens *e = (gam_ens *)calloc(1, sizeof(gam_ens));
     if (!e) return fail(GAM_E_NOMEM, "gam_ens_create: host allocation failed");
-    new (&e->ph[0]) std::vector<EnsPhase>();
-    new (&e->ph[1]) std::vector<EnsPhase>();
+    for (int q = 0; q < 4; q++) new (&e->ph[q]) std::vector<EnsPhase>();
+    e->direct = 1;
+    for (int q = 0; q < n; q++) e->direct = e->direct && plan_direct(members[q]);
+    const int nr = e->direct ? 4 : 2;
     e->n = n;
     e->m = (gam_ctx **)calloc(n, sizeof(gam_ctx *));
     e->cur0 = (int *)calloc(n, sizeof(int));
@@ -1131,25 +1226,31 @@ extern "C" int gam_ens_create(gam_ens **out, int n, gam_ctx *const *members)
         return fail(GAM_E_NOMEM, "gam_ens_create: host allocation failed");
     }
 
-    // record two steps of every member (enq_step swaps its buffers twice)
-    std::vector<std::vector<EnsLaunch>> rec[2];
-    rec[0].resize(n);
-    rec[1].resize(n);
+    // record two steps of every member (enq_step swaps its buffers twice), of
+    // each kind; the context's bookkeeping is put back after them
+    std::vector<std::vector<EnsLaunch>> rec[4];
+    for (int r = 0; r < nr; r++) rec[r].resize(n);
     for (int q = 0; q < n; q++) {
         gam_ctx *c = members[q];
         e->m[q] = c;
         e->cur0[q] = c->cur;
         e->gen0[q] = c->gen;
-        const int prof = c->prof;
+        const int prof = c->prof, std0[2] = {c->std[0], c->std[1]}, hf0 = c->hf;
         c->prof = 0;
         c->fork = c->concurrent;
-        for (int r = 0; r < 2; r++) {
+        for (int r = 0; r < nr; r++) {
+            c->std[0] = c->std[1] = 0;
+            c->direct = r >= 2;
             set_launch_recorder(&rec[r][q]);
-            enq_step(c);
+            enq_step(c, false);
         }
         set_launch_recorder(nullptr);
+        c->direct = 0;
         c->fork = 0;
         c->prof = prof;
+        c->std[0] = std0[0];
+        c->std[1] = std0[1];
+        c->hf = hf0;
     }
     // every member issues the same number of launches per step; at each
     // position the members are grouped by kernel (their launch plans may
@@ -1157,7 +1258,7 @@ extern "C" int gam_ens_create(gam_ens **out, int n, gam_ctx *const *members)
     auto lane_of = [&](int q, hipStream_t st) {
         return st == members[q]->aux[0] ? 1 : st == members[q]->aux[1] ? 2 : 0;
     };
-    for (int r = 0; r < 2; r++)
+    for (int r = 0; r < nr; r++)
         for (int q = 1; q < n; q++) {
             bool same = rec[r][q].size() == rec[r][0].size();
             for (size_t p = 0; same && p < rec[r][0].size(); p++) {
@@ -1178,7 +1279,7 @@ extern "C" int gam_ens_create(gam_ens **out, int n, gam_ctx *const *members)
         memcpy(host.data() + off, p, bytes);
         return off;
     };
-    for (int r = 0; r < 2; r++) {
+    for (int r = 0; r < nr; r++) {
         for (size_t p = 0; p < rec[r][0].size(); p++) {
             const int lane = lane_of(0, rec[r][0][p].stream);
             if (rec[r][0][p].mark) {
@@ -1249,7 +1350,7 @@ extern "C" int gam_ens_create(gam_ens **out, int n, gam_ctx *const *members)
     for (int q = 0; err == hipSuccess && q < 4; q++) err = hipEventCreateWithFlags(&e->ev[q], hipEventDisableTiming);
     if (err == hipSuccess) err = hipMalloc((void **)&e->dev, host.size());
     if (err == hipSuccess) err = hipMemcpy(e->dev, host.data(), host.size(), hipMemcpyHostToDevice);
-    for (int r = 0; err == hipSuccess && r < 2; r++) {
+    for (int r = 0; err == hipSuccess && r < nr; r++) {
         err = hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal);
         if (err != hipSuccess) break;
         const hipStream_t ls[3] = {e->stream, e->aux[0], e->aux[1]};
@@ -1289,11 +1390,23 @@ static int ens_enqueue(gam_ens *e, int nsteps)
     }
     e->parity = q0;
     for (int n = 0; n < nsteps; n++) {
-        HIPCHK(hipGraphLaunch(e->exec[e->parity], e->stream));
+        bool direct = e->direct;
+        for (int q = 0; q < e->n; q++) direct = direct && e->m[q]->std[0] && e->m[q]->std[1];
+        for (int q = 0; q < e->n; q++) {
+            gam_ctx *c = e->m[q];
+            c->cur = e->cur0[q] ^ e->parity;
+            if (direct && n + 1 == nsteps) {
+                const int rc = hf_keep(c, e->stream, S_old(c));
+                if (rc) return rc;
+            }
+            c->itgen++;
+            c->hf = direct ? 1 : 0;
+            c->cur ^= 1;
+            c->std[c->cur] = c->mp.doMHD ? 1 : 0;
+        }
+        HIPCHK(hipGraphLaunch(e->exec[e->parity + (direct ? 2 : 0)], e->stream));
         e->parity ^= 1;
     }
-    for (int q = 0; q < e->n; q++) e->m[q]->itgen++;
-    for (int q = 0; q < e->n; q++) e->m[q]->cur = e->cur0[q] ^ e->parity;
     return GAM_OK;
 }
 
@@ -1348,7 +1461,7 @@ extern "C" int gam_ens_launches_per_step(gam_ens *e, int *n)
 {
     if (!e || !n) return fail(GAM_E_ARG, "gam_ens_launches_per_step: NULL argument");
     int k = 0;
-    for (const EnsPhase &ph : e->ph[0]) k += ph.mark == 0;
+    for (const EnsPhase &ph : e->ph[e->direct ? 2 : 0]) k += ph.mark == 0;
     *n = k;
     return GAM_OK;
 }
@@ -1399,11 +1512,13 @@ extern "C" int gam_set_plan(gam_ctx *c, const int *plan)
 static int tune_time(gam_ctx *c, int slot, int reps, double *ms)
 {
     c->tune_slot = -1;
-    enq_step(c);
+    c->general += slot == TS_PREDICT;   // steps that run it
+    enq_step(c, false);
     c->tune_slot = slot;
     c->ntev = 0;
-    for (int r = 0; r < reps; r++) enq_step(c);
+    for (int r = 0; r < reps; r++) enq_step(c, false);
     c->tune_slot = -1;
+    c->general -= slot == TS_PREDICT;
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
     double tot = 0.0;
@@ -1444,13 +1559,15 @@ extern "C" int gam_autotune(gam_ctx *c, int reps)
     if (rc) return rc;
     graphs_drop(c);   // launch arguments change
     if (reps < 1 || reps > GAM_TUNE_MAXREPS) return fail(GAM_E_ARG, "gam_autotune: reps must be in 1..%d", GAM_TUNE_MAXREPS);
-    // snapshot State, oState and the clock; tuning takes real steps
+    if ((rc = hf_flush(c))) return rc;
+    // snapshot State, oState (with their primitives) and the clock; tuning
+    // takes real steps
     const size_t bytes = (size_t)S_NPL * c->g.N3 * sizeof(double);
     double *save = nullptr;
     HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipMalloc((void **)&save, 2 * bytes));
     Clock ck;
-    const int cur0 = c->cur;
+    const int cur0 = c->cur, std0[2] = {c->std[0], c->std[1]};
     const int prof = c->prof;
     hipError_t e = hipMemcpyAsync(save, c->st[0], bytes, hipMemcpyDeviceToDevice, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(save + bytes / sizeof(double), c->st[1], bytes, hipMemcpyDeviceToDevice, c->stream);
@@ -1503,6 +1620,12 @@ extern "C" int gam_autotune(gam_ctx *c, int reps)
     if (e == hipSuccess) e = hipMemcpyAsync(c->clk, &ck, sizeof(Clock), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     c->cur = cur0;
+    c->std[0] = std0[0];
+    c->std[1] = std0[1];
+    // the half state of the next step, which every tuning began with
+    c->hf = 0;
+    launch_predict(c->stream, c->plan.v[TS_PREDICT], c->g, c->mp, face_box(c->g), c->clk, S_cur(c), S_old(c), c->met,
+                   c->H);
     hipFree(save);
     if (rc) return rc;
     if (e != hipSuccess) return fail(GAM_E_HIP, "gam_autotune: %s", hipGetErrorString(e));
@@ -1652,7 +1775,7 @@ extern "C" int gam_adj_create_budget(gam_adj **out, gam_ctx *c, int nsteps, int 
     hipError_t e = hipSuccess;
 #define AALLOC(ptr, bytes) if (e == hipSuccess) e = hipMalloc((void **)&(ptr), (bytes))
     AALLOC(a->ck, (size_t)a->nck * 2 * CK_NPL * pl);
-    AALLOC(a->fin, 2 * S_NPL * pl);
+    AALLOC(a->fin, 2 * ST_NPL * pl);
     AALLOC(a->clkh, (size_t)(nsteps + 1) * sizeof(Clock));
     AALLOC(a->oclk, sizeof(Clock));
     AALLOC(a->tape, (size_t)(K + 2) * CK_NPL * pl);
@@ -1762,18 +1885,33 @@ static int adj_put(gam_adj *a, int n, const double *src, int npl)
     return GAM_OK;
 }
 
+// The adjoint's forward steps: with the predictor, whose planes the
+// transposes read; the states are then not those a plain step leaves.
+struct AdjSteps {
+    gam_ctx *c;
+    explicit AdjSteps(gam_ctx *x) : c(x) { c->general++; }
+    ~AdjSteps()
+    {
+        c->general--;
+        c->std[0] = c->std[1] = 0;
+    }
+};
+
 extern "C" int gam_adj_forward(gam_adj *a, double *J)
 {
     if (!a) return fail(GAM_E_ARG, "gam_adj_forward: NULL argument");
     if (!a->haveW) return fail(GAM_E_STATE, "gam_adj_forward: objective weights not set");
     gam_ctx *c = a->c;
     const long N3 = c->g.N3;
-    const size_t bytes = (size_t)S_NPL * N3 * sizeof(double);
+    const size_t bytes = (size_t)ST_NPL * N3 * sizeof(double);
     const size_t ckb = (size_t)CK_NPL * N3 * sizeof(double);
+    int rc = hf_flush(c);
+    if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     a->cur0 = c->cur;
     const int prof = c->prof;
     c->prof = 0;
+    AdjSteps general(c);
     HIPCHK(hipEventRecord(a->ev[0], c->stream));
     HIPCHK(hipMemcpyAsync(a->clkh, c->clk, sizeof(Clock), hipMemcpyDeviceToDevice, c->stream));
     // the last interval's states (and intermediates) go straight onto the
@@ -1813,9 +1951,8 @@ extern "C" int gam_adj_forward(gam_adj *a, double *J)
     HIPCHK(hipEventRecord(a->ev[1], c->stream));
     c->prof = prof;
     HIPCHK(hipMemcpyAsync(a->fin, S_cur(c), bytes, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(a->fin + (size_t)S_NPL * N3, S_old(c), bytes, hipMemcpyDeviceToDevice, c->stream));
-    int rc = adj_objective(a, S_cur(c), a->lam, J);
-    if (rc) return rc;
+    HIPCHK(hipMemcpyAsync(a->fin + (size_t)ST_NPL * N3, S_old(c), bytes, hipMemcpyDeviceToDevice, c->stream));
+    if ((rc = adj_objective(a, S_cur(c), a->lam, J))) return rc;
     HIPCHK(hipEventElapsedTime(&a->fwd_ms, a->ev[0], a->ev[1]));
     // the start oState's boundary values are those of its own time, or of
     // State's when the caller's forward starts from gam_init_run
@@ -1831,7 +1968,7 @@ extern "C" int gam_adj_forward(gam_adj *a, double *J)
 static int adj_restore_final(gam_adj *a)
 {
     gam_ctx *c = a->c;
-    int rc = adj_put(a, a->nsteps, a->fin, S_NPL);
+    int rc = adj_put(a, a->nsteps, a->fin, ST_NPL);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     return GAM_OK;
@@ -1885,13 +2022,13 @@ static void adj_step(gam_adj *a, int n, const StepIT *it, const double *Sn, cons
         // the hydrodynamic transposes read no face fluxes, but the dt share
         // of the update does
         if (c->mp.doMHD || pdt) {
-            for (int d = 0; d < 3; d++) {
-                Box fb = act_box(g);
-                if (d == 0) fb.i1 += 1; else if (d == 1) fb.j1 += 1; else fb.k1 += 1;
-                launch_flux(s, d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb, c->H, Sn, c->met, c->bg, c->gflx,
-                            c->mflx, c->vf + (long)3 * d * N3);
-            }
-            if (c->mp.doMHD) launch_vface_rim(s, g, c->H, c->met, c->vf);
+            const HalfSrc h = {c->H, Sn, nullptr, clk};
+            Box fb[3];
+            flux_boxes(g, fb);
+            for (int d = 0; d < 3; d++)
+                launch_flux(s, d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb[d], h, c->met, c->bg, c->gflx, c->mflx,
+                            c->vf + (long)3 * d * N3);
+            if (c->mp.doMHD) launch_vface_rim(s, g, h, c->met, c->vf);
         }
     }
     if (c->mp.doMHD) {
@@ -1948,6 +2085,9 @@ extern "C" int gam_adj_backward(gam_adj *a, double *gGas, double *gGasO, double 
         return fail(GAM_E_STATE, "gam_adj_backward: the inflow series changed length since gam_adj_create");
     if (a->dtMode >= 2 && a->dtrecMode != a->dtMode)
         return fail(GAM_E_STATE, "gam_adj_backward: dt mode %d needs a gam_adj_forward run in that mode", a->dtMode);
+    int rc = hf_flush(c);
+    if (rc) return rc;
+    AdjSteps general(c);
     HIPCHK(hipStreamSynchronize(s));
     HIPCHK(hipEventRecord(a->ev[2], s));
     HIPCHK(hipMemsetAsync(a->lam, 0, 3 * ADJ_SET * N3 * sizeof(double), s));
@@ -1957,8 +2097,7 @@ extern "C" int gam_adj_backward(gam_adj *a, double *gGas, double *gGasO, double 
         HIPCHK(hipMemsetAsync(a->gwq, 0, (size_t)WIND_COPIES * a->nw * 5 * sizeof(double), s));
         HIPCHK(hipMemsetAsync(a->gwb, 0, (size_t)WIND_COPIES * a->nw * 3 * sizeof(double), s));
     }
-    int rc = adj_objective(a, a->fin, lA, nullptr);
-    if (rc) return rc;
+    if ((rc = adj_objective(a, a->fin, lA, nullptr))) return rc;
     const int prof = c->prof;
     c->prof = 0;
     // Interval seg recomputed from its checkpoint onto tape pair buf: on the
@@ -2100,8 +2239,10 @@ static int adj_replay(gam_adj *a, const double *Gas, const double *oGas, const d
         if (!a->dts) HIPCHK(hipMalloc((void **)&a->dts, (size_t)a->nsteps * sizeof(double)));
         HIPCHK(hipMemcpy(a->dts, dts, (size_t)a->nsteps * sizeof(double), hipMemcpyHostToDevice));
     }
-    int rc = adj_put(a, 0, a->ck, CK_NPL);
+    int rc = hf_flush(c);
     if (rc) return rc;
+    AdjSteps general(c);
+    if ((rc = adj_put(a, 0, a->ck, CK_NPL))) return rc;
     if ((rc = upload(c, Gas, 0, 5, S_cur(c) + S_GAS * N3))) return rc;
     if (oGas && (rc = upload(c, oGas, 0, 5, S_old(c) + S_GAS * N3))) return rc;
     if (MF && (rc = upload(c, MF, 1, 3, S_cur(c) + S_MF * N3))) return rc;

@@ -30,6 +30,7 @@ __device__ __forceinline__ void finalize_clock(const MParm &m, Clock *clk, int m
 {
     Clock c = *clk;
     if (mode & FIN_ADVANCE) {          // applyUpdate: oState%time=State%time; State%time+=dt
+        c.whf = ab2_weight(clk);
         c.ost = c.st;
         c.st = c.st + c.dtA;
     }
@@ -136,7 +137,7 @@ struct GhostBoxes {
 template <bool FIELD>
 struct k_bc_copy {
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, const BcSet &bc,
-                                               const GhostBoxes &gb, Clock *clk, int finmode,
+                                               const GhostBoxes &gb, Clock *clk, int finmode, int writeW,
                                                double *__restrict__ S, const double *__restrict__ met) const
     {
         const int w = (int)bi.x, tid = (int)(threadIdx.x + BX * threadIdx.y);
@@ -186,6 +187,12 @@ struct k_bc_copy {
         if (sg != c) {
 #pragma unroll
             for (int v = 0; v < 5; v++) S[(S_GAS + v) * N3 + c] = U[v];
+        }
+        if (FIELD && writeW && cell) {
+            double W[5];
+            c2p_cell(m, U, W);
+#pragma unroll
+            for (int v = 0; v < 5; v++) S[(S_W + v) * N3 + c] = W[v];
         }
 #pragma unroll
         for (int d = 0; d < 3; d++)
@@ -381,7 +388,7 @@ void launch_bflux2fld(hipStream_t s, const Geo &g, const Box &cb, const Box &ski
 // it (gam_enforce_bcs).  field = true: inside a step; cell B of every ghost
 // cell from its faces instead (bFlux2Fld), and with finmode the time
 // bookkeeping, whose Model%t the inflow then reads ahead of it.
-void launch_bcs(hipStream_t s, const int *kind, bool field, int finmode, const Geo &g, const MParm &m, Clock *clk,
+void launch_bcs(hipStream_t s, const int *kind, bool field, bool writeW, int finmode, const Geo &g, const MParm &m, Clock *clk,
                 const WindDev &w, double *S, const double *met)
 {
     BcSet bc;
@@ -428,8 +435,8 @@ void launch_bcs(hipStream_t s, const int *kind, bool field, int finmode, const G
         }
         gb.start[6] = tot;
         const int fm = last ? finmode : 0;
-        if (f) launch_f<k_bc_copy<true>>(dim3((unsigned)tot), dim3(BX, BY), s, g, m, bc, gb, clk, fm, S, met);
-        else launch_f<k_bc_copy<false>>(dim3((unsigned)tot), dim3(BX, BY), s, g, m, bc, gb, clk, fm, S, met);
+        if (f) launch_f<k_bc_copy<true>>(dim3((unsigned)tot), dim3(BX, BY), s, g, m, bc, gb, clk, fm, writeW ? 1 : 0, S, met);
+        else launch_f<k_bc_copy<false>>(dim3((unsigned)tot), dim3(BX, BY), s, g, m, bc, gb, clk, fm, writeW ? 1 : 0, S, met);
     };
     if (all) copy(7, true);
     else if (per[2]) copy(6, true);

@@ -65,10 +65,12 @@ struct Clock {
     int status;     // sticky CalcDT status: 0 ok, 1 bad, 2 disaster
     int lastStatus; // status of the last CalcDT
     int pad;
+    double whf;     // AB2 weight of the last step's half state
 };
 
-// Plane indices: State buffer
-enum { S_GAS = 0, S_MF = 5, S_B = 8, S_E = 11, S_NPL = 14 };
+// Plane indices: State buffer.  S_W holds the primitives of the gas (CellC2P)
+// wherever a step has left them; the planes before it are the state itself.
+enum { S_GAS = 0, S_MF = 5, S_B = 8, S_E = 11, S_W = 14, S_NPL = 19, ST_NPL = S_W };
 // Half state buffer + primitive planes
 enum { H_GAS = 0, H_MF = 5, H_B = 8, H_WH = 11, H_WN = 16, H_NPL = 21 };
 // Metric planes

@@ -158,7 +158,7 @@ struct edge_geom {
 #define EMF_LDS (edge_geom<0>::LDS)
 static_assert(edge_geom<1>::LDS <= EMF_LDS && edge_geom<2>::LDS <= EMF_LDS, "LDS planes");
 
-template <int ED, int RM, bool BG, bool BORIS>
+template <int ED, int RM, bool BG, bool BORIS, bool DIR>
 struct edge_tile {
     using G = edge_geom<ED>;
     // face e of pair P: its place in the tile, as offsets from the tile's
@@ -196,6 +196,7 @@ struct edge_tile {
                                                const EdgeTile &t, const Clock *clk,
                                                const double *__restrict__ H,
                                                const double *__restrict__ S,
+                                               const double *__restrict__ O,
                                                const double *__restrict__ Vf,
                                                const double *__restrict__ met,
                                                const double *__restrict__ bg,
@@ -230,8 +231,17 @@ struct edge_tile {
 
         // the faces' loads
         double A1[Q1], V1[Q1][3], h1[Q1], l1[Q1], A2[Q2], h2[Q2], l2[Q2];
-        const double *mfH = H + H_MF * N3;
-        const double *mfL = m.doLFM ? S + S_MF * N3 : mfH;
+        // (half-state fluxes h and limiter fluxes l; DIR: of oState and State,
+        // extrapolated below)
+        const double *mfH = DIR ? O + S_MF * N3 : H + H_MF * N3;
+        const double *mfL = DIR || m.doLFM ? S + S_MF * N3 : mfH;
+        const double wt = DIR ? ab2_weight(clk) : 0.0;
+        auto extrapolate = [&](double &h, double &l) {
+            if (DIR) {
+                h = ab2(l, h, wt);
+                if (!m.doLFM) l = h;
+            }
+        };
 #pragma unroll
         for (int q = 0; q < Q1; q++) {
             int di, dj, dk;
@@ -266,8 +276,15 @@ struct edge_tile {
         {
             constexpr int E1 = (ED == 0) ? 1 : 0, E2 = (ED == 2) ? 1 : 2;
             const unsigned s1 = (unsigned)(8 * STRIDE<E1>(g)), s2 = (unsigned)(8 * STRIDE<E2>(g));
-            const double *Dh = pln(H, (H_GAS + DEN) * N3);
-            D[0] = ldp(Dh, oc); D[1] = ldp(Dh, oc - s1); D[2] = ldp(Dh, oc - s2); D[3] = ldp(Dh, oc - s1 - s2);
+            const unsigned od[4] = {oc, oc - s1, oc - s2, oc - s1 - s2};
+            const double *Dh = DIR ? pln(S, (S_W + DEN) * N3) : pln(H, (H_GAS + DEN) * N3);
+#pragma unroll
+            for (int q = 0; q < 4; q++) D[q] = ldp(Dh, od[q]);
+            if (DIR) {
+                const double *Do = pln(O, (S_W + DEN) * N3);
+#pragma unroll
+                for (int q = 0; q < 4; q++) D[q] = half_prim(m, DEN, D[q], ldp(Do, od[q]), wt);
+            }
         }
         // EdgeLRs' weighting (fields.F90:288-362), see edge_lr
 #pragma unroll
@@ -276,6 +293,7 @@ struct edge_tile {
             if (e < NF1) {
                 int di, dj, dk;
                 const int l = place<1>(e, di, dj, dk);
+                extrapolate(h1[q], l1[q]);
                 sA1[e] = A1[q];
 #pragma unroll
                 for (int d = 0; d < 3; d++) sV[d * NF1 + e] = A1[q] * V1[q][d];
@@ -289,6 +307,7 @@ struct edge_tile {
             if (e < NF2) {
                 int di, dj, dk;
                 const int l = place<2>(e, di, dj, dk);
+                extrapolate(h2[q], l2[q]);
                 sA2[e] = A2[q];
                 sq2[e] = h2[q] * fmin(A2[q] * (1.0 / GAM_TINY), 1.0);
                 if (l >= 0) sn2[l] = l2[q] * gam_rcp(dmax(A2[q], GAM_TINY));
@@ -336,19 +355,20 @@ struct edge_tile {
     }
 };
 
-template <int ED, int RM, bool BG, bool BORIS>
+template <int ED, int RM, bool BG, bool BORIS, bool DIR>
 struct k_emf_t {
     static constexpr int NT = BX * BY;
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, EdgeTile b, const Clock *clk,
                                                const double *__restrict__ H,
                                                const double *__restrict__ S,
+                                               const double *__restrict__ O,
                                                const double *__restrict__ Vf,
                                                const double *__restrict__ met,
                                                const double *__restrict__ bg,
                                                double *__restrict__ E) const
     {
         __shared__ double lds[edge_geom<ED>::LDS];
-        edge_tile<ED, RM, BG, BORIS>{}(lds, (int)bi.x, g, m, b, clk, H, S, Vf, met, bg, E);
+        edge_tile<ED, RM, BG, BORIS, DIR>{}(lds, (int)bi.x, g, m, b, clk, H, S, O, Vf, met, bg, E);
     }
 };
 
@@ -374,12 +394,13 @@ struct Emf3 {
     int start[2];     // first workgroup of edge direction 1, of direction 2
 };
 
-template <int RM, bool BG, bool BORIS>
+template <int RM, bool BG, bool BORIS, bool DIR>
 struct k_emf3 {
     static constexpr int NT = BX * BY;
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, const Emf3 &f, const Clock *clk,
                                                const double *__restrict__ H,
                                                const double *__restrict__ S,
+                                               const double *__restrict__ O,
                                                const double *__restrict__ Vf,
                                                const double *__restrict__ met,
                                                const double *__restrict__ bg,
@@ -388,18 +409,17 @@ struct k_emf3 {
         __shared__ double lds[EMF_LDS];
         const int w = (int)bi.x;
         if (w < f.start[0])
-            edge_tile<0, RM, BG, BORIS>{}(lds, w, g, m, f.t[0], clk, H, S, Vf + 3 * g.N3, met, bg, E);
+            edge_tile<0, RM, BG, BORIS, DIR>{}(lds, w, g, m, f.t[0], clk, H, S, O, Vf + 3 * g.N3, met, bg, E);
         else if (w < f.start[1])
-            edge_tile<1, RM, BG, BORIS>{}(lds, w - f.start[0], g, m, f.t[1], clk, H, S, Vf + 6 * g.N3, met, bg, E);
+            edge_tile<1, RM, BG, BORIS, DIR>{}(lds, w - f.start[0], g, m, f.t[1], clk, H, S, O, Vf + 6 * g.N3, met, bg, E);
         else
-            edge_tile<2, RM, BG, BORIS>{}(lds, w - f.start[1], g, m, f.t[2], clk, H, S, Vf, met, bg, E);
+            edge_tile<2, RM, BG, BORIS, DIR>{}(lds, w - f.start[1], g, m, f.t[2], clk, H, S, O, Vf, met, bg, E);
     }
 };
 
 template <int RM, bool BG, bool BO>
-static void emf3_t(hipStream_t s, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
-                   const double *H, const double *S, const double *Vf, const double *met, const double *bg,
-                   double *E)
+static void emf3_t(hipStream_t s, const Geo &g, const MParm &m, const Box *b, const HalfSrc &h,
+                   const double *Vf, const double *met, const double *bg, double *E)
 {
     Emf3 f;
     int tot = 0;
@@ -408,7 +428,9 @@ static void emf3_t(hipStream_t s, const Geo &g, const MParm &m, const Box *b, co
         tot += (int)xcd_grid(f.t[d].nb, f.t[d].xs);
         if (d < 2) f.start[d] = tot;
     }
-    launch_f<k_emf3<RM, BG, BO>>(dim3((unsigned)tot), dim3(BX, BY), s, g, m, f, clk, H, S, Vf, met, bg, E);
+    const dim3 gr((unsigned)tot), bl(BX, BY);
+    if (h.O) launch_f<k_emf3<RM, BG, BO, true>>(gr, bl, s, g, m, f, h.clk, h.H, h.S, h.O, Vf, met, bg, E);
+    else launch_f<k_emf3<RM, BG, BO, false>>(gr, bl, s, g, m, f, h.clk, h.H, h.S, h.O, Vf, met, bg, E);
 }
 
 bool emf3_ok(const int *plan)
@@ -418,31 +440,33 @@ bool emf3_ok(const int *plan)
     return true;
 }
 
-void launch_emf3(hipStream_t s, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
-                 const double *H, const double *S, const double *Vf, const double *met, const double *bg, double *E)
+void launch_emf3(hipStream_t s, const Geo &g, const MParm &m, const Box *b, const HalfSrc &h, const double *Vf,
+                 const double *met, const double *bg, double *E)
 {
     const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
     switch (sel) {
-    case 0: emf3_t<0, false, false>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 1: emf3_t<0, false, true>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 2: emf3_t<0, true, false>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 3: emf3_t<0, true, true>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 4: emf3_t<1, false, false>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 5: emf3_t<1, false, true>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 6: emf3_t<1, true, false>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    default: emf3_t<1, true, true>(s, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 0: emf3_t<0, false, false>(s, g, m, b, h, Vf, met, bg, E); break;
+    case 1: emf3_t<0, false, true>(s, g, m, b, h, Vf, met, bg, E); break;
+    case 2: emf3_t<0, true, false>(s, g, m, b, h, Vf, met, bg, E); break;
+    case 3: emf3_t<0, true, true>(s, g, m, b, h, Vf, met, bg, E); break;
+    case 4: emf3_t<1, false, false>(s, g, m, b, h, Vf, met, bg, E); break;
+    case 5: emf3_t<1, false, true>(s, g, m, b, h, Vf, met, bg, E); break;
+    case 6: emf3_t<1, true, false>(s, g, m, b, h, Vf, met, bg, E); break;
+    default: emf3_t<1, true, true>(s, g, m, b, h, Vf, met, bg, E); break;
     }
 }
 
 template <int ED, int RM, bool BG, bool BO>
-static void emf_t(hipStream_t s, int plan, const Geo &g, const MParm &m, const Box &b, const Clock *clk,
-                  const double *H, const double *S, const double *Vf, const double *met,
-                  const double *bg, double *E)
+static void emf_t(hipStream_t s, int plan, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                  const double *Vf, const double *met, const double *bg, double *E)
 {
+    const double *H = h.H, *S = h.S;
+    const Clock *clk = h.clk;
     if (plan == PLAN_LDS) {
         const EdgeTile t = edge_tiles(ED, b);
-        launch_f<k_emf_t<ED, RM, BG, BO>>(dim3(xcd_grid(t.nb, t.xs)), dim3(BX, BY), s, g, m, t, clk, H, S, Vf, met,
-                                          bg, E);
+        const dim3 gr(xcd_grid(t.nb, t.xs)), bl(BX, BY);
+        if (h.O) launch_f<k_emf_t<ED, RM, BG, BO, true>>(gr, bl, s, g, m, t, clk, H, S, h.O, Vf, met, bg, E);
+        else launch_f<k_emf_t<ED, RM, BG, BO, false>>(gr, bl, s, g, m, t, clk, H, S, h.O, Vf, met, bg, E);
         return;
     }
     const int ch = plan_chunk(plan);
@@ -456,28 +480,26 @@ static void emf_t(hipStream_t s, int plan, const Geo &g, const MParm &m, const B
 }
 
 template <int ED>
-static void emf_d(hipStream_t s, int ax, const Geo &g, const MParm &m, const Box &b, const Clock *clk,
-                  const double *H, const double *S, const double *Vf, const double *met,
-                  const double *bg, double *E)
+static void emf_d(hipStream_t s, int ax, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                  const double *Vf, const double *met, const double *bg, double *E)
 {
     const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
     switch (sel) {
-    case 0: emf_t<ED, 0, false, false>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 1: emf_t<ED, 0, false, true>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 2: emf_t<ED, 0, true, false>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 3: emf_t<ED, 0, true, true>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 4: emf_t<ED, 1, false, false>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 5: emf_t<ED, 1, false, true>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    case 6: emf_t<ED, 1, true, false>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
-    default: emf_t<ED, 1, true, true>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E); break;
+    case 0: emf_t<ED, 0, false, false>(s, ax, g, m, b, h, Vf, met, bg, E); break;
+    case 1: emf_t<ED, 0, false, true>(s, ax, g, m, b, h, Vf, met, bg, E); break;
+    case 2: emf_t<ED, 0, true, false>(s, ax, g, m, b, h, Vf, met, bg, E); break;
+    case 3: emf_t<ED, 0, true, true>(s, ax, g, m, b, h, Vf, met, bg, E); break;
+    case 4: emf_t<ED, 1, false, false>(s, ax, g, m, b, h, Vf, met, bg, E); break;
+    case 5: emf_t<ED, 1, false, true>(s, ax, g, m, b, h, Vf, met, bg, E); break;
+    case 6: emf_t<ED, 1, true, false>(s, ax, g, m, b, h, Vf, met, bg, E); break;
+    default: emf_t<ED, 1, true, true>(s, ax, g, m, b, h, Vf, met, bg, E); break;
     }
 }
 
-void launch_emf(hipStream_t s, int eD, int ax, const Geo &g, const MParm &m, const Box &b, const Clock *clk,
-                const double *H, const double *S, const double *Vf, const double *met,
-                const double *bg, double *E)
+void launch_emf(hipStream_t s, int eD, int ax, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                const double *Vf, const double *met, const double *bg, double *E)
 {
-    if (eD == 0) emf_d<0>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E);
-    else if (eD == 1) emf_d<1>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E);
-    else emf_d<2>(s, ax, g, m, b, clk, H, S, Vf, met, bg, E);
+    if (eD == 0) emf_d<0>(s, ax, g, m, b, h, Vf, met, bg, E);
+    else if (eD == 1) emf_d<1>(s, ax, g, m, b, h, Vf, met, bg, E);
+    else emf_d<2>(s, ax, g, m, b, h, Vf, met, bg, E);
 }

@@ -8,17 +8,17 @@
 // Fluxes, stress.F90:204-429, after BlockStateLRs): magnetic kinetic flux
 // with the B0 terms, Boris mag-HOGS, gas kinetic flux, HOGS and the nuke
 // term, times the face area, stored to gFlx/mFlx of direction D.  AT(p)
-// reads plane p at the face point, AT_M(p) one cell below it along D;
+// reads plane p at the face point; HALF_MF() is the half-state face flux,
+// HALF_DU the half-state gas less that of the cell below the face along D;
 // RECON_B(BL, BR) fills the magnetic L/R states (called only with MHD on,
 // after the metric loads, which keeps the register peak of the fused
 // kernel at that of the gas part); oc is the face's byte offset for the
 // stores.
 // ====================================================================
-template <int D, bool BG, bool BORIS, class AtF, class AtMF, class ReconB>
+template <int D, bool BG, bool BORIS, class AtF, class HalfF, class DuF, class ReconB>
 __device__ __forceinline__ void face_flux_lr(const Geo &g, const MParm &m,
-                                             const double *__restrict__ H,
                                              const double *__restrict__ met,
-                                             const double *__restrict__ bg, AtF AT, AtMF AT_M,
+                                             const double *__restrict__ bg, AtF AT, HalfF HALF_MF, DuF HALF_DU,
                                              ReconB RECON_B, const double *WL,
                                              const double *WR, double *BL, double *BR,
                                              unsigned oc,
@@ -48,7 +48,7 @@ __device__ __forceinline__ void face_flux_lr(const Geo &g, const MParm &m,
     if (m.doMHD) {
         RECON_B(BL, BR);
         const double iFaB = gam_rcp(faB);
-        const double Bn = AT(H + (H_MF + D) * N3) * iFaB;
+        const double Bn = HALF_MF() * iFaB;
         double B0[3] = {0.0, 0.0, 0.0}, B0n = 0.0;
         if (BG) {
 #pragma unroll
@@ -84,11 +84,10 @@ __device__ __forceinline__ void face_flux_lr(const Geo &g, const MParm &m,
             nuke = sqrt(vL * vL + vR * vR) / GAM_SQRT2_SP >= 1.5 * m.Ca;
         }
         if (nuke) {
+            double dU[5];
+            HALF_DU(dU);
 #pragma unroll
-            for (int v = 0; v < 5; v++) {
-                double dU = AT(H + (H_GAS + v) * N3) - AT_M(H + (H_GAS + v) * N3);
-                gF[v] = gF[v] - m.Ca * dU;
-            }
+            for (int v = 0; v < 5; v++) gF[v] = gF[v] - m.Ca * dU[v];
         }
     }
 #pragma unroll
@@ -166,8 +165,11 @@ struct k_flux {
         };
         double BL[3], BR[3];
         face_flux_lr<D, BG, BORIS>(
-            g, m, H, met, bg, [&](const double *p) { return LD(p, 4); },
-            [&](const double *p) { return LD(p, 3); }, recon_b, WL, WR, BL, BR, o[4], gflx, mflx);
+            g, m, met, bg, [&](const double *p) { return LD(p, 4); }, [&]() { return LD(H + (H_MF + D) * N3, 4); },
+            [&](double *dU) {
+                for (int v = 0; v < 5; v++) dU[v] = LD(H + (H_GAS + v) * N3, 4) - LD(H + (H_GAS + v) * N3, 3);
+            },
+            recon_b, WL, WR, BL, BR, o[4], gflx, mflx);
     }
 };
 
@@ -184,6 +186,10 @@ struct k_flux {
 // Two phases share the LDS planes: the five gas variables, then the three
 // field components, whose loads wait in registers meanwhile; 37 KB (33 for
 // D = 0) and 128 registers leave room for four workgroups per CU.
+// DIR: the half state is formed as the cells are staged, from the primitives
+// and cell B that the last two steps left (S_W, S_B of State and oState): as
+// many words as the predictor's planes, which are then neither written nor
+// read (HalfSrc says when).
 // The tile's 32 points are two whole 128-byte lines of every row.
 // Bound by memory traffic, close behind by FP64 issue (1075 vector
 // instructions per face; at 1580 the clock fell to 1.8 GHz).  256x256x384
@@ -202,7 +208,7 @@ struct FluxTile {
 
 #define FLUX_LDS ((8 + 3) * 376 > (8 + 7) * 32 * 6 + (8 + 3) * 32 * 5 ? (8 + 3) * 376 : (8 + 7) * 32 * 6 + (8 + 3) * 32 * 5)
 
-template <int D, int RM, bool BG, bool BORIS>
+template <int D, int RM, bool BG, bool BORIS, bool DIR>
 struct flux_tile {
     static constexpr int TI = 32, TA = 8;
     static constexpr int NE = D == 0 ? 376 : (TA + 7) * TI;   // cells staged (D = 0: at most)
@@ -214,6 +220,7 @@ struct flux_tile {
     __device__ __forceinline__ void operator()(double *lds, int w, const Geo &g, const MParm &m,
                                                const FluxTile &t, const double *__restrict__ H,
                                                const double *__restrict__ S,
+                                               const double *__restrict__ O, const Clock *clk,
                                                const double *__restrict__ met,
                                                const double *__restrict__ bg,
                                                double *__restrict__ gflx,
@@ -283,21 +290,64 @@ struct flux_tile {
         // limiter entry of a staged cell
         auto lim = [&](int e) { return e >= LO && e - LO < NL; };
 
+        // wq: volume-weighted half-state primitives, wl: limiter primitives,
+        // bq: half-state cell B (weighted below), bl: limiter cell B
         const double *pv = met + M_VOL * N3;
-        const double *Wv = H + H_WH * N3, *Wl = H + H_WN * N3;
-        const double *Bh = H + H_B * N3, *Bl = m.doLFM ? S + S_B * N3 : Bh;
-        double v[2], wq[2][5], wl[2][5], bq[2][3], bl[2][3];
+        double v[2], wq[2][5], wl[2][5], bq[2][3], bl[2][3], wt = 0.0;
+        if (DIR) {
+            wt = ab2_weight(clk);
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            v[q] = ldp(pv, oe[q]);
+            for (int q = 0; q < 2; q++) {
+                v[q] = ldp(pv, oe[q]);
 #pragma unroll
-            for (int n = 0; n < 5; n++) { wq[q][n] = ldp(pln(Wv, n * N3), oe[q]); wl[q][n] = ldp(pln(Wl, n * N3), oe[q]); }
-        }
-        if (m.doMHD) {
+                for (int n = 0; n < 5; n++) {
+                    wl[q][n] = ldp(pln(S, (S_W + n) * N3), oe[q]);
+                    wq[q][n] = ldp(pln(O, (S_W + n) * N3), oe[q]);
+                }
+            }
 #pragma unroll
             for (int q = 0; q < 2; q++)
 #pragma unroll
-                for (int x = 0; x < 3; x++) { bq[q][x] = ldp(pln(Bh, x * N3), oe[q]); bl[q][x] = ldp(pln(Bl, x * N3), oe[q]); }
+                for (int x = 0; x < 3; x++) {
+                    bl[q][x] = ldp(pln(S, (S_B + x) * N3), oe[q]);
+                    bq[q][x] = ldp(pln(O, (S_B + x) * N3), oe[q]);
+                }
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+#pragma unroll
+                for (int n = 0; n < 5; n++) {
+                    const double h = half_prim(m, n, wl[q][n], wq[q][n], wt);
+                    if (!m.doLFM) wl[q][n] = h;
+                    wq[q][n] = v[q] * h;
+                }
+#pragma unroll
+                for (int x = 0; x < 3; x++) {
+                    const double h = ab2(bl[q][x], bq[q][x], wt);
+                    if (!m.doLFM) bl[q][x] = h;
+                    bq[q][x] = h;
+                }
+            }
+        } else {
+            const double *Wv = H + H_WH * N3, *Wl = H + H_WN * N3;
+            const double *Bh = H + H_B * N3, *Bl = m.doLFM ? S + S_B * N3 : Bh;
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                v[q] = ldp(pv, oe[q]);
+#pragma unroll
+                for (int n = 0; n < 5; n++) {
+                    wq[q][n] = ldp(pln(Wv, n * N3), oe[q]);
+                    wl[q][n] = ldp(pln(Wl, n * N3), oe[q]);
+                }
+            }
+            if (m.doMHD) {
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+#pragma unroll
+                    for (int x = 0; x < 3; x++) {
+                        bq[q][x] = ldp(pln(Bh, x * N3), oe[q]);
+                        bl[q][x] = ldp(pln(Bl, x * N3), oe[q]);
+                    }
+            }
         }
 #pragma unroll
         for (int q = 0; q < 2; q++) {
@@ -335,7 +385,7 @@ struct flux_tile {
             // Mom2Face of this face from the same velocity stencil
             if (n >= 1 && n <= 3 && act) stp(Vf + (n - 1) * N3, oc, vel);
         }
-        if (m.doMHD) {
+        if (DIR || m.doMHD) {
             __syncthreads();
 #pragma unroll
             for (int q = 0; q < 2; q++) {
@@ -354,18 +404,38 @@ struct flux_tile {
         }
         if (act)
             face_flux_lr<D, BG, BORIS>(
-                g, m, H, met, bg, [&](const double *p) { return ldp(pln(p, 0), oc); },
-                [&](const double *p) { return ldp(p, oc - s8); },
+                g, m, met, bg, [&](const double *p) { return ldp(pln(p, 0), oc); },
+                [&]() {
+                    return DIR ? ab2(ldp(pln(S, (S_MF + D) * N3), oc), ldp(pln(O, (S_MF + D) * N3), oc), wt)
+                               : ldp(pln(H, (H_MF + D) * N3), oc);
+                },
+                [&](double *dU) {
+                    if (DIR) {
+                        double W[5], U[5], Ul[5];
+                        for (int n = 0; n < 5; n++)
+                            W[n] = half_prim(m, n, ldp(S + (S_W + n) * N3, oc), ldp(O + (S_W + n) * N3, oc), wt);
+                        p2c_cell(m, W, U);
+                        for (int n = 0; n < 5; n++)
+                            W[n] = half_prim(m, n, ldp(S + (S_W + n) * N3, oc - s8),
+                                             ldp(O + (S_W + n) * N3, oc - s8), wt);
+                        p2c_cell(m, W, Ul);
+                        for (int n = 0; n < 5; n++) dU[n] = U[n] - Ul[n];
+                    } else {
+                        for (int n = 0; n < 5; n++)
+                            dU[n] = ldp(H + (H_GAS + n) * N3, oc) - ldp(H + (H_GAS + n) * N3, oc - s8);
+                    }
+                },
                 [](double *, double *) {}, WL, WR, BL, BR, oc, gflx, mflx);
     }
 };
 
-template <int D, int RM, bool BG, bool BORIS>
+template <int D, int RM, bool BG, bool BORIS, bool DIR>
 struct k_flux_t {
     static constexpr int NT = 256;
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, FluxTile t,
                                                const double *__restrict__ H,
                                                const double *__restrict__ S,
+                                               const double *__restrict__ O, const Clock *clk,
                                                const double *__restrict__ met,
                                                const double *__restrict__ bg,
                                                double *__restrict__ gflx,
@@ -373,7 +443,7 @@ struct k_flux_t {
                                                double *__restrict__ Vf) const
     {
         __shared__ double lds[FLUX_LDS];
-        flux_tile<D, RM, BG, BORIS>{}(lds, (int)bi.x, g, m, t, H, S, met, bg, gflx, mflx, Vf);
+        flux_tile<D, RM, BG, BORIS, DIR>{}(lds, (int)bi.x, g, m, t, H, S, O, clk, met, bg, gflx, mflx, Vf);
     }
 };
 
@@ -402,12 +472,18 @@ static inline FluxTile flux_tiles(int D, const Box &b, bool alt)
 }
 
 template <int D, int RM, bool BG, bool BO>
-static void flux_t(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
-                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
+static void flux_t(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                   const double *met, const double *bg, double *gf, double *mf, double *vf)
 {
+    const double *H = h.H, *S = h.S;
     if (plan_ax(form) >= PLAN_LDS) {
         const FluxTile t = flux_tiles(D, b, form & 1);
-        launch_f<k_flux_t<D, RM, BG, BO>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, met, bg, gf, mf, vf);
+        if (h.O)
+            launch_f<k_flux_t<D, RM, BG, BO, true>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk, met, bg,
+                                                    gf, mf, vf);
+        else
+            launch_f<k_flux_t<D, RM, BG, BO, false>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk, met, bg,
+                                                     gf, mf, vf);
         return;
     }
     const int ch = plan_chunk(form);
@@ -421,18 +497,18 @@ static void flux_t(hipStream_t s, int form, const Geo &g, const MParm &m, const 
 }
 
 template <int D>
-static void flux_d(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
-                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
+static void flux_d(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                   const double *met, const double *bg, double *gf, double *mf, double *vf)
 {
     const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
     switch (sel) {
-    case 0: flux_t<D, 0, false, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 1: flux_t<D, 0, false, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 2: flux_t<D, 0, true, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 3: flux_t<D, 0, true, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 4: flux_t<D, 1, false, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 5: flux_t<D, 1, false, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 6: flux_t<D, 1, true, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    default: flux_t<D, 1, true, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
+    case 0: flux_t<D, 0, false, false>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 1: flux_t<D, 0, false, true>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 2: flux_t<D, 0, true, false>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 3: flux_t<D, 0, true, true>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 4: flux_t<D, 1, false, false>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 5: flux_t<D, 1, false, true>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 6: flux_t<D, 1, true, false>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    default: flux_t<D, 1, true, true>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
     }
 }

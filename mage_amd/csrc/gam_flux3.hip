@@ -15,12 +15,13 @@ struct Flux3 {
     int start[4];     // first workgroup of direction 1, of direction 2, of the rim; the end
 };
 
-template <int RM, bool BG, bool BORIS>
+template <int RM, bool BG, bool BORIS, bool DIR>
 struct k_flux3 {
     static constexpr int NT = 256;
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, const Flux3 &f,
                                                const double *__restrict__ H,
                                                const double *__restrict__ S,
+                                               const double *__restrict__ O, const Clock *clk,
                                                const double *__restrict__ met,
                                                const double *__restrict__ bg,
                                                double *__restrict__ gflx,
@@ -31,19 +32,19 @@ struct k_flux3 {
         const int w = (int)bi.x;
         const long N3 = g.N3;
         if (w < f.start[0])
-            flux_tile<0, RM, BG, BORIS>{}(lds, w, g, m, f.t[0], H, S, met, bg, gflx, mflx, Vf);
+            flux_tile<0, RM, BG, BORIS, DIR>{}(lds, w, g, m, f.t[0], H, S, O, clk, met, bg, gflx, mflx, Vf);
         else if (w < f.start[1])
-            flux_tile<1, RM, BG, BORIS>{}(lds, w - f.start[0], g, m, f.t[1], H, S, met, bg, gflx, mflx, Vf + 3 * N3);
+            flux_tile<1, RM, BG, BORIS, DIR>{}(lds, w - f.start[0], g, m, f.t[1], H, S, O, clk, met, bg, gflx, mflx, Vf + 3 * N3);
         else if (w < f.start[2])
-            flux_tile<2, RM, BG, BORIS>{}(lds, w - f.start[1], g, m, f.t[2], H, S, met, bg, gflx, mflx, Vf + 6 * N3);
+            flux_tile<2, RM, BG, BORIS, DIR>{}(lds, w - f.start[1], g, m, f.t[2], H, S, O, clk, met, bg, gflx, mflx, Vf + 6 * N3);
         else
-            vface_rim{}(w - f.start[2], g, f.rim, H, met, Vf);
+            vface_rim<DIR>{}(w - f.start[2], g, f.rim, H, S, O, clk, met, Vf);
     }
 };
 
 template <int RM, bool BG, bool BO>
-static void flux3_t(hipStream_t s, const int *form, const Geo &g, const MParm &m, const Box *b, const double *H,
-                    const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
+static void flux3_t(hipStream_t s, const int *form, const Geo &g, const MParm &m, const Box *b, const HalfSrc &h,
+                    const double *met, const double *bg, double *gf, double *mf, double *vf)
 {
     Flux3 f;
     int tot = 0;
@@ -55,7 +56,9 @@ static void flux3_t(hipStream_t s, const int *form, const Geo &g, const MParm &m
     f.rim = rim_set(g);
     if (m.doMHD) tot += f.rim.start[6];
     f.start[3] = tot;
-    launch_f<k_flux3<RM, BG, BO>>(dim3((unsigned)tot), dim3(BX, BY), s, g, m, f, H, S, met, bg, gf, mf, vf);
+    const dim3 gr((unsigned)tot), bl(BX, BY);
+    if (h.O) launch_f<k_flux3<RM, BG, BO, true>>(gr, bl, s, g, m, f, h.H, h.S, h.O, h.clk, met, bg, gf, mf, vf);
+    else launch_f<k_flux3<RM, BG, BO, false>>(gr, bl, s, g, m, f, h.H, h.S, h.O, h.clk, met, bg, gf, mf, vf);
 }
 
 bool flux3_ok(const int *form)
@@ -65,24 +68,26 @@ bool flux3_ok(const int *form)
     return true;
 }
 
-void launch_flux3(hipStream_t s, const int *form, const Geo &g, const MParm &m, const Box *b, const double *H,
-                  const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
+void launch_flux3(hipStream_t s, const int *form, const Geo &g, const MParm &m, const Box *b, const HalfSrc &h,
+                  const double *met, const double *bg, double *gf, double *mf, double *vf)
 {
     const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
     switch (sel) {
-    case 0: flux3_t<0, false, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 1: flux3_t<0, false, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 2: flux3_t<0, true, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 3: flux3_t<0, true, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 4: flux3_t<1, false, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 5: flux3_t<1, false, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    case 6: flux3_t<1, true, false>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
-    default: flux3_t<1, true, true>(s, form, g, m, b, H, S, met, bg, gf, mf, vf); break;
+    case 0: flux3_t<0, false, false>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 1: flux3_t<0, false, true>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 2: flux3_t<0, true, false>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 3: flux3_t<0, true, true>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 4: flux3_t<1, false, false>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 5: flux3_t<1, false, true>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    case 6: flux3_t<1, true, false>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
+    default: flux3_t<1, true, true>(s, form, g, m, b, h, met, bg, gf, mf, vf); break;
     }
 }
 
-void launch_vface_rim(hipStream_t s, const Geo &g, const double *H, const double *met, double *Vf)
+void launch_vface_rim(hipStream_t s, const Geo &g, const HalfSrc &h, const double *met, double *Vf)
 {
     const RimSet r = rim_set(g);
-    launch_f<k_vface_rim>(dim3((unsigned)r.start[6]), dim3(BX, BY), s, g, r, H, met, Vf);
+    const dim3 gr((unsigned)r.start[6]), bl(BX, BY);
+    if (h.O) launch_f<k_vface_rim<true>>(gr, bl, s, g, r, h.H, h.S, h.O, h.clk, met, Vf);
+    else launch_f<k_vface_rim<false>>(gr, bl, s, g, r, h.H, h.S, h.O, h.clk, met, Vf);
 }

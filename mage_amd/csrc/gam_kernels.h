@@ -83,38 +83,49 @@ enum {
 // Sets the message gam_last_error() returns ("msg: detail") and returns code.
 int gam_fail_(int code, const char *msg, const char *detail);
 
+// Where the fluxes and EMFs take the half state from: H, the predictor's
+// planes (O null); or, with O, State S and oState O themselves.  That needs
+// MHD and both states as a step leaves them: gas at or above the density
+// floor, its primitives in S_W, cell B that of the face fluxes in every cell
+// (ghosts too), where extrapolating cell B and primitives is extrapolating
+// face fluxes and gas; and launch plans of the LDS forms.
+struct HalfSrc {
+    const double *H, *S, *O;
+    const Clock *clk;
+};
+
 void launch_predict(hipStream_t s, int ax, const Geo &g, const MParm &m, const Box &fb, const Clock *clk,
-                    const double *S, const double *O, const double *met, double *H);
+                    const double *S, const double *O, const double *met, double *H, int hfonly = 0);
 // Mom2Face on the faces the EMF stencils read past the interface-flux faces
 // (the flux kernels write the rest): Vf planes [3*dT1 + comp]
-void launch_vface_rim(hipStream_t s, const Geo &g, const double *H, const double *met, double *Vf);
-void launch_emf(hipStream_t s, int eD, int ax, const Geo &g, const MParm &m, const Box &b, const Clock *clk,
-                const double *H, const double *S, const double *Vf, const double *met,
-                const double *bg, double *E);
+void launch_vface_rim(hipStream_t s, const Geo &g, const HalfSrc &h, const double *met, double *Vf);
+void launch_emf(hipStream_t s, int eD, int ax, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                const double *Vf, const double *met, const double *bg, double *E);
 // Interface fluxes of direction d, and Mom2Face of the same faces into
 // vf's three planes of direction d
-void launch_flux(hipStream_t s, int d, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
-                 const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
+void launch_flux(hipStream_t s, int d, int form, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                 const double *met, const double *bg, double *gf, double *mf, double *vf);
 // All three directions (forms of the three slots, face boxes b[3]) and, with
 // MHD, the Mom2Face rim in one launch; flux3_ok: the forms allow it
 bool flux3_ok(const int *form);
-void launch_flux3(hipStream_t s, const int *form, const Geo &g, const MParm &m, const Box *b, const double *H,
-                  const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
+void launch_flux3(hipStream_t s, const int *form, const Geo &g, const MParm &m, const Box *b, const HalfSrc &h,
+                  const double *met, const double *bg, double *gf, double *mf, double *vf);
 // the three edge directions (edge boxes b[3]) in one launch, if the plans of
 // the three slots allow it
 bool emf3_ok(const int *plan);
-void launch_emf3(hipStream_t s, const Geo &g, const MParm &m, const Box *b, const Clock *clk,
-                 const double *H, const double *S, const double *Vf, const double *met, const double *bg, double *E);
+void launch_emf3(hipStream_t s, const Geo &g, const MParm &m, const Box *b, const HalfSrc &h, const double *Vf,
+                 const double *met, const double *bg, double *E);
 // one face direction each, one source file each
-void launch_flux_i(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
-                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
-void launch_flux_j(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
-                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
-void launch_flux_k(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
-                   const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf);
+void launch_flux_i(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                   const double *met, const double *bg, double *gf, double *mf, double *vf);
+void launch_flux_j(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                   const double *met, const double *bg, double *gf, double *mf, double *vf);
+void launch_flux_k(hipStream_t s, int form, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                   const double *met, const double *bg, double *gf, double *mf, double *vf);
 void launch_update(hipStream_t s, int ax, const Geo &g, const MParm &m, const Box &fb, const Box &ctb,
                    const Box *eboxes, const Box &ab, const Box &dtb, Clock *clk, const double *So,
-                   double *Sn, const double *gf, const double *mf, const double *met, const double *bg);
+                   double *Sn, bool writeW, const double *gf, const double *mf, const double *met,
+                   const double *bg);
 void launch_calc_dt(hipStream_t s, const Geo &g, const MParm &m, const Box &dtb, Clock *clk,
                     const double *S, const double *met, const double *bg);
 // Clock fields set from the host: State%time (st) or oState%time; Model%t,
@@ -127,7 +138,8 @@ void launch_bflux2fld(hipStream_t s, const Geo &g, const Box &cb, const Box &ski
                       double *B, const double *met);
 // EnforceBCs of S: alone (field = false) or inside a step, with cell B of
 // the ghost cells from their faces and, with finmode, launch_finalize's work
-void launch_bcs(hipStream_t s, const int *kind, bool field, int finmode, const Geo &g, const MParm &m, Clock *clk,
+// writeW: also the primitives (S_W) of every ghost cell
+void launch_bcs(hipStream_t s, const int *kind, bool field, bool writeW, int finmode, const Geo &g, const MParm &m, Clock *clk,
                 const WindDev &w, double *S, const double *met);
 void launch_divb(hipStream_t s, const Geo &g, const Box &ab, const double *mf, const double *bg,
                  int useBG, double *part, int *nparts);

@@ -83,6 +83,22 @@ __device__ __forceinline__ double ab2(double q, double oq, double w)
     return q + w * (q - oq);
 }
 
+// Its weight from the clock at the start of a step (mhdgroup.F90:26-28)
+__device__ __forceinline__ double ab2_weight(const Clock *clk)
+{
+    const double st = clk->st, dtM = clk->dt;
+    double ost = clk->ost;
+    if (fabs(ost - st) < GAM_TINY) ost = st - dtM;
+    return (0.5 * clk->dtA) / (st - ost);
+}
+// Half-state primitive v from the primitives of State and oState
+// (PredictCell, mhdgroup.F90:528-561)
+__device__ __forceinline__ double half_prim(const MParm &m, int v, double q, double oq, double w)
+{
+    const double h = ab2(q, oq, w);
+    return v == DEN ? dmax(h, m.dFloor) : v == PRS ? dmax(h, m.pFloor) : h;
+}
+
 // ---------------------------------------------------------- limiter
 // PDM (recon.F90:275-301) and pdmLR (231-272) of one face's two sides.
 // The reference clips the interpolated value to [q1, q2] and takes back

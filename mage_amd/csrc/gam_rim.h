@@ -16,9 +16,11 @@ struct RimSet {
     int start[7];    // first workgroup of each slab
 };
 
+template <bool DIR>
 struct vface_rim {
     __device__ __forceinline__ void operator()(int w, const Geo &g, const RimSet &r,
-                                               const double *__restrict__ H,
+                                               const double *__restrict__ H, const double *__restrict__ S,
+                                               const double *__restrict__ O, const Clock *clk,
                                                const double *__restrict__ met,
                                                double *__restrict__ Vf) const
     {
@@ -37,22 +39,29 @@ struct vface_rim {
 #pragma unroll
         for (int n = 0; n < 8; n++) v8[n] = vol[c + (n - 4) * s];
         const double Vi = wsum8([&](int n) { return v8[n]; });
-        const double rVi = 1.0 / Vi;
+        const double rVi = gam_rcp(Vi), wt = DIR ? ab2_weight(clk) : 0.0;
 #pragma unroll
         for (int x = 0; x < 3; x++) {
             double q8[8];
 #pragma unroll
-            for (int n = 0; n < 8; n++) q8[n] = wv[x * N3 + c + (n - 4) * s];
+            for (int n = 0; n < 8; n++) {
+                const long p = c + (n - 4) * s;
+                q8[n] = DIR ? v8[n] * ab2(S[(S_W + 1 + x) * N3 + p], O[(S_W + 1 + x) * N3 + p], wt)
+                            : wv[x * N3 + p];
+            }
             Vf[(3 * d + x) * N3 + c] = mom2face(q8, Vi, rVi);
         }
     }
 };
 
+template <bool DIR>
 struct k_vface_rim {
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, RimSet r, const double *__restrict__ H,
-                                               const double *__restrict__ met, double *__restrict__ Vf) const
+                                               const double *__restrict__ S, const double *__restrict__ O,
+                                               const Clock *clk, const double *__restrict__ met,
+                                               double *__restrict__ Vf) const
     {
-        vface_rim{}((int)bi.x, g, r, H, met, Vf);
+        vface_rim<DIR>{}((int)bi.x, g, r, H, S, O, clk, met, Vf);
     }
 };
 

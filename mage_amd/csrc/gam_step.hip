@@ -2,7 +2,12 @@
 //
 // Kernel sequence of one stepGamera (gamapp.F90:73-113):
 //   k_predict    Predictor: AB2 face fluxes, half-step B and gas, plus the
-//                primitives used by the flux sweeps
+//                primitives used by the flux sweeps.  Only where the fluxes
+//                and EMFs cannot form the half state themselves (HalfSrc):
+//                without MHD, in the first two steps of a state that was put,
+//                and in the adjoint.  It moves 50 words per point, the step
+//                without it 8 more; 256x256x384 shell 14.46 -> 12.80 ms per
+//                step, 96x96x128 0.784 -> 0.691, 16^3 box 0.035 -> 0.032.
 //   k_flux_t     Lyon gas/magnetic fluxes, one per direction, and the face
 //                velocities (Mom2Face) of the same faces (gam_flux.h)
 //   k_vface_rim  face velocities the EMF stencils read past the flux faces
@@ -61,18 +66,14 @@ struct k_predict {
                                                const double *__restrict__ S,
                                                const double *__restrict__ O,
                                                const double *__restrict__ met,
-                                               double *__restrict__ H) const
+                                               double *__restrict__ H, int hfonly) const
     {
         TILE_IJK(fb);
         const long N3 = g.N3;
         const long c = IX(g, i, j, k);
         const unsigned oc = (unsigned)(c * 8);    // byte offset of the point
-        const double st = clk->st, dtM = clk->dt;
-        double ost = clk->ost;
-        if (fabs(ost - st) < GAM_TINY) ost = st - dtM;   // mhdgroup.F90:26-28
-        const double odt = st - ost;
-        const double pdt = 0.5 * clk->dtA;
-        const double w = pdt / odt;
+        // hfonly: the half state alone (H_GAS, H_MF, H_B) of the last step
+        const double w = hfonly ? clk->whf : ab2_weight(clk);
 
         double f[3];
 #pragma unroll
@@ -113,6 +114,7 @@ struct k_predict {
         p2c_cell(m, pW, pQ);
 #pragma unroll
         for (int v = 0; v < 5; v++) stp(H + (H_GAS + v) * N3, oc, pQ[v]);
+        if (hfonly) return;
         // primitives of the reconstruction stencils (half state), stored
         // multiplied by the cell volume: every use is the volume-weighted
         // interpolation <V q>/<V> (recon.F90:125-198, fields.F90:262-270), and
@@ -199,7 +201,7 @@ struct k_update {
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m,
                                                Tile ft, Box ctb, EdgeBoxes eb, Box ab, Box dtb,
                                                Clock *clk, const double *__restrict__ So,
-                                               double *__restrict__ Sn,
+                                               double *__restrict__ Sn, int writeW,
                                                const double *__restrict__ gflx,
                                                const double *__restrict__ mflx,
                                                const double *__restrict__ met,
@@ -327,6 +329,13 @@ struct k_update {
             }
 #pragma unroll
             for (int v = 0; v < 5; v++) stp(Sn + (S_GAS + v) * N3, oc, U[v]);
+            // primitives of the active cells (the boundary launch adds the ghosts')
+            if (writeW && in_box(ab, i, j, k)) {
+                double W[5];
+                c2p_cell(m, U, W);
+#pragma unroll
+                for (int v = 0; v < 5; v++) stp(Sn + (S_W + v) * N3, oc, W[v]);
+            }
             if (in_box(dtb, i, j, k)) {
                 double bx = Bn[0], by = Bn[1], bz = Bn[2];
                 if (BG) {
@@ -481,51 +490,52 @@ int plan_candidates(int slot, int *vals)
 }
 
 void launch_predict(hipStream_t s, int plan, const Geo &g, const MParm &m, const Box &fb, const Clock *clk,
-                    const double *S, const double *O, const double *met, double *H)
+                    const double *S, const double *O, const double *met, double *H, int hfonly)
 {
     const int ch = plan_chunk(plan);
     const Tile t = tile_of(fb, plan_ax(plan), ch);
-    if (ch == 512) launch_f<k_predict<512>>(tgrid(t), dim3(BX, 8), s, g, m, t, clk, S, O, met, H);
-    else if (ch == 128) launch_f<k_predict<128>>(tgrid(t), dim3(BX, 2), s, g, m, t, clk, S, O, met, H);
-    else launch_f<k_predict<>>(tgrid(t), dim3(BX, BY), s, g, m, t, clk, S, O, met, H);
+    if (ch == 512) launch_f<k_predict<512>>(tgrid(t), dim3(BX, 8), s, g, m, t, clk, S, O, met, H, hfonly);
+    else if (ch == 128) launch_f<k_predict<128>>(tgrid(t), dim3(BX, 2), s, g, m, t, clk, S, O, met, H, hfonly);
+    else launch_f<k_predict<>>(tgrid(t), dim3(BX, BY), s, g, m, t, clk, S, O, met, H, hfonly);
 }
 
-void launch_flux(hipStream_t s, int d, int form, const Geo &g, const MParm &m, const Box &b, const double *H,
-                 const double *S, const double *met, const double *bg, double *gf, double *mf, double *vf)
+void launch_flux(hipStream_t s, int d, int form, const Geo &g, const MParm &m, const Box &b, const HalfSrc &h,
+                 const double *met, const double *bg, double *gf, double *mf, double *vf)
 {
-    (d == 0 ? launch_flux_i : d == 1 ? launch_flux_j : launch_flux_k)(s, form, g, m, b, H, S, met, bg, gf, mf, vf);
+    (d == 0 ? launch_flux_i : d == 1 ? launch_flux_j : launch_flux_k)(s, form, g, m, b, h, met, bg, gf, mf, vf);
 }
 
 template <bool BG, bool BO>
 static void update_t(hipStream_t s, int plan, const Geo &g, const MParm &m, const Box &fb, const Box &ctb,
                      const EdgeBoxes &eb, const Box &ab, const Box &dtb, Clock *clk, const double *So,
-                     double *Sn, const double *gf, const double *mf, const double *met, const double *bg)
+                     double *Sn, int writeW, const double *gf, const double *mf, const double *met,
+                     const double *bg)
 {
     const int ch = plan_chunk(plan);
     const Tile t = tile_of(fb, plan_ax(plan), ch);
     if (ch == 512)
-        launch_f<k_update<BG, BO, 512>>(tgrid(t), dim3(BX, 8), s, g, m, t, ctb, eb, ab, dtb, clk, So, Sn, gf, mf,
+        launch_f<k_update<BG, BO, 512>>(tgrid(t), dim3(BX, 8), s, g, m, t, ctb, eb, ab, dtb, clk, So, Sn, writeW, gf, mf,
                                         met, bg);
     else if (ch == 128)
-        launch_f<k_update<BG, BO, 128>>(tgrid(t), dim3(BX, 2), s, g, m, t, ctb, eb, ab, dtb, clk, So, Sn, gf, mf,
+        launch_f<k_update<BG, BO, 128>>(tgrid(t), dim3(BX, 2), s, g, m, t, ctb, eb, ab, dtb, clk, So, Sn, writeW, gf, mf,
                                         met, bg);
     else
-        launch_f<k_update<BG, BO>>(tgrid(t), dim3(BX, BY), s, g, m, t, ctb, eb, ab, dtb, clk, So, Sn, gf, mf, met,
-                                   bg);
+        launch_f<k_update<BG, BO>>(tgrid(t), dim3(BX, BY), s, g, m, t, ctb, eb, ab, dtb, clk, So, Sn, writeW, gf, mf,
+                                   met, bg);
 }
 
 void launch_update(hipStream_t s, int plan, const Geo &g, const MParm &m, const Box &fb, const Box &ctb,
                    const Box *eboxes, const Box &ab, const Box &dtb, Clock *clk, const double *So,
-                   double *Sn, const double *gf, const double *mf, const double *met, const double *bg)
+                   double *Sn, bool writeW, const double *gf, const double *mf, const double *met, const double *bg)
 {
     EdgeBoxes eb;
     for (int d = 0; d < 3; d++) eb.e[d] = eboxes[d];
     const int sel = (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
     switch (sel) {
-    case 0: update_t<false, false>(s, plan, g, m, fb, ctb, eb, ab, dtb, clk, So, Sn, gf, mf, met, bg); break;
-    case 1: update_t<false, true>(s, plan, g, m, fb, ctb, eb, ab, dtb, clk, So, Sn, gf, mf, met, bg); break;
-    case 2: update_t<true, false>(s, plan, g, m, fb, ctb, eb, ab, dtb, clk, So, Sn, gf, mf, met, bg); break;
-    default: update_t<true, true>(s, plan, g, m, fb, ctb, eb, ab, dtb, clk, So, Sn, gf, mf, met, bg); break;
+    case 0: update_t<false, false>(s, plan, g, m, fb, ctb, eb, ab, dtb, clk, So, Sn, writeW, gf, mf, met, bg); break;
+    case 1: update_t<false, true>(s, plan, g, m, fb, ctb, eb, ab, dtb, clk, So, Sn, writeW, gf, mf, met, bg); break;
+    case 2: update_t<true, false>(s, plan, g, m, fb, ctb, eb, ab, dtb, clk, So, Sn, writeW, gf, mf, met, bg); break;
+    default: update_t<true, true>(s, plan, g, m, fb, ctb, eb, ab, dtb, clk, So, Sn, writeW, gf, mf, met, bg); break;
     }
 }
 
