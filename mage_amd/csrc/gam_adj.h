@@ -270,43 +270,43 @@ __device__ __forceinline__ void recon_lr_w_adj(double pdmb, double rVi, const do
 }
 
 // ---------------------------------------------------------- gas flux
-// One side of GasKinFlux (gas_kin): aF = adjoint of the flux contribution
-// gF (5), adW (may be null) that of the HOGS difference dW (5); adds into
-// aW (5).
-__device__ __forceinline__ void gas_kin_adj(double igm1, double s, const double *W, const double *T,
-                                            const double *aF, double *aW, const double *adW = nullptr)
+// One side of GasKinFlux (gas_kin_vt): N = the face normal, vt = the
+// velocity's part along the face, aF = adjoint of the flux contribution gF
+// (5), at = its momentum part along the face, adW (may be null) the adjoint
+// of the HOGS difference dW (5); adds into aW (5).
+__device__ __forceinline__ void gas_kin_adj_vt(double igm1, double s, const double *W, const double *N,
+                                               const double *vt, const double *aF, const double *at,
+                                               double *aW, const double *adW)
 {
     const double d = W[DEN], p = W[PRS], vx = W[1], vy = W[2], vz = W[3];
     const double e = 0.5 * d * (vx * vx + vy * vy + vz * vz) + p * igm1;
-    const double lam = d / (2 * p);
-    const double rl = rsqrt(lam);
-    const double sl = lam * rl;   // sqrt(lam)
-    const double vn = T[0] * vx + T[1] * vy + T[2] * vz;
-    const double vt1 = T[3] * vx + T[4] * vy + T[5] * vz;
-    const double vt2 = T[6] * vx + T[7] * vy + T[8] * vz;
+    const double id = gam_rcp(d);
+    double rl, sl;   // 1/sqrt(lam), sqrt(lam); lam = d / (2 p)
+    gam_sqrt_rsqrt(2 * p * id, rl, sl);
+    const double vn = N[0] * vx + N[1] * vy + N[2] * vz;
     const double z = s * sl * vn;
     double ez;
     const double vn0 = 0.5 * gam_erfc_exp(z, ez);
     const double vn1 = vn * vn0 - 0.5 * s * ez * (rl * GAM_RSQRT_PI);
-    // flux = (d vn1, T.(fn, ft1, ft2), (e + p/2) vn1 + p vn0 vn / 2)
-    const double afn = T[0] * aF[MOMX] + T[1] * aF[MOMY] + T[2] * aF[MOMZ];
-    const double aft1 = T[3] * aF[MOMX] + T[4] * aF[MOMY] + T[5] * aF[MOMZ];
-    const double aft2 = T[6] * aF[MOMX] + T[7] * aF[MOMY] + T[8] * aF[MOMZ];
+    // flux = (d vn1, N (d vn1 vn + p vn0) + d vn1 vt, (e + p/2) vn1 + p vn0 vn / 2)
+    const double afn = N[0] * aF[MOMX] + N[1] * aF[MOMY] + N[2] * aF[MOMZ];
+    const double aft = vt[0] * aF[MOMX] + vt[1] * aF[MOMY] + vt[2] * aF[MOMZ];
     const double aE = aF[ENER];
-    double avn1 = d * aF[DEN] + (e + 0.5 * p) * aE + d * vn * afn + d * vt1 * aft1 + d * vt2 * aft2;
+    const double a1 = aF[DEN] + vn * afn + aft;
+    const double avn1 = d * a1 + (e + 0.5 * p) * aE;
     double avn0 = 0.5 * p * vn * aE + p * afn;
     double avn = 0.5 * p * vn0 * aE + d * vn1 * afn;
     double ae = vn1 * aE;
     double ap = 0.5 * vn1 * aE + 0.5 * vn0 * vn * aE + vn0 * afn;
-    double ad = vn1 * aF[DEN] + vn * vn1 * afn + vt1 * vn1 * aft1 + vt2 * vn1 * aft2;
-    const double avt1 = d * vn1 * aft1, avt2 = d * vn1 * aft2;
-    double ae2 = 0.0, avx = 0.0, avy = 0.0, avz = 0.0;
+    double ad = vn1 * a1;
+    const double avt = d * vn1;
+    double avx = 0.0, avy = 0.0, avz = 0.0;
     if (adW) {   // dW += s (d, d v, e)
         ad += s * (adW[DEN] + vx * adW[MOMX] + vy * adW[MOMY] + vz * adW[MOMZ]);
         avx = s * d * adW[MOMX];
         avy = s * d * adW[MOMY];
         avz = s * d * adW[MOMZ];
-        ae2 = s * adW[ENER];
+        ae += s * adW[ENER];
     }
     // vn1 = vn vn0 - s ez rl / (2 sqrt(pi))
     avn += vn0 * avn1;
@@ -318,19 +318,29 @@ __device__ __forceinline__ void gas_kin_adj(double igm1, double s, const double 
     // z = s sqrt(lam) vn
     avn += s * sl * az;
     const double asl = s * vn * az;
-    const double alam = asl * 0.5 * rl - 0.5 * rl / lam * arl;
-    // lam = d / (2 p)
-    ad += alam / (2 * p);
-    ap += -lam / p * alam;
+    // sl = sqrt(lam), rl = 1/sqrt(lam), lam = d / (2 p): 1/(2 p) = lam / d
+    const double lam = sl * sl;
+    const double lid = lam * (0.5 * rl * (asl - rl * rl * arl)) * id;   // lam alam / d
+    ad += lid;
+    ap -= 2 * lam * lid;
     // e = d |v|^2 / 2 + p igm1
-    ae += ae2;
     ad += 0.5 * (vx * vx + vy * vy + vz * vz) * ae;
     ap += igm1 * ae;
     aW[DEN] += ad;
     aW[PRS] += ap;
-    aW[1] += d * vx * ae + T[0] * avn + T[3] * avt1 + T[6] * avt2 + avx;
-    aW[2] += d * vy * ae + T[1] * avn + T[4] * avt1 + T[7] * avt2 + avy;
-    aW[3] += d * vz * ae + T[2] * avn + T[5] * avt1 + T[8] * avt2 + avz;
+    aW[1] += d * vx * ae + N[0] * avn + avt * at[0] + avx;
+    aW[2] += d * vy * ae + N[1] * avn + avt * at[1] + avy;
+    aW[3] += d * vz * ae + N[2] * avn + avt * at[2] + avz;
+}
+
+// the same with the face's triad T (gas_kin)
+__device__ __forceinline__ void gas_kin_adj(double igm1, double s, const double *W, const double *T,
+                                            const double *aF, double *aW, const double *adW = nullptr)
+{
+    double vt[3], at[3];
+    face_tangent(T, W, vt);
+    face_tangent(T, aF, at);
+    gas_kin_adj_vt(igm1, s, W, T, vt, aF, at, aW, adW);
 }
 
 // ---------------------------------------------------------- magnetic flux
@@ -344,7 +354,7 @@ __device__ __forceinline__ void mag_kin_adj(const MParm &m, double s, const doub
                                             double *aB, double &aBn)
 {
     const double d = W[DEN], p = W[PRS];
-    const double id = 1.0 / d;
+    const double id = gam_rcp(d);
     const double b[3] = {B[0], B[1], B[2]};
     const double dPb = 0.5 * (b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
     double t[3] = {b[0], b[1], b[2]};
@@ -352,14 +362,13 @@ __device__ __forceinline__ void mag_kin_adj(const MParm &m, double s, const doub
         for (int x = 0; x < 3; x++) t[x] += B0[x];
     const double tt = t[0] * t[0] + t[1] * t[1] + t[2] * t[2];
     const double va2 = BG ? tt * id : 2 * dPb * id;
-    const double den = 1 + va2 * m.iCa2;
-    const double vac2 = BORIS ? va2 / den : va2;
+    const double iden = gam_rcp(1 + va2 * m.iCa2);
+    const double vac2 = BORIS ? va2 * iden : va2;
     const double n[3] = {T[0], T[1], T[2]};
     const double vn = n[0] * W[1] + n[1] * W[2] + n[2] * W[3];
-    const double lam = 1 / (2 * p * id + vac2);
-    const double sl = sqrt(lam);
+    double ic, sl, ez;   // sl = sqrt(lam), ic = 1/sl; 1/lam = 2 p/d + vac2
+    gam_sqrt_rsqrt(2 * p * id + vac2, ic, sl);
     const double z = s * sl * vn;
-    double ez;
     const double vn0 = 0.5 * gam_erfc_exp(z, ez);
     const double bdb0 = BG ? B0[0] * b[0] + B0[1] * b[1] + B0[2] * b[2] : 0.0;
     double avn0 = 0.0, ndot = 0.0, bdot = 0.0;
@@ -383,15 +392,17 @@ __device__ __forceinline__ void mag_kin_adj(const MParm &m, double s, const doub
     double at[3] = {0.0, 0.0, 0.0};
     for (int x = 0; x < 3; x++) at[x] = abbD * t[x];
     // VaD += sqrt(vac2) / 2
-    double avac2 = (vac2 > 0.0) ? 0.25 / sqrt(vac2) * aVaD : 0.0;
+    double sva, iva;
+    gam_sqrt_rsqrt(vac2, sva, iva);
+    double avac2 = (vac2 > 0.0) ? 0.25 * iva * aVaD : 0.0;
     const double az = -GAM_RSQRT_PI * ez * avn0;
     const double avn = s * sl * az;
-    const double alam = (s * vn * az) * 0.5 / sl;
-    const double aX = -lam * lam * alam;
+    // alam = s vn az / (2 sl), aX = -lam^2 alam
+    const double aX = -0.5 * (s * vn * az) * (sl * sl) * sl;
     const double ap = 2 * id * aX;
     double aid = 2 * p * aX;
     avac2 += aX;
-    const double ava2 = BORIS ? avac2 / (den * den) : avac2;
+    const double ava2 = BORIS ? avac2 * (iden * iden) : avac2;
     if (BG) {
         const double att = id * ava2;
         aid += tt * ava2;

@@ -24,8 +24,7 @@
 // the forward steps (k_dtmin_part / k_dtmin_record: the argmin cell and its
 // values before the boundary pass) and k_dt_inject carries the next step's
 // value back through it.
-#include "gam_adj.h"
-#include "gam_kernels.h"
+#include "gam_adj_flux.h"
 
 #define ABX 64
 #define ABY 4
@@ -835,136 +834,13 @@ __global__ __launch_bounds__(256) void k_update_adj_faces(Geo g, Box fb, Box ab,
                 ? dtA * (fa(0, i, j, k) - fa(0, i, j - 1, k) + fa(1, i - 1, j, k) - fa(1, i, j, k)) : 0.0;
 }
 
-// Interface fluxes' transpose with the magnetic terms: gas and magnetic
-// kinetic fluxes (background-field cross terms, Boris factor), HOGS, the
-// Boris mag-HOGS and nuke terms, L/R states of gas (H_WH, H_WN) and cell B
-// (H_B weighted by volume, limiter S_B), the normal flux Bn = H_MF / A.
-template <int D, int RM, bool BG, bool BORIS>
-__global__ __launch_bounds__(256, 2) void k_flux_adj_mhd(Geo g, MParm m, Box fb,
-                                                      const double *__restrict__ H,
-                                                      const double *__restrict__ S,
-                                                      const double *__restrict__ met,
-                                                      const double *__restrict__ bg,
-                                                      const double *__restrict__ ag,
-                                                      const double *__restrict__ amf,
-                                                      double *__restrict__ sc,
-                                                      double *__restrict__ aHMF,
-                                                      double *__restrict__ aHG)
-{
-    POINT_SLAB(fb);
-    const long N3 = g.N3;
-    const long c = IX(g, i, j, k);
-    const long s = STRIDE<D>(g);
-    // stencil point n of a plane: a 32-bit byte offset from the plane base
-    // (as k_flux), formed where it is used rather than kept in registers
-    // through the kernel; along i plain indexing lets the compiler merge
-    // neighbouring points
-    const unsigned oc = (unsigned)(c * 8), os = (unsigned)(s * 8);
-    auto LD = [&](const double *__restrict__ plane, int n) -> double {
-        if (D == 0) return plane[c + (n - 4)];
-        return ldp(plane, oc + (unsigned)(n - 4) * os);
-    };
-    double vol[8];
-    for (int n = 0; n < 8; n++) vol[n] = LD(met + M_VOL * N3, n);
-    const double rVi = 1.0 / wsum8([&](int n) { return vol[n]; });
-    double WL[5], WR[5], BL[3], BR[3];
-    for (int v = 0; v < 5; v++) {
-        double qv[8], nq[4];
-        for (int n = 0; n < 8; n++) qv[n] = LD(H + (H_WH + v) * N3, n);
-        for (int n = 0; n < 4; n++) nq[n] = LD(H + (H_WN + v) * N3, n + 2);
-        recon_lr_w<RM>(m.pdmb, rVi, nq, qv, WL[v], WR[v]);
-    }
-    const double *Bl = m.doLFM ? S + S_B * N3 : H + H_B * N3;
-    for (int x = 0; x < 3; x++) {
-        double q[8], nq[4];
-        for (int n = 0; n < 8; n++) q[n] = LD(H + (H_B + x) * N3, n);
-        for (int n = 0; n < 4; n++) nq[n] = LD(Bl + x * N3, n + 2);
-        recon_lr<RM>(m.pdmb, vol, rVi, nq, q, BL[x], BR[x]);
-    }
-    double T[9];
-    for (int q = 0; q < 9; q++) T[q] = ldp(met + (M_TF + q + 9 * D) * N3, oc);
-    const double faB = ldp(met + (M_FACE + D) * N3, oc);
-    const double iFaB = 1.0 / faB;
-    const double Bn = ldp(H + (H_MF + D) * N3, oc) * iFaB;
-    double B0[3] = {0, 0, 0}, B0n = 0.0;
-    if (BG) {
-        for (int x = 0; x < 3; x++) B0[x] = ldp(bg + (B_FCB0 + x + 3 * D) * N3, oc);
-        B0n = ldp(bg + (B_BFLUX0 + D) * N3, oc) * iFaB;
-    }
-    // forward pieces the adjoint needs: VaD, bbD and the HOGS differences dW
-    double mF[3] = {0, 0, 0}, bbD = 0.0, VaD = 0.0;
-    mag_kin<BG, BORIS>(m, -1.0, WL, BL, Bn, T, B0, B0n, mF, bbD, VaD);
-    mag_kin<BG, BORIS>(m, +1.0, WR, BR, Bn, T, B0, B0n, mF, bbD, VaD);
-    double gF[5] = {0, 0, 0, 0, 0}, dW[5] = {0, 0, 0, 0, 0};
-    gas_kin(m.igm1, -1.0, WL, T, gF, dW);
-    gas_kin(m.igm1, +1.0, WR, T, gF, dW);
-    // adjoint
-    double aF[5], adW[5], aM[3], aVaD = 0.0, abbD = 0.0;
-    double aL[5] = {0, 0, 0, 0, 0}, aR[5] = {0, 0, 0, 0, 0}, abL[3] = {0, 0, 0}, abR[3] = {0, 0, 0}, aBn = 0.0;
-    for (int v = 0; v < 5; v++) {
-        aF[v] = faB * ldp(ag + (v + 5 * D) * N3, oc);
-        adW[v] = -m.cHogH * VaD * aF[v];
-        aVaD += -m.cHogH * dW[v] * aF[v];
-    }
-    for (int x = 0; x < 3; x++) aM[x] = faB * ldp(amf + (x + 3 * D) * N3, oc);
-    if (BORIS) {
-        // mag-HOGS: mF -= cHogM VaD bbD (WR - WL)_v / Ca^2
-        for (int x = 0; x < 3; x++) {
-            const double dv = WR[1 + x] - WL[1 + x];
-            const double deeP = bbD * dv * m.iCa2;
-            aVaD += -m.cHogM * deeP * aM[x];
-            const double adeeP = -m.cHogM * VaD * aM[x];
-            abbD += dv * m.iCa2 * adeeP;
-            aR[1 + x] += bbD * m.iCa2 * adeeP;
-            aL[1 + x] -= bbD * m.iCa2 * adeeP;
-        }
-        // nuke: gF -= Ca (U(c) - U(c - s)) where the mean speed is large
-        const double vL = sqrt(WL[1] * WL[1] + WL[2] * WL[2] + WL[3] * WL[3]);
-        const double vR = sqrt(WR[1] * WR[1] + WR[2] * WR[2] + WR[3] * WR[3]);
-        const double vn = sqrt(vL * vL + vR * vR) / GAM_SQRT2_SP;
-        if (vn >= 1.5 * m.Ca)
-            for (int v = 0; v < 5; v++) {
-                AADD(aHG + v * N3 + c, -m.Ca * aF[v]);
-                AADD(aHG + v * N3 + c - s, m.Ca * aF[v]);
-            }
-    }
-    gas_kin_adj(m.igm1, -1.0, WL, T, aF, aL, adW);
-    gas_kin_adj(m.igm1, +1.0, WR, T, aF, aR, adW);
-    mag_kin_adj<BG, BORIS>(m, -1.0, WL, BL, Bn, T, B0, B0n, aM, aVaD, abbD, aL, abL, aBn);
-    mag_kin_adj<BG, BORIS>(m, +1.0, WR, BR, Bn, T, B0, B0n, aM, aVaD, abbD, aR, abR, aBn);
-    AADD(aHMF + D * N3 + c, aBn * iFaB);
-    // the reconstructions' transposes up to their linear stencils: per
-    // variable (gas 5, then B 3) the stencil scalars sl, sr and the four
-    // limiter adjoints, gathered into the cells by k_recon_adj_gather
-    for (int v = 0; v < 5; v++) {
-        double qv[8], nq[4], anq[4] = {0, 0, 0, 0}, sl, sr;
-        for (int n = 0; n < 8; n++) qv[n] = LD(H + (H_WH + v) * N3, n);
-        for (int n = 0; n < 4; n++) nq[n] = LD(H + (H_WN + v) * N3, n + 2);
-        recon_lr_w_adj_s<RM>(m.pdmb, rVi, nq, qv, aL[v], aR[v], anq, sl, sr);
-        *(double2 *)(sc + 6 * v * N3 + 2 * c) = make_double2(sl, sr);
-        for (int n = 0; n < 4; n++) stp(sc + (6 * v + 2 + n) * N3, oc, anq[n]);
-    }
-    for (int x = 0; x < 3; x++) {
-        double qv[8], nq[4], anq[4] = {0, 0, 0, 0}, sl, sr;
-        // the volumes are loaded again (cached) rather than kept live through
-        // the flux adjoint, which holds the kernel's register peak
-        for (int n = 0; n < 8; n++) qv[n] = LD(met + M_VOL * N3, n) * LD(H + (H_B + x) * N3, n);
-        for (int n = 0; n < 4; n++) nq[n] = LD(Bl + x * N3, n + 2);
-        recon_lr_w_adj_s<RM>(m.pdmb, rVi, nq, qv, abL[x], abR[x], anq, sl, sr);
-        const int v = 5 + x;
-        *(double2 *)(sc + 6 * v * N3 + 2 * c) = make_double2(sl, sr);
-        for (int n = 0; n < 4; n++) stp(sc + (6 * v + 2 + n) * N3, oc, anq[n]);
-    }
-}
-
 // The cell side of the reconstruction transposes of the three face
-// directions (k_flux_adj_mhd's scratch, 48 planes per direction) and of
-// Mom2Face (rv, aVf): one thread per cell sums what the faces whose
-// stencils hold it give it, with no atomics, and WRITES the half-state
+// directions (k_flux_adj_mhd's scratch) and of Mom2Face (rv, aVf): one
+// thread per cell adds what the one or two tiles of each direction that
+// reach it left, with no atomics, and WRITES the half-state
 // adjoints aWH (5), aWN (5) and aHB (3) of every cell; with the LFM
 // limiter the B limiter adjoints go into aSSB (3, added).  Faces of
 // direction D exist on the active box extended by one along D.
-template <int RM>
 __global__ __launch_bounds__(256) void k_recon_adj_gather(Geo g, Box cb, const double *__restrict__ sc,
                                                           const double *__restrict__ rv,
                                                           const double *__restrict__ aVf,
@@ -977,6 +853,7 @@ __global__ __launch_bounds__(256) void k_recon_adj_gather(Geo g, Box cb, const d
     const long c = IX(g, i, j, k);
     double gh[8], gn[8], av[3] = {0.0, 0.0, 0.0};
     for (int v = 0; v < 8; v++) gh[v] = gn[v] = 0.0;
+#pragma unroll
     for (int D = 0; D < 3; D++) {
         const long s = D == 0 ? 1 : D == 1 ? (long)g.P : g.PP;
         const int at = D == 0 ? i : D == 1 ? j : k;
@@ -995,29 +872,28 @@ __global__ __launch_bounds__(256) void k_recon_adj_gather(Geo g, Box cb, const d
                       : D == 1 ? (i >= g.is && i <= g.ie && k >= g.ks && k <= g.ke)
                                : (i >= g.is && i <= g.ie && j >= g.js && j <= g.je);
         if (!tr) continue;
-        const double *sd = sc + (long)48 * D * N3;
-#pragma unroll
-        for (int n = 0; n < 8; n++) {
-            const int fi = at - (n - 4);   // this cell is stencil point n of face fi
-            if (fi < lo || fi > hi) continue;
-            const long f = c - (n - 4) * s;
+        // the tiles of the cell's own face and of the first and last face
+        // whose stencils hold it
+        const int x = at - lo, n = hi - lo + 1;
+        const int x0 = x < 0 ? 0 : x < n ? x : n - 1, x1 = x > 3 ? x - 3 : 0, x2 = x + 4 < n ? x + 4 : n - 1;
+        bool two;
+        if (D == 0) {
+            const unsigned p = ((unsigned)(k - g.ks) * (unsigned)(g.je - g.js + 1) + (unsigned)(j - g.js)) * (unsigned)n;
+            const unsigned own = (p + (unsigned)x0) >> 8;
+            two = (p + (unsigned)x1) >> 8 != own || (p + (unsigned)x2) >> 8 != own;
+        } else {
+            two = x1 / FA_L != x0 / FA_L || x2 / FA_L != x0 / FA_L;
+        }
+        const double *sd = sc + (long)FLUXADJ_NPL * D * N3 + c;
+        for (int v = 0; v < 8; v++) {
+            gh[v] += sd[v * N3];
+            gn[v] += sd[(8 + v) * N3];
+        }
+        if (two)
             for (int v = 0; v < 8; v++) {
-                const double2 lr = *(const double2 *)(sd + 6 * v * N3 + 2 * f);
-                if (RM == 1) {
-                    if (n <= 6) gh[v] += UP7(n) * lr.x;
-                    if (n >= 1) gh[v] += UP7(7 - n) * lr.y;
-                } else {
-                    gh[v] += W8(n) * lr.x;
-                }
+                gh[v] += sd[(16 + v) * N3];
+                gn[v] += sd[(24 + v) * N3];
             }
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int fi = at - (q - 2);   // this cell is limiter point q of face fi
-            if (fi < lo || fi > hi) continue;
-            const long f = c - (q - 2) * s;
-            for (int v = 0; v < 8; v++) gn[v] += sd[(6 * v + 2 + q) * N3 + f];
-        }
     }
     for (int v = 0; v < 5; v++) {
         aWH[v * N3 + c] = gh[v] + ((v >= 1 && v <= 3) ? av[v - 1] : 0.0);
@@ -1490,9 +1366,10 @@ static void flux_adj_mhd_r(hipStream_t s, const Geo &g, const MParm &m, const Bo
                            const double *S, const double *met, const double *bg, const double *ag,
                            const double *amf, double *sc, double *aHMF, double *aHG)
 {
+    const AdjTile t = adj_tiles(D, fb);
 #define FLUXADJ(BG, BO)                                                                                      \
-    hipLaunchKernelGGL((k_flux_adj_mhd<D, RM, BG, BO>), agrid_slab(fb), dim3(ABT), 0, s, g, m, fb, H, S, met,      \
-                       bg, ag, amf, sc, aHMF, aHG)
+    hipLaunchKernelGGL((k_flux_adj_mhd<D, RM, BG, BO>), tgrid(t.t), dim3(256), 0, s, g, m, t, H, S, met, bg, ag,   \
+                       amf, sc, aHMF, aHG)
     if (m.doBG && m.doBoris) FLUXADJ(true, true);
     else if (m.doBG) FLUXADJ(true, false);
     else if (m.doBoris) FLUXADJ(false, true);
@@ -1523,12 +1400,8 @@ void launch_recon_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const 
                              double *aSSB)
 {
     const Box cb = cells_of(g);
-    if (m.rmeth)
-        hipLaunchKernelGGL(k_recon_adj_gather<1>, agrid_slab(cb), dim3(ABT), 0, s, g, cb, sc, rv, aVf, met,
-                           m.doLFM ? 1 : 0, aWH, aWN, aHB, aSSB);
-    else
-        hipLaunchKernelGGL(k_recon_adj_gather<0>, agrid_slab(cb), dim3(ABT), 0, s, g, cb, sc, rv, aVf, met,
-                           m.doLFM ? 1 : 0, aWH, aWN, aHB, aSSB);
+    hipLaunchKernelGGL(k_recon_adj_gather, agrid_slab(cb), dim3(ABT), 0, s, g, cb, sc, rv, aVf, met,
+                       m.doLFM ? 1 : 0, aWH, aWN, aHB, aSSB);
 }
 
 template <int ED, int RM, bool BG, bool BO>

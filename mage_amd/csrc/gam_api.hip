@@ -1680,7 +1680,7 @@ struct gam_adj {
     double *ahmf, *ahb;      // adjoints of H_MF, H_B (3 each)
     double *avf, *aur, *adm, *ae;   // Vf (9), Reynolds gas (5), dM (3), E (3)
     double *rv;              // Mom2Face normalisation per face direction (3)
-    double *fsc;             // flux-transpose scratch, 48 planes per face direction (MHD)
+    double *fsc;             // flux-transpose scratch, FLUXADJ_NPL planes per face direction (MHD)
     double *esc;             // EMF-transpose scratch, 16 planes per edge direction (MHD);
                              // the first planes of fsc: the EMF gather has read it before
                              // the flux transpose writes fsc
@@ -1794,7 +1794,7 @@ extern "C" int gam_adj_create_budget(gam_adj **out, gam_ctx *c, int nsteps, int 
     AALLOC(a->wgt, pl);
     AALLOC(a->part, pl);
     AALLOC(a->rv, 3 * pl);
-    if (c->mp.doMHD) AALLOC(a->fsc, 3 * 48 * pl);
+    if (c->mp.doMHD) AALLOC(a->fsc, 3 * FLUXADJ_NPL * pl);
     a->esc = a->fsc;
     for (int sd = 0; sd < 6; sd++)
         if (c->model.bc[sd] == GAM_BC_WIND) a->nw = c->wd.n;
@@ -2049,7 +2049,7 @@ static void adj_step(gam_adj *a, int n, const StepIT *it, const double *Sn, cons
             Box fb = act_box(g);
             if (d == 0) fb.i1 += 1; else if (d == 1) fb.j1 += 1; else fb.k1 += 1;
             launch_flux_adj_mhd(s, d, g, c->mp, fb, H, Sn, c->met, c->bg, a->ag, a->amf,
-                                a->fsc + (size_t)48 * d * N3, a->ahmf, a->ahg);
+                                a->fsc + (size_t)FLUXADJ_NPL * d * N3, a->ahmf, a->ahg);
         }
         launch_recon_adj_gather(s, g, c->mp, a->fsc, a->rv, a->avf, c->met, a->awh, a->awn, a->ahb,
                                 lB + S_B * N3);

@@ -204,14 +204,16 @@ void launch_update_adj_mhd(hipStream_t s, const Geo &g, const MParm &m, const Bo
                            const double *gflx, const double *mflx, const double *met, const double *bg,
                            double *aSn, double *aSo, double *aUr, double *adM, double *ag, double *amf,
                            double *aE, double *pdt);
-// pass 1 of the flux transpose: per face, the stencil scalars and limiter
-// adjoints of its 8 reconstructions into sc (48 planes: per variable the
-// pair (sl, sr) interleaved over two planes, then the four limiter
-// adjoints), aBn into aHMF, the Boris nuke term into aHG
+// pass 1 of the flux transpose: per tile of faces, the transposed
+// reconstructions summed over the tile's cells into sc (FLUXADJ_NPL planes:
+// weighted values and limiter values of the 8 variables, from the tile of
+// the cell's own face and from the neighbouring one), aBn into aHMF, the
+// Boris nuke term into aHG
+#define FLUXADJ_NPL 32
 void launch_flux_adj_mhd(hipStream_t s, int d, const Geo &g, const MParm &m, const Box &fb, const double *H,
                          const double *S, const double *met, const double *bg, const double *ag,
                          const double *amf, double *sc, double *aHMF, double *aHG);
-// pass 2 (all three directions' sc, 48 planes each) fused with the Mom2Face
+// pass 2 (all three directions' sc) fused with the Mom2Face
 // transpose: writes aWH, aWN, aHB of every cell
 void launch_recon_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const double *sc, const double *rv,
                              const double *aVf, const double *met, double *aWH, double *aWN, double *aHB,
