@@ -1,5 +1,6 @@
 // gam_emf.hip -- edge EMFs (CalcElecField, fields.F90:70-517).
 #include "gam_launch.h"
+#include <algorithm>
 
 // ====================================================================
 // Edge EMF: GetCornerV/GetCornerD/GetCornerB/EdgeLRs + VxB
@@ -137,7 +138,8 @@ struct k_emf {
 // ====================================================================
 struct EdgeTile {
     int i0, i1, j0, j1, k0, k1;   // edges
-    int ni, n1, nb;               // tiles along i, along the second axis; in all
+    int ni, nb;                   // tiles along i; in all
+    int bfirst;                   // ED = 1: numbered along i, j, k (else along i, the second axis, the third)
     FastDiv qi, q1;
     int xs;
 };
@@ -212,7 +214,8 @@ struct edge_tile {
         const int tid = (int)(threadIdx.x + BX * threadIdx.y);
         const long N3 = g.N3;
         const unsigned r = (unsigned)L / t.qi, r2 = r / t.q1;
-        const int ti = L - (int)r * t.ni, ta = (int)r - (int)r2 * t.n1, tb = (int)r2;
+        const int ti = L - (int)r * t.ni, rq = (int)r - (int)r2 * (int)t.q1.d;
+        const int ta = t.bfirst ? (int)r2 : rq, tb = t.bfirst ? rq : (int)r2;
         const int i0 = t.i0 + ti * G::TX;
         const int j0 = t.j0 + (ED == 0 ? 4 * ta : ED == 2 ? 8 * ta : tb);
         const int k0 = t.k0 + (ED == 0 ? 4 * tb : ED == 1 ? 8 * ta : tb);
@@ -372,26 +375,31 @@ struct k_emf_t {
     }
 };
 
-static inline EdgeTile edge_tiles(int ED, const Box &b)
+static inline EdgeTile edge_tiles(int ED, const Box &b, bool slabs = false)
 {
     EdgeTile t;
     t.i0 = b.i0; t.i1 = b.i1; t.j0 = b.j0; t.j1 = b.j1; t.k0 = b.k0; t.k1 = b.k1;
     const int nj = b.j1 - b.j0 + 1, nk = b.k1 - b.k0 + 1;
     t.ni = ED == 0 ? (b.i1 - b.i0 + 16) / 16 : (b.i1 - b.i0 + 32) / 32;
-    t.n1 = ED == 0 ? (nj + 3) / 4 : ED == 2 ? (nj + 7) / 8 : (nk + 7) / 8;
-    t.nb = t.ni * t.n1 * (ED == 0 ? (nk + 3) / 4 : ED == 2 ? nk : nj);
+    const int n1 = ED == 0 ? (nj + 3) / 4 : ED == 2 ? (nj + 7) / 8 : (nk + 7) / 8;
+    t.nb = t.ni * n1 * (ED == 0 ? (nk + 3) / 4 : ED == 2 ? nk : nj);
     t.qi = fast_div((unsigned)t.ni);
-    t.q1 = fast_div((unsigned)t.n1);
+    t.bfirst = ED == 1 && slabs;
+    t.q1 = fast_div((unsigned)(t.bfirst ? nj : n1));
     t.xs = xcd_shift(t.nb);
     return t;
 }
 
-// The three edge directions in one launch, one range of workgroups after
-// another.  Vf: the face velocities of all three directions; direction eD
+// The three edge directions in one launch, in turn slab by slab along k (as
+// k_flux3): they share face areas, fluxes and densities, which the second and
+// third then find in the memory-side cache.  256x256x384 shell 3.49 -> 3.30
+// ms, 192x192x256 1.33 -> 1.24, 96x96x128 0.182 -> 0.175; slabs of 16 the
+// same, of 24 3.34.  Vf: the face velocities of all three directions; direction eD
 // takes those of the faces along dT1.
 struct Emf3 {
     EdgeTile t[3];
-    int start[2];     // first workgroup of edge direction 1, of direction 2
+    int n[3];         // workgroups of each direction in a slab
+    FastDiv slab;     // by the workgroups of a slab
 };
 
 template <int RM, bool BG, bool BORIS, bool DIR>
@@ -408,12 +416,17 @@ struct k_emf3 {
     {
         __shared__ double lds[EMF_LDS];
         const int w = (int)bi.x;
-        if (w < f.start[0])
-            edge_tile<0, RM, BG, BORIS, DIR>{}(lds, w, g, m, f.t[0], clk, H, S, O, Vf + 3 * g.N3, met, bg, E);
-        else if (w < f.start[1])
-            edge_tile<1, RM, BG, BORIS, DIR>{}(lds, w - f.start[0], g, m, f.t[1], clk, H, S, O, Vf + 6 * g.N3, met, bg, E);
-        else
-            edge_tile<2, RM, BG, BORIS, DIR>{}(lds, w - f.start[1], g, m, f.t[2], clk, H, S, O, Vf, met, bg, E);
+        const int sl = (int)((unsigned)w / f.slab);
+        int r = w - sl * (int)f.slab.d;
+        if (r < f.n[0]) {
+            edge_tile<0, RM, BG, BORIS, DIR>{}(lds, sl * f.n[0] + r, g, m, f.t[0], clk, H, S, O, Vf + 3 * g.N3, met, bg, E);
+        } else if (r < f.n[0] + f.n[1]) {
+            r -= f.n[0];
+            edge_tile<1, RM, BG, BORIS, DIR>{}(lds, sl * f.n[1] + r, g, m, f.t[1], clk, H, S, O, Vf + 6 * g.N3, met, bg, E);
+        } else {
+            r -= f.n[0] + f.n[1];
+            edge_tile<2, RM, BG, BORIS, DIR>{}(lds, sl * f.n[2] + r, g, m, f.t[2], clk, H, S, O, Vf, met, bg, E);
+        }
     }
 };
 
@@ -423,11 +436,16 @@ static void emf3_t(hipStream_t s, const Geo &g, const MParm &m, const Box *b, co
 {
     Emf3 f;
     int tot = 0;
+    const EdgeTile t0 = edge_tiles(0, b[0]);
+    const int ns = t0.nb < 2048 ? 1 : std::min((b[0].k1 - b[0].k0 + 8) / 8, t0.nb / (16 << t0.xs));
     for (int d = 0; d < 3; d++) {
-        f.t[d] = edge_tiles(d, b[d]);
-        tot += (int)xcd_grid(f.t[d].nb, f.t[d].xs);
-        if (d < 2) f.start[d] = tot;
+        f.t[d] = edge_tiles(d, b[d], ns > 1);
+        const int run = 8 << f.t[d].xs;
+        f.n[d] = (f.t[d].nb + ns * run - 1) / (ns * run) * run;
+        tot += f.n[d];
     }
+    f.slab = fast_div((unsigned)tot);
+    tot *= ns;
     const dim3 gr((unsigned)tot), bl(BX, BY);
     if (h.O) launch_f<k_emf3<RM, BG, BO, true>>(gr, bl, s, g, m, f, h.clk, h.H, h.S, h.O, Vf, met, bg, E);
     else launch_f<k_emf3<RM, BG, BO, false>>(gr, bl, s, g, m, f, h.clk, h.H, h.S, h.O, Vf, met, bg, E);

@@ -201,7 +201,8 @@ struct k_flux {
 struct FluxTile {
     Tile t;                       // D = 0: the face rows; D = 1, 2: t.nb and t.xs
     int i0, i1, a0, a1, b0;       // D = 1, 2: faces along i and D, first along the third axis
-    int byD;                      // D = 1, 2: tiles numbered along D first (else along i)
+    int byD;                      // D = 1, 2: tiles numbered along i, D, the third axis (0),
+                                  // along D, i, the third axis (1) or along i, the third, D (2)
     FastDiv q1, q2;               // D = 1, 2: by the tiles of the first and the second of those
     FastDiv q7;                   // D = 0: by ni + 7
 };
@@ -266,10 +267,11 @@ struct flux_tile {
                 oe[q] = (unsigned)(8 * IX(g, t.t.b.i0 - 4 + (int)x, j, k));
             }
         } else {
-            // L runs along i first, or along D first (n1 tiles, byD)
+            // (byD says what x and y run along)
             const unsigned r = (unsigned)L / t.q1, x = (unsigned)L - r * t.q1.d;
             const unsigned r2 = r / t.q2, y = r - r2 * t.q2.d;
-            const int ti = (int)(t.byD ? y : x), ta = (int)(t.byD ? x : y), b = t.b0 + (int)r2;
+            const int ti = (int)(t.byD == 1 ? y : x), ta = (int)(t.byD == 1 ? x : t.byD ? r2 : y);
+            const int b = t.b0 + (int)(t.byD == 2 ? y : r2);
             const int i0 = t.i0 + ti * TI, a0 = t.a0 + ta * TA;
             // a cell past the box reads the last one inside (only lanes of
             // faces outside the box use it)
@@ -447,9 +449,9 @@ struct k_flux_t {
     }
 };
 
-// The tiles of one direction's faces (box b); alt: the other numbering
-// (PLAN_LDS_D)
-static inline FluxTile flux_tiles(int D, const Box &b, bool alt)
+// The tiles of one direction's faces (box b); alt: their numbering (byD;
+// 1: PLAN_LDS_D, for D = 0 the other row order)
+static inline FluxTile flux_tiles(int D, const Box &b, int alt)
 {
     FluxTile t;
     t.t = tile_of(b, D == 0 && alt ? 2 : 1);
@@ -466,7 +468,8 @@ static inline FluxTile flux_tiles(int D, const Box &b, bool alt)
         t.t.nb = nti * nta * (D == 1 ? b.k1 - b.k0 + 1 : b.j1 - b.j0 + 1);
         t.t.xs = xcd_shift(t.t.nb);
         t.q1 = fast_div((unsigned)(alt ? nta : nti));
-        t.q2 = fast_div((unsigned)(alt ? nti : nta));
+        if (alt == 2) t.q1 = fast_div((unsigned)nti);
+        t.q2 = fast_div((unsigned)(alt == 2 ? (D == 1 ? b.k1 - b.k0 + 1 : b.j1 - b.j0 + 1) : alt ? nti : nta));
     }
     return t;
 }
