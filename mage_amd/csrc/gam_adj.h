@@ -535,37 +535,69 @@ struct EdgeAdj {
     double V1[3][8], mH1[8], mL1[4], mH2[8], mL2[4], D4[4];
 };
 
-// forward (k_emf's arithmetic), also returning the pieces the adjoint needs
+// the forward's pieces, in edge_lr's and edge_value's forms
+struct EdgeFwd {
+    double qv1[8], nq1[4], qv2[8], nq2[4], iA1, iA2, l1, r1, l2, r2;   // reconstructions
+    double rdA, v1, v2, ivD;               // corner velocity; 1/|v| (0 for v = 0)
+    double detT, b1, b2, Jd, Xb, Xd, ivA;  // vA = sqrt(X(b^2, D)), Xb, Xd its derivatives, 1/vA
+    double vsum, vDiff, E;
+};
+template <int RM, bool BORIS>
+__device__ __forceinline__ void edge_forward(const MParm &m, const EdgeIn &in, EdgeFwd &f)
+{
+    for (int n = 0; n < 8; n++) {
+        f.qv1[n] = in.mH1[n] * dmin(in.A1[n] * (1.0 / GAM_TINY), 1.0);
+        f.qv2[n] = in.mH2[n] * dmin(in.A2[n] * (1.0 / GAM_TINY), 1.0);
+    }
+    for (int n = 0; n < 4; n++) {
+        f.nq1[n] = in.mL1[n] * gam_rcp(dmax(in.A1[n + 2], GAM_TINY));
+        f.nq2[n] = in.mL2[n] * gam_rcp(dmax(in.A2[n + 2], GAM_TINY));
+    }
+    const double A1i = wsum8([&](int n) { return in.A1[n]; });
+    f.iA1 = gam_rcp(A1i);
+    f.iA2 = gam_rcp(wsum8([&](int n) { return in.A2[n]; }));
+    recon_lr_w<RM>(m.pdmb, f.iA1, f.nq1, f.qv1, f.l1, f.r1);
+    recon_lr_w<RM>(m.pdmb, f.iA2, f.nq2, f.qv2, f.l2, f.r2);
+    f.rdA = gam_rcp(dmax(A1i, GAM_TINY));
+    double vc[3];
+    for (int d = 0; d < 3; d++) vc[d] = in.AV[d] * f.rdA;
+    f.v1 = vc[0] * in.te1[0] + vc[1] * in.te1[1] + vc[2] * in.te1[2];
+    f.v2 = vc[0] * in.te2[0] + vc[1] * in.te2[1] + vc[2] * in.te2[2];
+    const double vv = f.v1 * f.v1 + f.v2 * f.v2;
+    double vD;
+    gam_sqrt_rsqrt(vv, vD, f.ivD);
+    if (!(vv > 0.0)) vD = f.ivD = 0.0;
+    const double Dc = 0.25 * (in.D4[0] + in.D4[1] + in.D4[2] + in.D4[3]);
+    const double bT1 = 0.5 * (f.l1 + f.r1), bT2 = 0.5 * (f.l2 + f.r2);
+    f.Jd = (f.r2 - f.l2) - (f.r1 - f.l1);
+    const double xni = in.tb[0], yni = in.tb[1], xnj = in.tb[2], ynj = in.tb[3];
+    f.detT = gam_rcp(xni * ynj - xnj * yni);
+    f.b1 = f.detT * (ynj * bT1 - yni * bT2) + in.b01;
+    f.b2 = f.detT * (-(xnj * bT1) + xni * bT2) + in.b02;
+    // X = b^2 / D, with Boris Ca^2 b^2 / (Ca^2 D + b^2)
+    const double bb = f.b1 * f.b1 + f.b2 * f.b2, Ca2 = m.Ca * m.Ca;
+    const double iq = gam_rcp(BORIS ? Ca2 * Dc + bb : Dc);
+    const double X = BORIS ? Ca2 * bb * iq : bb * iq;
+    f.Xb = BORIS ? Ca2 * iq * (Ca2 * Dc * iq) : iq;
+    f.Xd = BORIS ? -X * Ca2 * iq : -X * iq;
+    double vA;
+    gam_sqrt_rsqrt(X, vA, f.ivA);
+    if (!(X > 0.0)) vA = f.ivA = 0.0;
+    f.vsum = vD + vA;
+    f.vDiff = dmin(f.vsum, in.cap);
+    f.E = (-(f.v1 * f.b2 - f.v2 * f.b1) + m.Vd0 * f.vDiff * f.Jd) * in.edge;
+}
 template <int RM, bool BORIS>
 __device__ __forceinline__ double edge_emf(const MParm &m, const EdgeIn &in, double *l1, double *r1,
                                            double *l2, double *r2)
 {
-    const double rdA = 1.0 / dmax(wsum8([&](int n) { return in.A1[n]; }), GAM_TINY);
-    double vc[3];
-    for (int d = 0; d < 3; d++) vc[d] = in.AV[d] * rdA;
-    const double v1 = vc[0] * in.te1[0] + vc[1] * in.te1[1] + vc[2] * in.te1[2];
-    const double v2 = vc[0] * in.te2[0] + vc[1] * in.te2[1] + vc[2] * in.te2[2];
-    double vDiff = sqrt(v1 * v1 + v2 * v2);
-    const double Dc = 0.25 * (in.D4[0] + in.D4[1] + in.D4[2] + in.D4[3]);
-    double q[8], nq[4];
-    for (int n = 0; n < 8; n++) q[n] = in.mH1[n] / dmax(in.A1[n], GAM_TINY);
-    for (int n = 0; n < 4; n++) nq[n] = in.mL1[n] / dmax(in.A1[n + 2], GAM_TINY);
-    const double Vi1 = wsum8([&](int n) { return in.A1[n]; });
-    recon_lr<RM>(m.pdmb, in.A1, 1.0 / Vi1, nq, q, *l1, *r1);
-    for (int n = 0; n < 8; n++) q[n] = in.mH2[n] / dmax(in.A2[n], GAM_TINY);
-    for (int n = 0; n < 4; n++) nq[n] = in.mL2[n] / dmax(in.A2[n + 2], GAM_TINY);
-    const double Vi2 = wsum8([&](int n) { return in.A2[n]; });
-    recon_lr<RM>(m.pdmb, in.A2, 1.0 / Vi2, nq, q, *l2, *r2);
-    const double bT1 = 0.5 * (*l1 + *r1), bT2 = 0.5 * (*l2 + *r2);
-    const double Jd = (*r2 - *l2) - (*r1 - *l1);
-    const double xni = in.tb[0], yni = in.tb[1], xnj = in.tb[2], ynj = in.tb[3];
-    const double detT = 1.0 / (xni * ynj - xnj * yni);
-    const double b1 = detT * (ynj * bT1 - yni * bT2) + in.b01;
-    const double b2 = detT * (-(xnj * bT1) + xni * bT2) + in.b02;
-    double vA = sqrt(b1 * b1 + b2 * b2) / sqrt(Dc);
-    if (BORIS) vA = m.Ca * vA / sqrt(m.Ca * m.Ca + vA * vA);
-    vDiff = dmin(vDiff + vA, in.cap);
-    return (-(v1 * b2 - v2 * b1) + m.Vd0 * vDiff * Jd) * in.edge;
+    EdgeFwd f;
+    edge_forward<RM, BORIS>(m, in, f);
+    *l1 = f.l1;
+    *r1 = f.r1;
+    *l2 = f.l2;
+    *r2 = f.r2;
+    return f.E;
 }
 
 // edge_emf's transpose up to its linear stencils (gathered by the cell and
@@ -584,67 +616,32 @@ struct EdgeAdjS {
 template <int RM, bool BORIS>
 __device__ __forceinline__ void edge_emf_adj_s(const MParm &m, const EdgeIn &in, double aE, EdgeAdjS &o)
 {
-    double l1, r1, l2, r2;
-    o.E = edge_emf<RM, BORIS>(m, in, &l1, &r1, &l2, &r2);
-    // forward pieces again
-    const double rdA = 1.0 / dmax(wsum8([&](int n) { return in.A1[n]; }), GAM_TINY);
-    double vc[3];
-    for (int d = 0; d < 3; d++) vc[d] = in.AV[d] * rdA;
-    const double v1 = vc[0] * in.te1[0] + vc[1] * in.te1[1] + vc[2] * in.te1[2];
-    const double v2 = vc[0] * in.te2[0] + vc[1] * in.te2[1] + vc[2] * in.te2[2];
-    const double vD = sqrt(v1 * v1 + v2 * v2);
-    const double Dc = 0.25 * (in.D4[0] + in.D4[1] + in.D4[2] + in.D4[3]);
-    const double bT1 = 0.5 * (l1 + r1), bT2 = 0.5 * (l2 + r2);
-    const double Jd = (r2 - l2) - (r1 - l1);
+    EdgeFwd f;
+    edge_forward<RM, BORIS>(m, in, f);
+    o.E = f.E;
     const double xni = in.tb[0], yni = in.tb[1], xnj = in.tb[2], ynj = in.tb[3];
-    const double detT = 1.0 / (xni * ynj - xnj * yni);
-    const double b1 = detT * (ynj * bT1 - yni * bT2) + in.b01;
-    const double b2 = detT * (-(xnj * bT1) + xni * bT2) + in.b02;
-    const double nb = sqrt(b1 * b1 + b2 * b2);
-    const double u = nb / sqrt(Dc);
-    double vA = u;
-    if (BORIS) vA = m.Ca * u / sqrt(m.Ca * m.Ca + u * u);
-    const double vsum = vD + vA;
-    const double vDiff = dmin(vsum, in.cap);
     // adjoint
     const double ae = in.edge * aE;
-    double av1 = -b2 * ae, av2 = b1 * ae, ab1 = v2 * ae, ab2 = -v1 * ae;
-    const double avDiff = m.Vd0 * Jd * ae, aJd = m.Vd0 * vDiff * ae;
-    const double avs = (vsum < in.cap) ? avDiff : 0.0;
-    o.acap = (vsum < in.cap) ? 0.0 : avDiff;
-    double au = avs;
-    if (BORIS) {
-        const double c2 = m.Ca * m.Ca + u * u;
-        au = avs * m.Ca * m.Ca * m.Ca / (c2 * sqrt(c2));
-    }
-    const double anb = au / sqrt(Dc);
-    const double aDc = -0.5 * u / Dc * au;
-    if (nb > 0.0) { ab1 += b1 / nb * anb; ab2 += b2 / nb * anb; }
-    const double abT1 = detT * (ynj * ab1 - xnj * ab2);
-    const double abT2 = detT * (-yni * ab1 + xni * ab2);
-    double al1 = aJd + 0.5 * abT1, ar1 = -aJd + 0.5 * abT1;
-    double al2 = -aJd + 0.5 * abT2, ar2 = aJd + 0.5 * abT2;
-    if (vD > 0.0) { av1 += v1 / vD * avs; av2 += v2 / vD * avs; }
+    double av1 = -f.b2 * ae, av2 = f.b1 * ae, ab1 = f.v2 * ae, ab2 = -f.v1 * ae;
+    const double avDiff = m.Vd0 * f.Jd * ae, aJd = m.Vd0 * f.vDiff * ae;
+    const double avs = (f.vsum < in.cap) ? avDiff : 0.0;
+    o.acap = (f.vsum < in.cap) ? 0.0 : avDiff;
+    const double aX = 0.5 * f.ivA * avs;
+    ab1 += 2 * f.b1 * (f.Xb * aX);
+    ab2 += 2 * f.b2 * (f.Xb * aX);
+    o.aDc = f.Xd * aX;
+    const double abT1 = f.detT * (ynj * ab1 - xnj * ab2);
+    const double abT2 = f.detT * (-yni * ab1 + xni * ab2);
+    const double al1 = aJd + 0.5 * abT1, ar1 = -aJd + 0.5 * abT1;
+    const double al2 = -aJd + 0.5 * abT2, ar2 = aJd + 0.5 * abT2;
+    av1 += f.v1 * f.ivD * avs;
+    av2 += f.v2 * f.ivD * avs;
     // edge B reconstructions
-    {
-        double qv[8], nq[4];
-        for (int n = 0; n < 8; n++) qv[n] = in.A1[n] * (in.mH1[n] / dmax(in.A1[n], GAM_TINY));
-        for (int n = 0; n < 4; n++) nq[n] = in.mL1[n] / dmax(in.A1[n + 2], GAM_TINY);
-        const double Vi = wsum8([&](int n) { return in.A1[n]; });
-        for (int n = 0; n < 4; n++) o.anq1[n] = 0.0;
-        recon_lr_w_adj_s<RM>(m.pdmb, 1.0 / Vi, nq, qv, al1, ar1, o.anq1, o.sl1, o.sr1);
-    }
-    {
-        double qv[8], nq[4];
-        for (int n = 0; n < 8; n++) qv[n] = in.A2[n] * (in.mH2[n] / dmax(in.A2[n], GAM_TINY));
-        for (int n = 0; n < 4; n++) nq[n] = in.mL2[n] / dmax(in.A2[n + 2], GAM_TINY);
-        const double Vi = wsum8([&](int n) { return in.A2[n]; });
-        for (int n = 0; n < 4; n++) o.anq2[n] = 0.0;
-        recon_lr_w_adj_s<RM>(m.pdmb, 1.0 / Vi, nq, qv, al2, ar2, o.anq2, o.sl2, o.sr2);
-    }
-    // corner velocity and density
-    for (int d = 0; d < 3; d++) o.sv[d] = rdA * (in.te1[d] * av1 + in.te2[d] * av2);
-    o.aDc = aDc;
+    for (int n = 0; n < 4; n++) o.anq1[n] = o.anq2[n] = 0.0;
+    recon_lr_w_adj_s<RM>(m.pdmb, f.iA1, f.nq1, f.qv1, al1, ar1, o.anq1, o.sl1, o.sr1);
+    recon_lr_w_adj_s<RM>(m.pdmb, f.iA2, f.nq2, f.qv2, al2, ar2, o.anq2, o.sl2, o.sr2);
+    // corner velocity
+    for (int d = 0; d < 3; d++) o.sv[d] = f.rdA * (in.te1[d] * av1 + in.te2[d] * av2);
 }
 
 // the stencil weight of point n of the transposes split above

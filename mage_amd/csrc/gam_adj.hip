@@ -85,9 +85,10 @@ __device__ __forceinline__ void slab_row(const Box &b, unsigned nj, unsigned R, 
     }
 }
 
-#define POINT_SLAB(b)                                                                            \
+#define POINT_SLAB(b) POINT_SLAB_AT(b, blockIdx.x)
+#define POINT_SLAB_AT(b, w_)                                                                          \
     const unsigned ni_ = (unsigned)((b).i1 - (b).i0 + 1), nj_ = (unsigned)((b).j1 - (b).j0 + 1); \
-    const unsigned L_ = (blockIdx.x & ~127u) + ((blockIdx.x & 7u) << 4) + ((blockIdx.x >> 3) & 15u); \
+    const unsigned L_ = ((w_) & ~127u) + (((w_) & 7u) << 4) + (((w_) >> 3) & 15u); \
     const unsigned p_ = L_ * ABT + threadIdx.x;                                                  \
     if (p_ >= ni_ * nj_ * (unsigned)((b).k1 - (b).k0 + 1)) return;                               \
     const unsigned R_ = p_ / ni_;                                                                \
@@ -913,17 +914,17 @@ __global__ __launch_bounds__(256) void k_recon_adj_gather(Geo g, Box cb, const d
 // the half-state and limiter face fluxes and the half-state density by
 // k_emf_adj_gather.
 template <int ED, int RM, bool BG, bool BORIS>
-__global__ __launch_bounds__(256, 2) void k_emf_adj(Geo g, MParm m, Box eb, const Clock *clk,
-                                                 const double *__restrict__ H,
-                                                 const double *__restrict__ S,
-                                                 const double *__restrict__ Vf,
-                                                 const double *__restrict__ met,
-                                                 const double *__restrict__ bg,
-                                                 const double *__restrict__ aE,
-                                                 double *__restrict__ sc,
-                                                 double *__restrict__ pdt)
+__device__ __forceinline__ void emf_adj_edge(unsigned w, const Geo &g, const MParm &m, const Box &eb, const Clock *clk,
+                                             const double *__restrict__ H,
+                                             const double *__restrict__ S,
+                                             const double *__restrict__ Vf,
+                                             const double *__restrict__ met,
+                                             const double *__restrict__ bg,
+                                             const double *__restrict__ aE,
+                                             double *__restrict__ sc,
+                                             double *__restrict__ pdt)
 {
-    POINT_SLAB(eb);
+    POINT_SLAB_AT(eb, w);
     constexpr int T1 = (ED == 0) ? 1 : (ED == 1) ? 2 : 0;
     constexpr int T2 = (ED == 0) ? 2 : (ED == 1) ? 0 : 1;
     constexpr int E1 = (ED == 0) ? 1 : 0;
@@ -957,7 +958,7 @@ __global__ __launch_bounds__(256, 2) void k_emf_adj(Geo g, MParm m, Box eb, cons
     in.b01 = BG ? bg[(B_EDGB0 + 0 + 2 * ED) * N3 + c] : 0.0;
     in.b02 = BG ? bg[(B_EDGB0 + 1 + 2 * ED) * N3 + c] : 0.0;
     in.edge = met[(M_EDGE + ED) * N3 + c];
-    in.cap = m.CFL * in.edge / clk->dt;
+    in.cap = m.CFL * in.edge * gam_rcp(clk->dt);
     EdgeAdjS o;
     const double aEc = aE[ED * N3 + c];
     edge_emf_adj_s<RM, BORIS>(m, in, aEc, o);
@@ -972,6 +973,33 @@ __global__ __launch_bounds__(256, 2) void k_emf_adj(Geo g, MParm m, Box eb, cons
     // the stencil scalar pairs interleaved over planes 3-4 and 9-10
     *(double2 *)(sc + 3 * N3 + 2 * c) = make_double2(o.sl1, o.sr1);
     *(double2 *)(sc + 9 * N3 + 2 * c) = make_double2(o.sl2, o.sr2);
+}
+
+// The workgroups of the three edge directions one after another.  With pdt,
+// to which every direction adds at the same points, a launch holds one.
+struct EmfAdj3 {
+    Box e[3];
+    unsigned start[2];   // first workgroup of direction 1, of direction 2
+};
+
+template <int RM, bool BG, bool BORIS>
+__global__ __launch_bounds__(256, 2) void k_emf_adj(Geo g, MParm m, EmfAdj3 f, const Clock *clk,
+                                                 const double *__restrict__ H,
+                                                 const double *__restrict__ S,
+                                                 const double *__restrict__ Vf,
+                                                 const double *__restrict__ met,
+                                                 const double *__restrict__ bg,
+                                                 const double *__restrict__ aE,
+                                                 double *__restrict__ sc,
+                                                 double *__restrict__ pdt)
+{
+    const unsigned w = blockIdx.x;
+    if (w < f.start[0])
+        emf_adj_edge<0, RM, BG, BORIS>(w, g, m, f.e[0], clk, H, S, Vf, met, bg, aE, sc, pdt);
+    else if (w < f.start[1])
+        emf_adj_edge<1, RM, BG, BORIS>(w - f.start[0], g, m, f.e[1], clk, H, S, Vf, met, bg, aE, sc + 16 * g.N3, pdt);
+    else
+        emf_adj_edge<2, RM, BG, BORIS>(w - f.start[1], g, m, f.e[2], clk, H, S, Vf, met, bg, aE, sc + 32 * g.N3, pdt);
 }
 
 // Edge EMF transpose, pass 2: one thread per face position x (every
@@ -1361,38 +1389,39 @@ void launch_update_adj_mhd(hipStream_t s, const Geo &g, const MParm &m, const Bo
                        adM, aSn, aSo, ag, amf, aE);
 }
 
-template <int D, int RM>
-static void flux_adj_mhd_r(hipStream_t s, const Geo &g, const MParm &m, const Box &fb, const double *H,
+template <int RM, bool BG, bool BO>
+static void flux_adj_mhd_t(hipStream_t s, const Geo &g, const MParm &m, const Box *fb, const double *H,
                            const double *S, const double *met, const double *bg, const double *ag,
                            const double *amf, double *sc, double *aHMF, double *aHG)
 {
-    const AdjTile t = adj_tiles(D, fb);
-#define FLUXADJ(BG, BO)                                                                                      \
-    hipLaunchKernelGGL((k_flux_adj_mhd<D, RM, BG, BO>), tgrid(t.t), dim3(256), 0, s, g, m, t, H, S, met, bg, ag,   \
-                       amf, sc, aHMF, aHG)
-    if (m.doBG && m.doBoris) FLUXADJ(true, true);
-    else if (m.doBG) FLUXADJ(true, false);
-    else if (m.doBoris) FLUXADJ(false, true);
-    else FLUXADJ(false, false);
-#undef FLUXADJ
+    FluxAdj3 f;
+    unsigned tot = 0;
+    for (int d = 0; d < 3; d++) {
+        f.t[d] = adj_tiles(d, fb[d]);
+        tot += tgrid(f.t[d].t).x;
+        if (d < 2) f.start[d] = (int)tot;
+    }
+    hipLaunchKernelGGL((k_flux_adj_mhd<RM, BG, BO>), dim3(tot), dim3(256), 0, s, g, m, f, H, S, met, bg, ag, amf, sc,
+                       aHMF, aHG);
 }
 
-template <int D>
-static void flux_adj_mhd_d(hipStream_t s, const Geo &g, const MParm &m, const Box &fb, const double *H,
-                           const double *S, const double *met, const double *bg, const double *ag,
-                           const double *amf, double *sc, double *aHMF, double *aHG)
-{
-    if (m.rmeth) flux_adj_mhd_r<D, 1>(s, g, m, fb, H, S, met, bg, ag, amf, sc, aHMF, aHG);
-    else flux_adj_mhd_r<D, 0>(s, g, m, fb, H, S, met, bg, ag, amf, sc, aHMF, aHG);
-}
-
-void launch_flux_adj_mhd(hipStream_t s, int d, const Geo &g, const MParm &m, const Box &fb, const double *H,
+void launch_flux_adj_mhd(hipStream_t s, const Geo &g, const MParm &m, const Box *fb, const double *H,
                          const double *S, const double *met, const double *bg, const double *ag,
                          const double *amf, double *sc, double *aHMF, double *aHG)
 {
-    if (d == 0) flux_adj_mhd_d<0>(s, g, m, fb, H, S, met, bg, ag, amf, sc, aHMF, aHG);
-    else if (d == 1) flux_adj_mhd_d<1>(s, g, m, fb, H, S, met, bg, ag, amf, sc, aHMF, aHG);
-    else flux_adj_mhd_d<2>(s, g, m, fb, H, S, met, bg, ag, amf, sc, aHMF, aHG);
+    const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
+#define FLUXADJ(RM, BG, BO) flux_adj_mhd_t<RM, BG, BO>(s, g, m, fb, H, S, met, bg, ag, amf, sc, aHMF, aHG)
+    switch (sel) {
+    case 0: FLUXADJ(0, false, false); break;
+    case 1: FLUXADJ(0, false, true); break;
+    case 2: FLUXADJ(0, true, false); break;
+    case 3: FLUXADJ(0, true, true); break;
+    case 4: FLUXADJ(1, false, false); break;
+    case 5: FLUXADJ(1, false, true); break;
+    case 6: FLUXADJ(1, true, false); break;
+    default: FLUXADJ(1, true, true); break;
+    }
+#undef FLUXADJ
 }
 
 void launch_recon_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const double *sc, const double *rv,
@@ -1404,22 +1433,30 @@ void launch_recon_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const 
                        m.doLFM ? 1 : 0, aWH, aWN, aHB, aSSB);
 }
 
-template <int ED, int RM, bool BG, bool BO>
-static void emf_adj_t(hipStream_t s, const Geo &g, const MParm &m, const Box &eb, const Clock *clk,
+template <int RM, bool BG, bool BO>
+static void emf_adj_t(hipStream_t s, const Geo &g, const MParm &m, const Box *eb, const Clock *clk,
                       const double *H, const double *S, const double *Vf, const double *met, const double *bg,
                       const double *aE, double *sc, double *pdt)
 {
-    hipLaunchKernelGGL((k_emf_adj<ED, RM, BG, BO>), agrid_slab(eb), dim3(ABT), 0, s, g, m, eb, clk, H, S, Vf, met,
-                       bg, aE, sc + (size_t)16 * ED * g.N3, pdt);
+    for (int q = 0; q < (pdt ? 3 : 1); q++) {
+        EmfAdj3 f;
+        unsigned tot = 0;
+        for (int d = 0; d < 3; d++) {
+            f.e[d] = eb[d];
+            if (!pdt || d == q) tot += agrid_slab(eb[d]).x;
+            if (d < 2) f.start[d] = tot;
+        }
+        hipLaunchKernelGGL((k_emf_adj<RM, BG, BO>), dim3(tot), dim3(ABT), 0, s, g, m, f, clk, H, S, Vf, met, bg, aE, sc,
+                           pdt);
+    }
 }
 
-template <int ED>
-static void emf_adj_d(hipStream_t s, const Geo &g, const MParm &m, const Box &eb, const Clock *clk,
-                      const double *H, const double *S, const double *Vf, const double *met, const double *bg,
-                      const double *aE, double *sc, double *pdt)
+void launch_emf_adj(hipStream_t s, const Geo &g, const MParm &m, const Box *eb, const Clock *clk,
+                    const double *H, const double *S, const double *Vf, const double *met, const double *bg,
+                    const double *aE, double *sc, double *pdt)
 {
     const int sel = (m.rmeth ? 4 : 0) + (m.doBG ? 2 : 0) + (m.doBoris ? 1 : 0);
-#define EMFADJ(RM, BG, BO) emf_adj_t<ED, RM, BG, BO>(s, g, m, eb, clk, H, S, Vf, met, bg, aE, sc, pdt)
+#define EMFADJ(RM, BG, BO) emf_adj_t<RM, BG, BO>(s, g, m, eb, clk, H, S, Vf, met, bg, aE, sc, pdt)
     switch (sel) {
     case 0: EMFADJ(0, false, false); break;
     case 1: EMFADJ(0, false, true); break;
@@ -1431,15 +1468,6 @@ static void emf_adj_d(hipStream_t s, const Geo &g, const MParm &m, const Box &eb
     default: EMFADJ(1, true, true); break;
     }
 #undef EMFADJ
-}
-
-void launch_emf_adj(hipStream_t s, int ed, const Geo &g, const MParm &m, const Box &eb, const Clock *clk,
-                    const double *H, const double *S, const double *Vf, const double *met, const double *bg,
-                    const double *aE, double *sc, double *pdt)
-{
-    if (ed == 0) emf_adj_d<0>(s, g, m, eb, clk, H, S, Vf, met, bg, aE, sc, pdt);
-    else if (ed == 1) emf_adj_d<1>(s, g, m, eb, clk, H, S, Vf, met, bg, aE, sc, pdt);
-    else emf_adj_d<2>(s, g, m, eb, clk, H, S, Vf, met, bg, aE, sc, pdt);
 }
 
 void launch_emf_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const Box *eboxes, const double *sc,

@@ -53,26 +53,36 @@ static inline AdjTile adj_tiles(int D, const Box &b)
     return t;
 }
 
+template <int D> struct adj_geom {
+    static constexpr int NE = D == 0 ? 376 : (FA_L + 7) * FA_I;   // cells staged (D = 0: at most)
+    static constexpr int NL = D == 0 ? 376 : (FA_L + 3) * FA_I;   // limiter cells staged
+    static constexpr int SN = D == 0 ? 1 : FA_I;                  // LDS step of the stencil
+    static constexpr int LO = D == 0 ? 0 : 2 * FA_I;              // first staged cell with a limiter entry
+    static constexpr int G0 = 7 * SN;                             // zero slots before the first face's
+    static constexpr int NS = G0 + NE;                            // face slots, zero where no face is
+    static constexpr int LDS = 9 * NE + 8 * NL + 6 * NS;
+};
+#define FLUXADJ_LDS (adj_geom<0>::LDS)
+static_assert(adj_geom<1>::LDS <= FLUXADJ_LDS, "LDS planes");
+
+// workgroup w of the launch's range for direction D; lds: FLUXADJ_LDS doubles
 template <int D, int RM, bool BG, bool BORIS>
-__global__ __launch_bounds__(256, 2) void k_flux_adj_mhd(Geo g, MParm m, AdjTile t,
-                                                      const double *__restrict__ H,
-                                                      const double *__restrict__ S,
-                                                      const double *__restrict__ met,
-                                                      const double *__restrict__ bg,
-                                                      const double *__restrict__ ag,
-                                                      const double *__restrict__ amf,
-                                                      double *__restrict__ sc,
-                                                      double *__restrict__ aHMF,
-                                                      double *__restrict__ aHG)
+__device__ __forceinline__ void flux_adj_tile(double *lds, int w, const Geo &g, const MParm &m, const AdjTile &t,
+                                              const double *__restrict__ H,
+                                              const double *__restrict__ S,
+                                              const double *__restrict__ met,
+                                              const double *__restrict__ bg,
+                                              const double *__restrict__ ag,
+                                              const double *__restrict__ amf,
+                                              double *__restrict__ sc,
+                                              double *__restrict__ aHMF,
+                                              double *__restrict__ aHG)
 {
-    constexpr int NE = D == 0 ? 376 : (FA_L + 7) * FA_I;   // cells staged (D = 0: at most)
-    constexpr int NL = D == 0 ? 376 : (FA_L + 3) * FA_I;   // limiter cells staged
-    constexpr int SN = D == 0 ? 1 : FA_I;                  // LDS step of the stencil
-    constexpr int LO = D == 0 ? 0 : 2 * FA_I;              // first staged cell with a limiter entry
-    constexpr int G0 = 7 * SN;                             // zero slots before the first face's
-    constexpr int NS = G0 + NE;                            // face slots, zero where no face is
-    __shared__ double sv[NE], sq[8][NE], sl[8][NL], ss[6][NS];
-    const int L = xcd_tile((int)blockIdx.x, t.t.xs);
+    using A = adj_geom<D>;
+    constexpr int NE = A::NE, NL = A::NL, SN = A::SN, LO = A::LO, G0 = A::G0, NS = A::NS;
+    // volumes; weighted values and limiter values by variable; face slots
+    double *const sv = lds, *const sq = lds + NE, *const sl = sq + 8 * NE, *const ss = sl + 8 * NL;
+    const int L = xcd_tile(w, t.t.xs);
     if (L >= t.t.nb) return;                   // whole workgroup
     const int tid = (int)threadIdx.x;
     const long N3 = g.N3;
@@ -158,23 +168,23 @@ __global__ __launch_bounds__(256, 2) void k_flux_adj_mhd(Geo g, MParm m, AdjTile
             if (put[q]) {
                 sv[e] = v[q];
 #pragma unroll
-                for (int n = 0; n < 8; n++) sq[n][e] = n < 5 ? wq[q][n] : v[q] * wq[q][n];
+                for (int n = 0; n < 8; n++) sq[n * NE + e] = n < 5 ? wq[q][n] : v[q] * wq[q][n];
                 if (e >= LO && e - LO < NL)
 #pragma unroll
-                    for (int n = 0; n < 8; n++) sl[n][e - LO] = wl[q][n];
+                    for (int n = 0; n < 8; n++) sl[n * NL + e - LO] = wl[q][n];
             }
         }
         for (int e = tid; e < NS; e += 256)
 #pragma unroll
-            for (int n = 0; n < 6; n++) ss[n][e] = 0.0;
+            for (int n = 0; n < 6; n++) ss[n * NS + e] = 0.0;
     }
     __syncthreads();
     const double rVi = gam_rcp(wsum8([&](int n) { return sv[f0 + n * SN]; }));
     auto stencil = [&](int v, double *qv, double *nq) {
 #pragma unroll
-        for (int n = 0; n < 8; n++) qv[n] = sq[v][f0 + n * SN];
+        for (int n = 0; n < 8; n++) qv[n] = sq[v * NE + f0 + n * SN];
 #pragma unroll
-        for (int n = 0; n < 4; n++) nq[n] = sl[v][f0 + (D == 0 ? n + 2 : n * SN)];
+        for (int n = 0; n < 4; n++) nq[n] = sl[v * NL + f0 + (D == 0 ? n + 2 : n * SN)];
     };
     // adjoints of the left and right states: gas 5, B 3
     double aL[8], aR[8];
@@ -273,10 +283,10 @@ __global__ __launch_bounds__(256, 2) void k_flux_adj_mhd(Geo g, MParm m, AdjTile
             double qv[8], nq[4], an[4] = {0, 0, 0, 0}, l, r;
             stencil(v, qv, nq);
             recon_lr_w_adj_s<RM>(m.pdmb, rVi, nq, qv, aL[v], aR[v], an, l, r);
-            ss[0][fs] = l;
-            ss[1][fs] = r;
+            ss[fs] = l;
+            ss[NS + fs] = r;
 #pragma unroll
-            for (int n = 0; n < 4; n++) ss[2 + n][fs] = an[n];
+            for (int n = 0; n < 4; n++) ss[(2 + n) * NS + fs] = an[n];
         }
         __syncthreads();
 #pragma unroll
@@ -288,17 +298,46 @@ __global__ __launch_bounds__(256, 2) void k_flux_adj_mhd(Geo g, MParm m, AdjTile
 #pragma unroll
             for (int n = 0; n < 8; n++) {
                 if (RM == 1) {
-                    if (n <= 6) gh += UP7(n) * ss[0][e - n * SN];
-                    if (n >= 1) gh += UP7(7 - n) * ss[1][e - n * SN];
+                    if (n <= 6) gh += UP7(n) * ss[e - n * SN];
+                    if (n >= 1) gh += UP7(7 - n) * ss[NS + e - n * SN];
                 } else {
-                    gh += W8(n) * ss[0][e - n * SN];
+                    gh += W8(n) * ss[e - n * SN];
                 }
             }
 #pragma unroll
-            for (int n = 0; n < 4; n++) gn += ss[2 + n][e - (n + 2) * SN];
+            for (int n = 0; n < 4; n++) gn += ss[(2 + n) * NS + e - (n + 2) * SN];
             pc[q][v * N3] = gh;
             pc[q][(8 + v) * N3] = gn;
         }
         if (v < 7) __syncthreads();
     }
+}
+
+// The workgroups of the three directions one after another, as k_flux3
+struct FluxAdj3 {
+    AdjTile t[3];
+    int start[2];     // first workgroup of direction 1, of direction 2
+};
+
+template <int RM, bool BG, bool BORIS>
+__global__ __launch_bounds__(256, 2) void k_flux_adj_mhd(Geo g, MParm m, FluxAdj3 f,
+                                                      const double *__restrict__ H,
+                                                      const double *__restrict__ S,
+                                                      const double *__restrict__ met,
+                                                      const double *__restrict__ bg,
+                                                      const double *__restrict__ ag,
+                                                      const double *__restrict__ amf,
+                                                      double *__restrict__ sc,
+                                                      double *__restrict__ aHMF,
+                                                      double *__restrict__ aHG)
+{
+    __shared__ double lds[FLUXADJ_LDS];
+    const int w = (int)blockIdx.x;
+    const long ns = FLUXADJ_NPL * g.N3;
+    if (w < f.start[0])
+        flux_adj_tile<0, RM, BG, BORIS>(lds, w, g, m, f.t[0], H, S, met, bg, ag, amf, sc, aHMF, aHG);
+    else if (w < f.start[1])
+        flux_adj_tile<1, RM, BG, BORIS>(lds, w - f.start[0], g, m, f.t[1], H, S, met, bg, ag, amf, sc + ns, aHMF, aHG);
+    else
+        flux_adj_tile<2, RM, BG, BORIS>(lds, w - f.start[1], g, m, f.t[2], H, S, met, bg, ag, amf, sc + 2 * ns, aHMF, aHG);
 }

@@ -210,7 +210,7 @@ void launch_update_adj_mhd(hipStream_t s, const Geo &g, const MParm &m, const Bo
 // the cell's own face and from the neighbouring one), aBn into aHMF, the
 // Boris nuke term into aHG
 #define FLUXADJ_NPL 32
-void launch_flux_adj_mhd(hipStream_t s, int d, const Geo &g, const MParm &m, const Box &fb, const double *H,
+void launch_flux_adj_mhd(hipStream_t s, const Geo &g, const MParm &m, const Box *fb, const double *H,
                          const double *S, const double *met, const double *bg, const double *ag,
                          const double *amf, double *sc, double *aHMF, double *aHG);
 // pass 2 (all three directions' sc) fused with the Mom2Face
@@ -219,7 +219,7 @@ void launch_recon_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const 
                              const double *aVf, const double *met, double *aWH, double *aWN, double *aHB,
                              double *aSSB);
 // pass 1 of the edge EMF transpose: 16 planes per edge direction into sc
-void launch_emf_adj(hipStream_t s, int ed, const Geo &g, const MParm &m, const Box &eb, const Clock *clk,
+void launch_emf_adj(hipStream_t s, const Geo &g, const MParm &m, const Box *eb, const Clock *clk,
                     const double *H, const double *S, const double *Vf, const double *met, const double *bg,
                     const double *aE, double *sc, double *pdt);
 // pass 2: writes aVf, aHMF and aHG at every point (adds the limiter parts
