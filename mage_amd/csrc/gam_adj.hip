@@ -558,13 +558,12 @@ __device__ __forceinline__ void move_adj(double *p, long dst, long src)
 // one cell-B plane (each plane's chain of moves is independent of the
 // others', so they run in parallel instead of one after another).
 template <int SIDE>
-__global__ void k_bc_periodic_adj(Geo g, Box t, double *__restrict__ aS)
+__device__ __forceinline__ void bc_periodic_adj(const Geo &g, const Box &t, int z, double *__restrict__ aS)
 {
     const int a = t.i0 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
     const int b = t.j0 + (int)blockIdx.y;
     if (a > t.i1 || b > t.j1) return;
     const long N3 = g.N3;
-    const int z = (int)blockIdx.z;
     const int pl = z <= 5 ? S_GAS + z - 1 : S_B + z - 6;
     double *mf = aS + S_MF * N3;
     for (int n = 4; n >= 1; n--) {
@@ -595,6 +594,16 @@ __global__ void k_bc_periodic_adj(Geo g, Box t, double *__restrict__ aS)
         }
         if (z > 0 && gi <= g.ieg && gj <= g.jeg && gk <= g.keg) move_adj(aS + pl * N3, d, s);
     }
+}
+
+// With 18 blocks along z also the axis's other side (the two sides share no
+// ghost and, with more than 8 cells between them, no source).
+template <int SIDE>
+__global__ void k_bc_periodic_adj(Geo g, Box t, double *__restrict__ aS)
+{
+    const int z = (int)blockIdx.z;
+    if (z < 9) bc_periodic_adj<SIDE>(g, t, z, aS);
+    else bc_periodic_adj<SIDE ^ 1>(g, t, z - 9, aS);
 }
 
 // Transpose of the zero-gradient / sphere BC copies with the magnetic
@@ -810,29 +819,35 @@ __global__ __launch_bounds__(256) void k_update_adj_faces(Geo g, Box fb, Box ab,
         const bool face = i >= g.is && j >= g.js && k >= g.ks && i <= g.ie + (d == 0) &&
                           j <= g.je + (d == 1) && k <= g.ke + (d == 2);
         if (!face) continue;
-        const long cl = c - st[d];
+        // adH (in aUr), adM hold values at active cells only: the others' place
+        // is taken by the active cell on the face's other side, with weight 0
         const bool up = inside(ab, i, j, k);
         const bool lo = inside(ab, i - (d == 0), j - (d == 1), k - (d == 2));
-        const double wu = up ? 1.0 / met[M_VOL * N3 + c] : 0.0;
-        const double wl = lo ? 1.0 / met[M_VOL * N3 + cl] : 0.0;
-        // adH (in aUr), adM hold values at active cells only
+        const long cu = up ? c : c - st[d], cl = lo ? c - st[d] : c;
+        const double iu = gam_rcp(met[M_VOL * N3 + cu]), il = gam_rcp(met[M_VOL * N3 + cl]);
+        const double wu = up ? iu : 0.0, wl = lo ? il : 0.0;
+#pragma unroll
         for (int v = 0; v < 5; v++)
-            ag[(v + 5 * d) * N3 + c] = (up ? wu * aUr[v * N3 + c] : 0.0) - (lo ? wl * aUr[v * N3 + cl] : 0.0);
+            ag[(v + 5 * d) * N3 + c] = wu * aUr[v * N3 + cu] - wl * aUr[v * N3 + cl];
+#pragma unroll
         for (int x = 0; x < 3; x++)
-            amf[(x + 3 * d) * N3 + c] = (up ? wu * adM[x * N3 + c] : 0.0) - (lo ? wl * adM[x * N3 + cl] : 0.0);
+            amf[(x + 3 * d) * N3 + c] = wu * adM[x * N3 + cu] - wl * adM[x * N3 + cl];
     }
     const double *aF = aSn + S_MF * N3;   // adjoint of the new face fluxes
     for (int d = 0; d < 3; d++) aSo[(S_MF + d) * N3 + c] += aF[d * N3 + c];
     // CT: new flux(d, f) = old - dtA * (curl of E around f); gather per edge
     auto fa = [&](int d, int ii, int jj, int kk) -> double {
-        return inside(ctb, ii, jj, kk) ? aF[d * N3 + IX(g, ii, jj, kk)] : 0.0;
+        const bool ok = inside(ctb, ii, jj, kk);
+        const double x = aF[d * N3 + (ok ? IX(g, ii, jj, kk) : c)];
+        return ok ? x : 0.0;
     };
-    aE[c] = inside(eb.e[0], i, j, k)
-                ? dtA * (fa(1, i, j, k) - fa(1, i, j, k - 1) + fa(2, i, j - 1, k) - fa(2, i, j, k)) : 0.0;
-    aE[N3 + c] = inside(eb.e[1], i, j, k)
-                ? dtA * (fa(0, i, j, k - 1) - fa(0, i, j, k) + fa(2, i, j, k) - fa(2, i - 1, j, k)) : 0.0;
-    aE[2 * N3 + c] = inside(eb.e[2], i, j, k)
-                ? dtA * (fa(0, i, j, k) - fa(0, i, j - 1, k) + fa(1, i - 1, j, k) - fa(1, i, j, k)) : 0.0;
+    const double f0 = fa(0, i, j, k), f1 = fa(1, i, j, k), f2 = fa(2, i, j, k);
+    const double e0 = dtA * (f1 - fa(1, i, j, k - 1) + fa(2, i, j - 1, k) - f2);
+    const double e1 = dtA * (fa(0, i, j, k - 1) - f0 + f2 - fa(2, i - 1, j, k));
+    const double e2 = dtA * (f0 - fa(0, i, j - 1, k) + fa(1, i - 1, j, k) - f1);
+    aE[c] = inside(eb.e[0], i, j, k) ? e0 : 0.0;
+    aE[N3 + c] = inside(eb.e[1], i, j, k) ? e1 : 0.0;
+    aE[2 * N3 + c] = inside(eb.e[2], i, j, k) ? e2 : 0.0;
 }
 
 // The cell side of the reconstruction transposes of the three face
@@ -1011,7 +1026,57 @@ __global__ __launch_bounds__(256, 2) void k_emf_adj(Geo g, MParm m, EmfAdj3 f, c
 // of each direction around it (aHG's density; its other planes get 0).
 // aVf, aHMF and aHG are WRITTEN at every point (the flux transpose adds
 // into aHMF and aHG afterwards).  sc: 16 planes per edge direction from
-// k_emf_adj; edges exist in eb.
+// k_emf_adj; edges exist in eb.  Blocks y = 0, 1, 2 take the faces of one
+// direction each and y = 3 the cells: one thread for all of them is a chain
+// of some 190 loads, most behind a test (one thread: 279 us on a 96x96x128 shell, 27 on a 32x24x27
+// box; split 245 and 13; loads without a branch, of the point
+// itself where there is no edge, 346 and 26).
+template <int RM, int T>
+__device__ __forceinline__ void emf_adj_face(const Geo &g, const EdgeBoxes &eb, const double *__restrict__ sc,
+                                             const double *__restrict__ met, int lfm, int i, int j, int k,
+                                             double *__restrict__ aVf, double *__restrict__ aHMF,
+                                             double *__restrict__ aSSMF)
+{
+    const long N3 = g.N3;
+    const long c = IX(g, i, j, k);
+    const long st[3] = {1, (long)g.P, g.PP};
+    const int EDa = (T + 2) % 3, Da = (T + 1) % 3;   // edges with T1 = T, stencil along T2
+    const int EDb = (T + 1) % 3, Db = (T + 2) % 3;   // edges with T2 = T, stencil along T1
+    const double *sa = sc + (long)16 * EDa * N3, *sb = sc + (long)16 * EDb * N3;
+    double sv[3] = {0.0, 0.0, 0.0}, sh = 0.0, sn = 0.0;
+#pragma unroll
+    for (int n = 0; n < 8; n++) {
+        int e3[3] = {i, j, k};
+        e3[Da] -= n - 4;
+        if (inside(eb.e[EDa], e3[0], e3[1], e3[2])) {
+            const long e = c - (n - 4) * st[Da];
+            for (int d = 0; d < 3; d++) sv[d] += W8(n) * sa[d * N3 + e];
+            const double2 lr = *(const double2 *)(sa + 3 * N3 + 2 * e);
+            sh += stencil_adj<RM>(n, lr.x, lr.y);
+        }
+        int e4[3] = {i, j, k};
+        e4[Db] -= n - 4;
+        if (inside(eb.e[EDb], e4[0], e4[1], e4[2])) {
+            const long e = c - (n - 4) * st[Db];
+            const double2 lr = *(const double2 *)(sb + 9 * N3 + 2 * e);
+            sh += stencil_adj<RM>(n, lr.x, lr.y);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        int e3[3] = {i, j, k};
+        e3[Da] -= q - 2;
+        if (inside(eb.e[EDa], e3[0], e3[1], e3[2])) sn += sa[(5 + q) * N3 + c - (q - 2) * st[Da]];
+        int e4[3] = {i, j, k};
+        e4[Db] -= q - 2;
+        if (inside(eb.e[EDb], e4[0], e4[1], e4[2])) sn += sb[(11 + q) * N3 + c - (q - 2) * st[Db]];
+    }
+    const double A = met[(M_FACE + T) * N3 + c], iAm = gam_rcp(dmax(A, GAM_TINY));
+    for (int d = 0; d < 3; d++) aVf[(3 * T + d) * N3 + c] = A * sv[d];
+    aHMF[T * N3 + c] = dmin(A * (1.0 / GAM_TINY), 1.0) * sh + (lfm ? 0.0 : sn * iAm);
+    if (lfm) aSSMF[T * N3 + c] += sn * iAm;
+}
+
 template <int RM>
 __global__ __launch_bounds__(256) void k_emf_adj_gather(Geo g, Box fb, EdgeBoxes eb, const double *__restrict__ sc,
                                                         const double *__restrict__ met, int lfm,
@@ -1019,47 +1084,12 @@ __global__ __launch_bounds__(256) void k_emf_adj_gather(Geo g, Box fb, EdgeBoxes
                                                         double *__restrict__ aHG, double *__restrict__ aSSMF)
 {
     POINT_SLAB(fb);
+    if (blockIdx.y == 0) { emf_adj_face<RM, 0>(g, eb, sc, met, lfm, i, j, k, aVf, aHMF, aSSMF); return; }
+    if (blockIdx.y == 1) { emf_adj_face<RM, 1>(g, eb, sc, met, lfm, i, j, k, aVf, aHMF, aSSMF); return; }
+    if (blockIdx.y == 2) { emf_adj_face<RM, 2>(g, eb, sc, met, lfm, i, j, k, aVf, aHMF, aSSMF); return; }
     const long N3 = g.N3;
     const long c = IX(g, i, j, k);
     const long st[3] = {1, (long)g.P, g.PP};
-#pragma unroll
-    for (int T = 0; T < 3; T++) {
-        const int EDa = (T + 2) % 3, Da = (T + 1) % 3;   // edges with T1 = T, stencil along T2
-        const int EDb = (T + 1) % 3, Db = (T + 2) % 3;   // edges with T2 = T, stencil along T1
-        const double *sa = sc + (long)16 * EDa * N3, *sb = sc + (long)16 * EDb * N3;
-        double sv[3] = {0.0, 0.0, 0.0}, sh = 0.0, sn = 0.0;
-#pragma unroll
-        for (int n = 0; n < 8; n++) {
-            int e3[3] = {i, j, k};
-            e3[Da] -= n - 4;
-            if (inside(eb.e[EDa], e3[0], e3[1], e3[2])) {
-                const long e = c - (n - 4) * st[Da];
-                for (int d = 0; d < 3; d++) sv[d] += W8(n) * sa[d * N3 + e];
-                const double2 lr = *(const double2 *)(sa + 3 * N3 + 2 * e);
-                sh += stencil_adj<RM>(n, lr.x, lr.y);
-            }
-            int e4[3] = {i, j, k};
-            e4[Db] -= n - 4;
-            if (inside(eb.e[EDb], e4[0], e4[1], e4[2])) {
-                const long e = c - (n - 4) * st[Db];
-                const double2 lr = *(const double2 *)(sb + 9 * N3 + 2 * e);
-                sh += stencil_adj<RM>(n, lr.x, lr.y);
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            int e3[3] = {i, j, k};
-            e3[Da] -= q - 2;
-            if (inside(eb.e[EDa], e3[0], e3[1], e3[2])) sn += sa[(5 + q) * N3 + c - (q - 2) * st[Da]];
-            int e4[3] = {i, j, k};
-            e4[Db] -= q - 2;
-            if (inside(eb.e[EDb], e4[0], e4[1], e4[2])) sn += sb[(11 + q) * N3 + c - (q - 2) * st[Db]];
-        }
-        const double A = met[(M_FACE + T) * N3 + c], Am = dmax(A, GAM_TINY);
-        for (int d = 0; d < 3; d++) aVf[(3 * T + d) * N3 + c] = A * sv[d];
-        aHMF[T * N3 + c] = (A / Am) * sh + (lfm ? 0.0 : sn / Am);
-        if (lfm) aSSMF[T * N3 + c] += sn / Am;
-    }
     if (i <= g.ieg && j <= g.jeg && k <= g.keg) {
         double sd = 0.0;
 #pragma unroll
@@ -1129,19 +1159,25 @@ __global__ __launch_bounds__(256) void k_predict_mf_adj(Geo g, Box fb, const Clo
     for (int d = 0; d < 3; d++) {
         double a = aHMF[d * N3 + c];
         const double *xf = met + (long)(M_XFC + 3 * d) * N3;
-        if (cin) {
-            const double iv = 1.0 / met[M_VOL * N3 + c];
+        {
+            const double iv = gam_rcp(met[M_VOL * N3 + c]);
+            double t = 0.0;
+#pragma unroll
             for (int x = 0; x < 3; x++)
-                a += aHB[x * N3 + c] * iv * (-xf[x * N3 + c] + met[(M_XYZCC + x) * N3 + c]);
+                t += aHB[x * N3 + c] * iv * (-xf[x * N3 + c] + met[(M_XYZCC + x) * N3 + c]);
+            a += cin ? t : 0.0;
         }
         const int at = d == 0 ? i : d == 1 ? j : k;
         const int lo = d == 0 ? g.isg : d == 1 ? g.jsg : g.ksg;
         const bool oin = at - 1 >= lo && (d == 0 || i <= g.ieg) && (d == 1 || j <= g.jeg) && (d == 2 || k <= g.keg);
-        if (oin) {
-            const long cm = c - (d == 0 ? 1 : d == 1 ? (long)g.P : g.PP);
-            const double iv = 1.0 / met[M_VOL * N3 + cm];
+        {
+            const long cm = oin ? c - (d == 0 ? 1 : d == 1 ? (long)g.P : g.PP) : c;
+            const double iv = gam_rcp(met[M_VOL * N3 + cm]);
+            double t = 0.0;
+#pragma unroll
             for (int x = 0; x < 3; x++)
-                a += aHB[x * N3 + cm] * iv * (xf[x * N3 + c] - met[(M_XYZCC + x) * N3 + cm]);
+                t += aHB[x * N3 + cm] * iv * (xf[x * N3 + c] - met[(M_XYZCC + x) * N3 + cm]);
+            a += oin ? t : 0.0;
         }
         aS[(S_MF + d) * N3 + c] += (1.0 + w) * a;
         aO[(S_MF + d) * N3 + c] = -w * a;
@@ -1318,14 +1354,14 @@ void launch_cellb_adj(hipStream_t s, const Geo &g, int all, double *aS, const do
 }
 
 template <int SIDE>
-static void bcp_adj_side(hipStream_t s, const Geo &g, double *aS)
+static void bcp_adj_side(hipStream_t s, const Geo &g, double *aS, bool both)
 {
     Box t;
     if (SIDE <= 1) { t.i0 = g.jsg; t.i1 = g.jeg + 1; t.j0 = g.ksg; t.j1 = g.keg + 1; }
     else if (SIDE <= 3) { t.i0 = g.isg; t.i1 = g.ieg + 1; t.j0 = g.ksg; t.j1 = g.keg + 1; }
     else { t.i0 = g.isg; t.i1 = g.ieg + 1; t.j0 = g.jsg; t.j1 = g.jeg + 1; }
     t.k0 = t.k1 = 0;
-    const dim3 gr((unsigned)((t.i1 - t.i0 + 64) / 64), (unsigned)(t.j1 - t.j0 + 1), 9);
+    const dim3 gr((unsigned)((t.i1 - t.i0 + 64) / 64), (unsigned)(t.j1 - t.j0 + 1), both ? 18 : 9);
     hipLaunchKernelGGL(k_bc_periodic_adj<SIDE>, gr, dim3(64), 0, s, g, t, aS);
 }
 
@@ -1345,7 +1381,7 @@ static void bcc_adj_side(hipStream_t s, const Geo &g, double *aS, const double *
 // transpose of one side's BC with magnetic fields; kind as gam_model.bc
 void launch_bc_mhd_adj(hipStream_t s, int side, int kind, const Geo &g, double *aS, const double *met)
 {
-    if (kind == 0) { launch_bc_periodic_adj(s, side, g, aS); return; }
+    if (kind == 0) { launch_bc_periodic_adj(s, side, g, aS, false); return; }
     switch (side) {
     case 0: if (kind == 2) bcc_adj_side<0, 2>(s, g, aS, met); else bcc_adj_side<0, 1>(s, g, aS, met); break;
     case 1: if (kind == 3) bcc_adj_side<1, 3>(s, g, aS, met); else bcc_adj_side<1, 1>(s, g, aS, met); break;
@@ -1356,15 +1392,15 @@ void launch_bc_mhd_adj(hipStream_t s, int side, int kind, const Geo &g, double *
     }
 }
 
-void launch_bc_periodic_adj(hipStream_t s, int side, const Geo &g, double *aS)
+void launch_bc_periodic_adj(hipStream_t s, int side, const Geo &g, double *aS, bool both)
 {
     switch (side) {
-    case 0: bcp_adj_side<0>(s, g, aS); break;
-    case 1: bcp_adj_side<1>(s, g, aS); break;
-    case 2: bcp_adj_side<2>(s, g, aS); break;
-    case 3: bcp_adj_side<3>(s, g, aS); break;
-    case 4: bcp_adj_side<4>(s, g, aS); break;
-    default: bcp_adj_side<5>(s, g, aS); break;
+    case 0: bcp_adj_side<0>(s, g, aS, both); break;
+    case 1: bcp_adj_side<1>(s, g, aS, both); break;
+    case 2: bcp_adj_side<2>(s, g, aS, both); break;
+    case 3: bcp_adj_side<3>(s, g, aS, both); break;
+    case 4: bcp_adj_side<4>(s, g, aS, both); break;
+    default: bcp_adj_side<5>(s, g, aS, both); break;
     }
 }
 
@@ -1476,11 +1512,12 @@ void launch_emf_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const Bo
     const Box fb = faces_of(g);
     EdgeBoxes eb;
     for (int d = 0; d < 3; d++) eb.e[d] = eboxes[d];
+    const dim3 gr(agrid_slab(fb).x, 4);
     if (m.rmeth)
-        hipLaunchKernelGGL(k_emf_adj_gather<1>, agrid_slab(fb), dim3(ABT), 0, s, g, fb, eb, sc, met,
+        hipLaunchKernelGGL(k_emf_adj_gather<1>, gr, dim3(ABT), 0, s, g, fb, eb, sc, met,
                            m.doLFM ? 1 : 0, aVf, aHMF, aHG, aSSMF);
     else
-        hipLaunchKernelGGL(k_emf_adj_gather<0>, agrid_slab(fb), dim3(ABT), 0, s, g, fb, eb, sc, met,
+        hipLaunchKernelGGL(k_emf_adj_gather<0>, gr, dim3(ABT), 0, s, g, fb, eb, sc, met,
                            m.doLFM ? 1 : 0, aVf, aHMF, aHG, aSSMF);
 }
 

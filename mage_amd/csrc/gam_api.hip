@@ -1983,6 +1983,11 @@ static void adj_bcs(gam_adj *a, double *l, const double *S, const Clock *bclk)
     for (int sd = 5; sd >= 0; sd--) {
         if (c->model.bc[sd] == GAM_BC_WIND)
             launch_bc_wind_adj(c->stream, c->g, c->mp, bclk, c->wd, S, l, c->met, a->gwq, a->gwb);
+        else if (c->mp.doMHD && (sd & 1) && c->model.bc[sd] == 0 && c->model.bc[sd - 1] == 0 &&
+                 (sd == 5 ? c->g.Nkp : sd == 3 ? c->g.Njp : c->g.Nip) > 8) {
+            launch_bc_periodic_adj(c->stream, sd, c->g, l, true);
+            sd--;
+        }
         else if (c->mp.doMHD) launch_bc_mhd_adj(c->stream, sd, c->model.bc[sd], c->g, l, c->met);
         else launch_bc_adj(c->stream, sd, c->model.bc[sd] == GAM_BC_PERIODIC ? 0 : 1, c->g, l);
     }

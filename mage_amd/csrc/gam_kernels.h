@@ -192,7 +192,8 @@ void launch_dt_record(hipStream_t s, const Geo &g, const MParm &m, const Box &dt
 void launch_dt_inject(hipStream_t s, const Geo &g, const MParm &m, const double *rec, const double *mu,
                       double *lam);
 void launch_cellb_adj(hipStream_t s, const Geo &g, int all, double *aS, const double *met);
-void launch_bc_periodic_adj(hipStream_t s, int side, const Geo &g, double *aS);
+// both: the two sides of its axis, which must have more than 8 cells
+void launch_bc_periodic_adj(hipStream_t s, int side, const Geo &g, double *aS, bool both);
 void launch_bc_mhd_adj(hipStream_t s, int side, int kind, const Geo &g, double *aS, const double *met);
 // transpose of the inflow BC; adds the series adjoint into gQ (n,5), gB (n,3),
 // each WIND_COPIES consecutive copies of those arrays (the caller sums them)
