@@ -773,9 +773,14 @@ static void enq_fluxes_emfs_apart(gam_ctx *c, const HalfSrc &h, const Box *eb, d
 }
 
 // Whether the launch plan's fluxes and EMFs can form the half state themselves.
+// (Boris and the background field are nothing without a magnetic field.)
+static bool keeps_prims(const gam_ctx *c)
+{
+    return c->mp.doMHD || (!c->mp.doBG && !c->mp.doBoris);
+}
 static bool plan_direct(const gam_ctx *c)
 {
-    return c->mp.doMHD && flux3_ok(&c->plan.v[TS_FLUX_I]) && emf3_ok(&c->plan.v[TS_EMF_I]);
+    return keeps_prims(c) && flux3_ok(&c->plan.v[TS_FLUX_I]) && emf3_ok(&c->plan.v[TS_EMF_I]);
 }
 // Whether the next step will.
 static bool step_direct(const gam_ctx *c)
@@ -862,7 +867,7 @@ static int enq_step(gam_ctx *c, bool keep = true)
     // the boundary launch does the time bookkeeping, unless CalcDT's argmin
     // is recorded, which needs the new dt before it, or an ensemble's launches
     const bool apart = c->dtrec || launch_recorder();
-    const bool writeW = c->mp.doMHD && !c->general && !c->snx;
+    const bool writeW = keeps_prims(c) && !c->general && !c->snx;
     const bool direct = step_direct(c);
     if (direct && keep) {
         const int rc = hf_keep(c, c->stream, S_old(c));
@@ -1402,7 +1407,7 @@ static int ens_enqueue(gam_ens *e, int nsteps)
             c->itgen++;
             c->hf = direct ? 1 : 0;
             c->cur ^= 1;
-            c->std[c->cur] = c->mp.doMHD ? 1 : 0;
+            c->std[c->cur] = keeps_prims(c) ? 1 : 0;
         }
         HIPCHK(hipGraphLaunch(e->exec[e->parity + (direct ? 2 : 0)], e->stream));
         e->parity ^= 1;

@@ -186,7 +186,7 @@ struct k_flux {
 // Two phases share the LDS planes: the five gas variables, then the three
 // field components, whose loads wait in registers meanwhile; 37 KB (33 for
 // D = 0) and 128 registers leave room for four workgroups per CU.
-// DIR: the half state is formed as the cells are staged, from the primitives
+// DIR (1; 2 without a magnetic field): the half state is formed as the cells are staged, from the primitives
 // and cell B that the last two steps left (S_W, S_B of State and oState): as
 // many words as the predictor's planes, which are then neither written nor
 // read (HalfSrc says when).
@@ -209,7 +209,7 @@ struct FluxTile {
 
 #define FLUX_LDS ((8 + 3) * 376 > (8 + 7) * 32 * 6 + (8 + 3) * 32 * 5 ? (8 + 3) * 376 : (8 + 7) * 32 * 6 + (8 + 3) * 32 * 5)
 
-template <int D, int RM, bool BG, bool BORIS, bool DIR>
+template <int D, int RM, bool BG, bool BORIS, int DIR>
 struct flux_tile {
     static constexpr int TI = 32, TA = 8;
     static constexpr int NE = D == 0 ? 376 : (TA + 7) * TI;   // cells staged (D = 0: at most)
@@ -297,6 +297,7 @@ struct flux_tile {
         const double *pv = met + M_VOL * N3;
         double v[2], wq[2][5], wl[2][5], bq[2][3], bl[2][3], wt = 0.0;
         if (DIR) {
+            if (DIR == 2) __builtin_assume(!m.doMHD);
             wt = ab2_weight(clk);
 #pragma unroll
             for (int q = 0; q < 2; q++) {
@@ -307,13 +308,15 @@ struct flux_tile {
                     wq[q][n] = ldp(pln(O, (S_W + n) * N3), oe[q]);
                 }
             }
+            if (DIR == 1) {
 #pragma unroll
-            for (int q = 0; q < 2; q++)
+                for (int q = 0; q < 2; q++)
 #pragma unroll
-                for (int x = 0; x < 3; x++) {
-                    bl[q][x] = ldp(pln(S, (S_B + x) * N3), oe[q]);
-                    bq[q][x] = ldp(pln(O, (S_B + x) * N3), oe[q]);
-                }
+                    for (int x = 0; x < 3; x++) {
+                        bl[q][x] = ldp(pln(S, (S_B + x) * N3), oe[q]);
+                        bq[q][x] = ldp(pln(O, (S_B + x) * N3), oe[q]);
+                    }
+            }
 #pragma unroll
             for (int q = 0; q < 2; q++) {
 #pragma unroll
@@ -322,6 +325,16 @@ struct flux_tile {
                     if (!m.doLFM) wl[q][n] = h;
                     wq[q][n] = v[q] * h;
                 }
+                if (DIR == 2 && m.doLFM && wl[q][DEN] <= m.dFloor) {
+                    // only a hydrodynamic update leaves densities below the
+                    // floor, where the limiter's velocity and pressure
+                    // (c2p_block) are not S_W's (c2p_cell)
+                    double U[5];
+#pragma unroll
+                    for (int n = 0; n < 5; n++) U[n] = ldp(S + (S_GAS + n) * N3, oe[q]);
+                    c2p_block(m, U, wl[q]);
+                }
+                if (DIR == 2) continue;
 #pragma unroll
                 for (int x = 0; x < 3; x++) {
                     const double h = ab2(bl[q][x], bq[q][x], wt);
@@ -383,11 +396,11 @@ struct flux_tile {
 #pragma unroll
         for (int n = 0; n < 5; n++) {
             double vel;
-            recon(n, WL[n], WR[n], n >= 1 && n <= 3 ? &vel : nullptr);
+            recon(n, WL[n], WR[n], DIR != 2 && n >= 1 && n <= 3 ? &vel : nullptr);
             // Mom2Face of this face from the same velocity stencil
-            if (n >= 1 && n <= 3 && act) stp(Vf + (n - 1) * N3, oc, vel);
+            if (DIR != 2 && n >= 1 && n <= 3 && act) stp(Vf + (n - 1) * N3, oc, vel);
         }
-        if (DIR || m.doMHD) {
+        if (DIR == 1 || (DIR == 0 && m.doMHD)) {
             __syncthreads();
 #pragma unroll
             for (int q = 0; q < 2; q++) {
@@ -431,7 +444,7 @@ struct flux_tile {
     }
 };
 
-template <int D, int RM, bool BG, bool BORIS, bool DIR>
+template <int D, int RM, bool BG, bool BORIS, int DIR>
 struct k_flux_t {
     static constexpr int NT = 256;
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, FluxTile t,
@@ -481,12 +494,15 @@ static void flux_t(hipStream_t s, int form, const Geo &g, const MParm &m, const 
     const double *H = h.H, *S = h.S;
     if (plan_ax(form) >= PLAN_LDS) {
         const FluxTile t = flux_tiles(D, b, form & 1);
-        if (h.O)
-            launch_f<k_flux_t<D, RM, BG, BO, true>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk, met, bg,
-                                                    gf, mf, vf);
+        if (!h.O)
+            launch_f<k_flux_t<D, RM, BG, BO, 0>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk, met, bg, gf,
+                                                 mf, vf);
+        else if (BG || BO || m.doMHD)
+            launch_f<k_flux_t<D, RM, BG, BO, 1>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk, met, bg, gf,
+                                                 mf, vf);
         else
-            launch_f<k_flux_t<D, RM, BG, BO, false>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk, met, bg,
-                                                     gf, mf, vf);
+            launch_f<k_flux_t<D, RM, BG, BO, BG || BO ? 1 : 2>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk,
+                                                                met, bg, gf, mf, vf);
         return;
     }
     const int ch = plan_chunk(form);

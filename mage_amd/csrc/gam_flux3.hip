@@ -22,7 +22,7 @@ struct Flux3 {
     int start[2];     // first workgroup of the rim; the end
 };
 
-template <int RM, bool BG, bool BORIS, bool DIR>
+template <int RM, bool BG, bool BORIS, int DIR>
 struct k_flux3 {
     static constexpr int NT = 256;
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, const Flux3 &f,
@@ -39,7 +39,7 @@ struct k_flux3 {
         const int w = (int)bi.x;
         const long N3 = g.N3;
         if (w >= f.start[0]) {
-            vface_rim<DIR>{}(w - f.start[0], g, f.rim, H, S, O, clk, met, Vf);
+            vface_rim<DIR != 0>{}(w - f.start[0], g, f.rim, H, S, O, clk, met, Vf);
             return;
         }
         const int sl = (int)((unsigned)w / f.slab);
@@ -80,8 +80,11 @@ static void flux3_t(hipStream_t s, const int *form, const Geo &g, const MParm &m
     if (m.doMHD) tot += f.rim.start[6];
     f.start[1] = tot;
     const dim3 gr((unsigned)tot), bl(BX, BY);
-    if (h.O) launch_f<k_flux3<RM, BG, BO, true>>(gr, bl, s, g, m, f, h.H, h.S, h.O, h.clk, met, bg, gf, mf, vf);
-    else launch_f<k_flux3<RM, BG, BO, false>>(gr, bl, s, g, m, f, h.H, h.S, h.O, h.clk, met, bg, gf, mf, vf);
+    if (!h.O) launch_f<k_flux3<RM, BG, BO, 0>>(gr, bl, s, g, m, f, h.H, h.S, h.O, h.clk, met, bg, gf, mf, vf);
+    else if (BG || BO || m.doMHD)
+        launch_f<k_flux3<RM, BG, BO, 1>>(gr, bl, s, g, m, f, h.H, h.S, h.O, h.clk, met, bg, gf, mf, vf);
+    else
+        launch_f<k_flux3<RM, BG, BO, BG || BO ? 1 : 2>>(gr, bl, s, g, m, f, h.H, h.S, h.O, h.clk, met, bg, gf, mf, vf);
 }
 
 bool flux3_ok(const int *form)
