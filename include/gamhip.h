@@ -228,10 +228,10 @@ int gam_get_solver(gam_ctx *ctx, int which, double *out);
  * launch shapes that give the same results: the chunk tiling of the box's
  * points, value = row order (1 = j fastest, 2 = k fastest, 3 = slabs of 8
  * j-rows) + 8 x chunk extent (0: 256 points per workgroup, 1: 512,
- * 2: 128), and the LDS-staged forms: 4 for the EMFs; for the fluxes 4 (tiles numbered
- * along i first; i fluxes: rows j fastest) and 5 (along the flux direction
- * first; rows k fastest).  For the j and k fluxes 6 and 7 are other names
- * of 4 and 5.
+ * 2: 128).  The LDS-staged forms are EMF 1, 2 and 3 (one form), i flux 1
+ * and 2 (its two row orders), and for the j and k fluxes 4 (tiles numbered
+ * along i first) and 5 (along the flux direction first), with 6 and 7 as
+ * other names of 4 and 5.
  * gam_autotune times every candidate of every slot on the context's own
  * grid (reps steps per candidate, hipEvents around that slot's launch),
  * keeps the fastest (the current shape unless another is more than 1 %

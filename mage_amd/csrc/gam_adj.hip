@@ -9,10 +9,10 @@
 //
 // Adjoint planes hold the derivative of the objective with respect to the
 // same-named forward plane; an adjoint state set has the State layout's
-// first 11 planes (gas 5, face flux 3, cell B 3).  The MHD flux and EMF
-// transposes are split at their linear stencils: a per-face (per-edge)
-// pass writes stencil scalars to scratch planes and a per-cell (per-face)
-// gather sums them, with no atomics.  The other kernels whose forward
+// first 11 planes (gas 5, face flux 3, cell B 3).  The MHD flux transpose
+// (gam_adj_flux.h) sums its transposed stencils over tiles of cells, the EMF
+// transpose writes stencil scalars per edge, and a per-cell (per-face) gather
+// adds the tiles (the scalars), with no atomics.  The other kernels whose forward
 // gathers over a stencil (the hydrodynamic flux, cell B, the boundary
 // scatter of the inflow and outer-wall BCs) scatter with FP64 atomic adds
 // (hardware global_atomic_add_f64); the rest gather.  dt is the forward
@@ -1028,9 +1028,9 @@ __global__ __launch_bounds__(256, 2) void k_emf_adj(Geo g, MParm m, EmfAdj3 f, c
 // into aHMF and aHG afterwards).  sc: 16 planes per edge direction from
 // k_emf_adj; edges exist in eb.  Blocks y = 0, 1, 2 take the faces of one
 // direction each and y = 3 the cells: one thread for all of them is a chain
-// of some 190 loads, most behind a test (one thread: 279 us on a 96x96x128 shell, 27 on a 32x24x27
-// box; split 245 and 13; loads without a branch, of the point
-// itself where there is no edge, 346 and 26).
+// of some 190 loads, most behind a test (96x96x128 shell 279 us, 32x24x27
+// box 27; split 245 and 13; in one thread without branches, the point itself
+// loaded where there is no edge, 346 and 26).
 template <int RM, int T>
 __device__ __forceinline__ void emf_adj_face(const Geo &g, const EdgeBoxes &eb, const double *__restrict__ sc,
                                              const double *__restrict__ met, int lfm, int i, int j, int k,
@@ -1108,10 +1108,10 @@ __global__ __launch_bounds__(256) void k_emf_adj_gather(Geo g, Box fb, EdgeBoxes
     }
 }
 
-// Mom2Face (k_vface): face velocity of direction d at face f =
+// Mom2Face (mom2face): face velocity of direction d at face f =
 // sum_n W8(n) V_n v_n / sum_n W8(n) V_n over the 8 cells along d (cells
 // past the k ends of the grid left out).  rv[d] = that normalisation,
-// 1 / max(sum_n W8(n) V_n, tiny), at each face k_vface writes (0
+// 1 / max(sum_n W8(n) V_n, tiny), at each face with a velocity (0
 // elsewhere); geometry only, formed once per adjoint run.
 __global__ __launch_bounds__(256) void k_vface_rv(Geo g, Box cb, const double *__restrict__ met,
                                                   double *__restrict__ rv)

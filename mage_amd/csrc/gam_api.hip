@@ -1594,7 +1594,7 @@ extern "C" int gam_autotune(gam_ctx *c, int reps)
         rc = tune_time(c, slot, reps, &best);
         for (int q = 0; q < n && rc == GAM_OK; q++) {
             if (v[q] == bestv) continue;
-            if (v[q] >= PLAN_LDS + PLAN_ALIAS && v[q] < 8) continue;   // another name of a shape
+            if (plan_alias(slot, v[q])) continue;
             c->plan.v[slot] = v[q];
             double ms = 0.0;
             rc = tune_time(c, slot, reps, &ms);

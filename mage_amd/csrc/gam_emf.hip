@@ -454,7 +454,7 @@ static void emf3_t(hipStream_t s, const Geo &g, const MParm &m, const Box *b, co
 bool emf3_ok(const int *plan)
 {
     for (int d = 0; d < 3; d++)
-        if (plan[d] != PLAN_LDS) return false;
+        if (!emf_lds(plan[d])) return false;
     return true;
 }
 
@@ -480,7 +480,7 @@ static void emf_t(hipStream_t s, int plan, const Geo &g, const MParm &m, const B
 {
     const double *H = h.H, *S = h.S;
     const Clock *clk = h.clk;
-    if (plan == PLAN_LDS) {
+    if (emf_lds(plan)) {
         const EdgeTile t = edge_tiles(ED, b);
         const dim3 gr(xcd_grid(t.nb, t.xs)), bl(BX, BY);
         if (h.O) launch_f<k_emf_t<ED, RM, BG, BO, true>>(gr, bl, s, g, m, t, clk, H, S, h.O, Vf, met, bg, E);
@@ -491,10 +491,8 @@ static void emf_t(hipStream_t s, int plan, const Geo &g, const MParm &m, const B
     const Tile t = tile_of(b, plan_ax(plan), ch);
     if (ch == 512)
         launch_f<k_emf<ED, RM, BG, BO, 512>>(tgrid(t), dim3(BX, 8), s, g, m, t, clk, H, S, Vf, met, bg, E);
-    else if (ch == 128)
-        launch_f<k_emf<ED, RM, BG, BO, 128>>(tgrid(t), dim3(BX, 2), s, g, m, t, clk, H, S, Vf, met, bg, E);
     else
-        launch_f<k_emf<ED, RM, BG, BO>>(tgrid(t), dim3(BX, BY), s, g, m, t, clk, H, S, Vf, met, bg, E);
+        launch_f<k_emf<ED, RM, BG, BO, 128>>(tgrid(t), dim3(BX, 2), s, g, m, t, clk, H, S, Vf, met, bg, E);
 }
 
 template <int ED>

@@ -492,8 +492,8 @@ static void flux_t(hipStream_t s, int form, const Geo &g, const MParm &m, const 
                    const double *met, const double *bg, double *gf, double *mf, double *vf)
 {
     const double *H = h.H, *S = h.S;
-    if (plan_ax(form) >= PLAN_LDS) {
-        const FluxTile t = flux_tiles(D, b, form & 1);
+    if (flux_lds(D, form)) {
+        const FluxTile t = flux_tiles(D, b, flux_alt(D, form));
         if (!h.O)
             launch_f<k_flux_t<D, RM, BG, BO, 0>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk, met, bg, gf,
                                                  mf, vf);
@@ -511,8 +511,9 @@ static void flux_t(hipStream_t s, int form, const Geo &g, const MParm &m, const 
         launch_f<k_flux<D, RM, BG, BO, 512>>(tgrid(t), dim3(BX, 8), s, g, m, t, H, S, met, bg, gf, mf, vf);
     else if (ch == 128)
         launch_f<k_flux<D, RM, BG, BO, 128>>(tgrid(t), dim3(BX, 2), s, g, m, t, H, S, met, bg, gf, mf, vf);
-    else
-        launch_f<k_flux<D, RM, BG, BO>>(tgrid(t), dim3(BX, BY), s, g, m, t, H, S, met, bg, gf, mf, vf);
+    else if (D != 0)
+        launch_f<k_flux<D, RM, BG, BO, D == 0 ? 128 : BX * BY>>(tgrid(t), dim3(BX, BY), s, g, m, t, H, S, met, bg, gf,
+                                                                mf, vf);
 }
 
 template <int D>

@@ -68,7 +68,7 @@ static void flux3_t(hipStream_t s, const int *form, const Geo &g, const MParm &m
     const Tile t0 = tile_of(b[0], 1);
     const int ns = t0.nb < 2048 ? 1 : std::min((b[0].k1 - b[0].k0 + 8) / 8, t0.nb / (16 << t0.xs));
     for (int d = 0; d < 3; d++) {
-        f.t[d] = flux_tiles(d, b[d], d == 2 && ns > 1 ? 2 : form[d] & 1);
+        f.t[d] = flux_tiles(d, b[d], d == 2 && ns > 1 ? 2 : flux_alt(d, form[d]));
         const int run = 8 << f.t[d].t.xs;
         f.n[d] = (f.t[d].t.nb + ns * run - 1) / (ns * run) * run;
         tot += f.n[d];
@@ -90,7 +90,7 @@ static void flux3_t(hipStream_t s, const int *form, const Geo &g, const MParm &m
 bool flux3_ok(const int *form)
 {
     for (int d = 0; d < 3; d++)
-        if (plan_ax(form[d]) < PLAN_LDS) return false;
+        if (!flux_lds(d, form[d])) return false;
     return true;
 }
 

@@ -54,11 +54,13 @@ void order_record(hipStream_t s, hipEvent_t e, int ev);
 void order_wait(hipStream_t s, hipEvent_t e, int ev);
 
 // Launch plan: the shape of every tunable launch of the step.  Values
-// 1, 2, 3 are the Tile row orders (ax1: j fastest, k fastest, j-slabs);
-// PLAN_LDS selects the LDS-staged EMFs; it and PLAN_LDS_D the LDS-staged
-// interface fluxes, tiles numbered along i first or along the flux direction first (i fluxes: rows j
-// or k fastest).  PLAN_ALIAS added to either names the same launch: plans
-// saved when these were separate shapes stay valid.
+// 1, 2, 3 are the Tile row orders (ax1: j fastest, k fastest, j-slabs), + 8
+// or 16 for chunks of 512 or 128 points instead of 256.  The LDS-staged
+// forms stand where direct loads in chunks of 256 were never faster: EMF 1,
+// 2, 3 (one form), i flux 1 and 2 (its two row orders); j and k flux
+// PLAN_LDS and PLAN_LDS_D (tiles numbered along i first, or along the flux
+// direction first), which PLAN_ALIAS added to either also names.  So plans
+// saved when these were other shapes stay valid and take the new ones.
 enum { TS_PREDICT = 0, TS_EMF_I, TS_EMF_J, TS_EMF_K, TS_FLUX_I, TS_FLUX_J, TS_FLUX_K, TS_UPDATE,
        TS_COUNT };
 #define PLAN_LDS 4
@@ -67,6 +69,15 @@ enum { TS_PREDICT = 0, TS_EMF_I, TS_EMF_J, TS_EMF_K, TS_FLUX_I, TS_FLUX_J, TS_FL
 struct Plan {
     int v[TS_COUNT];
 };
+static inline bool emf_lds(int v) { return v <= 3; }
+static inline bool flux_lds(int d, int v) { return d == 0 ? v <= 2 : (v & 7) >= PLAN_LDS; }
+static inline int flux_alt(int d, int v) { return d == 0 ? v == 2 : v & 1; }   // the other numbering
+// v names the same launch as a smaller value of the slot
+static inline bool plan_alias(int slot, int v)
+{
+    if (slot >= TS_EMF_I && slot <= TS_EMF_K) return v == 2 || v == 3;
+    return v >= PLAN_LDS + PLAN_ALIAS && v < 8;
+}
 Plan default_plan();
 // candidate values of a slot; returns their number
 int plan_candidates(int slot, int *vals);

@@ -459,10 +459,10 @@ Plan default_plan()
     // pointwise but for the next row and plane: row order 1 takes the
     // 256x256x384 step from 16.28 to 16.09 ms for either (slabs: 3)
     p.v[TS_PREDICT] = 1;
-    p.v[TS_EMF_I] = PLAN_LDS;
-    p.v[TS_EMF_J] = PLAN_LDS;
-    p.v[TS_EMF_K] = PLAN_LDS;
-    p.v[TS_FLUX_I] = PLAN_LDS;
+    p.v[TS_EMF_I] = 1;
+    p.v[TS_EMF_J] = 1;
+    p.v[TS_EMF_K] = 1;
+    p.v[TS_FLUX_I] = 1;
     p.v[TS_FLUX_J] = PLAN_LDS;
     p.v[TS_FLUX_K] = PLAN_LDS;
     p.v[TS_UPDATE] = 1;
@@ -477,14 +477,11 @@ int plan_candidates(int slot, int *vals)
     // row order x chunk size (256, 512, 128 points per workgroup)
     for (int c = 0; c < 3; c++)
         for (int a = 1; a <= maxax; a++) vals[n++] = a + 8 * c;
-    if (slot >= TS_EMF_I && slot <= TS_EMF_K) vals[n++] = PLAN_LDS;
-    if (slot >= TS_FLUX_I && slot <= TS_FLUX_K) {
+    if (slot == TS_FLUX_J || slot == TS_FLUX_K) {
         vals[n++] = PLAN_LDS;
         vals[n++] = PLAN_LDS_D;
-        if (slot != TS_FLUX_I) {
-            vals[n++] = PLAN_LDS + PLAN_ALIAS;
-            vals[n++] = PLAN_LDS_D + PLAN_ALIAS;
-        }
+        vals[n++] = PLAN_LDS + PLAN_ALIAS;
+        vals[n++] = PLAN_LDS_D + PLAN_ALIAS;
     }
     return n;
 }
