@@ -31,12 +31,12 @@ FP64_PEAK_TFLOPS = 78.6        # MI355X FP64 vector
 # Algorithmic FP64 words per cell-update of the whole step (state 19 read +
 # 14 written, metrics 79, dipole background 24): 136 words = 1088 B.
 STEP_BYTES_PER_CELL = 8 * (19 + 14 + 79 + 24)
-# Algorithmic words of one interface-flux launch, per face: stencil inputs
-# counted once per cell (half-state 5, limiter state 5, half B 3, limiter B
-# 3, volume 1), face data (Tf 9, area 1, half-state flux 1, fcB0 3,
-# bFlux0 1) and outputs (gas 5, magnetic 3, face velocity 3): 43 words =
-# 344 B.
-FLUX_BYTES_PER_FACE = 8 * 43
+# Algorithmic words of one direction's interface fluxes, per face: stencil
+# inputs counted once per cell (primitives of State and oState 5 each, their
+# cell B 3 each, volume 1), face data (normal 3, area 1, face flux of State
+# and oState 1 each, fcB0 3, bFlux0 1) and outputs (gas 5, magnetic 3, face
+# velocity 3): 38 words = 304 B.
+FLUX_BYTES_PER_FACE = 8 * 38
 # rocprofv3 summaries of the headline workload: FETCH_SIZE/WRITE_SIZE per
 # dispatch with the copy-kernel calibration, and the FP64 VALU instruction
 # counts per dispatch (written by the profiling runs recorded in the files).
@@ -88,10 +88,11 @@ def _summary_rows(path, prefix, col):
 
 
 def flux_traffic(path=PMC_SUMMARY):
-    """Calibrated HBM bytes per interface-flux dispatch from the committed
-    PMC summary (mean over the three directions), or None without one."""
-    vals = _summary_rows(path, "`k_flux", 5)
-    return sum(vals) / len(vals) if vals else None
+    """Calibrated HBM bytes of one direction's interface fluxes (a third of
+    the merged dispatch's) from the committed PMC summary, or None without
+    one."""
+    vals = _summary_rows(path, "`k_flux3", 5)
+    return sum(vals) / len(vals) / 3 if vals else None
 
 
 def step_flops(path=FLOP_SUMMARY):
@@ -564,7 +565,7 @@ def main():
         "launch_plan": plan,
         "roofline": {
             "bound": "hbm",
-            "kernel": "k_flux (interface fluxes and face velocities of one face direction per launch)",
+            "kernel": "k_flux3 (interface fluxes and face velocities; per face direction, a third of the launch)",
             "achieved": flux_gbs,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
