@@ -853,16 +853,22 @@ __global__ __launch_bounds__(256) void k_update_adj_faces(Geo g, Box fb, Box ab,
 // The cell side of the reconstruction transposes of the three face
 // directions (k_flux_adj_mhd's scratch) and of Mom2Face (rv, aVf): one
 // thread per cell adds what the one or two tiles of each direction that
-// reach it left, with no atomics, and WRITES the half-state
-// adjoints aWH (5), aWN (5) and aHB (3) of every cell; with the LFM
-// limiter the B limiter adjoints go into aSSB (3, added).  Faces of
-// direction D exist on the active box extended by one along D.
-__global__ __launch_bounds__(256) void k_recon_adj_gather(Geo g, Box cb, const double *__restrict__ sc,
+// reach it left, with no atomics, and carries the half-state adjoints on
+// through the predictor's gas transpose (with the half-state gas adjoint aHG
+// of the EMF's corner density) in the same thread: into aS and aO.  WRITES
+// the half-state cell-B adjoint aHB (3) of every cell; with the LFM limiter
+// the B limiter adjoints go into aS's cell B.  Faces of direction D exist on
+// the active box extended by one along D.
+__global__ __launch_bounds__(256) void k_recon_adj_gather(Geo g, MParm m, Box cb, const Clock *clk,
+                                                          const double *__restrict__ sc,
                                                           const double *__restrict__ rv,
                                                           const double *__restrict__ aVf,
-                                                          const double *__restrict__ met, int lfm,
-                                                          double *__restrict__ aWH, double *__restrict__ aWN,
-                                                          double *__restrict__ aHB, double *__restrict__ aSSB)
+                                                          const double *__restrict__ met,
+                                                          const double *__restrict__ S,
+                                                          const double *__restrict__ O,
+                                                          const double *__restrict__ aHG,
+                                                          double *__restrict__ aHB, double *__restrict__ aS,
+                                                          double *__restrict__ aO, double *__restrict__ pw)
 {
     POINT_SLAB(cb);
     const long N3 = g.N3;
@@ -911,15 +917,28 @@ __global__ __launch_bounds__(256) void k_recon_adj_gather(Geo g, Box cb, const d
                 gn[v] += sd[(24 + v) * N3];
             }
     }
-    for (int v = 0; v < 5; v++) {
-        aWH[v * N3 + c] = gh[v] + ((v >= 1 && v <= 3) ? av[v - 1] : 0.0);
-        aWN[v * N3 + c] = gn[v];
-    }
     const double V = met[M_VOL * N3 + c];
     for (int x = 0; x < 3; x++) {
-        aHB[x * N3 + c] = V * gh[5 + x] + (lfm ? 0.0 : gn[5 + x]);
-        if (lfm) aSSB[x * N3 + c] += gn[5 + x];
+        gh[1 + x] += av[x];
+        aHB[x * N3 + c] = V * gh[5 + x] + (m.doLFM ? 0.0 : gn[5 + x]);
+        if (m.doLFM) aS[(S_B + x) * N3 + c] += gn[5 + x];
     }
+    const double w = ab2_weight(clk);
+    double Q[5], oQ[5], ahg[5], aQ[5] = {0, 0, 0, 0, 0}, aoQ[5] = {0, 0, 0, 0, 0}, aw = 0.0;
+    for (int v = 0; v < 5; v++) {
+        Q[v] = S[(S_GAS + v) * N3 + c];
+        oQ[v] = O[(S_GAS + v) * N3 + c];
+        ahg[v] = aHG[v * N3 + c];
+    }
+    predict_cell_adj(m, Q, oQ, w, V, ahg, gh, gn, aQ, aoQ, pw ? &aw : nullptr);
+    if (pw) pw[c] = aw;
+    for (int v = 0; v < 5; v++) {
+        aS[v * N3 + c] += aQ[v];
+        aO[v * N3 + c] = aoQ[v];
+    }
+    // oState's cell B does not enter the step (the predictor forms the half
+    // state's B from the extrapolated face fluxes)
+    for (int x = 0; x < 3; x++) aO[(S_B + x) * N3 + c] = 0.0;
 }
 
 // Edge EMF transpose (k_emf), pass 1: per edge, the pieces of
@@ -1185,42 +1204,6 @@ __global__ __launch_bounds__(256) void k_predict_mf_adj(Geo g, Box fb, const Clo
     }
 }
 
-// predictor gas transpose with the half-state gas adjoint (the EMF's
-// corner density) included
-__global__ __launch_bounds__(256) void k_predict_adj_mhd(Geo g, MParm m, Box cb, const Clock *clk,
-                                                         const double *__restrict__ S,
-                                                         const double *__restrict__ O,
-                                                         const double *__restrict__ met,
-                                                         const double *__restrict__ aHG,
-                                                         const double *__restrict__ aWH,
-                                                         const double *__restrict__ aWN,
-                                                         double *__restrict__ aS,
-                                                         double *__restrict__ aO,
-                                                         double *__restrict__ pw)
-{
-    POINT_IN(cb);
-    const long N3 = g.N3;
-    const long c = IX(g, i, j, k);
-    const double w = ab2_weight(clk);
-    double Q[5], oQ[5], ahg[5], awh[5], awn[5], aQ[5] = {0, 0, 0, 0, 0}, aoQ[5] = {0, 0, 0, 0, 0}, aw = 0.0;
-    for (int v = 0; v < 5; v++) {
-        Q[v] = S[(S_GAS + v) * N3 + c];
-        oQ[v] = O[(S_GAS + v) * N3 + c];
-        ahg[v] = aHG[v * N3 + c];
-        awh[v] = aWH[v * N3 + c];
-        awn[v] = aWN[v * N3 + c];
-    }
-    predict_cell_adj(m, Q, oQ, w, met[M_VOL * N3 + c], ahg, awh, awn, aQ, aoQ, pw ? &aw : nullptr);
-    if (pw) pw[c] = aw;
-    for (int v = 0; v < 5; v++) {
-        aS[v * N3 + c] += aQ[v];
-        aO[v * N3 + c] = aoQ[v];
-    }
-    // oState's cell B does not enter the step (the predictor forms the half
-    // state's B from the extrapolated face fluxes)
-    for (int x = 0; x < 3; x++) aO[(S_B + x) * N3 + c] = 0.0;
-}
-
 // ------------------------------------------------------------ launchers
 void launch_adj_objective(hipStream_t s, const Geo &g, const MParm &m, const double *S,
                           const double *wgt, double *aS, double *part, int *nparts)
@@ -1460,13 +1443,13 @@ void launch_flux_adj_mhd(hipStream_t s, const Geo &g, const MParm &m, const Box 
 #undef FLUXADJ
 }
 
-void launch_recon_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const double *sc, const double *rv,
-                             const double *aVf, const double *met, double *aWH, double *aWN, double *aHB,
-                             double *aSSB)
+void launch_recon_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const Clock *clk, const double *sc,
+                             const double *rv, const double *aVf, const double *met, const double *S,
+                             const double *O, const double *aHG, double *aHB, double *aS, double *aO, double *pw)
 {
     const Box cb = cells_of(g);
-    hipLaunchKernelGGL(k_recon_adj_gather, agrid_slab(cb), dim3(ABT), 0, s, g, cb, sc, rv, aVf, met,
-                       m.doLFM ? 1 : 0, aWH, aWN, aHB, aSSB);
+    hipLaunchKernelGGL(k_recon_adj_gather, agrid_slab(cb), dim3(ABT), 0, s, g, m, cb, clk, sc, rv, aVf, met, S, O, aHG,
+                       aHB, aS, aO, pw);
 }
 
 template <int RM, bool BG, bool BO>
@@ -1527,15 +1510,11 @@ void launch_vface_rv(hipStream_t s, const Geo &g, const double *met, double *rv)
     hipLaunchKernelGGL(k_vface_rv, agrid(cb), dim3(ABT), 0, s, g, cb, met, rv);
 }
 
-void launch_predict_adj_mhd(hipStream_t s, const Geo &g, const MParm &m, const Clock *clk, const double *S,
-                            const double *O, const double *met, const double *aHG, const double *aWH,
-                            const double *aWN, double *aHB, double *aHMF, double *aS, double *aO, double *pw)
+void launch_predict_mf_adj(hipStream_t s, const Geo &g, const Clock *clk, const double *S, const double *O,
+                           const double *met, double *aHB, double *aHMF, double *aS, double *aO, double *pw)
 {
-    const Box cb = cells_of(g), fb = faces_of(g);
-    hipLaunchKernelGGL(k_predict_adj_mhd, agrid(cb), dim3(ABT), 0, s, g, m, cb, clk, S, O, met, aHG, aWH,
-                       aWN, aS, aO, pw);
-    hipLaunchKernelGGL(k_predict_mf_adj, agrid(fb), dim3(ABT), 0, s, g, fb, clk, met, aHB, aHMF, aS, aO, S, O,
-                       pw);
+    const Box fb = faces_of(g);
+    hipLaunchKernelGGL(k_predict_mf_adj, agrid(fb), dim3(ABT), 0, s, g, fb, clk, met, aHB, aHMF, aS, aO, S, O, pw);
 }
 
 // ============================================================ inflow BC

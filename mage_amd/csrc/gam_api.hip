@@ -1681,7 +1681,7 @@ struct gam_adj {
     hipEvent_t evR[2], evA[2];   // recompute of a pair done / adjoint done reading it
     double *lam;             // three adjoint state sets (ADJ_SET planes each)
     double *ag, *amf;        // adjoints of gFlx (15) and mFlx (9)
-    double *awh, *awn, *ahg; // adjoints of H_WH, H_WN, H_GAS (5 each)
+    double *awh, *awn, *ahg; // adjoints of H_WH, H_WN (hydrodynamic only), H_GAS (5 each)
     double *ahmf, *ahb;      // adjoints of H_MF, H_B (3 each)
     double *avf, *aur, *adm, *ae;   // Vf (9), Reynolds gas (5), dM (3), E (3)
     double *rv;              // Mom2Face normalisation per face direction (3)
@@ -1787,8 +1787,10 @@ extern "C" int gam_adj_create_budget(gam_adj **out, gam_ctx *c, int nsteps, int 
     AALLOC(a->lam, 3 * ADJ_SET * pl);
     AALLOC(a->ag, 15 * pl);
     AALLOC(a->amf, 9 * pl);
-    AALLOC(a->awh, 5 * pl);
-    AALLOC(a->awn, 5 * pl);
+    if (!c->mp.doMHD) {
+        AALLOC(a->awh, 5 * pl);
+        AALLOC(a->awn, 5 * pl);
+    }
     AALLOC(a->ahg, 5 * pl);
     AALLOC(a->ahmf, 3 * pl);
     AALLOC(a->ahb, 3 * pl);
@@ -2051,7 +2053,7 @@ static void adj_step(gam_adj *a, int n, const StepIT *it, const double *Sn, cons
                               lA, lB, a->aur, a->adm, a->ag, a->amf, a->ae, pdt);
         // the EMF transpose first: its gather writes aVf, aHMF and aHG whole,
         // the flux transpose adds into aHMF and aHG, and its gather writes
-        // aWH, aWN and aHB whole (no plane needs zeroing)
+        // aHB whole and goes on through the predictor (no plane needs zeroing)
         launch_emf_adj(s, g, c->mp, eb, clk, H, Sn, vf, c->met, c->bg, a->ae, a->esc, pdt);
         launch_emf_adj_gather(s, g, c->mp, eb, a->esc, c->met, a->avf, a->ahmf, a->ahg, lB + S_MF * N3);
         Box fb[3] = {act_box(g), act_box(g), act_box(g)};
@@ -2059,10 +2061,8 @@ static void adj_step(gam_adj *a, int n, const StepIT *it, const double *Sn, cons
         fb[1].j1 += 1;
         fb[2].k1 += 1;
         launch_flux_adj_mhd(s, g, c->mp, fb, H, Sn, c->met, c->bg, a->ag, a->amf, a->fsc, a->ahmf, a->ahg);
-        launch_recon_adj_gather(s, g, c->mp, a->fsc, a->rv, a->avf, c->met, a->awh, a->awn, a->ahb,
-                                lB + S_B * N3);
-        launch_predict_adj_mhd(s, g, c->mp, clk, Sn, On, c->met, a->ahg, a->awh, a->awn, a->ahb, a->ahmf, lB, lC,
-                               pw);
+        launch_recon_adj_gather(s, g, c->mp, clk, a->fsc, a->rv, a->avf, c->met, Sn, On, a->ahg, a->ahb, lB, lC, pw);
+        launch_predict_mf_adj(s, g, clk, Sn, On, c->met, a->ahb, a->ahmf, lB, lC, pw);
     } else {
         adj_bcs(a, lA, Sn1, bclk);
         dt_inject();

@@ -225,11 +225,11 @@ void launch_update_adj_mhd(hipStream_t s, const Geo &g, const MParm &m, const Bo
 void launch_flux_adj_mhd(hipStream_t s, const Geo &g, const MParm &m, const Box *fb, const double *H,
                          const double *S, const double *met, const double *bg, const double *ag,
                          const double *amf, double *sc, double *aHMF, double *aHG);
-// pass 2 (all three directions' sc) fused with the Mom2Face
-// transpose: writes aWH, aWN, aHB of every cell
-void launch_recon_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const double *sc, const double *rv,
-                             const double *aVf, const double *met, double *aWH, double *aWN, double *aHB,
-                             double *aSSB);
+// pass 2 (all three directions' sc) fused with the Mom2Face transpose and the
+// predictor's gas transpose: into aS, aO; writes aHB of every cell
+void launch_recon_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const Clock *clk, const double *sc,
+                             const double *rv, const double *aVf, const double *met, const double *S,
+                             const double *O, const double *aHG, double *aHB, double *aS, double *aO, double *pw);
 // pass 1 of the edge EMF transpose: 16 planes per edge direction into sc
 void launch_emf_adj(hipStream_t s, const Geo &g, const MParm &m, const Box *eb, const Clock *clk,
                     const double *H, const double *S, const double *Vf, const double *met, const double *bg,
@@ -239,6 +239,5 @@ void launch_emf_adj(hipStream_t s, const Geo &g, const MParm &m, const Box *eb, 
 void launch_emf_adj_gather(hipStream_t s, const Geo &g, const MParm &m, const Box *eboxes, const double *sc,
                            const double *met, double *aVf, double *aHMF, double *aHG, double *aSSMF);
 void launch_vface_rv(hipStream_t s, const Geo &g, const double *met, double *rv);
-void launch_predict_adj_mhd(hipStream_t s, const Geo &g, const MParm &m, const Clock *clk, const double *S,
-                            const double *O, const double *met, const double *aHG, const double *aWH,
-                            const double *aWN, double *aHB, double *aHMF, double *aS, double *aO, double *pw);
+void launch_predict_mf_adj(hipStream_t s, const Geo &g, const Clock *clk, const double *S, const double *O,
+                           const double *met, double *aHB, double *aHMF, double *aS, double *aO, double *pw);
