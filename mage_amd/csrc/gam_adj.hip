@@ -57,7 +57,7 @@ static inline dim3 agrid(const Box &b)
 // points of one (j, k) along i) in slabs of RBA j-rows, j fastest within a
 // slab, then k, then the next slab, cut into 256-point chunks of which
 // each XCD takes runs of 16 (as the step's launches do, see XCD_RUN in
-// gam_step.hip).  The rows at j +- 4 and at
+// gam_launch.h).  The rows at j +- 4 and at
 // k +- 4 of a point are then at most 4 RBA rows away in the order the
 // workgroups run, so the 8-point stencils of neighbouring workgroups meet
 // in L2; with the plane-by-plane order of POINT_IN the k neighbours lie a
