@@ -196,7 +196,9 @@ struct k_flux {
 // shell, per launch: a 64 x 4 tile staged one variable at a time took 2.35
 // ms for D = 1, 2 (9.15 GB), direct loads 2.02 ms for D = 0 (9.1 GB); this
 // form 1.75-1.84 ms and 1.92 ms (9.0 GB at 5.0 TB/s; the streaming rate of
-// 32 read and 11 written planes is 5.2-5.5).
+// 32 read and 11 written planes is 5.2-5.5).  With the normal alone of
+// orthonormal triads and the directions in slabs (k_flux3) 1.68 ms a direction
+// (9.6 GB at 5.7 TB/s).
 // ====================================================================
 struct FluxTile {
     Tile t;                       // D = 0: the face rows; D = 1, 2: t.nb and t.xs
