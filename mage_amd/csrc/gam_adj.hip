@@ -992,7 +992,7 @@ __device__ __forceinline__ void emf_adj_edge(unsigned w, const Geo &g, const MPa
     in.b01 = BG ? bg[(B_EDGB0 + 0 + 2 * ED) * N3 + c] : 0.0;
     in.b02 = BG ? bg[(B_EDGB0 + 1 + 2 * ED) * N3 + c] : 0.0;
     in.edge = met[(M_EDGE + ED) * N3 + c];
-    in.cap = m.CFL * in.edge * gam_rcp(clk->dt);
+    in.cap = m.CFL * in.edge / clk->dt;   // infinite for dt = 0, as the step's
     EdgeAdjS o;
     const double aEc = aE[ED * N3 + c];
     edge_emf_adj_s<RM, BORIS>(m, in, aEc, o);
