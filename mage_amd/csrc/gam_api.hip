@@ -203,7 +203,7 @@ extern "C" int gam_create(gam_ctx **out, const gam_dims *d, const gam_model *m)
     MParm &p = c->mp;
     p.gamma = m->gamma; p.CFL = m->CFL; p.Vd0 = m->Vd0; p.Ca = m->Ca; p.cHogH = m->cHogH;
     p.cHogM = m->cHogM; p.pdmb = m->pdmb; p.dFloor = m->dFloor; p.pFloor = m->pFloor;
-    p.tFin = m->tFin; p.dt0 = m->dt0; p.limDT0 = m->limDT0;
+    p.tFin = m->tFin; p.limDT0 = m->limDT0;
     p.igm1 = 1.0 / (m->gamma - 1.0);
     p.iCa2 = 1.0 / (m->Ca * m->Ca);
     p.doMHD = m->doMHD; p.doBoris = m->doBoris; p.doBG = m->doBackground; p.doLFM = m->doLFMLim;
@@ -254,6 +254,7 @@ extern "C" int gam_create(gam_ctx **out, const gam_dims *d, const gam_model *m)
     if (e == hipSuccess) {
         Clock ck;
         memset(&ck, 0, sizeof(ck));
+        ck.dt0 = m->dt0;
         double h = GAM_HUGE;
         memcpy(&ck.dtBits, &h, sizeof(double));
         e = hipMemcpy(c->clk, &ck, sizeof(Clock), hipMemcpyHostToDevice);
@@ -635,8 +636,9 @@ extern "C" int gam_set_dt0(gam_ctx *c, double dt0)
 {
     if (!c) return fail(GAM_E_ARG, "gam_set_dt0: NULL context");
     if (!(dt0 >= 0.0)) return fail(GAM_E_ARG, "gam_set_dt0: dt0 must be >= 0");
+    launch_clock_dt0(c->stream, c->clk, dt0);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
-    c->mp.dt0 = dt0;
     c->model.dt0 = dt0;
     return GAM_OK;
 }
@@ -644,7 +646,7 @@ extern "C" int gam_set_dt0(gam_ctx *c, double dt0)
 extern "C" int gam_get_dt0(gam_ctx *c, double *dt0)
 {
     if (!c || !dt0) return fail(GAM_E_ARG, "gam_get_dt0: NULL argument");
-    *dt0 = c->mp.dt0;
+    *dt0 = c->model.dt0;
     return GAM_OK;
 }
 
@@ -1926,7 +1928,7 @@ static int adj_put(gam_adj *a, int n, const double *src, int npl)
     c->cur = a->cur0 ^ (n & 1);
     HIPCHK(hipMemcpyAsync(S_cur(c), src, bytes, hipMemcpyDeviceToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(S_old(c), src + (size_t)npl * c->g.N3, bytes, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->clk, a->clkh + n, sizeof(Clock), hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->clk, a->clkh + n, CLOCK_TIME, hipMemcpyDeviceToDevice, c->stream));
     return GAM_OK;
 }
 
@@ -2172,7 +2174,7 @@ extern "C" int gam_adj_backward(gam_adj *a, double *gGas, double *gGasO, double 
         int r = GAM_OK;
         if (hipMemcpyAsync(slot(1), ck, bytes, hipMemcpyDeviceToDevice, c->stream) ||
             hipMemcpyAsync(slot(0), ck + (size_t)CK_NPL * N3, bytes, hipMemcpyDeviceToDevice, c->stream) ||
-            hipMemcpyAsync(c->clk, a->clkh + s0, sizeof(Clock), hipMemcpyDeviceToDevice, c->stream))
+            hipMemcpyAsync(c->clk, a->clkh + s0, CLOCK_TIME, hipMemcpyDeviceToDevice, c->stream))
             r = fail(GAM_E_HIP, "gam_adj_backward: tape copy failed");
         c->st[c->cur] = slot(1);
         c->st[1 - c->cur] = slot(0);

@@ -46,11 +46,11 @@ __device__ __forceinline__ void finalize_clock(const MParm &m, Clock *clk, int m
         double dt = dtMin;
         if (c.ts > 0) {
             if (c.dt / dtMin >= 10) st = st > 1 ? st : 1;
-            if ((m.dt0 > GAM_TINY) && (dtMin / m.dt0 <= m.limDT0)) st = st > 1 ? st : 1;
+            if ((c.dt0 > GAM_TINY) && (dtMin / c.dt0 <= m.limDT0)) st = st > 1 ? st : 1;
             if (dtMin <= GAM_TINY) st = 2;
         }
         if ((c.t + dt) > m.tFin) dt = dmax(m.tFin - c.t, GAM_TINY);
-        if (m.dt0 > GAM_TINY && dt > (10.0 * m.dt0)) dt = 10.0 * m.dt0;
+        if (c.dt0 > GAM_TINY && dt > (10.0 * c.dt0)) dt = 10.0 * c.dt0;
         c.dtRet = dt;
         c.lastStatus = st;
         c.status = c.status > st ? c.status : st;

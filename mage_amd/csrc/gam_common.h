@@ -9,6 +9,7 @@
 // in the reference's (isg:ieg[+1], ...) Fortran arrays.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #define GAM_TINY 1.0e-12
@@ -36,7 +37,7 @@ struct EdgeBoxes { Box e[3]; };
 
 struct MParm {
     double gamma, CFL, Vd0, Ca, cHogH, cHogM, pdmb, dFloor, pFloor;
-    double tFin, dt0, limDT0;
+    double tFin, limDT0;
     double igm1;    // 1/(gamma-1)
     double iCa2;    // 1/Ca^2
     int doMHD, doBoris, doBG, doLFM, rmeth;
@@ -66,7 +67,12 @@ struct Clock {
     int lastStatus; // status of the last CalcDT
     int pad;
     double whf;     // AB2 weight of the last step's half state
+    // Model%dt0, kept here and not in MParm: captured graphs and ensemble
+    // records hold MParm by value.  Last, as no part of a recorded time: what
+    // puts a recorded clock back copies the CLOCK_TIME bytes before it.
+    double dt0;
 };
+enum { CLOCK_TIME = offsetof(Clock, dt0) };
 
 // Plane indices: State buffer.  S_W holds the primitives of the gas (CellC2P)
 // wherever a step has left them; the planes before it are the state itself.

@@ -140,10 +140,11 @@ void launch_update(hipStream_t s, int ax, const Geo &g, const MParm &m, const Bo
 void launch_calc_dt(hipStream_t s, const Geo &g, const MParm &m, const Box &dtb, Clock *clk,
                     const double *S, const double *met, const double *bg);
 // Clock fields set from the host: State%time (st) or oState%time; Model%t,
-// dt, ts; AdvanceMHD's dt
+// dt, ts; AdvanceMHD's dt; Model%dt0
 void launch_clock_state(hipStream_t s, Clock *clk, bool st, double time);
 void launch_clock_time(hipStream_t s, Clock *clk, double t, double dt, int ts);
 void launch_clock_dta(hipStream_t s, Clock *clk, double dt);
+void launch_clock_dt0(hipStream_t s, Clock *clk, double dt0);
 void launch_finalize(hipStream_t s, const MParm &m, Clock *clk, int mode);
 void launch_bflux2fld(hipStream_t s, const Geo &g, const Box &cb, const Box &skip, const double *mf,
                       double *B, const double *met);

@@ -437,6 +437,7 @@ __global__ void k_clock_time(Clock *clk, double t, double dt, int ts)
     clk->ts = ts;
 }
 __global__ void k_clock_dta(Clock *clk, double dt) { clk->dtA = dt; }
+__global__ void k_clock_dt0(Clock *clk, double dt0) { clk->dt0 = dt0; }
 
 // Zero the E entries outside the active EMF boxes (CalcElecField zeroes E
 // before filling the active edges, fields.F90:89).
@@ -578,6 +579,10 @@ void launch_clock_time(hipStream_t s, Clock *clk, double t, double dt, int ts)
 void launch_clock_dta(hipStream_t s, Clock *clk, double dt)
 {
     LAUNCH(k_clock_dta, dim3(1), dim3(1), s, clk, dt);
+}
+void launch_clock_dt0(hipStream_t s, Clock *clk, double dt0)
+{
+    LAUNCH(k_clock_dt0, dim3(1), dim3(1), s, clk, dt0);
 }
 
 void launch_mask_e(hipStream_t s, const Geo &g, const Box &all, const Box *eboxes, double *E)
