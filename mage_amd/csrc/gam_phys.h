@@ -105,7 +105,9 @@ __device__ __forceinline__ double half_prim(const MParm &m, int v, double q, dou
 // what it exceeds q1 by more than 2b |q1 - q0| where the two slopes agree in
 // sign, all of it where they do not: that is the clip of the value to the
 // interval from q1 to q1 + minmod(q2 - q1, 2b (q1 - q0)), written here
-// without sign selects (21 instructions for both sides instead of 54).
+// without sign selects (23 instructions for both sides instead of 54).  fmin
+// and fmax drop a NaN, the reference's form hands on one in n[0] or n[3]: so
+// do the products with 0 here (as NaN also an infinity there), two of the 23.
 // n[4] the limiter values around the face (between n[1] and n[2]), l and r
 // the interpolated values of the two sides.
 __device__ __forceinline__ void pdm_lr(double b, const double *n, double l, double r, double &ql,
@@ -115,8 +117,8 @@ __device__ __forceinline__ void pdm_lr(double b, const double *n, double l, doub
     const double mL = b2 * (n[1] - n[0]), mR = b2 * (n[3] - n[2]);
     const double hiL = n[1] + fmax(0.0, fmin(d, mL)), loL = n[1] + fmin(0.0, fmax(d, mL));
     const double hiR = n[2] - fmin(0.0, fmax(d, mR)), loR = n[2] - fmax(0.0, fmin(d, mR));
-    ql = fmax(loL, fmin(l, hiL));
-    qr = fmax(loR, fmin(r, hiR));
+    ql = fmax(loL, fmin(l, hiL)) + 0.0 * mL;
+    qr = fmax(loR, fmin(r, hiR)) + 0.0 * mR;
 }
 
 // Volume-weighted reconstruction + limiting for one variable at one face:
