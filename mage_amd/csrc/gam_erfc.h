@@ -48,7 +48,9 @@ GAM_HD inline double gam_erfc_exp(double z, double &e)
 #pragma unroll
     for (int n = 24; n >= 0; n--) q = std::fma(q, u, GAM_ERFC_Q[n]);
     const double hi = a * a;
-    const double lo = hi < 1.0e300 ? std::fma(a, a, -hi) : 0.0;   // 0 for a = inf
+    // 0 for a = inf; a NaN goes through here into both results (the fmin above
+    // and gam_exp_neg drop it)
+    const double lo = hi >= 1.0e300 ? 0.0 : std::fma(a, a, -hi);
     e = gam_exp_neg(-hi);
     e = std::fma(-e, lo, e);
     const double r = t * e * q;

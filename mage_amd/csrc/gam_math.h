@@ -71,7 +71,7 @@ GAM_HD inline double gam_sqrt(double x)
 
 // exp(x) for x <= 0: x = n ln 2 + r with |r| <= ln(2) / 2, the Taylor
 // polynomial of degree 13 in r (remainder below 5e-18) and a scaling by
-// 2^n; 0 below -800 (and for -inf).
+// 2^n; 0 below -800 (and for -inf, and for NaN).
 GAM_HD inline double gam_exp_neg(double x)
 {
     x = std::fmax(x, -800.0);
