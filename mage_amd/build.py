@@ -76,6 +76,18 @@ def build_restart_lib():
     return RES_LIB
 
 
+# gam_math.h and gam_erfc.h evaluated on the device, for their test
+MATH_LIB = os.path.join(ROOT, "tests", "libdevmath.so")
+
+
+def build_math_test_lib():
+    tmp = MATH_LIB + ".tmp"
+    _run([HIPCC] + FLAGS + ["-shared", os.path.join(ROOT, "tests", "device_math.hip"), "-o", tmp])
+    os.replace(tmp, MATH_LIB)
+    return MATH_LIB
+
+
 if __name__ == "__main__":
     print(build_lib(verbose="-v" in sys.argv))
     print(build_restart_lib())
+    print(build_math_test_lib())

@@ -5,10 +5,12 @@
 // the clock it costs) as by memory: on gfx950 a correctly rounded division
 // is ~11 vector instructions, a square root ~14 and exp ~30, each 4 cycles.
 // These forms take 5, 9-12 and 18.  They start from the hardware's seeds
-// (v_rcp_f64, v_rsq_f64) and take two Newton steps, which leaves 1 ulp;
-// arguments are positive and normal (densities, pressures, squared speeds,
-// sums of face areas), and a zero or infinite argument gives NaN where the
-// plain form gives an infinity or 0, except where noted.
+// (v_rcp_f64, v_rsq_f64) and take two Newton steps, which leaves a relative
+// 2^-53 (2.5 times that for the reciprocal square root).  Arguments are normal
+// and, but for gam_rcp's (an edge's determinant has either sign), positive:
+// densities, pressures, squared speeds, sums of face areas.  A zero or infinite
+// argument gives NaN where the plain form gives an infinity or 0, except where
+// noted; what a caller may set to 0 (Model%dt) is divided by.
 // The host builds (CPU tests) use the plain operations.
 #pragma once
 #include <cmath>
