@@ -15,7 +15,7 @@
  *  - Host arrays are the reference's own Fortran arrays: column-major, i
  *    fastest, ghost lower bounds isg=1-nG.  The state, grid, background and
  *    adjoint-gradient arrays may also be device memory of the context's GPU
- *    in that same layout (the copies use hipMemcpyDefault).  Cell arrays are
+ *    in that same layout (kernels on the context's stream read and write it).  Cell arrays are
  *    (Ni,Nj,Nk[,comp...]) with Ni=Nip+2nG, face/edge arrays are
  *    (Ni+1,Nj+1,Nk+1[,comp...]) exactly as allocated by gamutils.F90:169-201
  *    (allocState/allocGridVec) and init.F90:793-1072 (Corners2Grid).

@@ -359,6 +359,16 @@ static int download(gam_ctx *c, const double *src, int face, int ncomp, double *
     return GAM_OK;
 }
 
+// ncomp planes of n zeros to the caller's array, host or device memory.
+static int put_zero(gam_ctx *c, double *dst, size_t n, int ncomp)
+{
+    HIPCHK(hipMemsetAsync(c->stage, 0, n * sizeof(double), c->stream));
+    for (int q = 0; q < ncomp; q++)
+        HIPCHK(hipMemcpyAsync(dst + q * n, c->stage, n * sizeof(double), hipMemcpyDefault, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return GAM_OK;
+}
+
 // The device clock as it is once everything enqueued so far has run: one
 // copy to pinned memory behind it and one wait.
 static int read_clock(gam_ctx *c, Clock *ck)
@@ -594,7 +604,7 @@ extern "C" int gam_get_state(gam_ctx *c, int which, double *Gas, double *magFlux
         if (Gas && (rc = download(c, c->H + H_GAS * N3, 0, 5, Gas))) return rc;
         if (magFlux && (rc = download(c, c->H + H_MF * N3, 1, 3, magFlux))) return rc;
         if (Bxyz && (rc = download(c, c->H + H_B * N3, 0, 3, Bxyz))) return rc;
-        if (Efld) memset(Efld, 0, sizeof(double) * (size_t)c->g.Ni * c->g.Nj * c->g.Nk * 3);
+        if (Efld && (rc = put_zero(c, Efld, (size_t)c->g.Ni * c->g.Nj * c->g.Nk, 3))) return rc;
         if (time) *time = 0.0;
         return GAM_OK;
     }
