@@ -50,7 +50,8 @@ struct gam_ctx {
     MParm mp;
     Geo g;
     hipStream_t stream;
-    double *st[2];        // State / oState buffers (S_NPL planes each)
+    double *st[2];        // State / oState buffers (snpl planes each)
+    int snpl;             // S_NPL, or ST_NPL: without the primitives
     int cur;              // which of st[] is State
     unsigned gen;         // bumped whenever recorded launch arguments change
     double *H;            // half state + primitive planes
@@ -58,7 +59,7 @@ struct gam_ctx {
     double *bg;           // background planes (+9 scratch)
     double *gflx, *mflx, *vf;
     double *stage;        // one-plane staging buffer for layout conversion
-    double *part;         // reduction partials
+    double *part;         // reduction partials: the staging buffer, never in use at once
     Clock *clk;
     Clock *hclk;          // pinned host copy of *clk (read_clock)
     double *wind;         // device wind series
@@ -178,6 +179,60 @@ static int prof_flush(gam_ctx *c)
 // ------------------------------------------------------------ create
 extern "C" const char *gam_last_error(void) { return g_err; }
 
+static void free_planes(gam_ctx *c)
+{
+    double **bufs[] = {&c->st[0], &c->st[1], &c->H, &c->met, &c->bg, &c->gflx, &c->mflx, &c->vf, &c->stage};
+    for (double **b : bufs) {
+        if (*b) hipFree(*b);
+        *b = nullptr;
+    }
+    c->part = nullptr;
+}
+
+// Index space and planes of a context.  prims: S_W planes in the State
+// buffers; compact: rows of whole 64-byte lines instead of 128.  Leaves
+// nothing allocated where it fails; past GAM_MEM_LIMIT (bytes, from the
+// environment) it fails as a full device does.
+static hipError_t alloc_planes(gam_ctx *c, bool prims, bool compact)
+{
+    Geo &g = c->g;
+    const gam_dims &d = c->dims;
+    g.Nip = d.Nip; g.Njp = d.Njp; g.Nkp = d.Nkp;
+    g.Ni = d.Nip + 8; g.Nj = d.Njp + 8; g.Nk = d.Nkp + 8;
+    g.is = 1; g.ie = d.Nip; g.js = 1; g.je = d.Njp; g.ks = 1; g.ke = d.Nkp;
+    g.isg = -3; g.ieg = g.ie + 4; g.jsg = -3; g.jeg = g.je + 4; g.ksg = -3; g.keg = g.ke + 4;
+    // rows of whole 128-byte lines with the first active cell i = is at the
+    // start of one (index 16), the i ghosts below it at the end of the row
+    // before: tiles of 16 or 32 points from i = is read whole lines.  The last
+    // row of the last plane then ends past it.
+    const int line = compact ? 8 : 16;
+    g.P = (g.Ni + 1 + line - 1) / line * line;
+    g.PP = (long)g.P * (g.Nj + 1);
+    g.c0 = line - g.is - (long)g.P * g.jsg - g.PP * g.ksg;
+    const long n3 = g.PP * (g.Nk + 1) + (compact ? 0 : 16);
+    g.N3 = (n3 + 63) / 64 * 64;
+    c->snpl = prims ? S_NPL : ST_NPL;
+    struct { double **p; int n; } want[] = {
+        {&c->st[0], c->snpl}, {&c->st[1], c->snpl}, {&c->H, H_NPL}, {&c->met, M_NPL}, {&c->bg, B_NPL + 9},
+        {&c->gflx, 15}, {&c->mflx, 9}, {&c->vf, 9}, {&c->stage, 1}};
+    const char *lim = getenv("GAM_MEM_LIMIT");
+    size_t left = lim ? (size_t)strtoull(lim, nullptr, 10) : (size_t)-1;
+    hipError_t e = hipSuccess;
+    for (auto &w : want) {
+        const size_t bytes = (size_t)w.n * g.N3 * sizeof(double);
+        if (e == hipSuccess && bytes > left) e = hipErrorOutOfMemory;
+        left -= bytes;
+        if (e == hipSuccess) e = hipMalloc((void **)w.p, bytes);
+        if (e == hipSuccess) e = hipMemset(*w.p, 0, bytes);
+    }
+    c->part = c->stage;
+    if (e != hipSuccess) {
+        free_planes(c);
+        hipGetLastError();   // the failure is reported by value
+    }
+    return e;
+}
+
 extern "C" int gam_create(gam_ctx **out, const gam_dims *d, const gam_model *m)
 {
     if (!out || !d || !m) return fail(GAM_E_ARG, "gam_create: NULL argument");
@@ -209,46 +264,23 @@ extern "C" int gam_create(gam_ctx **out, const gam_dims *d, const gam_model *m)
     p.doMHD = m->doMHD; p.doBoris = m->doBoris; p.doBG = m->doBackground; p.doLFM = m->doLFMLim;
     p.rmeth = m->rmeth;
 
-    Geo &g = c->g;
-    g.Nip = d->Nip; g.Njp = d->Njp; g.Nkp = d->Nkp;
-    g.Ni = d->Nip + 8; g.Nj = d->Njp + 8; g.Nk = d->Nkp + 8;
-    g.is = 1; g.ie = d->Nip; g.js = 1; g.je = d->Njp; g.ks = 1; g.ke = d->Nkp;
-    g.isg = -3; g.ieg = g.ie + 4; g.jsg = -3; g.jeg = g.je + 4; g.ksg = -3; g.keg = g.ke + 4;
-    // rows of whole 128-byte lines with the first active cell i = is at the
-    // start of one (index 16), the i ghosts below it at the end of the row
-    // before: tiles of 16 or 32 points from i = is read whole lines
-    g.P = (g.Ni + 1 + 15) / 16 * 16;
-    g.PP = (long)g.P * (g.Nj + 1);
-    g.c0 = 16 - g.is - (long)g.P * g.jsg - g.PP * g.ksg;
-    long n3 = g.PP * (g.Nk + 1) + 16;
-    g.N3 = (n3 + 63) / 64 * 64;
-    const size_t pl = (size_t)g.N3 * sizeof(double);
-
     int rc = GAM_OK;
-    hipError_t e = hipSuccess;
-#define ALLOC(ptr, nplanes)                                                   \
-    if (e == hipSuccess) {                                                    \
-        e = hipMalloc((void **)&(ptr), (size_t)(nplanes) * pl);              \
-        if (e == hipSuccess) e = hipMemset((ptr), 0, (size_t)(nplanes) * pl); \
-    }
-    e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
+    hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     for (int q = 0; e == hipSuccess && q < 2; q++) e = hipStreamCreateWithFlags(&c->aux[q], hipStreamNonBlocking);
     for (int q = 0; e == hipSuccess && q < 6; q++) e = hipEventCreateWithFlags(&c->fev[q], hipEventDisableTiming);
     {
         const char *cv = getenv("GAM_CONCURRENT");
         c->concurrent = (cv && cv[0] == '0') ? 0 : 1;
     }
-    ALLOC(c->st[0], S_NPL);
-    ALLOC(c->st[1], S_NPL);
-    ALLOC(c->H, H_NPL);
-    ALLOC(c->met, M_NPL);
-    ALLOC(c->bg, B_NPL + 9);
-    ALLOC(c->gflx, 15);
-    ALLOC(c->mflx, 9);
-    ALLOC(c->vf, 9);
-    ALLOC(c->stage, 1);
-    ALLOC(c->part, 1);
-#undef ALLOC
+    // Primitives beside the states and rows of whole 128-byte lines, where
+    // both fit; else 208 planes of 64-byte rows, whose steps run the predictor
+    // (96x96x128 shell 0.816 ms per step in place of 0.669, 256x256x384 14.5 in
+    // place of 12.5).
+    const bool prims = p.doMHD || (!p.doBG && !p.doBoris);
+    if (e == hipSuccess) {
+        e = alloc_planes(c, prims, false);
+        if (e == hipErrorOutOfMemory) e = alloc_planes(c, false, true);
+    }
     if (e == hipSuccess) e = hipMalloc((void **)&c->clk, sizeof(Clock));
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->hclk, sizeof(Clock), hipHostMallocDefault);
     if (e == hipSuccess) {
@@ -284,8 +316,8 @@ extern "C" int gam_destroy(gam_ctx *c)
     if (!c) return GAM_OK;
     if (c->stream) hipStreamSynchronize(c->stream);
     graphs_drop(c);
-    double *bufs[] = {c->st[0], c->st[1], c->H, c->met, c->bg, c->gflx, c->mflx, c->vf, c->stage, c->part, c->wind};
-    for (double *b : bufs) if (b) hipFree(b);
+    free_planes(c);
+    if (c->wind) hipFree(c->wind);
     if (c->clk) hipFree(c->clk);
     if (c->hclk) hipHostFree(c->hclk);
     for (int q = 0; q < (int)(sizeof(c->ev) / sizeof(c->ev[0])); q++) if (c->ev[q]) hipEventDestroy(c->ev[q]);
@@ -785,11 +817,12 @@ static void enq_fluxes_emfs_apart(gam_ctx *c, const HalfSrc &h, const Box *eb, d
         }
 }
 
-// Whether the launch plan's fluxes and EMFs can form the half state themselves.
-// (Boris and the background field are nothing without a magnetic field.)
+// Whether steps leave the primitives, and whether the launch plan's fluxes and
+// EMFs can form the half state themselves.  (Boris and the background field
+// are nothing without a magnetic field: those contexts go without.)
 static bool keeps_prims(const gam_ctx *c)
 {
-    return c->mp.doMHD || (!c->mp.doBG && !c->mp.doBoris);
+    return c->snpl == S_NPL;
 }
 static bool plan_direct(const gam_ctx *c)
 {
@@ -1617,7 +1650,7 @@ extern "C" int gam_autotune(gam_ctx *c, int reps)
     if ((rc = hf_flush(c))) return rc;
     // snapshot State, oState (with their primitives) and the clock; tuning
     // takes real steps
-    const size_t bytes = (size_t)S_NPL * c->g.N3 * sizeof(double);
+    const size_t bytes = (size_t)c->snpl * c->g.N3 * sizeof(double);
     double *save = nullptr;
     HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipMalloc((void **)&save, 2 * bytes));
