@@ -236,7 +236,9 @@ int gam_get_solver(gam_ctx *ctx, int which, double *out);
  * along i first) and 5 (along the flux direction first), with 6 and 7 as
  * other names of 4 and 5.
  * gam_autotune times every candidate of every slot on the context's own
- * grid (reps steps per candidate, hipEvents around that slot's launch),
+ * grid (reps steps per candidate; hipEvents around the predictor's or the
+ * update's launch, and around whole steps for the flux and EMF slots, which
+ * decide whether a step needs the predictor and how many launches it makes),
  * keeps the fastest (the current shape unless another is more than 1 %
  * faster), keeps the resulting plan only if 4 x reps whole graph-replayed
  * steps also run more than 1 % faster with it than with the plan it

@@ -731,7 +731,11 @@ static void enq_bcs(gam_ctx *c, double *S, Clock *clk = nullptr)
     launch_bcs(c->stream, c->model.bc, false, false, 0, c->g, c->mp, clk ? clk : c->clk, c->wd, S, c->met);
 }
 
-// While a slot is being tuned, its launches are bracketed by events.
+// While a slot is being tuned, its launch is bracketed by events: of the
+// predictor and the update themselves, of the fluxes and EMFs whole steps, as
+// their shapes decide which launches a step makes (merged or apart, with the
+// predictor or without).
+static bool tuned_whole(int slot) { return slot != TS_PREDICT && slot != TS_UPDATE; }
 static void tune_mark(gam_ctx *c, int slot)
 {
     if (c->tune_slot != slot || c->ntev >= 2 * GAM_TUNE_MAXREPS) return;
@@ -748,13 +752,12 @@ static void flux_boxes(const Geo &g, Box *fb)
 
 // The fluxes of every direction and the Mom2Face rim as one launch, if the
 // plan's shapes allow it for them and for the EMFs; false: nothing enqueued.
-// While a slot is tuned its launch stays apart, and so do those of an
-// ensemble's first steps, with the predictor (whose branches the batched graph
-// runs side by side).
+// The launches of an ensemble's first steps, with the predictor, stay apart
+// (their branches run side by side in the batched graph).
 static bool enq_fluxes_merged(gam_ctx *c, const HalfSrc &h)
 {
     const int *form = &c->plan.v[TS_FLUX_I];
-    if (c->tune_slot >= 0 || (launch_recorder() && !c->direct) || !flux3_ok(form) || !emf3_ok(&c->plan.v[TS_EMF_I])) return false;
+    if ((launch_recorder() && !c->direct) || !flux3_ok(form) || !emf3_ok(&c->plan.v[TS_EMF_I])) return false;
     Box fb[3];
     flux_boxes(c->g, fb);
     prof_begin(c, KG_FLUX);
@@ -763,7 +766,8 @@ static bool enq_fluxes_merged(gam_ctx *c, const HalfSrc &h)
     return true;
 }
 
-// One launch per direction of the fluxes and EMFs.  Inside a captured graph
+// One launch per direction of the fluxes and EMFs, from the predictor's
+// planes (a step without it takes the merged launches).  Inside a captured graph
 // (fork) the j and k fluxes and the EMFs that take their face velocities run
 // on two more streams: the graph then has three branches between the
 // predictor and the update, which the device may overlap.  The launches and
@@ -786,10 +790,8 @@ static void enq_fluxes_emfs_apart(gam_ctx *c, const HalfSrc &h, const Box *eb, d
     flux_boxes(g, fb);
     for (int d = 0; d < 3; d++) {
         prof_begin(c, KG_FLUX);
-        tune_mark(c, TS_FLUX_I + d);
         launch_flux(fs[d], d, c->plan.v[TS_FLUX_I + d], g, c->mp, fb[d], h, c->met, c->bg, c->gflx, c->mflx,
                     c->vf + (long)3 * d * N3);
-        tune_mark(c, TS_FLUX_I + d);
         prof_end(c, KG_FLUX);
     }
     if (!c->mp.doMHD) return;
@@ -804,10 +806,8 @@ static void enq_fluxes_emfs_apart(gam_ctx *c, const HalfSrc &h, const Box *eb, d
         // edge direction eD takes the face velocities along dT1
         const int dT1 = (eD == 0) ? 1 : (eD == 1) ? 2 : 0;
         prof_begin(c, KG_EMF);
-        tune_mark(c, TS_EMF_I + eD);
         launch_emf(fs[dT1], eD, c->plan.v[TS_EMF_I + eD], g, c->mp, eb[eD], h, c->vf + (long)3 * dT1 * N3, c->met,
                    c->bg, E);
-        tune_mark(c, TS_EMF_I + eD);
         prof_end(c, KG_EMF);
     }
     if (fork)
@@ -1596,15 +1596,20 @@ extern "C" int gam_set_plan(gam_ctx *c, const int *plan)
     return GAM_OK;
 }
 
-// Time one slot's launches over reps steps (after one untimed step).
+// Time one slot over reps steps, after two untimed ones: the shape's first,
+// and, after steps that ran the predictor, as many as still must.
 static int tune_time(gam_ctx *c, int slot, int reps, double *ms)
 {
     c->tune_slot = -1;
     c->general += slot == TS_PREDICT;   // steps that run it
-    enq_step(c, false);
+    for (int r = 0; r < 2; r++) enq_step(c, false);
     c->tune_slot = slot;
     c->ntev = 0;
-    for (int r = 0; r < reps; r++) enq_step(c, false);
+    for (int r = 0; r < reps; r++) {
+        if (tuned_whole(slot)) tune_mark(c, slot);
+        enq_step(c, false);
+        if (tuned_whole(slot)) tune_mark(c, slot);
+    }
     c->tune_slot = -1;
     c->general -= slot == TS_PREDICT;
     HIPCHK(hipGetLastError());
@@ -1667,6 +1672,16 @@ extern "C" int gam_autotune(gam_ctx *c, int reps)
     }
     c->prof = 0;
     const Plan start = c->plan;
+    // The forms without the predictor are one choice: a plan that has only
+    // some of its fluxes and EMFs in them gains nothing by the next one.
+    if (keeps_prims(c) && !plan_direct(c)) {
+        const Plan d = default_plan();
+        double apart = 0.0, merged = 0.0;
+        rc = tune_time(c, TS_FLUX_I, reps, &apart);
+        for (int q = TS_EMF_I; q <= TS_FLUX_K; q++) c->plan.v[q] = d.v[q];
+        if (rc == GAM_OK) rc = tune_time(c, TS_FLUX_I, reps, &merged);
+        if (rc != GAM_OK || !(merged < 0.99 * apart)) c->plan = start;
+    }
     // the current shape is timed first and another replaces it only when
     // more than 1 % faster, so timing noise does not flip near-equal shapes
     for (int slot = 0; slot < TS_COUNT && rc == GAM_OK; slot++) {

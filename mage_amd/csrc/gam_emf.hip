@@ -359,20 +359,20 @@ struct edge_tile {
     }
 };
 
-template <int ED, int RM, bool BG, bool BORIS, bool DIR>
+// one edge direction, from the predictor's planes
+template <int ED, int RM, bool BG, bool BORIS>
 struct k_emf_t {
     static constexpr int NT = BX * BY;
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, EdgeTile b, const Clock *clk,
                                                const double *__restrict__ H,
                                                const double *__restrict__ S,
-                                               const double *__restrict__ O,
                                                const double *__restrict__ Vf,
                                                const double *__restrict__ met,
                                                const double *__restrict__ bg,
                                                double *__restrict__ E) const
     {
         __shared__ double lds[edge_geom<ED>::LDS];
-        edge_tile<ED, RM, BG, BORIS, DIR>{}(lds, (int)bi.x, g, m, b, clk, H, S, O, Vf, met, bg, E);
+        edge_tile<ED, RM, BG, BORIS, false>{}(lds, (int)bi.x, g, m, b, clk, H, S, nullptr, Vf, met, bg, E);
     }
 };
 
@@ -484,8 +484,7 @@ static void emf_t(hipStream_t s, int plan, const Geo &g, const MParm &m, const B
     if (emf_lds(plan)) {
         const EdgeTile t = edge_tiles(ED, b);
         const dim3 gr(xcd_grid(t.nb, t.xs)), bl(BX, BY);
-        if (h.O) launch_f<k_emf_t<ED, RM, BG, BO, true>>(gr, bl, s, g, m, t, clk, H, S, h.O, Vf, met, bg, E);
-        else launch_f<k_emf_t<ED, RM, BG, BO, false>>(gr, bl, s, g, m, t, clk, H, S, h.O, Vf, met, bg, E);
+        launch_f<k_emf_t<ED, RM, BG, BO>>(gr, bl, s, g, m, t, clk, H, S, Vf, met, bg, E);
         return;
     }
     const int ch = plan_chunk(plan);

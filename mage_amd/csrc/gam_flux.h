@@ -446,13 +446,13 @@ struct flux_tile {
     }
 };
 
-template <int D, int RM, bool BG, bool BORIS, int DIR>
+// one direction, from the predictor's planes
+template <int D, int RM, bool BG, bool BORIS>
 struct k_flux_t {
     static constexpr int NT = 256;
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, MParm m, FluxTile t,
                                                const double *__restrict__ H,
                                                const double *__restrict__ S,
-                                               const double *__restrict__ O, const Clock *clk,
                                                const double *__restrict__ met,
                                                const double *__restrict__ bg,
                                                double *__restrict__ gflx,
@@ -460,7 +460,7 @@ struct k_flux_t {
                                                double *__restrict__ Vf) const
     {
         __shared__ double lds[FLUX_LDS];
-        flux_tile<D, RM, BG, BORIS, DIR>{}(lds, (int)bi.x, g, m, t, H, S, O, clk, met, bg, gflx, mflx, Vf);
+        flux_tile<D, RM, BG, BORIS, 0>{}(lds, (int)bi.x, g, m, t, H, S, nullptr, nullptr, met, bg, gflx, mflx, Vf);
     }
 };
 
@@ -496,15 +496,7 @@ static void flux_t(hipStream_t s, int form, const Geo &g, const MParm &m, const 
     const double *H = h.H, *S = h.S;
     if (flux_lds(D, form)) {
         const FluxTile t = flux_tiles(D, b, flux_alt(D, form));
-        if (!h.O)
-            launch_f<k_flux_t<D, RM, BG, BO, 0>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk, met, bg, gf,
-                                                 mf, vf);
-        else if (BG || BO || m.doMHD)
-            launch_f<k_flux_t<D, RM, BG, BO, 1>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk, met, bg, gf,
-                                                 mf, vf);
-        else
-            launch_f<k_flux_t<D, RM, BG, BO, BG || BO ? 1 : 2>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, h.O, h.clk,
-                                                                met, bg, gf, mf, vf);
+        launch_f<k_flux_t<D, RM, BG, BO>>(tgrid(t.t), dim3(BX, BY), s, g, m, t, H, S, met, bg, gf, mf, vf);
         return;
     }
     const int ch = plan_chunk(form);

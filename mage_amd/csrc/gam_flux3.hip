@@ -19,7 +19,7 @@ struct Flux3 {
     RimSet rim;
     int n[3];         // workgroups of each direction in a slab
     FastDiv slab;     // by the workgroups of a slab
-    int start[2];     // first workgroup of the rim; the end
+    int rim0;         // first workgroup of the rim
 };
 
 template <int RM, bool BG, bool BORIS, int DIR>
@@ -38,8 +38,8 @@ struct k_flux3 {
         __shared__ double lds[FLUX_LDS];
         const int w = (int)bi.x;
         const long N3 = g.N3;
-        if (w >= f.start[0]) {
-            vface_rim<DIR != 0>{}(w - f.start[0], g, f.rim, H, S, O, clk, met, Vf);
+        if (w >= f.rim0) {
+            vface_rim<DIR != 0>{}(w - f.rim0, g, f.rim, H, S, O, clk, met, Vf);
             return;
         }
         const int sl = (int)((unsigned)w / f.slab);
@@ -75,10 +75,9 @@ static void flux3_t(hipStream_t s, const int *form, const Geo &g, const MParm &m
     }
     f.slab = fast_div((unsigned)tot);
     tot *= ns;
-    f.start[0] = tot;
+    f.rim0 = tot;
     f.rim = rim_set(g);
     if (m.doMHD) tot += f.rim.start[6];
-    f.start[1] = tot;
     const dim3 gr((unsigned)tot), bl(BX, BY);
     if (!h.O) launch_f<k_flux3<RM, BG, BO, 0>>(gr, bl, s, g, m, f, h.H, h.S, h.O, h.clk, met, bg, gf, mf, vf);
     else if (BG || BO || m.doMHD)
@@ -113,7 +112,5 @@ void launch_flux3(hipStream_t s, const int *form, const Geo &g, const MParm &m, 
 void launch_vface_rim(hipStream_t s, const Geo &g, const HalfSrc &h, const double *met, double *Vf)
 {
     const RimSet r = rim_set(g);
-    const dim3 gr((unsigned)r.start[6]), bl(BX, BY);
-    if (h.O) launch_f<k_vface_rim<true>>(gr, bl, s, g, r, h.H, h.S, h.O, h.clk, met, Vf);
-    else launch_f<k_vface_rim<false>>(gr, bl, s, g, r, h.H, h.S, h.O, h.clk, met, Vf);
+    launch_f<k_vface_rim>(dim3((unsigned)r.start[6]), dim3(BX, BY), s, g, r, h.H, met, Vf);
 }

@@ -107,6 +107,7 @@ struct HalfSrc {
 
 void launch_predict(hipStream_t s, int ax, const Geo &g, const MParm &m, const Box &fb, const Clock *clk,
                     const double *S, const double *O, const double *met, double *H, int hfonly = 0);
+// Launches of one direction each take the half state from h.H (h.O null).
 // Mom2Face on the faces the EMF stencils read past the interface-flux faces
 // (the flux kernels write the rest): Vf planes [3*dT1 + comp]
 void launch_vface_rim(hipStream_t s, const Geo &g, const HalfSrc &h, const double *met, double *Vf);

@@ -54,14 +54,12 @@ struct vface_rim {
     }
 };
 
-template <bool DIR>
 struct k_vface_rim {
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g, RimSet r, const double *__restrict__ H,
-                                               const double *__restrict__ S, const double *__restrict__ O,
-                                               const Clock *clk, const double *__restrict__ met,
+                                               const double *__restrict__ met,
                                                double *__restrict__ Vf) const
     {
-        vface_rim<DIR>{}((int)bi.x, g, r, H, S, O, clk, met, Vf);
+        vface_rim<false>{}((int)bi.x, g, r, H, nullptr, nullptr, nullptr, met, Vf);
     }
 };
 
