@@ -8,25 +8,18 @@ The adjoint runs the same kernels on either layout: 1e-12.
 """
 import numpy as np
 import pytest
-import torch
 
 from helpers import box_case, compare_state, rel_linf, shell_case
+from hip_runtime import used
 from mage_amd import gamhip, problems as pb
 
 pytestmark = pytest.mark.gpu
-KEYS = ("Gas", "magFlux", "Bxyz", "Efld")
 
 
 def _planes(N, n):
     """Bytes of n planes of 64-byte rows."""
     pts = (N[0] + 16) * (N[1] + 9) * (N[2] + 9)
     return n * 8 * ((pts + 63) // 64 * 64)
-
-
-def _used():
-    torch.cuda.synchronize()
-    free, total = torch.cuda.mem_get_info()
-    return total - free
 
 
 def test_footprint_and_refusal(monkeypatch):
@@ -38,22 +31,22 @@ def test_footprint_and_refusal(monkeypatch):
     for limit in (None, need, need - 1):
         if limit is not None:
             monkeypatch.setenv("GAM_MEM_LIMIT", str(limit))
-        u0 = _used()
+        u0 = used()
         if limit == need - 1:
             with pytest.raises(gamhip.GamError) as ei:
                 gamhip.GamHip(*N, p)
             assert ei.value.code == -2      # GAM_E_HIP, as on a full device
-            assert _used() - u0 <= slack
+            assert used() - u0 <= slack
             continue
         g = gamhip.GamHip(*N, p)
-        used = _used() - u0
-        print("limit %s: %.1f MiB" % (limit, used / 2 ** 20), flush=True)
+        mem = used() - u0
+        print("limit %s: %.1f MiB" % (limit, mem / 2 ** 20), flush=True)
         if limit is None:
-            assert used >= _planes(N, 218)
+            assert mem >= _planes(N, 218)
         else:
-            assert used <= need + slack
+            assert mem <= need + slack
         g.close()
-        assert _used() - u0 <= slack
+        assert used() - u0 <= slack
 
 
 def _case(kind, rmeth):
