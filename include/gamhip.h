@@ -213,7 +213,8 @@ int gam_time_steps(gam_ctx *ctx, int nsteps, double *ms);
 /* Per-kernel-group timing: when enabled, every launch group of the step is
  * bracketed by hipEvents on the context's stream.  gam_kernel_times()
  * returns accumulated milliseconds and launch counts per group in the
- * order of gam_kernel_group_name(). */
+ * order of gam_kernel_group_name().  Groups whose work is part of another
+ * launch count 0 (mom2face in the flux launch, bflux2fld_ghosts in bcs). */
 #define GAM_KG_COUNT 8
 int gam_set_profiling(gam_ctx *ctx, int on);
 int gam_kernel_times(gam_ctx *ctx, double *ms, int *counts);
@@ -261,8 +262,10 @@ int gam_tune_candidates(int slot, int *values);
  * one gamApp_T per process and has no batched form; an ensemble here is a
  * set of contexts (each one stepGamera instance, gamapp.F90:73-113, with
  * its own grid size, grid, background, inflow series, state and clock)
- * whose steps are issued as one launch per kernel covering every member,
- * and whose whole step is one captured hipGraph.  Every member's results
+ * whose steps are issued as launches that cover many members: every member
+ * in one launch per kernel where the step runs the predictor, else up to
+ * three chains of launches, each over a third of them.  The whole step is
+ * one captured hipGraph.  Every member's results
  * are those of stepping it on its own.
  * ------------------------------------------------------------------- */
 typedef struct gam_ens gam_ens;
@@ -289,7 +292,7 @@ int gam_ens_create(gam_ens **out, int n, gam_ctx *const *members);
 int gam_ens_run(gam_ens *e, int nsteps);
 /* Same, bracketed by hipEvents on the ensemble's stream; ms = elapsed time. */
 int gam_ens_time_steps(gam_ens *e, int nsteps, double *ms);
-/* Kernel launches per step of every member (= graph nodes per step). */
+/* Kernel launches per step of the ensemble (= kernel nodes of its graph). */
 int gam_ens_launches_per_step(gam_ens *e, int *n);
 int gam_ens_destroy(gam_ens *e);
 

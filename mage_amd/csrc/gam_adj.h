@@ -153,7 +153,7 @@ __device__ __forceinline__ void clip_adj(double a, double b, double qI, double a
     aqI += toQ ? aq : 0.0;
 }
 
-// PDM (pdm_one)
+// PDM (recon.F90:275-301), one side of pdm_lr
 __device__ __forceinline__ void pdm_one_adj(double b, double q0, double q1, double q2, double qI,
                                             double aout, double &aq0, double &aq1, double &aq2,
                                             double &aqI)
@@ -176,7 +176,7 @@ __device__ __forceinline__ void pdm_one_adj(double b, double q0, double q1, doub
     clip_adj(q1, q2, qI, aqN, aq1, aq2, aqI);
 }
 
-// pdmLR (pdm_pair)
+// pdmLR (recon.F90:231-272), both sides of pdm_lr with one value
 __device__ __forceinline__ void pdm_pair_adj(double b, double v0, double v1, double v2, double v3,
                                              double qi, double aql, double aqr, double &av0,
                                              double &av1, double &av2, double &av3, double &aqi)

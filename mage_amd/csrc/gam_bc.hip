@@ -73,12 +73,11 @@ struct k_finalize {
 // ====================================================================
 struct k_bflux2fld {
     __device__ __forceinline__ void operator()(const uint3 bi, Geo g,
-                                               Tile cb, Box skip, const double *__restrict__ mf,
+                                               Tile cb, const double *__restrict__ mf,
                                                double *__restrict__ B,
                                                const double *__restrict__ met) const
     {
         TILE_IJK(cb);
-        if (in_box(skip, i, j, k)) return;
         const long N3 = g.N3, c = IX(g, i, j, k);
         double b[3];
         cell_b(g, met, c, mf[c], mf[N3 + c], mf[2 * N3 + c], mf[c + 1], mf[N3 + c + g.P],
@@ -378,11 +377,11 @@ void launch_finalize(hipStream_t s, const MParm &m, Clock *clk, int mode)
     launch_f<k_finalize>(dim3(1), dim3(64), s, m, clk, mode);
 }
 
-void launch_bflux2fld(hipStream_t s, const Geo &g, const Box &cb, const Box &skip, const double *mf,
+void launch_bflux2fld(hipStream_t s, const Geo &g, const Box &cb, const double *mf,
                       double *B, const double *met)
 {
     const Tile t = tile_of(cb, 1);
-    launch_f<k_bflux2fld>(tgrid(t), dim3(BX, BY), s, g, t, skip, mf, B, met);
+    launch_f<k_bflux2fld>(tgrid(t), dim3(BX, BY), s, g, t, mf, B, met);
 }
 
 // EnforceBCs on S.  field = false: the sides alone, with cell B as they copy

@@ -96,10 +96,11 @@ int gam_fail_(int code, const char *msg, const char *detail);
 
 // Where the fluxes and EMFs take the half state from: H, the predictor's
 // planes (O null); or, with O, State S and oState O themselves.  That needs
-// MHD and both states as a step leaves them: gas at or above the density
-// floor, its primitives in S_W, cell B that of the face fluxes in every cell
-// (ghosts too), where extrapolating cell B and primitives is extrapolating
-// face fluxes and gas; and launch plans of the LDS forms.
+// both states as a step leaves them: the primitives of their gas in S_W and,
+// with MHD, gas at or above the density floor and cell B that of the face
+// fluxes in every cell (ghosts too), where extrapolating cell B and primitives
+// is extrapolating face fluxes and gas; and launch plans of the LDS forms.
+// (A hydrodynamic step applies no floor: its fluxes see to densities below it.)
 struct HalfSrc {
     const double *H, *S, *O;
     const Clock *clk;
@@ -147,7 +148,7 @@ void launch_clock_time(hipStream_t s, Clock *clk, double t, double dt, int ts);
 void launch_clock_dta(hipStream_t s, Clock *clk, double dt);
 void launch_clock_dt0(hipStream_t s, Clock *clk, double dt0);
 void launch_finalize(hipStream_t s, const MParm &m, Clock *clk, int mode);
-void launch_bflux2fld(hipStream_t s, const Geo &g, const Box &cb, const Box &skip, const double *mf,
+void launch_bflux2fld(hipStream_t s, const Geo &g, const Box &cb, const double *mf,
                       double *B, const double *met);
 // EnforceBCs of S: alone (field = false) or inside a step, with cell B of
 // the ghost cells from their faces and, with finmode, launch_finalize's work

@@ -211,7 +211,8 @@ __device__ __forceinline__ void gas_kin_vt(double igm1, double s, const double *
     dW[MOMZ] = dW[MOMZ] + s * d * vz;
     dW[ENER] = dW[ENER] + s * e;
 }
-// with the face triad T (N, T1, T2)
+// with the face triad T (N, T1, T2): the forward of gas_kin_adj, which the CPU
+// tests difference
 __device__ __forceinline__ void gas_kin(double igm1, double s, const double *W, const double *T,
                                         double *gF, double *dW)
 {

@@ -4,14 +4,19 @@
 //   k_predict    Predictor: AB2 face fluxes, half-step B and gas, plus the
 //                primitives used by the flux sweeps.  Only where the fluxes
 //                and EMFs cannot form the half state themselves (HalfSrc):
-//                without MHD, in the first two steps of a state that was put,
-//                and in the adjoint.  It moves 50 words per point, the step
+//                in the first two steps of a state that was put, in the
+//                adjoint, with launch plans of direct loads and in contexts
+//                without the primitives' planes (hydrodynamic ones with the
+//                Boris or background option, full devices).  It moves 50
+//                words per point, the step
 //                without it 8 more; 256x256x384 shell 14.46 -> 12.80 ms per
 //                step, 96x96x128 0.784 -> 0.691, 16^3 box 0.035 -> 0.032.
-//   k_flux_t     Lyon gas/magnetic fluxes, one per direction, and the face
-//                velocities (Mom2Face) of the same faces (gam_flux.h)
-//   k_vface_rim  face velocities the EMF stencils read past the flux faces
-//   k_emf        edge EMFs (gam_emf.hip)
+//   k_flux3      Lyon gas/magnetic fluxes of the three directions, the face
+//                velocities (Mom2Face) of the same faces and of those the EMF
+//                stencils read past them (gam_flux3.hip, gam_flux.h)
+//   k_emf3       edge EMFs of the three directions (gam_emf.hip)
+//                (k_flux_t or k_flux, k_vface_rim, k_emf_t or k_emf: the same
+//                one direction at a time, after k_predict)
 //   k_update     CT face-flux update, cell B of the new state, flux
 //                divergence, Reynolds, Maxwell/Boris and the CFL
 //                min-reduction of the new state

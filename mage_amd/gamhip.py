@@ -362,8 +362,8 @@ class GamHip:
 
 
 class GamEnsemble:
-    """Independent contexts stepped together: one launch per step kernel
-    over all members, one captured hipGraph per step.  The members stay
+    """Independent contexts stepped together: launches that cover many
+    members, one captured hipGraph per step.  The members stay
     usable as GamHip objects (state transfers show the ensemble's
     progress); they must outlive the ensemble."""
 
