@@ -56,8 +56,8 @@ __device__ __forceinline__ double edge_value(const MParm &m, const double *vc, d
     const double bb = b1 * b1 + b2 * b2, Ca2 = m.Ca * m.Ca;
     const double vA = gam_sqrt(BORIS ? Ca2 * bb * gam_rcp(Ca2 * Dc + bb) : bb * gam_rcp(Dc));
     vDiff = vDiff + vA;
-    // a true division: no cap (infinite) where Model%dt is 0
-    vDiff = dmin(vDiff, m.CFL * edge / dt);
+    // no cap (infinite) where Model%dt is 0
+    vDiff = dmin(vDiff, m.CFL * edge * (dt != 0.0 ? gam_rcp(dt) : HUGE_VAL));
     const double e = -(v1 * b2 - v2 * b1) + m.Vd0 * vDiff * Jd;
     return e * edge;
 }

@@ -10,7 +10,7 @@
 // and, but for gam_rcp's (an edge's determinant has either sign), positive:
 // densities, pressures, squared speeds, sums of face areas.  A zero or infinite
 // argument gives NaN where the plain form gives an infinity or 0, except where
-// noted; what a caller may set to 0 (Model%dt) is divided by.
+// noted; what a caller may set to 0 (Model%dt) is tested first or divided by.
 // The host builds (CPU tests) use the plain operations.
 #pragma once
 #include <cmath>
