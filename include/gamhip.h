@@ -102,8 +102,9 @@ const char *gam_last_error(void);
 /* Allocate device storage for one Grid/State/Solver set.
  * Replaces the allocations of Hatch/initSolver (init.F90:38-59, 486-508).
  * Where the device has no room for the planes that let steps go without the
- * predictor (or they pass GAM_MEM_LIMIT bytes, from the environment), the
- * context does without them: 208 planes in place of 218, slower steps. */
+ * predictor, the context does without them: 208 planes in place of 218, slower
+ * steps.  GAM_MEM_LIMIT (bytes, in the environment) bounds a context's planes,
+ * and gam_autotune's snapshot beside them, as a full device would. */
 int gam_create(gam_ctx **ctx, const gam_dims *dims, const gam_model *model);
 int gam_destroy(gam_ctx *ctx);
 /* The sizes the context was created with. */

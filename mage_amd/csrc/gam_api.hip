@@ -54,6 +54,7 @@ struct gam_ctx {
     hipStream_t stream;
     double *st[2];        // State / oState buffers (snpl planes each)
     int snpl;             // S_NPL, or ST_NPL: without the primitives
+    size_t bytes;         // of all planes
     int cur;              // which of st[] is State
     unsigned gen;         // bumped whenever recorded launch arguments change
     double *H;            // half state + primitive planes
@@ -191,10 +192,20 @@ static void free_planes(gam_ctx *c)
     c->part = nullptr;
 }
 
+// hipMalloc, which past GAM_MEM_LIMIT (bytes, from the environment; used: what
+// the context has) fails as on a full device.
+static hipError_t limited_malloc(double **p, size_t bytes, size_t used)
+{
+    const char *lim = getenv("GAM_MEM_LIMIT");
+    hipError_t e = lim && used + bytes > (size_t)strtoull(lim, nullptr, 10) ? hipErrorOutOfMemory
+                                                                          : hipMalloc((void **)p, bytes);
+    if (e != hipSuccess) hipGetLastError();   // the failure is reported by value
+    return e;
+}
+
 // Index space and planes of a context.  prims: S_W planes in the State
 // buffers; compact: rows of whole 64-byte lines instead of 128.  Leaves
-// nothing allocated where it fails; past GAM_MEM_LIMIT (bytes, from the
-// environment) it fails as a full device does.
+// nothing allocated where it fails.
 static hipError_t alloc_planes(gam_ctx *c, bool prims, bool compact)
 {
     Geo &g = c->g;
@@ -217,21 +228,16 @@ static hipError_t alloc_planes(gam_ctx *c, bool prims, bool compact)
     struct { double **p; int n; } want[] = {
         {&c->st[0], c->snpl}, {&c->st[1], c->snpl}, {&c->H, H_NPL}, {&c->met, M_NPL}, {&c->bg, B_NPL + 9},
         {&c->gflx, 15}, {&c->mflx, 9}, {&c->vf, 9}, {&c->stage, 1}};
-    const char *lim = getenv("GAM_MEM_LIMIT");
-    size_t left = lim ? (size_t)strtoull(lim, nullptr, 10) : (size_t)-1;
     hipError_t e = hipSuccess;
+    c->bytes = 0;
     for (auto &w : want) {
         const size_t bytes = (size_t)w.n * g.N3 * sizeof(double);
-        if (e == hipSuccess && bytes > left) e = hipErrorOutOfMemory;
-        left -= bytes;
-        if (e == hipSuccess) e = hipMalloc((void **)w.p, bytes);
+        if (e == hipSuccess) e = limited_malloc(w.p, bytes, c->bytes);
         if (e == hipSuccess) e = hipMemset(*w.p, 0, bytes);
+        c->bytes += bytes;
     }
     c->part = c->stage;
-    if (e != hipSuccess) {
-        free_planes(c);
-        hipGetLastError();   // the failure is reported by value
-    }
+    if (e != hipSuccess) free_planes(c);
     return e;
 }
 
@@ -1653,12 +1659,18 @@ extern "C" int gam_autotune(gam_ctx *c, int reps)
     graphs_drop(c);   // launch arguments change
     if (reps < 1 || reps > GAM_TUNE_MAXREPS) return fail(GAM_E_ARG, "gam_autotune: reps must be in 1..%d", GAM_TUNE_MAXREPS);
     if ((rc = hf_flush(c))) return rc;
-    // snapshot State, oState (with their primitives) and the clock; tuning
-    // takes real steps
-    const size_t bytes = (size_t)c->snpl * c->g.N3 * sizeof(double);
+    // snapshot State, oState (with their primitives, where there is room: else
+    // the next two steps run the predictor) and the clock; tuning takes real
+    // steps
+    int npl = c->snpl;
     double *save = nullptr;
     HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMalloc((void **)&save, 2 * bytes));
+    const size_t pl = (size_t)c->g.N3 * sizeof(double);
+    if (limited_malloc(&save, 2 * npl * pl, c->bytes) != hipSuccess) {
+        npl = ST_NPL;
+        HIPCHK(limited_malloc(&save, 2 * npl * pl, c->bytes));
+    }
+    const size_t bytes = npl * pl;
     Clock ck;
     const int cur0 = c->cur, std0[2] = {c->std[0], c->std[1]};
     const int prof = c->prof;
@@ -1723,8 +1735,8 @@ extern "C" int gam_autotune(gam_ctx *c, int reps)
     if (e == hipSuccess) e = hipMemcpyAsync(c->clk, &ck, sizeof(Clock), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     c->cur = cur0;
-    c->std[0] = std0[0];
-    c->std[1] = std0[1];
+    c->std[0] = npl == c->snpl && std0[0];
+    c->std[1] = npl == c->snpl && std0[1];
     // the half state of the next step, which every tuning began with
     c->hf = 0;
     launch_predict(c->stream, c->plan.v[TS_PREDICT], c->g, c->mp, face_box(c->g), c->clk, S_cur(c), S_old(c), c->met,

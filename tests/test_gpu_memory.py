@@ -81,6 +81,7 @@ def test_results_without_room(kind, rmeth, monkeypatch):
     assert max(rel_linf(h[k], ho[k]) for k in ("Gas", "magFlux", "Bxyz")) <= 1e-12
     d = g.divb()
     assert np.isfinite(d)
+    monkeypatch.delenv("GAM_MEM_LIMIT")     # (it bounds a tuning run's snapshot too)
     g.autotune(reps=1)
     g.close()
     # the adjoint, against the context with every plane
@@ -100,3 +101,39 @@ def test_results_without_room(kind, rmeth, monkeypatch):
     assert abs(grads[0][0] - grads[1][0]) <= 1e-12 * abs(grads[0][0])
     for x, y in zip(grads[0][1:], grads[1][1:]):
         assert rel_linf(x, y) <= 1e-12
+
+
+def test_autotune_without_room_for_the_primitives(monkeypatch):
+    """The snapshot of a tuning run takes the two states' 28 planes, with
+    their primitives 38 where there is room: the run goes on within 1e-12
+    (two steps through the predictor) or bit for bit."""
+    N = (24, 11, 13)
+    pts = ((24 + 9 + 15) // 16 * 16) * (N[1] + 9) * (N[2] + 9) + 16
+    plane = 8 * ((pts + 63) // 64 * 64)
+    ref = _case("shell", "7UP")[0]
+    ref.init_run()
+    ref.run(8)
+    for planes, ok in ((218 + 38, True), (218 + 28, True), (218 + 27, False)):
+        monkeypatch.delenv("GAM_MEM_LIMIT", raising=False)
+        g = _case("shell", "7UP")[0]
+        g.init_run()
+        g.run(4)
+        plan, s0, t0 = g.get_plan(), g.get_state(), g.get_time()
+        monkeypatch.setenv("GAM_MEM_LIMIT", str(planes * plane))
+        if ok:
+            g.autotune(reps=1)
+            g.set_plan(plan)
+        else:
+            with pytest.raises(gamhip.GamError) as ei:
+                g.autotune(reps=1)
+            assert ei.value.code == -2
+        assert g.get_time() == t0
+        s1 = g.get_state()
+        for k in ("Gas", "magFlux", "Bxyz", "Efld"):
+            assert np.array_equal(s0[k], s1[k])
+        g.run(4)
+        a, b = g.get_state(), ref.get_state()
+        for k in ("Gas", "magFlux", "Bxyz", "Efld"):
+            assert rel_linf(a[k], b[k]) <= (1e-12 if planes == 218 + 28 else 0.0), (planes, k)
+        g.close()
+    ref.close()
