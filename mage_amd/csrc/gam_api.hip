@@ -413,7 +413,7 @@ static int put_zero(gam_ctx *c, double *dst, size_t n, int ncomp)
 // copy to pinned memory behind it and one wait.
 static int read_clock(gam_ctx *c, Clock *ck)
 {
-    HIPCHK(hipMemcpyAsync(c->hclk, c->clk, sizeof(Clock), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(c->hclk, c->clk, CLOCK_TIME, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     *ck = *c->hclk;
     return GAM_OK;
@@ -1088,7 +1088,7 @@ extern "C" int gam_run(gam_ctx *c, int nsteps)
 
 // gamAdvanceModel (gamtypessub.F90:74-90): one stepGamera, then more while
 // Model%t < t0 + dt.  The loop condition needs Model%t, so every step ends
-// with a 64-byte clock read; a CalcDT failure ends the loop with its code,
+// with an 80-byte clock read; a CalcDT failure ends the loop with its code,
 // where the reference prints and stops (step.F90:136-151).
 extern "C" int gam_advance_model(gam_ctx *c, double dt, int *nsteps)
 {

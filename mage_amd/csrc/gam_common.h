@@ -71,7 +71,9 @@ struct Clock {
     // records hold MParm by value.  Last, as no part of a recorded time: what
     // puts a recorded clock back copies the CLOCK_TIME bytes before it.
     double dt0;
+    double pad0;    // whole 16-byte words, also in arrays of clocks: copies of others are slower
 };
+static_assert(offsetof(Clock, dt0) % 16 == 0 && sizeof(Clock) % 16 == 0, "clock copies");
 enum { CLOCK_TIME = offsetof(Clock, dt0) };
 
 // Plane indices: State buffer.  S_W holds the primitives of the gas (CellC2P)
